@@ -382,10 +382,42 @@ template <> struct V4<double> {
     typedef double4 t;
     static __device__ double4 make(double a, double b, double c, double d) { return make_double4(a, b, c, d); }
 };
-// v_rsq_f32 directly (1 ulp): pair distances squared are far above the denormal range, so the
+// 1 / r^3 (POT: 1 / r) from r^2 = x in FP64, 0 for x = 0.  v_rsq_f64 gives y with a relative error
+// of about 2^-24; with y2 = fl(y y) and e = 1 - x y2 one step of third order,
+//   1 / r = y (1 + e (1/2 + 3/8 e)),  1 / r^3 = y^3 (1 + e (3/2 + 15/8 e)),
+// leaves the next term (about 2^-70) far below the roundings: at most 1.25 ulp for the cube (the
+// rounding of y2 enters e as well and half cancels), against 1.5 ulp of 1 / (x sqrt(x)), in 6
+// instructions and the v_rsq instead of about 25.  Arguments whose powers leave the normal range
+// (x < 2^-670, x = 0, infinities, NaN) take the IEEE operations.
+// inv_power_regular gives the value where inv_power_rank is below INV_POWER_ODD.
+constexpr unsigned INV_POWER_ODD = (unsigned)(2 * 670) << 20;
+__device__ __forceinline__ unsigned inv_power_rank(double x) {   // negative x and NaN rank high
+    return (unsigned)__double2hiint(x) - ((unsigned)(1023 - 670) << 20);
+}
+template <bool POT>
+__device__ __forceinline__ double inv_power_regular(double x) {
+    double c = POT ? 0.5 : 1.5;
+    asm("" : "+v"(c));   // in a register: as a literal it is moved anew before every accumulating FMA
+    const double y = __builtin_amdgcn_rsq(x), y2 = y * y, e = fma_t(-x, y2, 1.0), w = POT ? y : y2 * y;
+    return fma_t(w, e * fma_t(e, POT ? 0.375 : 1.875, c), w);
+}
+template <bool POT>
+__device__ __forceinline__ double inv_power_ieee(double x) {
+    return x == 0.0 ? 0.0 : POT ? 1.0 / sqrt(x) : 1.0 / (x * sqrt(x));
+}
+template <bool POT>
+__device__ __forceinline__ double inv_power(double x) {
+    double f = inv_power_regular<POT>(x);
+    if (__builtin_expect(inv_power_rank(x) >= INV_POWER_ODD, 0)) f = inv_power_ieee<POT>(x);
+    return f;
+}
+// FP32: v_rsq_f32 directly (1 ulp): pair distances squared are far above the denormal range, so the
 // denormal-scaling wrapper of rsqrtf is not needed
-__device__ __forceinline__ float rsqrt_t(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ double rsqrt_t(double x) { return 1.0 / sqrt(x); }
+template <bool POT>
+__device__ __forceinline__ float inv_power(float x) {
+    const float ri = x > 0.0f ? __builtin_amdgcn_rsqf(x) : 0.0f;
+    return POT ? ri : ri * ri * ri;
+}
 // P0[j] = (hi(y_j - o), q_x), P1[j] = (lo(y_j - o), q_y), P2[j] = q_z for every source slot j
 template <class R>
 __global__ void k_pack_sources(int n, const double* __restrict__ origin, const double* __restrict__ sxyz,
@@ -477,16 +509,15 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
                     }
                     // fused multiply-adds (explicit: this library is built without contraction)
                     const R r2 = fma_t(dx, dx, fma_t(dy, dy, dz * dz));
-                    const R ri = r2 > (R)0 ? rsqrt_t(r2) : (R)0;
+                    const R ip = inv_power<POT>(r2);
                     if (POT) {
-                        f0 = fma_t(qx, ri, f0);
-                        f1 = fma_t(qy, ri, f1);
-                        f2 = fma_t(qz, ri, f2);
+                        f0 = fma_t(qx, ip, f0);
+                        f1 = fma_t(qy, ip, f1);
+                        f2 = fma_t(qz, ip, f2);
                     } else {
-                        const R ri3 = ri * ri * ri;
-                        f0 = fma_t(fma_t(qy, dz, -qz * dy), ri3, f0);
-                        f1 = fma_t(fma_t(qz, dx, -qx * dz), ri3, f1);
-                        f2 = fma_t(fma_t(qx, dy, -qy * dx), ri3, f2);
+                        f0 = fma_t(fma_t(qy, dz, -qz * dy), ip, f0);
+                        f1 = fma_t(fma_t(qz, dx, -qx * dz), ip, f1);
+                        f2 = fma_t(fma_t(qx, dy, -qy * dx), ip, f2);
                     }
                 }
                 a0 += f0;
@@ -697,8 +728,7 @@ __global__ __launch_bounds__(64) void k_p2p_bem(const int* __restrict__ leaves, 
             for (int j = sbegin[s]; j < send[s]; j++) {
                 const double q0 = sxyz[3 * j] - x, q1 = sxyz[3 * j + 1] - y, q2 = sxyz[3 * j + 2] - z;
                 const double r2 = q0 * q0 + q1 * q1 + q2 * q2;
-                if (r2 == 0.0) continue;
-                const double r3 = 1.0 / (r2 * sqrt(r2)), d = sd[j];
+                const double r3 = inv_power<false>(r2), d = sd[j];
                 const double v0 = sv[3 * j], v1 = sv[3 * j + 1], v2 = sv[3 * j + 2];
                 a0 += (q0 * d + (q1 * v2 - q2 * v1)) * r3;
                 a1 += (q1 * d + (q2 * v0 - q0 * v2)) * r3;
@@ -750,49 +780,64 @@ __global__ void k_assemble(const int* __restrict__ slots, int n, const double* _
 // ---------------------------------------------------------------- direct sum (FP64)
 // B(x) = scale sum_j q_j x (x - y_j) / |x - y_j|^3 (POT: A(x) = scale sum_j q_j / |x - y_j|),
 // math::calcBioSavartLaplace (integration.cpp:101-120).  The sources are cut into nsplit
-// contiguous ranges: workgroup (b, s) sums range s for the 256 targets of block b (sources staged
-// in LDS) into partial[s][t][3]; k_direct_reduce adds the nsplit partials of each target in range
-// order (deterministic) and scales.  Splitting the sources keeps every CU busy when the targets
-// are few (16,384 targets are 64 workgroups).
+// contiguous ranges: the wave (b, s) sums range s for the 64 targets of block b into
+// partial[s][t][3]; k_direct_reduce adds the nsplit partials of each target in a fixed order
+// (deterministic) and scales.  Splitting the sources keeps every SIMD busy when the targets are few.
+//
+// Bound by FP64 VALU issue.  A source is the same for all lanes, so its six doubles come through
+// scalar loads straight into the arithmetic (no LDS staging, no barriers), four sources in flight;
+// with inv_power and explicit fused multiply-adds a pair costs about half the instructions of an
+// IEEE square root and division without contraction.  1,048,576 sources x 16,384 targets: 33.0 ->
+// 17.5 ms (9.8e11 pairs/s; the start of the Newton step from v_rsq_f32 instead, with the two
+// conversions, 20.8 ms).
 template <bool POT>
-__global__ __launch_bounds__(256) void k_direct_partial(const double* __restrict__ sxyz, const double* __restrict__ sq,
-                                                        int ns, const double* __restrict__ txyz, int nt,
-                                                        double* __restrict__ partial) {
-    __shared__ double3 sp[256];
-    __shared__ double3 sqq[256];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x, split = blockIdx.y, nsplit = gridDim.y;
+__global__ __launch_bounds__(64) void k_direct_partial(const double* __restrict__ sxyz, const double* __restrict__ sq,
+                                                       int ns, const double* __restrict__ txyz, int nt,
+                                                       double* __restrict__ partial) {
+    const int t = blockIdx.x * 64 + threadIdx.x, split = blockIdx.y, nsplit = gridDim.y;
     const long long per = ((long long)ns + nsplit - 1) / nsplit;
     const int j_begin = (int)min((long long)ns, per * split), j_end = (int)min((long long)ns, per * (split + 1));
     double x = 0, y = 0, z = 0;
     if (t < nt) { x = txyz[3 * t]; y = txyz[3 * t + 1]; z = txyz[3 * t + 2]; }
     double a0 = 0, a1 = 0, a2 = 0;
-    for (int j0 = j_begin; j0 < j_end; j0 += 256) {
-        int j = j0 + threadIdx.x;
-        __syncthreads();
-        if (j < j_end) {
-            sp[threadIdx.x] = make_double3(sxyz[3 * j], sxyz[3 * j + 1], sxyz[3 * j + 2]);
-            sqq[threadIdx.x] = make_double3(sq[3 * j], sq[3 * j + 1], sq[3 * j + 2]);
+    auto add = [&](double dx, double dy, double dz, double f, double qx, double qy, double qz) {
+        if (POT) {
+            a0 = fma_t(qx, f, a0);
+            a1 = fma_t(qy, f, a1);
+            a2 = fma_t(qz, f, a2);
+        } else {
+            a0 = fma_t(fma_t(qy, dz, -qz * dy), f, a0);
+            a1 = fma_t(fma_t(qz, dx, -qx * dz), f, a1);
+            a2 = fma_t(fma_t(qx, dy, -qy * dx), f, a2);
         }
-        __syncthreads();
-        int nj = min(256, j_end - j0);
-        for (int jj = 0; jj < nj; jj++) {
-            double dx = x - sp[jj].x, dy = y - sp[jj].y, dz = z - sp[jj].z;
-            double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 == 0.0) continue;
-            double r = sqrt(r2);
-            double3 q = sqq[jj];
-            if (POT) {
-                double ri = 1.0 / r;
-                a0 += q.x * ri;
-                a1 += q.y * ri;
-                a2 += q.z * ri;
-            } else {
-                double r3 = 1.0 / (r2 * r);
-                a0 += (q.y * dz - q.z * dy) * r3;
-                a1 += (q.z * dx - q.x * dz) * r3;
-                a2 += (q.x * dy - q.y * dx) * r3;
-            }
+    };
+    int j = j_begin;
+    for (; j + 4 <= j_end; j += 4) {
+        double v[12], q[12], r2[4], f[4];
+#pragma unroll
+        for (int e = 0; e < 12; e++) {
+            v[e] = sxyz[3 * (size_t)j + e];
+            q[e] = sq[3 * (size_t)j + e];
         }
+        unsigned rank = 0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const double dx = x - v[3 * u], dy = y - v[3 * u + 1], dz = z - v[3 * u + 2];
+            r2[u] = fma_t(dx, dx, fma_t(dy, dy, dz * dz));
+            f[u] = inv_power_regular<POT>(r2[u]);
+            rank = max(rank, inv_power_rank(r2[u]));
+        }
+        if (__builtin_expect(rank >= INV_POWER_ODD, 0))   // one test for the four keeps their chains interleaved
+            for (int u = 0; u < 4; u++) f[u] = inv_power<POT>(r2[u]);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            add(x - v[3 * u], y - v[3 * u + 1], z - v[3 * u + 2], f[u], q[3 * u], q[3 * u + 1], q[3 * u + 2]);
+    }
+    for (; j < j_end; j++) {
+        const double* v = sxyz + 3 * (size_t)j;
+        const double* q = sq + 3 * (size_t)j;
+        const double dx = x - v[0], dy = y - v[1], dz = z - v[2];
+        add(dx, dy, dz, inv_power<POT>(fma_t(dx, dx, fma_t(dy, dy, dz * dz))), q[0], q[1], q[2]);
     }
     if (t < nt) {
         double* o = partial + ((size_t)split * nt + t) * 3;
@@ -802,20 +847,26 @@ __global__ __launch_bounds__(256) void k_direct_partial(const double* __restrict
     }
 }
 
-__global__ void k_direct_reduce(const double* __restrict__ partial, int nt, int nsplit, double scale,
+// 2^lg lanes per output value (target * 3 + component): lane g adds the partials g, g + 2^lg, ...
+// in range order, then the lanes are summed pairwise.  With hundreds of ranges and few targets one
+// lane per value would be a chain of as many loads.
+__global__ void k_direct_reduce(const double* __restrict__ partial, int nt, int nsplit, int lg, double scale,
                                 double* __restrict__ B) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;   // target * 3 + component
-    if (i >= 3 * nt) return;
+    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long i = id >> lg, n = 3ll * nt;
+    const int g = (int)(id & ((1 << lg) - 1));
     double acc = 0;
-    for (int s = 0; s < nsplit; s++) acc += partial[(size_t)s * 3 * nt + i];
-    B[i] = acc * scale;
+    if (i < n)
+        for (int s = g; s < nsplit; s += 1 << lg) acc += partial[(size_t)s * n + i];
+    for (int o = 1; o < (1 << lg); o <<= 1) acc += __shfl_xor(acc, o);
+    if (i < n && g == 0) B[i] = acc * scale;
 }
 
 int direct_splits(int ns, int nt) {
-    // about 4 workgroups per CU in total, each range at least 4,096 sources
-    const int tb = std::max(1, blocks(nt));
-    int s = std::max(1, 4 * num_cus() / tb);
-    s = std::min(s, std::max(1, ns / 4096));
+    // 16 waves per CU in total (4 per SIMD hide the arithmetic latency), each range at least 1,024 sources
+    const int tb = std::max(1, blocks(nt, 64));
+    int s = std::max(1, 16 * num_cus() / tb);
+    s = std::min(s, std::max(1, ns / 1024));
     return s;
 }
 
@@ -823,10 +874,12 @@ void launch_direct(bool pot, const double* sxyz, const double* sq, int ns, const
                    double* out, double* partial, int nsplit, hipStream_t st) {
     if (!nt) return;
     if (nsplit < 1) throw Error(1, "direct sum: at least one source range");
-    dim3 grid(blocks(nt), nsplit);
-    if (pot) k_direct_partial<true><<<grid, 256, 0, st>>>(sxyz, sq, ns, txyz, nt, partial);
-    else k_direct_partial<false><<<grid, 256, 0, st>>>(sxyz, sq, ns, txyz, nt, partial);
-    k_direct_reduce<<<blocks(3 * (long long)nt), 256, 0, st>>>(partial, nt, nsplit, scale, out);
+    dim3 grid(blocks(nt, 64), nsplit);
+    if (pot) k_direct_partial<true><<<grid, 64, 0, st>>>(sxyz, sq, ns, txyz, nt, partial);
+    else k_direct_partial<false><<<grid, 64, 0, st>>>(sxyz, sq, ns, txyz, nt, partial);
+    int lg = 0;
+    while (lg < 6 && (2 << lg) <= nsplit) lg++;
+    k_direct_reduce<<<blocks((3ll * nt) << lg), 256, 0, st>>>(partial, nt, nsplit, lg, scale, out);
     FMM_HIP(hipGetLastError());
 }
 
