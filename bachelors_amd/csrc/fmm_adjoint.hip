@@ -8,7 +8,7 @@
 //   M2L^T : mu_s += T_M2L^T lambda_t over all far pairs;
 //   M2M^T : top-down, mu_child += T_M2M^T mu_parent;
 //   P2M^T : dL/dq_j = sum_lm mu(l,m) R_lm(u_j);
-//   P2P^T : dL/dq_j += sum_{close targets i} (x_i - y_j) x g_i / |x_i - y_j|^3;
+//   P2P^T : dL/dq_j += sum_{close targets i} g_i x (y_j - x_i) / |y_j - x_i|^3;
 // and dL/dw_j = J_j . dL/dq_j.  The backward pass consumes no forward expansion (B is
 // linear in w), so nothing per level is stored for it: the same expansion-sized
 // workspaces are reused, and only the trees, lists and operator tables of the forward
@@ -161,58 +161,21 @@ __global__ __launch_bounds__(64) void k_p2m_adj(const int* __restrict__ leaves, 
     }
 }
 
-// near field transposed: per target leaf, targets staged in LDS; lanes walk the sources
-// of each close node and add their gradient with one FP64 atomic per source and leaf
-template <class R>
-__global__ __launch_bounds__(64) void k_p2p_adj(const int* __restrict__ leaves, const double* __restrict__ tcenter,
-                                                const int* __restrict__ tbegin, const int* __restrict__ tend,
-                                                const int* __restrict__ close_begin, const int* __restrict__ close_end,
-                                                const int* __restrict__ close_s, const int* __restrict__ sbegin,
-                                                const int* __restrict__ send, const double* __restrict__ sxyz,
-                                                const double* __restrict__ txyz, const double* __restrict__ g,
-                                                double* __restrict__ gq) {
-    __shared__ R tx[64], ty[64], tz[64], g0[64], g1[64], g2[64];
-    const int leaf = leaves[blockIdx.x];
-    const int lane = threadIdx.x;
-    const double cx = tcenter[3 * leaf], cy = tcenter[3 * leaf + 1], cz = tcenter[3 * leaf + 2];
-    const int cb = close_begin[leaf], ce = close_end[leaf];
-    for (int k0 = tbegin[leaf]; k0 < tend[leaf]; k0 += 64) {
-        int nk = min(64, tend[leaf] - k0);
-        __syncthreads();
-        if (lane < nk) {
-            int k = k0 + lane;
-            tx[lane] = (R)(txyz[3 * k] - cx); ty[lane] = (R)(txyz[3 * k + 1] - cy); tz[lane] = (R)(txyz[3 * k + 2] - cz);
-            g0[lane] = (R)g[3 * k]; g1[lane] = (R)g[3 * k + 1]; g2[lane] = (R)g[3 * k + 2];
-        }
-        __syncthreads();
-        for (int ci = cb; ci < ce; ci++) {
-            int s = close_s[ci];
-            for (int j = sbegin[s] + lane; j < send[s]; j += 64) {
-                R yx = (R)(sxyz[3 * j] - cx), yy = (R)(sxyz[3 * j + 1] - cy), yz = (R)(sxyz[3 * j + 2] - cz);
-                R a0 = 0, a1 = 0, a2 = 0;
-                for (int i = 0; i < nk; i++) {
-                    R dx = tx[i] - yx, dy = ty[i] - yy, dz = tz[i] - yz;
-                    R r2 = dx * dx + dy * dy + dz * dz;
-                    R ri = r2 > (R)0 ? (R)1 / sqrt(r2) : (R)0;
-                    R ri3 = ri * ri * ri;
-                    // (d x g) / r^3
-                    a0 += (dy * g2[i] - dz * g1[i]) * ri3;
-                    a1 += (dz * g0[i] - dx * g2[i]) * ri3;
-                    a2 += (dx * g1[i] - dy * g0[i]) * ri3;
-                }
-                unsafeAtomicAdd(&gq[3 * j], (double)a0);
-                unsafeAtomicAdd(&gq[3 * j + 1], (double)a1);
-                unsafeAtomicAdd(&gq[3 * j + 2], (double)a2);
-            }
-        }
-    }
+// close_t[order[k]]: the targets of the close pairs in the order of their sources
+__global__ void k_gather_close(const int* __restrict__ order, const int* __restrict__ close_t, int n,
+                               int* __restrict__ out) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = close_t[order[i]];
 }
 
+// dL/dw = J . dL/dq, the far part gq plus the near part gn (may be null)
 __global__ void k_weights(const int* __restrict__ slots, int n, const double* __restrict__ sJ,
-                          const double* __restrict__ gq, double* __restrict__ dLdw) {
+                          const double* __restrict__ gq, const double* __restrict__ gn, double* __restrict__ dLdw) {
     int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    dLdw[slots[k]] = sJ[3 * k] * gq[3 * k] + sJ[3 * k + 1] * gq[3 * k + 1] + sJ[3 * k + 2] * gq[3 * k + 2];
+    double g[3];
+    for (int c = 0; c < 3; c++) g[c] = gq[3 * k + c] + (gn ? gn[3 * k + c] : 0.0);
+    dLdw[slots[k]] = sJ[3 * k] * g[0] + sJ[3 * k + 1] * g[1] + sJ[3 * k + 2] * g[2];
 }
 
 
@@ -286,23 +249,24 @@ void run_adjoint(AdjointState& S, const AdjointArgs& a, const double* dLdB, doub
                                                              Ts.end.as<int>(), Ts.level.as<int>(), a.sigS, a.sxyz,
                                                              (const float*)mu, a.p, a.Lp, gq);
     }
-    // P2P^T
-    if (a.near_field && a.n_tgt_leaves) {
-        const Lists& L = *a.lists;
-        if (f64)
-            k_p2p_adj<double><<<a.n_tgt_leaves, 64, 0, st>>>(a.tgt_leaves, Tt.center.as<double>(), Tt.begin.as<int>(),
-                                                            Tt.end.as<int>(), L.close_begin.as<int>(),
-                                                            L.close_end.as<int>(), L.close_s.as<int>(),
-                                                            Ts.begin.as<int>(), Ts.end.as<int>(), a.sxyz, a.txyz, g, gq);
-        else
-            k_p2p_adj<float><<<a.n_tgt_leaves, 64, 0, st>>>(a.tgt_leaves, Tt.center.as<double>(), Tt.begin.as<int>(),
-                                                           Tt.end.as<int>(), L.close_begin.as<int>(),
-                                                           L.close_end.as<int>(), L.close_s.as<int>(),
-                                                           Ts.begin.as<int>(), Ts.end.as<int>(), a.sxyz, a.txyz, g, gq);
+    // P2P^T: the targets, packed with the strengths g, summed at the sources of every source leaf
+    const Lists& L = *a.lists;
+    double* gn = nullptr;
+    if (a.near_field && a.n_src_leaves && L.num_close) {
+        const size_t rs = f64 ? sizeof(double) : sizeof(float), nt_ = (size_t)std::max(nts, 1);
+        gn = S.gn.get<double>(3 * (size_t)std::max(nss, 1));
+        void *P0 = S.P0.reserve(4 * rs * nt_), *P1 = S.P1.reserve(4 * rs * nt_), *P2 = S.P2.reserve(rs * nt_);
+        launch_pack_sources(f64, nts, Ts.center.as<double>(), a.txyz, g, P0, P1, P2, st);
+        build_pair_index(L.close_s.as<int>(), L.num_close, Ts.num_nodes, S.close_ix, st);
+        int* ct = S.close_t.get<int>(L.num_close);
+        k_gather_close<<<blocks(L.num_close), 256, 0, st>>>(S.close_ix.order.as<int>(), L.close_t.as<int>(),
+                                                            L.num_close, ct);
+        launch_p2p_transposed(f64, a.src_leaves, a.n_src_leaves, Ts, Tt, S.close_ix.begin.as<int>(),
+                              S.close_ix.end.as<int>(), ct, P0, P1, P2, a.sxyz, gn, st);
     }
     // dL/dw = J . dL/dq (input order; sources outside the root keep 0)
     FMM_HIP(hipMemsetAsync(dLdw, 0, (size_t)std::max(a.ns, 1) * sizeof(double), st));
-    k_weights<<<blocks(nss), 256, 0, st>>>(Ts.slots.as<int>(), nss, a.sJ, gq, dLdw);
+    k_weights<<<blocks(nss), 256, 0, st>>>(Ts.slots.as<int>(), nss, a.sJ, gq, gn, dLdw);
     FMM_HIP(hipGetLastError());
 }
 

@@ -42,6 +42,9 @@ struct AdjointState {
     DevBuf g, lam, mu, gq, Gexp;
     PairIndex m2l_ix;   // far pairs by source node
     DevBuf slab;        // transposed M2L result per (pair, component)
+    DevBuf gn;          // near field at the sources
+    PairIndex close_ix; // close pairs by source node
+    DevBuf close_t, P0, P1, P2;   // their targets in that order; the targets packed with g
 };
 
 // dLdw (input order) = transposed FMM applied to dLdB (input order); device pointers.

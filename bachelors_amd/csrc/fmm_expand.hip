@@ -441,7 +441,9 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
 // below 8; lane = target * G + g takes sources g, g + G, ...).  Lane partials are summed over
 // the G lanes, then over the 4 waves in a fixed order, and written once.
 // POT: the vector potential sum_j q_j / |x - y_j| instead of B.
-template <class R, bool POT, int UNROLL>
+// UP: the leaf takes the lists of its ancestors as well (parent[] up to the root): the transposed
+// near field, where a source leaf is reached through the close pairs of any node that holds it.
+template <class R, bool POT, int UNROLL, bool UP = false>
 __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegin, const int* __restrict__ tend,
                                          const int* __restrict__ close_begin, const int* __restrict__ close_end,
                                          const int* __restrict__ close_s, const double* __restrict__ origin,
@@ -450,13 +452,12 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
                                          const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
                                          const double* __restrict__ txyz, double* __restrict__ Bnear,
                                          typename V4<R>::t (*s0)[64], typename V4<R>::t (*s1)[64], R (*s2)[64],
-                                         double (*red)[3][64]) {
+                                         double (*red)[3][64], const int* __restrict__ parent = nullptr) {
     typedef typename V4<R>::t v4;
     constexpr bool split = sizeof(R) == 4;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tb = tbegin[leaf], te = tend[leaf];
-    const int cb = close_begin[leaf], ce = close_end[leaf];
-    if (cb >= ce) {
+    if (!UP && close_begin[leaf] >= close_end[leaf]) {
         for (int k = tb + tid; k < te; k += 256) Bnear[3 * k] = Bnear[3 * k + 1] = Bnear[3 * k + 2] = 0.0;
         return;
     }
@@ -482,7 +483,8 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
         // the close list's 64-source chunks, in list order, dealt round-robin to the waves (an
         // internal close node can hold most of a leaf's sources)
         int run = 0;   // chunks of the close nodes before ci
-        for (int ci = cb; ci < ce; ci++) {
+        for (int node = leaf; node >= 0; node = UP ? parent[node] : -1)
+        for (int ci = close_begin[node], ce = close_end[node]; ci < ce; ci++) {
             const int s = close_s[ci];
             const int sb = sbegin[s], se = send[s];
             const int nch = (se - sb + 63) >> 6;
@@ -566,6 +568,28 @@ __global__ __launch_bounds__(256) void k_p2p(const int* __restrict__ leaves, con
     __shared__ R s2[4][64];
     __shared__ double red[4][3][64];
     p2p_leaf<R, POT, 4>(leaves[blockIdx.x], tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send, P0, P1, P2, txyz, Bnear, s0, s1, s2, red);
+}
+
+// The transposed near field (adjoint): per useful source leaf, sum_i g_i x (y_j - x_i) / |y_j - x_i|^3
+// over the targets x_i (strengths g_i, packed as P0, P1, P2) of every target leaf that is close to the
+// leaf or to one of its ancestors.  The roles of the forward near field are swapped, so the pairs run
+// in the same body: no atomics, and a sum whose order is fixed.  Bound by VALU issue like the forward
+// one; one wave per target leaf adding to the sources by FP64 atomics, its differences in plain FP32,
+// took 14.2 ms where this takes about 2 (262,147 x 131,101 clustered points, 3.6e8 pairs) and had put
+// 1.5e-6 into the FP32 gradient, now 1.4e-7.
+template <class R>
+__global__ __launch_bounds__(256) void k_p2p_transposed(
+    const int* __restrict__ leaves, const int* __restrict__ sbegin, const int* __restrict__ send,
+    const int* __restrict__ parent, const int* __restrict__ close_begin, const int* __restrict__ close_end,
+    const int* __restrict__ close_t, const double* __restrict__ origin, const int* __restrict__ tbegin,
+    const int* __restrict__ tend, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
+    const R* __restrict__ P2, const double* __restrict__ sxyz, double* __restrict__ out) {
+    __shared__ typename V4<R>::t s0[4][64];
+    __shared__ typename V4<R>::t s1[4][64];
+    __shared__ R s2[4][64];
+    __shared__ double red[4][3][64];
+    p2p_leaf<R, false, 4, true>(leaves[blockIdx.x], sbegin, send, close_begin, close_end, close_t, origin, tbegin, tend,
+                                P0, P1, P2, sxyz, out, s0, s1, s2, red, parent);
 }
 
 // The same near field as a small persistent grid taking leaves from a queue (an atomic counter
@@ -1017,6 +1041,22 @@ void launch_p2p_queue(bool f64, const int* leaves, int nleaves, const TreeDev& T
                                                         close_begin, close_end, close_s, S.center.as<double>(),
                                                         S.begin.as<int>(), S.end.as<int>(), (const float4*)P0,
                                                         (const float4*)P1, (const float*)P2, txyz, Bnear);
+    FMM_HIP(hipGetLastError());
+}
+void launch_p2p_transposed(bool f64, const int* leaves, int nleaves, const TreeDev& S, const TreeDev& T,
+                           const int* close_begin, const int* close_end, const int* close_t, const void* P0,
+                           const void* P1, const void* P2, const double* sxyz, double* out, hipStream_t st) {
+    if (!nleaves) return;
+    if (f64)
+        k_p2p_transposed<double><<<nleaves, 256, 0, st>>>(
+            leaves, S.begin.as<int>(), S.end.as<int>(), S.parent.as<int>(), close_begin, close_end, close_t,
+            S.center.as<double>(), T.begin.as<int>(), T.end.as<int>(), (const double4*)P0, (const double4*)P1,
+            (const double*)P2, sxyz, out);
+    else
+        k_p2p_transposed<float><<<nleaves, 256, 0, st>>>(
+            leaves, S.begin.as<int>(), S.end.as<int>(), S.parent.as<int>(), close_begin, close_end, close_t,
+            S.center.as<double>(), T.begin.as<int>(), T.end.as<int>(), (const float4*)P0, (const float4*)P1,
+            (const float*)P2, sxyz, out);
     FMM_HIP(hipGetLastError());
 }
 void launch_p2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,

@@ -33,6 +33,12 @@ void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, cons
 void launch_p2p_queue(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S,
                       const int* close_begin, const int* close_end, const int* close_s, const void* P0, const void* P1,
                       const void* P2, const double* txyz, double* Bnear, int* queue, int grid, hipStream_t st);
+// the transposed near field at the sources (slot order, written whole for the leaves given): the
+// targets are packed by launch_pack_sources with their strengths, relative to the same origin (the
+// source root's centre); close_begin / close_end / close_t: the close targets of every source node
+void launch_p2p_transposed(bool f64, const int* leaves, int nleaves, const TreeDev& S, const TreeDev& T,
+                           const int* close_begin, const int* close_end, const int* close_t, const void* P0,
+                           const void* P1, const void* P2, const double* sxyz, double* out, hipStream_t st);
 void launch_assemble(const int* slots, int n, const double* Bfar, const double* Bnear, double scale, double* B,
                      hipStream_t st);
 // L2P / P2P of the vector potential A (the calcA counterparts of launch_l2p / launch_p2p)

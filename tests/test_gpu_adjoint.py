@@ -92,3 +92,32 @@ def test_adjoint_gradient_vs_finite_differences_and_direct():
     Bs = O.direct_B(src, wstar, tgt)
     gd = O.direct_grad_w(src, w, tgt, Bs)
     assert rel_l2(grad, gd) < 1e-4
+
+
+@pytest.mark.parametrize("ns,nt,cap_s,cap_t", [(2, 1, 2, 1), (700, 300, 4, 200), (700, 300, 300, 3), (65, 64, 64, 64),
+                                               (5000, 129, 8, 128)])
+def test_transposed_near_field_is_the_transpose(ns, nt, cap_s, cap_t):
+    """The near field summed at the source leaves through their ancestors' close pairs: leaf
+    capacities far apart (close source nodes are then internal, or targets' leaves much larger), single
+    points, and one point per 64-lane block, by g.B(w) = w.B^T g with g = B(w) (1 + U[-1/2, 1/2])
+    (FP64 rounding, as above)."""
+    import ctypes
+
+    import torch
+    import bachelors_amd as fm
+    rng = np.random.default_rng(31 + ns + nt)
+    src = shell_sources(rng, ns)
+    w = rng.uniform(0.5, 1.5, ns)
+    tgt = rng.uniform(-1.2, 1.2, (nt, 3))
+    F = fm.FMM(order=6, source_leaf_capacity=cap_s, target_leaf_capacity=cap_t, precision="fp64", frame=1)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    B = F.run(1.0)
+    g = torch.from_numpy(B * (1 + rng.uniform(-0.5, 0.5, B.shape))).cuda()
+    gw = torch.empty(ns, dtype=torch.float64, device="cuda")
+    F.adjoint_weights_dev(1.0, ctypes.c_void_p(g.data_ptr()), ctypes.c_void_p(gw.data_ptr()))
+    F.synchronize()
+    lhs, rhs = float((B * g.cpu().numpy()).sum()), float((w * gw.cpu().numpy()).sum())
+    assert F.stats()["close_pairs"] > 0
+    F.close()
+    assert abs(lhs - rhs) <= 1e-11 * abs(lhs)
