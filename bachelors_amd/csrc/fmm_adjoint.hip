@@ -222,10 +222,10 @@ void run_adjoint(AdjointState& S, const AdjointArgs& a, const double* dLdB, doub
     if (a.m2l.ntiles) {
         const int npairs = a.lists->num_far;
         build_pair_index(a.m2l.dst, npairs, Ts.num_nodes, S.m2l_ix, st);
-        void* slab = S.slab.reserve((size_t)3 * npairs * a.Lp * es);
-        class_gemm(a.prec, a.down_ops, a.down_ops_lo, a.m2l.tiles, a.m2l.ntiles, a.m2l.src, a.m2l.dst, lam, slab,
-                   a.Lp, EPI_STORE, st, true);
-        reduce_pairs(f64, S.m2l_ix, slab, a.Lp, a.Lp, mu, st);
+        const int L = (a.p + 1) * (a.p + 1), R = m2l_slab_rows(a.prec, L, a.Lp);
+        void* slab = a.slab->reserve((size_t)3 * npairs * R * es);
+        m2l_gemm(a.prec, a.down_ops, a.down_ops_lo, a.m2l.tiles, a.m2l.ntiles, a.m2l.src, lam, slab, L, a.Lp, st, true);
+        reduce_pairs(f64, S.m2l_ix, slab, R, a.Lp, mu, st);
     }
     // M2M^T top-down (forward child -> parent; here parent -> child, one write per child)
     for (int k = 1; k < Ts.num_levels; k++) {

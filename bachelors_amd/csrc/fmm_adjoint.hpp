@@ -34,6 +34,7 @@ struct AdjointArgs {
     int n_up_ops, n_down_ops;
     std::vector<PassView> m2m_levels, l2l_levels;   // indexed by child level
     PassView m2l;                                   // src = far_t, dst = far_s (already transposed roles)
+    DevBuf* slab;       // workspace: the M2L's result per (pair, component), free after the forward pass
     double scale;
     int nt, ns;
 };
@@ -41,7 +42,6 @@ struct AdjointArgs {
 struct AdjointState {
     DevBuf g, lam, mu, gq, Gexp;
     PairIndex m2l_ix;   // far pairs by source node
-    DevBuf slab;        // transposed M2L result per (pair, component)
     DevBuf gn;          // near field at the sources
     PairIndex close_ix; // close pairs by source node
     DevBuf close_t, P0, P1, P2;   // their targets in that order; the targets packed with g

@@ -1408,6 +1408,7 @@ int fmm_adjoint_weights_dev(fmm_ctx* c, double current, const double* dLdB, doub
                          c->lists.far_s.as<int>(), 64};
         a.n_up_ops = c->up_ops.nops;
         a.n_down_ops = c->down_ops.nops;
+        a.slab = &c->m2l_slab;
         a.scale = current * REF_MU0 / (4.0 * REF_PI);
         a.nt = c->nt;
         a.ns = c->ns;

@@ -13,7 +13,7 @@
 // next step's global loads issued before the current step's MFMAs (one barrier per step).
 //
 // Precisions:
-//   F64    : v_mfma_f64_16x16x4f64 (C register r holds row 4r + lane/16);
+//   F64    : v_mfma_f64_16x16x4f64 (rows permuted so that C register r holds row 4(lane/16) + r);
 //   F32    : v_mfma_f32_16x16x4f32 (C register r holds row 4(lane/16) + r), FP32 accumulate;
 //   BF16X3 : v_mfma_f32_16x16x32_bf16 on A = Ah + Al (tables split offline from FP64) and
 //            B = Bh + Bl (split on load): C += Al Bh + Ah Bl + Ah Bh, FP32 accumulate.
@@ -25,18 +25,18 @@ namespace fmm {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BN = 64;
 
-// hardware float atomics (global_atomic_add_f32/f64) on coarse-grained device memory
-__device__ __forceinline__ void add_out(float* p, float v, int epi) {
-    if (epi == EPI_ATOMIC) unsafeAtomicAdd(p, v);
-    else *p += v;
-}
-__device__ __forceinline__ void add_out(double* p, double v, int epi) {
-    if (epi == EPI_ATOMIC) unsafeAtomicAdd(p, v);
-    else *p += v;
+// The operator row that lane li supplies as row li of a 16-row MFMA block.  The FP64 MFMA returns
+// rows r, 4 + r, ... in register r of lane group g (row 4r + g), the FP32 one rows 4g + r; with the
+// rows of an FP64 block read in the order 4 (li mod 4) + li / 4, register r of group g holds row
+// 4g + r too, so a lane writes 32 consecutive bytes and its column's four lanes a 128-byte line
+// instead of four 32-byte pieces.
+template <class T> __device__ __forceinline__ int mfma_row(int li) {
+    return sizeof(T) == 8 ? 4 * (li & 3) + (li >> 2) : li;
 }
 
 template <class T> struct Vec4;
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void k_gemm(const T* __restrict__ ops, const G
 #pragma unroll
             for (int a = 0; a < RB; a++) {
                 if (!live[a]) continue;   // uniform over the wave
-                af[a] = As[cur][kk][16 * (wave + 4 * a) + (lane & 15)];
+                af[a] = As[cur][kk][16 * (wave + 4 * a) + mfma_row<T>(lane & 15)];
 #pragma unroll
                 for (int b = 0; b < 4; b++) {
                     if constexpr (sizeof(T) == 8)
@@ -167,42 +167,20 @@ __global__ __launch_bounds__(256) void k_gemm(const T* __restrict__ ops, const G
         if (epi == EPI_STORE) {
             T* out = dst_exp + (size_t)col * Lp;
 #pragma unroll
-            for (int a = 0; a < RB; a++) {
-                const int r0 = 16 * (wave + 4 * a);
-                if constexpr (sizeof(T) == 8) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) out[r0 + 4 * r + (lane >> 4)] = acc[a][b][r];
-                } else {
-                    *(float4*)(out + r0 + 4 * (lane >> 4)) =
-                        make_float4(acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]);
-                }
-            }
+            for (int a = 0; a < RB; a++) *(acc_t*)(out + 16 * (wave + 4 * a) + 4 * (lane >> 4)) = acc[a][b];
             continue;
         }
         int pair = col / 3, comp = col - 3 * pair;
         T* dst = dst_exp + ((size_t)pair_dst[pair] * 3 + comp) * Lp;
-        if constexpr (sizeof(T) == 4) {
-            if (epi == EPI_ADD) {   // a lane's four rows are consecutive: one 16-byte read-modify-write
+        if (epi == EPI_ADD) {   // a lane's four rows are consecutive: one vector read-modify-write
 #pragma unroll
-                for (int a = 0; a < RB; a++) {
-                    float4* q = (float4*)(dst + 16 * (wave + 4 * a) + 4 * (lane >> 4));
-                    float4 v = *q;
-                    v.x += acc[a][b][0];
-                    v.y += acc[a][b][1];
-                    v.z += acc[a][b][2];
-                    v.w += acc[a][b][3];
-                    *q = v;
-                }
-                continue;
-            }
+            for (int a = 0; a < RB; a++) *(acc_t*)(dst + 16 * (wave + 4 * a) + 4 * (lane >> 4)) += acc[a][b];
+            continue;
         }
 #pragma unroll
         for (int a = 0; a < RB; a++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                int rr = (sizeof(T) == 8) ? (4 * r + (lane >> 4)) : (4 * (lane >> 4) + r);
-                add_out(dst + 16 * (wave + 4 * a) + rr, (T)acc[a][b][r], epi);
-            }
+#pragma unroll   // hardware float atomics on coarse-grained device memory
+            for (int r = 0; r < 4; r++) unsafeAtomicAdd(dst + 16 * (wave + 4 * a) + 4 * (lane >> 4) + r, (T)acc[a][b][r]);
     }
 }
 
@@ -348,7 +326,7 @@ __global__ __launch_bounds__(256) void k_gemm_bf16x3(const __bf16* __restrict__ 
 #pragma unroll
         for (int a = 0; a < RB; a++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) add_out(dst + a * 16 + 4 * (lane >> 4) + r, acc[a][b][r], epi);
+            for (int r = 0; r < 4; r++) unsafeAtomicAdd(dst + a * 16 + 4 * (lane >> 4) + r, acc[a][b][r]);
     }
 }
 
@@ -357,13 +335,13 @@ __global__ __launch_bounds__(256) void k_gemm_bf16x3(const __bf16* __restrict__ 
 // owns the 16 columns [16w, 16w + 16) of the 64-column tile and all NB row blocks, so an odd
 // block count leaves no wave idle.  Each column is written to the per-pair slab with row
 // stride R (rows >= L are zero: the operators are zero there).
-constexpr int lds_stride(int rows, int words_per_elem) {
-    // rows + pad with the stride = 16 (mod 64) 4-byte words: the four K-rows read at once by the
-    // 16-lane groups of a wave fall on disjoint LDS banks
-    return words_per_elem == 1 ? rows + ((16 - rows % 64) + 64) % 64 : rows + ((8 - rows % 32) + 32) % 32;
-}
-
-template <class T, int NB>
+// TRANS applies T^T (the adjoint): a thread then loads one k and four consecutive rows of a
+// quad, k fastest over the lanes, so that the scattered LDS stores of a wave fall on 64 banks.
+// Matrix cores are busy 66-68 % of the time (counters).  Measured: 2.02 million FP64 pairs at p = 12
+// 8.2 -> 7.4 ms (128-byte stores 0.55, fragments read block by block 0.25); the transposed product of
+// 1.6 million FP32 pairs at p = 14 5.5 ms (7.0 with the whole-panel kernel).  Three workgroups per CU
+// instead of two (K steps of 8) or columns loaded 2 to 4 K steps ahead: 7.2 - 8.5 and 5.6 - 6.2 ms.
+template <class T, int NB, bool TRANS>
 __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, const GemmTile* __restrict__ tiles,
                                                   const int* __restrict__ pair_src, const T* __restrict__ src_exp,
                                                   T* __restrict__ slab, int Lp) {
@@ -396,7 +374,9 @@ __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, con
 #pragma unroll
         for (int j = 0; j < NQ; j++) {
             int qi = tid + 256 * j;
-            if (qi < NB * 64) ra[j] = V::load(A + (size_t)(qi >> 2) * Lp + k0 + (qi & 3) * 4);
+            if (qi < NB * 64)
+                ra[j] = V::load(TRANS ? A + (size_t)(k0 + (qi & 15)) * Lp + (qi >> 4) * 4
+                                      : A + (size_t)(qi >> 2) * Lp + k0 + (qi & 3) * 4);
         }
         if (bptr) rb = V::load(bptr + k0 + bq);
     };
@@ -404,7 +384,12 @@ __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, con
 #pragma unroll
         for (int j = 0; j < NQ; j++) {
             int qi = tid + 256 * j;
-            if (qi < NB * 64) *(v4*)&As[buf][qi >> 2][(qi & 3) * 4] = ra[j];
+            if (qi >= NB * 64) continue;
+            if (TRANS)
+#pragma unroll
+                for (int i = 0; i < 4; i++) As[buf][(qi >> 4) * 4 + i][qi & 15] = V::get(ra[j], i);
+            else
+                *(v4*)&As[buf][qi >> 2][(qi & 3) * 4] = ra[j];
         }
         if (bptr) *(v4*)&Bs[buf][bc][bq] = rb;
         else *(v4*)&Bs[buf][bc][bq] = V::zero();
@@ -419,19 +404,24 @@ __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, con
         const int cur = kt & 1;
         if (kt + 1 < NK) gload((kt + 1) * BK);
         const v4 bf = *(const v4*)&Bs[cur][wave * 16 + li][4 * g];
-        v4 af[NB];
+        // two row blocks at a time: their fragments are read while the previous blocks' MFMAs run, and
+        // consecutive MFMAs update different accumulators
 #pragma unroll
-        for (int a = 0; a < NB; a++) af[a] = *(const v4*)&As[cur][a * 16 + li][4 * g];
-        // consecutive MFMAs update different accumulators (no back-to-back dependence)
+        for (int a0 = 0; a0 < NB; a0 += 2) {
+            v4 af[2];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+            for (int a = a0; a < a0 + 2 && a < NB; a++)
+                af[a - a0] = *(const v4*)&As[cur][a * 16 + mfma_row<T>(li)][4 * g];
 #pragma unroll
-            for (int a = 0; a < NB; a++) {
-                if constexpr (sizeof(T) == 8)
-                    acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(V::get(af[a], j), V::get(bf, j), acc[a], 0, 0, 0);
-                else
-                    acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(V::get(af[a], j), V::get(bf, j), acc[a], 0, 0, 0);
-            }
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int a = a0; a < a0 + 2 && a < NB; a++) {
+                    if constexpr (sizeof(T) == 8)
+                        acc[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(V::get(af[a - a0], j), V::get(bf, j), acc[a], 0, 0, 0);
+                    else
+                        acc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(V::get(af[a - a0], j), V::get(bf, j), acc[a], 0, 0, 0);
+                }
+        }
         if (kt + 1 < NK) lstore(cur ^ 1);
         __syncthreads();
     }
@@ -444,8 +434,8 @@ __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, con
 #pragma unroll
     for (int a = 0; a < NB; a++) {
         if constexpr (sizeof(T) == 8) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) __builtin_nontemporal_store(acc[a][r], out + a * 16 + 4 * r + g);
+            __builtin_nontemporal_store(f64x2{acc[a][0], acc[a][1]}, (f64x2*)(out + a * 16 + 4 * g));
+            __builtin_nontemporal_store(f64x2{acc[a][2], acc[a][3]}, (f64x2*)(out + a * 16 + 4 * g + 2));
         } else {
             __builtin_nontemporal_store(acc[a], (f32x4*)(out + a * 16 + 4 * g));
         }
@@ -877,14 +867,14 @@ void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float*
     throw Error(4, "FP16 M2L: no kernel instance for this order");
 }
 
-template <int NB>
+template <int NB, bool TRANS>
 static void launch_m2l_nb(Precision prec, const void* ops, const GemmTile* d_tiles, int ntiles, const int* pair_src,
                           const void* src_exp, void* slab, int Lp, hipStream_t st) {
     if (prec == Precision::F64)
-        k_gemm_m2l<double, NB><<<ntiles, 256, 0, st>>>((const double*)ops, d_tiles, pair_src, (const double*)src_exp,
+        k_gemm_m2l<double, NB, TRANS><<<ntiles, 256, 0, st>>>((const double*)ops, d_tiles, pair_src, (const double*)src_exp,
                                                        (double*)slab, Lp);
     else
-        k_gemm_m2l<float, NB><<<ntiles, 256, 0, st>>>((const float*)ops, d_tiles, pair_src, (const float*)src_exp,
+        k_gemm_m2l<float, NB, TRANS><<<ntiles, 256, 0, st>>>((const float*)ops, d_tiles, pair_src, (const float*)src_exp,
                                                       (float*)slab, Lp);
     FMM_HIP(hipGetLastError());
 }
@@ -902,22 +892,29 @@ int m2l_slab_rows(Precision prec, int L, int Lp) {
     }
 }
 
-void m2l_gemm(Precision prec, const void* ops, const void* ops_lo, const GemmTile* d_tiles, int ntiles,
-              const int* pair_src, const void* src_exp, void* slab, int L, int Lp, hipStream_t st) {
+template <bool TRANS>
+static void m2l_gemm_go(Precision prec, const void* ops, const void* ops_lo, const GemmTile* d_tiles, int ntiles,
+                        const int* pair_src, const void* src_exp, void* slab, int L, int Lp, hipStream_t st) {
     if (ntiles == 0) return;
     const int R = m2l_slab_rows(prec, L, Lp);
-    if (R == Lp) {   // the whole-panel kernel (BF16x3, or an L without a padded-to-16 instance)
-        class_gemm(prec, ops, ops_lo, d_tiles, ntiles, pair_src, nullptr, src_exp, slab, Lp, EPI_STORE, st);
+    if (R == Lp) {   // the whole-panel kernel (BF16x3, or an L that fills whole panels)
+        class_gemm(prec, ops, ops_lo, d_tiles, ntiles, pair_src, nullptr, src_exp, slab, Lp, EPI_STORE, st, TRANS);
         return;
     }
 #define FMM_NB(N) \
-    case N: launch_m2l_nb<N>(prec, ops, d_tiles, ntiles, pair_src, src_exp, slab, Lp, st); break;
+    case N: launch_m2l_nb<N, TRANS>(prec, ops, d_tiles, ntiles, pair_src, src_exp, slab, Lp, st); break;
     switch (R / 16) {
         FMM_NB(1) FMM_NB(2) FMM_NB(3) FMM_NB(4) FMM_NB(6) FMM_NB(7) FMM_NB(8) FMM_NB(9) FMM_NB(11) FMM_NB(13)
         FMM_NB(15) FMM_NB(16) FMM_NB(19) FMM_NB(21) FMM_NB(23) FMM_NB(25) FMM_NB(28)
         default: throw Error(4, "no padded-row M2L kernel for this order");
     }
 #undef FMM_NB
+}
+
+void m2l_gemm(Precision prec, const void* ops, const void* ops_lo, const GemmTile* d_tiles, int ntiles,
+              const int* pair_src, const void* src_exp, void* slab, int L, int Lp, hipStream_t st, bool transpose) {
+    if (transpose) m2l_gemm_go<true>(prec, ops, ops_lo, d_tiles, ntiles, pair_src, src_exp, slab, L, Lp, st);
+    else m2l_gemm_go<false>(prec, ops, ops_lo, d_tiles, ntiles, pair_src, src_exp, slab, L, Lp, st);
 }
 
 template <int RB, bool TR, bool MU>
@@ -1057,7 +1054,6 @@ __device__ __forceinline__ float4 load_stream(const float4* p) {
     return make_float4(v[0], v[1], v[2], v[3]);
 }
 __device__ __forceinline__ double2 load_stream(const double2* p) {
-    typedef double f64x2 __attribute__((ext_vector_type(2)));
     f64x2 v = __builtin_nontemporal_load((const f64x2*)p);
     return make_double2(v[0], v[1]);
 }

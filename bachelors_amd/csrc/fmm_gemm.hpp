@@ -55,7 +55,8 @@ void reduce_pairs(bool f64, PairIndex& ix, const void* slab, int R, int Lp, void
 int m2l_slab_rows(Precision prec, int L, int Lp);
 // M2L of all classes into the slab [3 * pairs][m2l_slab_rows] (column 3 pair + component).
 void m2l_gemm(Precision prec, const void* ops, const void* ops_lo, const GemmTile* d_tiles, int ntiles,
-              const int* pair_src, const void* src_exp, void* slab, int L, int Lp, hipStream_t st);
+              const int* pair_src, const void* src_exp, void* slab, int L, int Lp, hipStream_t st,
+              bool transpose = false);
 
 // F16X3 M2L (FP16 split products on MFMA, equilibrated by powers of 2): operator rows
 // m2l_f16_rows(L), K padded to Kp = m2l_f16_kpad(L); the multipoles enter split by split_columns

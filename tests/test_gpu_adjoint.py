@@ -121,3 +121,22 @@ def test_transposed_near_field_is_the_transpose(ns, nt, cap_s, cap_t):
     assert F.stats()["close_pairs"] > 0
     F.close()
     assert abs(lhs - rhs) <= 1e-11 * abs(lhs)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
+@pytest.mark.parametrize("order", [1, 2, 4, 5, 6, 8, 9, 11, 13, 15, 17, 18, 20])
+def test_transposed_m2l_at_every_row_padding(order, precision, tol):
+    """The transposed M2L with rows padded to multiples of 16 (one kernel instance per block count) at
+    orders of each count, with classes of a few to a few hundred columns, by the same identity."""
+    import torch
+    from bachelors_amd.torch_fmm import FMMBiotSavart
+    rng, src, w, tgt = _case(40 + order, ns=1500, nt=900)
+    F = FMMBiotSavart(src, tgt, order=order, cap=24, precision=precision)
+    wt = torch.tensor(w, dtype=torch.float64, device="cuda", requires_grad=True)
+    B = F(wt)
+    g = B.detach() * (1 + torch.tensor(rng.uniform(-0.5, 0.5, (len(tgt), 3)), device="cuda"))
+    (B * g).sum().backward()
+    lhs = float((B.detach() * g).sum())
+    rhs = float((wt.detach() * wt.grad).sum())
+    assert F._fmm.stats()["far_pairs"] > 0
+    assert abs(lhs - rhs) <= tol * abs(lhs)
