@@ -12,7 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libbachelors_fmm.so")
-SOURCES = ["fmm_prims.hip", "fmm_tree.hip", "fmm_lists.hip", "fmm_tables.hip", "fmm_gemm.hip", "fmm_expand.hip",
+SOURCES = ["fmm_prims.hip", "fmm_tree.hip", "fmm_lists.hip", "fmm_groups.hip", "fmm_tables.hip", "fmm_gemm.hip", "fmm_expand.hip",
            "fmm_treecode.hip", "fmm_adjoint.hip", "fmm_capi.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -20,6 +20,7 @@
 #include "fmm_adjoint.hpp"
 #include "fmm_expand.hpp"
 #include "fmm_gemm.hpp"
+#include "fmm_groups.hpp"
 #include "fmm_lists.hpp"
 #include "fmm_prims.hpp"
 #include "fmm_tables.hpp"
@@ -161,14 +162,16 @@ struct fmm_ctx {
     DevBuf pp_tiles;                             // per-pair path: tiles of one chunk
     Lists lists;
     ListScratch lscr;
-    PairIndex m2l_ix;                            // far pairs by target node
+    PairIndex m2l_ix;                            // far pairs (F16X3: their groups) by target node
+    FarGroups groups;                            // F16X3: far pairs grouped by target and source parent
     // F16X3: per-coefficient scales dm, the M2L tables split in FP16 (their FP32 staging), the
     // multipole column scales; down_l2l = L2L operators ahead of the M2L ones in the down tables
     DevBuf dm, m2l_hi, m2l_lo, m2l_rinv, m2l_work, cscale, Mhl;   // Mhl: split multipoles (hi | lo)
+    DevBuf cratio, cpinv;                        // column scales against the siblings' smallest, and 1 / that
     DevBuf queues;   // work counters: [0, 8) the M2L GEMM's per-XCD tiles, [8] the near-field leaves
     int down_l2l = 0;
     const OpSpec* down_specs = nullptr;          // device specs of the down tables
-    DevBuf m2l_slab;                             // M2L result per (pair, component)
+    DevBuf m2l_slab;                             // M2L result per (pair or group, component)
     // evaluation
     DevBuf Bfar, Bnear, Bout;
     DevBuf Afar, Anear, Aout;                    // vector potential (calcA)
@@ -229,10 +232,6 @@ void join_default_stream(fmm_ctx* c) {
 }
 
 bool nonempty_host(const TreeDev& T, int n) { return T.h_first_child[n] >= 0 || T.h_npts[n] > 0; }
-
-// columns per M2L tile: the FP16 split kernel takes 128 (two 16-column blocks per wave, each
-// operator fragment read from LDS once for both; measured 2.37 -> 2.09 ms on the 1M workload)
-int m2l_tile_cols(const fmm_ctx* c) { return c->prec == Precision::F16X3 ? 128 : 64; }
 
 // F16X3: the scale of real coefficient i = (l, m), a power of 2 with dm_i max |R_i(u)| in
 // (0.5, 1] over |u| <= sqrt(3) (the scaled position of any point in its box), so every scaled
@@ -461,7 +460,7 @@ void stage_leaves(fmm_ctx* c) {
             split.dm = c->dm.as<float>();
             split.Kp = kp;
             split.cscale = c->cscale.get<float>(ncols);
-            split.hl = c->Mhl.get<_Float16>((size_t)2 * ncols * kp);
+            split.hl = c->Mhl.get<_Float16>((size_t)2 * (ncols + 1) * kp);
         }
         launch_p2m(c->f64(), c->src_leaves.as<int>(), (int)c->h_src_leaves.size(), c->S, c->sigS,
                    c->sxyz.as<double>(), c->sq.as<double>(), c->p, c->Lp, M, c->stream, split);
@@ -644,7 +643,7 @@ void downward_per_pair(fmm_ctx* c) {
             run_per_pair(c, OPK_L2L, P.src, P.dst, P.npairs, T, T, c->sigT, c->sigT, Lx, Lx, false);
     }
     c->down_ops.nops = 0;
-    c->m2l_pass.ntiles = 0;
+    c->m2l_pass = Pass();
     c->rec(E_L2L);
     c->stage = ST_DOWN;
 }
@@ -660,8 +659,12 @@ void stage_lists(fmm_ctx* c, hipStream_t ls, hipEvent_t far_ready, const std::fu
     // the pair index (a sort of the far pairs by target) is queued as soon as the far pairs are,
     // ahead of the close lists
     build_lists(c->lists, c->lscr, c->S, c->T, c->cfg.mac_scale, shared, ls, far_ready, [&] {
-        if (shared) build_pair_index(c->lists.far_t.as<int>(), c->lists.num_far, c->T.num_nodes, c->m2l_ix, ls);
         if (after_far) after_far();
+        if (shared && c->prec == Precision::F16X3)
+            build_far_groups(c->groups, c->m2l_ix, c->lists, c->lscr.flag.as<uint32_t>(), c->lscr.pos.as<uint32_t>(),
+                             c->S, c->T, ls);
+        else if (shared)
+            build_pair_index(c->lists.far_t.as<int>(), c->lists.num_far, c->T.num_nodes, c->m2l_ix, ls);
     });
     c->rec_on(E_LISTS, ls);
     c->lists_ready = true;
@@ -715,25 +718,25 @@ void translate_tables(fmm_ctx* c, hipStream_t st) {
     } else if (O.nops) {
         build_tables(c, O, d, st);
     }
-    // the M2L tiles (planned while the tables are built)
+    // the M2L tiles (planned while the tables are built; F16X3: those of the groups, made with the lists)
     Pass& P = c->m2l_pass;
-    {
+    P = Pass();
+    P.npairs = c->lists.num_far;
+    if (c->prec != Precision::F16X3) {
         std::vector<int> cop(nc);
         for (int i = 0; i < nc; i++) cop[i] = n_l2l + i;
         std::vector<GemmTile> tiles;
-        plan_tiles(c->lists.h_class_begin, cop, tiles, m2l_tile_cols(c));
+        plan_tiles(c->lists.h_class_begin, cop, tiles);
         Staging& sg = c->m2l_stage;
         sg.begin();
         const size_t o_tiles = sg.put(tiles);
-        P.npairs = c->lists.num_far;
         P.ntiles = (int)tiles.size();
-        P.width = m2l_tile_cols(c);
         P.tiles = (const GemmTile*)(sg.send(st) + o_tiles);
     }
     // the pair reduction writes every local expansion whole; cleared here only when it will not run
     size_t n = (size_t)T.num_nodes * 3 * c->Lp;
     void* Lx = c->Lx.reserve(n * c->esize());
-    if (!P.ntiles) FMM_HIP(hipMemsetAsync(Lx, 0, n * c->esize(), st));
+    if (!P.npairs) FMM_HIP(hipMemsetAsync(Lx, 0, n * c->esize(), st));
     c->rec_on(E_TABLES, st);
 }
 
@@ -744,8 +747,10 @@ void split_for_gemm(fmm_ctx* c) {
     const int ncols = 3 * c->S.num_nodes, kp = m2l_f16_kpad(c->L);
     const bool leaves = c->leaves_split;   // the P2M wrote its leaves' columns
     split_columns(c->M.as<float>(), ncols, c->L, c->Lp, kp, c->dm.as<float>(), c->cscale.get<float>(ncols),
-                  c->Mhl.get<_Float16>((size_t)2 * ncols * kp), c->stream,
+                  c->Mhl.get<_Float16>((size_t)2 * (ncols + 1) * kp), c->stream,
                   leaves ? c->S.first_child.as<int>() : nullptr, leaves ? c->S.npts.as<int>() : nullptr);
+    sibling_scales(c->S.parent.as<int>(), c->S.first_child.as<int>(), c->S.num_nodes, c->cscale.as<float>(),
+                   c->cratio.get<float>(ncols + 1), c->cpinv.get<float>(ncols + 1), c->stream);
 }
 
 // Part 2 (stream A, after the tables and the multipoles): the M2L of all classes in one launch
@@ -757,19 +762,23 @@ void translate_gemm(fmm_ctx* c, hipEvent_t gemm_after = nullptr, bool split_done
     const OpTables& O = c->down_ops;
     const Pass& P = c->m2l_pass;
     const bool f16 = c->prec == Precision::F16X3;
-    if (f16 && P.ntiles && !split_done) split_for_gemm(c);
+    if (f16 && P.npairs && !split_done) split_for_gemm(c);
     if (gemm_after) FMM_HIP(hipStreamWaitEvent(st, gemm_after, 0));
+    const int R = m2l_slab_rows(c->prec, c->L, c->Lp);
+    if (f16) {
+        group_row_scales(c->groups, c->m2l_rinv.as<float>(), c->L, st);
+        FMM_HIP(hipMemsetAsync(c->queues.as<int>() + 8, 0, sizeof(int), st));   // the near field's leaves
+    }
     c->rec(E_GEMM0);
-    if (P.ntiles) {
-        const int R = m2l_slab_rows(c->prec, c->L, c->Lp);
+    if (P.npairs && f16) {
+        void* slab = c->m2l_slab.reserve((size_t)3 * c->groups.num * R * c->esize());
+        m2l_gemm_f16x3(c->m2l_hi.as<_Float16>(), c->m2l_lo.as<_Float16>(), c->m2l_rinv.as<float>(), c->groups,
+                       c->Mhl.as<_Float16>(), c->cratio.as<float>(), c->cpinv.as<float>(), 3 * c->S.num_nodes, (float*)slab,
+                       c->L, c->queues.get<int>(16), st);
+    } else if (P.npairs) {
         void* slab = c->m2l_slab.reserve((size_t)3 * P.npairs * R * c->esize());
-        if (f16)
-            m2l_gemm_f16x3(c->m2l_hi.as<_Float16>(), c->m2l_lo.as<_Float16>(), c->m2l_rinv.as<float>(), c->down_l2l,
-                           P.tiles, P.ntiles, m2l_tile_cols(c), c->lists.far_s.as<int>(), c->Mhl.as<_Float16>(),
-                           c->cscale.as<float>(), (float*)slab, c->L, c->queues.get<int>(16), st);
-        else
-            m2l_gemm(c->prec, ops_ptr(c, O), O.lo.ptr, P.tiles, P.ntiles, c->lists.far_s.as<int>(), c->M.ptr, slab,
-                     c->L, c->Lp, st);
+        m2l_gemm(c->prec, ops_ptr(c, O), O.lo.ptr, P.tiles, P.ntiles, c->lists.far_s.as<int>(), c->M.ptr, slab, c->L,
+                 c->Lp, st);
     }
     c->rec(E_M2L_GEMM);
     FMM_HIP(hipEventRecord(c->j_gemm, st));
@@ -782,7 +791,7 @@ void translate_finish(fmm_ctx* c) {
     OpTables& O = c->down_ops;
     const int nlev = T.num_levels;
     void* Lx = c->Lx.ptr;
-    if (c->m2l_pass.ntiles) {
+    if (c->m2l_pass.npairs) {
         reduce_pairs(c->f64(), c->m2l_ix, c->m2l_slab.ptr, m2l_slab_rows(c->prec, c->L, c->Lp), c->Lp, Lx, st);
     }
     c->rec(E_M2L);
@@ -843,6 +852,13 @@ __global__ void k_fill_nan(double* p, size_t n) {
     if (i < n) p[i] = __longlong_as_double(0x7ff8000000000000ll);
 }
 
+// near field of the target leaves left in the queue, by a persistent grid on stream ps
+void p2p_from_queue(fmm_ctx* c, hipStream_t ps, int grid, bool beside) {
+    launch_p2p_queue(c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S, c->lists.close_begin.as<int>(),
+                     c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->nP0.ptr, c->nP1.ptr, c->nP2.ptr,
+                     c->txyz.as<double>(), c->Bnear.as<double>(), c->queues.as<int>() + 8, grid, beside, ps);
+}
+
 // near field on stream ps (needs the lists and the packed sources)
 void stage_p2p(fmm_ctx* c, hipStream_t ps, bool queue = false) {
     int nts = c->T.num_slots;
@@ -856,10 +872,7 @@ void stage_p2p(fmm_ctx* c, hipStream_t ps, bool queue = false) {
                          c->lists.close_s.as<int>(), c->txyz.as<double>(), Bnear, nullptr, ps);
     } else if (c->cfg.near_field && queue) {
         // one persistent workgroup per CU beside the M2L GEMM (see run_fused)
-        launch_p2p_queue(c->f64(), c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S,
-                         c->lists.close_begin.as<int>(), c->lists.close_end.as<int>(), c->lists.close_s.as<int>(),
-                         c->nP0.ptr, c->nP1.ptr, c->nP2.ptr, c->txyz.as<double>(), Bnear, c->queues.get<int>(16) + 8,
-                         num_cus(), ps);
+        p2p_from_queue(c, ps, num_cus(), true);
     } else if (c->cfg.near_field) {
         launch_p2p(c->f64(), c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S, c->lists.close_begin.as<int>(),
                    c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->nP0.ptr, c->nP1.ptr, c->nP2.ptr,
@@ -981,7 +994,7 @@ void run_fused(fmm_ctx* c, double current, double* Bdev) {
     // GEMM workgroup.  Otherwise the P2P follows the GEMM (beside the GEMMs of one workgroup per
     // tile it only slows them).
     const bool p2p_beside = c->prec == Precision::F16X3 && c->cfg.near_field == FMM_NEAR_P2P &&
-                            m2l_tile_cols(c) == 128 && m2l_f16x3_persistent(c->L);
+                            m2l_f16x3_persistent(c->L);
     std::exception_ptr side_error;
     auto post = [&](int& state, int v) {
         {
@@ -1047,8 +1060,8 @@ void run_fused(fmm_ctx* c, double current, double* Bdev) {
             // the GEMM starts after the lists' last kernels (the pair index sort): beside the
             // persistent GEMM a sort whose blocks wait on each other crawled (17 ms instead of
             // 0.1), holding back the near field queued after it; normally the lists end first
-            translate_gemm(c, lists_state == 1 ? c->j_lists : nullptr, split_early);
-            post(gemm_state, 1);
+            if (lists_state == 1) translate_gemm(c, c->j_lists, split_early);
+            post(gemm_state, lists_state);   // 2: the side thread failed, its error is rethrown below
         } else {
             post(gemm_state, 2);
         }
@@ -1069,6 +1082,9 @@ void run_fused(fmm_ctx* c, double current, double* Bdev) {
         FMM_HIP(hipEventRecord(c->j_p2p, Bs));
     }
     stage_l2p(c);
+    // the leaves that the near field beside the GEMM has not taken: the chip is free now, and one
+    // workgroup per CU would take until long after
+    if (p2p_beside) p2p_from_queue(c, A, 8 * num_cus(), false);
     FMM_HIP(hipStreamWaitEvent(A, c->j_p2p, 0));
     stage_assemble(c, current, Bdev);
 }
@@ -1383,11 +1399,10 @@ int fmm_adjoint_weights_dev(fmm_ctx* c, double current, const double* dLdB, doub
             plan_tiles(cb, cop, tiles);
             stage_pass(sg, c->m2m_adj_pass[k], all_s, all_d, tiles);
         }
-        // M2L^T runs on class_gemm (tiles of at most 64 columns); the forward M2L tiles may be
-        // wider (F16X3 plans 128), so the transposed pass gets its own 64-column tiles
+        // the M2L^T's 64-column tiles of the far pairs (the forward M2L of F16X3 runs on groups of them)
         size_t o_m2l_tiles = 0;
         int n_m2l_tiles = 0;
-        if (c->m2l_pass.ntiles) {
+        if (c->m2l_pass.npairs) {
             const int nc = c->lists.num_classes;
             std::vector<int> cop(nc);
             for (int i = 0; i < nc; i++) cop[i] = c->down_l2l + i;

@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "fmm_expand.hpp"
+#include "fmm_gemm.hpp"
 #include "fmm_recip.hpp"
 
 namespace fmm {
@@ -190,7 +191,7 @@ __global__ __launch_bounds__(64) void k_p2m(const int* __restrict__ leaves, cons
                     mx = fmaxf(mx, fabsf(x[r]));
                 }
                 for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-                const float sc = mx > 0.0f ? exp2f((float)(-(ilogbf(mx) + 1))) : 1.0f;
+                const float sc = column_scale(mx);
                 const size_t col = (size_t)leaf * 3 + cc;
                 if (lane == 0) cscale[col] = sc;
                 _Float16* dst = hl + col * 2 * Kp;
@@ -592,16 +593,19 @@ __global__ __launch_bounds__(256) void k_p2p_transposed(
                                 P0, P1, P2, sxyz, out, s0, s1, s2, red, parent);
 }
 
-// The same near field as a small persistent grid taking leaves from a queue (an atomic counter
-// that starts at 0), with a register budget of 56 per lane: one workgroup per CU fits beside the
-// F16X3 M2L GEMM's, so the near field runs on the VALU slots the GEMM leaves idle.
-template <class R, bool POT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(10))) void k_p2p_queue(
-    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ tbegin,
-    const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
-    const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
-    const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
-    const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
+// The same near field as a persistent grid taking leaves from a queue (an atomic counter that starts at
+// 0), two forms of which may share a queue: BESIDE with a register budget of 56 per lane (no unrolling),
+// one workgroup of which fits on a CU beside the F16X3 M2L GEMM's, so the near field runs on the VALU
+// slots the GEMM leaves idle, and the plain one for the leaves left when the GEMM is done.
+template <class R, bool POT, bool BESIDE>
+__device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, int nleaves, int* __restrict__ queue,
+                                               const int* __restrict__ tbegin, const int* __restrict__ tend,
+                                               const int* __restrict__ close_begin, const int* __restrict__ close_end,
+                                               const int* __restrict__ close_s, const double* __restrict__ origin,
+                                               const int* __restrict__ sbegin, const int* __restrict__ send,
+                                               const typename V4<R>::t* __restrict__ P0,
+                                               const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
+                                               const double* __restrict__ txyz, double* __restrict__ Bnear) {
     __shared__ typename V4<R>::t s0[4][64];
     __shared__ typename V4<R>::t s1[4][64];
     __shared__ R s2[4][64];
@@ -613,8 +617,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(10))) void 
         const int i = next;
         __syncthreads();   // every thread has read next before thread 0 takes the following leaf
         if (i >= nleaves) break;
-        p2p_leaf<R, POT, 1>(leaves[i], tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send, P0, P1, P2, txyz, Bnear, s0, s1, s2, red);
+        p2p_leaf<R, POT, BESIDE ? 1 : 4>(leaves[i], tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send,
+                                         P0, P1, P2, txyz, Bnear, s0, s1, s2, red);
     }
+}
+template <class R, bool POT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(10))) void k_p2p_queue(
+    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ tbegin,
+    const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
+    const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
+    const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
+    const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
+    p2p_queue_body<R, POT, true>(leaves, nleaves, queue, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+                                 send, P0, P1, P2, txyz, Bnear);
+}
+template <class R, bool POT>
+__global__ __launch_bounds__(256) void k_p2p_queue_rest(
+    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ tbegin,
+    const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
+    const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
+    const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
+    const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
+    p2p_queue_body<R, POT, false>(leaves, nleaves, queue, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+                                  send, P0, P1, P2, txyz, Bnear);
 }
 
 // ---------------------------------------------------------------- Problem::BEM
@@ -1025,22 +1050,15 @@ void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, cons
                 const double* txyz, double* Bnear, hipStream_t st) {
     p2p_launch<false>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Bnear, st);
 }
-void launch_p2p_queue(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S,
-                      const int* close_begin, const int* close_end, const int* close_s, const void* P0, const void* P1,
-                      const void* P2, const double* txyz, double* Bnear, int* queue, int grid, hipStream_t st) {
+void launch_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                      const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
+                      const double* txyz, double* Bnear, int* queue, int grid, bool beside, hipStream_t st) {
     if (!nleaves) return;
     if (grid < 1) throw Error(1, "near field: empty persistent grid");
-    FMM_HIP(hipMemsetAsync(queue, 0, sizeof(int), st));
-    if (f64)
-        k_p2p_queue<double, false><<<grid, 256, 0, st>>>(leaves, nleaves, queue, T.begin.as<int>(), T.end.as<int>(),
-                                                         close_begin, close_end, close_s, S.center.as<double>(),
-                                                         S.begin.as<int>(), S.end.as<int>(), (const double4*)P0,
-                                                         (const double4*)P1, (const double*)P2, txyz, Bnear);
-    else
-        k_p2p_queue<float, false><<<grid, 256, 0, st>>>(leaves, nleaves, queue, T.begin.as<int>(), T.end.as<int>(),
-                                                        close_begin, close_end, close_s, S.center.as<double>(),
-                                                        S.begin.as<int>(), S.end.as<int>(), (const float4*)P0,
-                                                        (const float4*)P1, (const float*)P2, txyz, Bnear);
+    (beside ? k_p2p_queue<float, false> : k_p2p_queue_rest<float, false>)<<<grid, 256, 0, st>>>(
+        leaves, nleaves, queue, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
+        S.center.as<double>(), S.begin.as<int>(), S.end.as<int>(), (const float4*)P0, (const float4*)P1,
+        (const float*)P2, txyz, Bnear);
     FMM_HIP(hipGetLastError());
 }
 void launch_p2p_transposed(bool f64, const int* leaves, int nleaves, const TreeDev& S, const TreeDev& T,

@@ -19,6 +19,7 @@
 //            B = Bh + Bl (split on load): C += Al Bh + Ah Bl + Ah Bh, FP32 accumulate.
 // TRANS applies T^T (the adjoint passes) by reading the operator column-wise.
 #include "fmm_gemm.hpp"
+#include "fmm_groups.hpp"
 #include "fmm_prims.hpp"
 
 namespace fmm {
@@ -453,122 +454,223 @@ __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, con
 //                                   evaluation by k_split_columns into FP16 hi and lo parts)
 // so T M = diag(rinv) (A_eq B_eq) diag(1/s), applied in the epilogue.  Rows R = 16 NB >= L,
 // K padded to Kp = 32 NKS >= L (zero operator columns and multipole rows beyond L).
-// Layout and schedule follow k_gemm_m2l: wave w owns the tile's columns [16w, 16w + 16) and all
-// NB row blocks; one LDS buffer refilled from registers whose loads overlap the MFMAs.
+//
+// A column is a component of one group of far pairs: up to 8 children of one source node that are far
+// from one target (fmm_groups.hpp).  A tile runs over the K steps of every child in the union of its
+// groups' masks, one operator per child; columns whose group lacks that child take zeros.  The children
+// have operators and columns of their own scales, so on the way into LDS the operator rows are brought
+// to the largest 1 / rs of the class (rows times rinv / cls_rinv) and the columns to the smallest
+// scale of the siblings (ratio), powers of 2 at most 1: a value keeps FP16's 22 split bits relative to
+// the largest term of the group's sum.  The epilogue applies cls_rinv and 1 / that scale (pinv) and
+// stores one slab block per group.
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+// eight halves on their way from memory to LDS.  As a half vector the compiler takes each register apart
+// and together again wherever a load is conditional (300 instructions per K step, more than all others)
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ i32x4 scaled(i32x4 v, _Float16 s) {
+    return __builtin_bit_cast(i32x4, __builtin_bit_cast(half8, v) * s);
+}
 
-template <int NB, int NKS, int NC>
-__global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(const _Float16* __restrict__ ops_hi,
-                                                        const _Float16* __restrict__ ops_lo,
-                                                        const float* __restrict__ ops_rinv,
-                                                        const GemmTile* __restrict__ tiles,
-                                                        const int* __restrict__ pair_src,
-                                                        const _Float16* __restrict__ src_hl,
-                                                        const float* __restrict__ cscale, float* __restrict__ slab,
-                                                        int op_base) {
-    constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK + 8;   // LDS row stride: 80 bytes
+// LDS rows of 32 halves without padding, their four 16-byte chunks permuted by the row: chunk q of row r
+// lies at q ^ f(r / 4 mod 4), f = 0, 2, 3, 1.  16-byte LDS reads are served in lane groups
+// 0-3, 12-15, 20-23, 24-27 and 4-7, 8-11, 16-19, 28-31 (and those + 32): with lane = 16 g + i reading
+// chunk g of row i, each group then covers all 64 banks once, and so do the stores of 8 consecutive lanes
+// (two whole rows).  Rows padded to 80 bytes conflicted in half of all LDS cycles.
+__device__ __forceinline__ int lds_chunk(int q, int row) {
+    const int b1 = (row >> 3) & 1, b0 = (row >> 2) & 1;
+    return q ^ (2 * (b1 ^ b0) + b1);
+}
+
+struct M2LGroupArgs {
+    const _Float16 *ops_hi, *ops_lo;
+    const float* ops_rinv;
+    const GroupTile* tiles;
+    const int* cls_ops;
+    const float* cls_rinv;
+    const int* grp_fc;
+    const int* grp_mask;
+    const _Float16* src_hl;
+    const float* ratio;
+    const float* pinv;
+    float* slab;
+    int ntiles, zero_col;   // the column of zeros
+};
+
+// What the threads of a workgroup load of the current child of a tile: the operator's rows
+// (tid >> 2) + 64 j and the columns (tid >> 2) + 64 c, 8 consecutive k each, and their scales.  Every
+// load is unconditional (rows beyond R are clamped and not stored, columns whose group lacks the child
+// read the column of zeros behind the nodes'): after a load that may have been skipped the compiler
+// cannot count the loads in flight and waits for all of them, the ones issued steps ahead included.
+template <int R, int Kp, int NQ>
+struct M2LTileLoads {
+    const M2LGroupArgs& A;
+    GroupTile tile;
+    int tid, wave, bq, sq;           // wave: uniform; bq, sq: first k of this thread's chunk, its place in LDS
+    int col[2], gm[2];               // multipole column of child 0 and child mask of the columns' groups
+    const _Float16 *ah, *al;         // operator parts (uniform)
+    const _Float16* b[2];
+    __device__ __forceinline__ M2LTileLoads(const M2LGroupArgs& A_, const GroupTile& t, int tid_)
+        : A(A_), tile(t), tid(tid_), wave(__builtin_amdgcn_readfirstlane(tid_ >> 6)), bq((tid_ & 3) * 8),
+          sq(8 * lds_chunk(tid_ & 3, tid_ >> 2)) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int cl = (tid >> 2) + 64 * c;
+            const bool valid = cl < 3 * tile.ng;
+            const int g = tile.g0 + (valid ? cl / 3 : 0);
+            col[c] = 3 * A.grp_fc[g] + cl % 3;
+            gm[c] = valid ? A.grp_mask[g] : 0;
+        }
+    }
+    __device__ __forceinline__ int row(int j) const {
+        const int r = (tid >> 2) + 64 * j;
+        return 64 * (j + 1) <= R ? r : min(r, R - 1);
+    }
+    // a wave stages 16 rows at a time: all of them exist or none
+    __device__ __forceinline__ bool has_rows(int j) const { return 64 * (j + 1) <= R || 16 * wave + 64 * j < R; }
+    __device__ __forceinline__ size_t op(int o) const { return (size_t)A.cls_ops[8 * (size_t)tile.cls + o]; }
+    __device__ __forceinline__ void set_columns(int o, bool any = true) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const bool in = any && ((gm[c] >> o) & 1);
+            b[c] = A.src_hl + (size_t)(in ? col[c] + 3 * o : A.zero_col) * 2 * Kp + bq;
+        }
+    }
+    __device__ __forceinline__ void set_rows(int o) {
+        ah = A.ops_hi + op(o) * R * Kp;
+        al = A.ops_lo + op(o) * R * Kp;
+    }
+    __device__ __forceinline__ void scales(int o, _Float16 (&rs)[NQ], _Float16 (&cs)[2]) const {
+#pragma unroll
+        for (int c = 0; c < 2; c++) cs[c] = (_Float16)A.ratio[(gm[c] >> o) & 1 ? col[c] + 3 * o : A.zero_col];
+        const float *ro = A.ops_rinv + op(o) * R, *rc = A.cls_rinv + (size_t)tile.cls * R;
+#pragma unroll
+        for (int j = 0; j < NQ; j++)   // both are powers of 2: the quotient by their exponents
+            rs[j] = (_Float16)__int_as_float(__float_as_int(ro[row(j)]) - __float_as_int(rc[row(j)]) + 0x3f800000);
+    }
+    __device__ __forceinline__ void aload1(int j, int k0, i32x4& h, i32x4& l) const {
+        const unsigned o = (unsigned)(row(j) * Kp + k0 + bq);
+        h = *(const i32x4*)(ah + o);
+        l = *(const i32x4*)(al + o);
+    }
+    __device__ __forceinline__ void aload(int k0, i32x4 (&h)[NQ], i32x4 (&l)[NQ]) const {
+#pragma unroll
+        for (int j = 0; j < NQ; j++) aload1(j, k0, h[j], l[j]);
+    }
+    __device__ __forceinline__ void bload(int k0, i32x4 (&h)[2], i32x4 (&l)[2]) const {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            h[c] = *(const i32x4*)(b[c] + 2 * k0);
+            l[c] = *(const i32x4*)(b[c] + 2 * k0 + 32);
+        }
+    }
+    template <int S>
+    __device__ __forceinline__ void astore1(int j, _Float16 rs, const i32x4& h, const i32x4& l, _Float16 (*Ah)[S],
+                                            _Float16 (*Al)[S]) const {
+        const i32x4 hs = scaled(h, rs), ls = scaled(l, rs);
+        if (has_rows(j)) {
+            *(i32x4*)&Ah[(tid >> 2) + 64 * j][sq] = hs;
+            *(i32x4*)&Al[(tid >> 2) + 64 * j][sq] = ls;
+        }
+    }
+    template <int S>
+    __device__ __forceinline__ void bstore(const _Float16 (&cs)[2], const i32x4 (&h)[2], const i32x4 (&l)[2],
+                                           _Float16 (*Bh)[S], _Float16 (*Bl)[S]) const {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            *(i32x4*)&Bh[(tid >> 2) + 64 * c][sq] = scaled(h[c], cs[c]);
+            *(i32x4*)&Bl[(tid >> 2) + 64 * c][sq] = scaled(l[c], cs[c]);
+        }
+    }
+    template <int S>
+    __device__ __forceinline__ void store(const _Float16 (&rs)[NQ], const _Float16 (&cs)[2], const i32x4 (&ah_)[NQ],
+                                          const i32x4 (&al_)[NQ], const i32x4 (&bh)[2], const i32x4 (&bl)[2],
+                                          _Float16 (*Ah)[S], _Float16 (*Al)[S], _Float16 (*Bh)[S],
+                                          _Float16 (*Bl)[S]) const {
+        bstore<S>(cs, bh, bl, Bh, Bl);
+#pragma unroll
+        for (int j = 0; j < NQ; j++) astore1<S>(j, rs[j], ah_[j], al_[j], Ah, Al);
+    }
+    // column cl of the tile: the slab block's column and the scale to undo
+    __device__ __forceinline__ float* column(int cl, float& sinv) const {
+        const int g = tile.g0 + cl / 3, comp = cl % 3;
+        sinv = A.pinv[3 * A.grp_fc[g] + comp];
+        return A.slab + (3 * (size_t)g + comp) * R;
+    }
+};
+
+// Small orders (and the largest, whose two LDS buffers do not fit): wave w owns the tile's columns
+// [32w, 32w + 32) and all NB row blocks; one LDS buffer refilled from registers whose loads overlap the
+// MFMAs, two workgroups per CU.
+template <int NB, int NKS>
+__global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
+    constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK;
     constexpr int NQ = (4 * R + 255) / 256;                          // A: 8-half vectors per thread and part
-    constexpr int W = 64 * NC;                                       // tile columns (NC blocks of 16 per wave)
     __shared__ __attribute__((aligned(16))) _Float16 Ah[R][S];
     __shared__ __attribute__((aligned(16))) _Float16 Al[R][S];
-    __shared__ __attribute__((aligned(16))) _Float16 Bh[W][S];
-    __shared__ __attribute__((aligned(16))) _Float16 Bl[W][S];
+    __shared__ __attribute__((aligned(16))) _Float16 Bh[128][S];
+    __shared__ __attribute__((aligned(16))) _Float16 Bl[128][S];
     // each XCD works on a contiguous eighth of the tiles (a bijection of the grid)
     const int nt = gridDim.x, xcd = blockIdx.x & 7, q = nt >> 3, rem = nt & 7;
     const int t = xcd * q + min(xcd, rem) + (blockIdx.x >> 3);
-    const GemmTile tile = tiles[t];
+    const GroupTile tile = A.tiles[t];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
-    const int op = tile.op - op_base;   // tile.op numbers the operators of all down passes
-    const _Float16* Ahg = ops_hi + (size_t)op * R * Kp;
-    const _Float16* Alg = ops_lo + (size_t)op * R * Kp;
-    // B staging: columns bc + 64 c, k = bq .. bq + 7 of each K step, from the multipoles split
-    // beforehand (split_columns): equilibrated FP16 hi and lo parts, [column][K step][hi | lo]
-    const int bc = tid >> 2, bq = (tid & 3) * 8;
-    const _Float16* bph[NC];
-    const _Float16* bpl[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-        bph[c] = bpl[c] = nullptr;
-        if (bc + 64 * c < tile.ncol) {
-            const int col = tile.col0 + bc + 64 * c, pair = col / 3, comp = col - 3 * pair;
-            const size_t sc = (size_t)pair_src[pair] * 3 + comp;
-            bph[c] = src_hl + sc * 2 * Kp;
-            bpl[c] = bph[c] + 32;
-        }
-    }
-    half8 rah[NQ], ral[NQ];
-    half8 rbh[NC], rbl[NC];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int j = 0; j < NQ; j++) {
-            const int qi = tid + 256 * j;
-            if (qi < 4 * R) {
-                const size_t o = (size_t)(qi >> 2) * Kp + k0 + (qi & 3) * 8;
-                rah[j] = *(const half8*)(Ahg + o);
-                ral[j] = *(const half8*)(Alg + o);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const half8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-            rbh[c] = bph[c] ? *(const half8*)(bph[c] + 2 * k0 + bq) : z;
-            rbl[c] = bpl[c] ? *(const half8*)(bpl[c] + 2 * k0 + bq) : z;
-        }
-    };
-    auto lstore = [&]() {
-#pragma unroll
-        for (int j = 0; j < NQ; j++) {
-            const int qi = tid + 256 * j;
-            if (qi < 4 * R) {
-                *(half8*)&Ah[qi >> 2][(qi & 3) * 8] = rah[j];
-                *(half8*)&Al[qi >> 2][(qi & 3) * 8] = ral[j];
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            *(half8*)&Bh[bc + 64 * c][bq] = rbh[c];
-            *(half8*)&Bl[bc + 64 * c][bq] = rbl[c];
-        }
-    };
-    f32x4 acc[NB][NC];
+    M2LTileLoads<R, Kp, NQ> ld(A, tile, tid);
+    _Float16 rs[NQ], cs[2];
+    i32x4 rah[NQ], ral[NQ], rbh[2], rbl[2];
+    f32x4 acc[NB][2];
 #pragma unroll
     for (int a = 0; a < NB; a++)
 #pragma unroll
-        for (int c = 0; c < NC; c++) acc[a][c] = f32x4{0, 0, 0, 0};
-    gload(0);
-    for (int kt = 0; kt < NKS; kt++) {
-        lstore();
-        __syncthreads();
-        if (kt + 1 < NKS) gload((kt + 1) * BK);
-        const int kk = 8 * g;
-        half8 bh[NC], bl[NC];
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            bh[c] = *(const half8*)&Bh[wave * 16 * NC + 16 * c + li][kk];
-            bl[c] = *(const half8*)&Bl[wave * 16 * NC + 16 * c + li][kk];
-        }
-#pragma unroll
-        for (int a = 0; a < NB; a++) {
-            const half8 ah = *(const half8*)&Ah[a * 16 + li][kk];
-            const half8 al = *(const half8*)&Al[a * 16 + li][kk];
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[c], acc[a][c], 0, 0, 0);
-                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[c], acc[a][c], 0, 0, 0);
-                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[c], acc[a][c], 0, 0, 0);
+        for (int c = 0; c < 2; c++) acc[a][c] = f32x4{0, 0, 0, 0};
+    int m = tile.mask;
+    auto open = [&](int o) {
+        ld.set_columns(o);
+        ld.set_rows(o);
+        ld.scales(o, rs, cs);
+    };
+    open(__builtin_ctz(m));
+    ld.aload(0, rah, ral);
+    ld.bload(0, rbh, rbl);
+    while (m) {
+        m &= m - 1;
+        for (int kt = 0; kt < NKS; kt++) {
+            ld.template store<S>(rs, cs, rah, ral, rbh, rbl, Ah, Al, Bh, Bl);
+            __syncthreads();
+            if (kt + 1 < NKS || m) {
+                if (kt + 1 == NKS) open(__builtin_ctz(m));
+                const int k0 = kt + 1 < NKS ? (kt + 1) * BK : 0;
+                ld.aload(k0, rah, ral);
+                ld.bload(k0, rbh, rbl);
             }
+            const int kk = 8 * lds_chunk(g, li);
+            half8 bh[2], bl[2];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                bh[c] = *(const half8*)&Bh[wave * 32 + 16 * c + li][kk];
+                bl[c] = *(const half8*)&Bl[wave * 32 + 16 * c + li][kk];
+            }
+#pragma unroll
+            for (int a = 0; a < NB; a++) {
+                const half8 ah = *(const half8*)&Ah[a * 16 + li][kk];
+                const half8 al = *(const half8*)&Al[a * 16 + li][kk];
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[c], acc[a][c], 0, 0, 0);
+                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[c], acc[a][c], 0, 0, 0);
+                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[c], acc[a][c], 0, 0, 0);
+                }
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
     // epilogue: undo the scales; the slab is written once and read once (nontemporal)
-    const float* rv = ops_rinv + (size_t)op * R;
+    const float* rv = A.cls_rinv + (size_t)tile.cls * R;
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-        const int cl = wave * 16 * NC + 16 * c + li;
-        if (cl >= tile.ncol) continue;
-        const int col = tile.col0 + cl, pair = col / 3, comp = col - 3 * pair;
-        const float sinv = 1.0f / cscale[pair_src[pair] * 3 + comp];
-        float* out = slab + (size_t)col * R;
+    for (int c = 0; c < 2; c++) {
+        const int cl = wave * 32 + 16 * c + li;
+        if (cl >= 3 * tile.ng) continue;
+        float sinv;
+        float* out = ld.column(cl, sinv);
 #pragma unroll
         for (int a = 0; a < NB; a++) {
             const float4 r = *(const float4*)(rv + a * 16 + 4 * g);
@@ -579,22 +681,17 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(const _Float16* __restri
     }
 }
 
-// The 128-column F16X3 M2L with the waves on a 2 x 2 grid: wave (wr, wc) owns the row blocks
-// [wr NB0, wr NB0 + NB0) below NB (NB0 = ceil(NB / 2)) and the tile columns [64 wc, 64 wc + 64),
-// so it reads half the operator rows and half the columns from LDS per K step (a wave tile of
-// 16 NB0 x 64 instead of 16 NB x 32: about a third less LDS traffic per MFMA).  Staging, numerics
-// and epilogue as k_gemm_m2l_f16x3.
+// The waves on a 2 x 2 grid: wave (wr, wc) owns the row blocks [wr NB0, wr NB0 + NB0) below NB
+// (NB0 = ceil(NB / 2)) and the tile columns [64 wc, 64 wc + 64), so it reads half the operator rows and
+// half the columns from LDS per K step (a wave tile of 16 NB0 x 64 instead of 16 NB x 32: about a
+// third less LDS traffic per MFMA).  Two LDS buffers, one barrier per K step; the multipole columns
+// (gathered from HBM) are loaded BD K steps ahead, the operator rows (shared by the tiles of one
+// class, mostly L2 hits) one step ahead, across the boundary from one child to the next.
 template <int NB, int NKS, int BD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_gemm_m2l_f16x3_q(
-                                                          const _Float16* __restrict__ ops_hi,
-                                                          const _Float16* __restrict__ ops_lo,
-                                                          const float* __restrict__ ops_rinv,
-                                                          const GemmTile* __restrict__ tiles,
-                                                          const int* __restrict__ pair_src,
-                                                          const _Float16* __restrict__ src_hl,
-                                                          const float* __restrict__ cscale, float* __restrict__ slab,
-                                                          int op_base, int ntiles, int* __restrict__ xq) {
-    constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK + 8;   // LDS row stride: 80 bytes
+__global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_gemm_m2l_f16x3_q(M2LGroupArgs A,
+                                                                                                int* __restrict__ xq) {
+    static_assert(NKS % BD == 0 && (BD == 2 || BD == 1), "the column register sets are indexed statically");
+    constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK;
     constexpr int NQ = (4 * R + 255) / 256;                          // A: 8-half vectors per thread and part
     constexpr int W = 128, NB0 = (NB + 1) / 2;
     __shared__ __attribute__((aligned(16))) _Float16 Ah[2][R][S];
@@ -602,14 +699,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
     __shared__ __attribute__((aligned(16))) _Float16 Bh[2][W][S];
     __shared__ __attribute__((aligned(16))) _Float16 Bl[2][W][S];
     // persistent: the grid (a multiple of 8, workgroup b on XCD b mod 8) walks the tiles, each
-    // XCD a contiguous eighth of them (one class's operator shared in one L2) taken from that
+    // XCD a contiguous eighth of them (one class's operators shared in one L2) taken from that
     // XCD's counter xq[xcd] (zero at launch), so a workgroup that starts late (its CU busy)
     // takes fewer tiles, and then from the other XCDs' eighths; a workgroup starts its next tile
     // while its last stores drain.  The
     // register budget leaves room for one near-field workgroup (k_p2p_queue) per CU.
-    const int xcd = blockIdx.x & 7, q = ntiles >> 3, rem = ntiles & 7;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
-    const int wr = wave & 1, wc = wave >> 1, rb0 = wr * NB0;
+    const int xcd = blockIdx.x & 7, q = A.ntiles >> 3, rem = A.ntiles & 7;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, li = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave & 1, wc = wave >> 1, rb0 = wr * NB0;
     __shared__ int next_tile;
     int from = xcd;   // (thread 0) the eighth this workgroup draws from: its XCD's, then the others'
     for (;;) {
@@ -628,120 +725,114 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
             next_tile = t;
         }
         __syncthreads();
-        const int it = next_tile;   // read before the K loop's barriers; rewritten only after them
+        // read before the K loop's barriers, rewritten only after them; the same in every lane, so what
+        // follows from it stays in scalar registers
+        const int it = __builtin_amdgcn_readfirstlane(next_tile);
         if (it < 0) break;
-        const GemmTile tile = tiles[it];
-        const int op = tile.op - op_base;
-        const _Float16* Ahg = ops_hi + (size_t)op * R * Kp;
-        const _Float16* Alg = ops_lo + (size_t)op * R * Kp;
-        const int bc = tid >> 2, bq = (tid & 3) * 8;
-        const _Float16* bph[2];
-        const _Float16* bpl[2];
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            bph[c] = bpl[c] = nullptr;
-            if (bc + 64 * c < tile.ncol) {
-                const int col = tile.col0 + bc + 64 * c, pair = col / 3, comp = col - 3 * pair;
-                const size_t sc = (size_t)pair_src[pair] * 3 + comp;
-                bph[c] = src_hl + sc * 2 * Kp;
-                bpl[c] = bph[c] + 32;
-            }
-        }
-        half8 rah[NQ], ral[NQ];
-        half8 rbh[BD][2], rbl[BD][2];   // [set][c]: the multipole columns of BD K steps in flight
-        auto aload = [&](int k0) {
-#pragma unroll
-            for (int j = 0; j < NQ; j++) {
-                const int qi = tid + 256 * j;
-                if (qi < 4 * R) {
-                    const size_t o = (size_t)(qi >> 2) * Kp + k0 + (qi & 3) * 8;
-                    rah[j] = *(const half8*)(Ahg + o);
-                    ral[j] = *(const half8*)(Alg + o);
-                }
-            }
-        };
-        auto bload = [&](int set, int k0) {
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const half8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-                rbh[set][c] = bph[c] ? *(const half8*)(bph[c] + 2 * k0 + bq) : z;
-                rbl[set][c] = bpl[c] ? *(const half8*)(bpl[c] + 2 * k0 + bq) : z;
-            }
-        };
-        auto lstore = [&](int buf, int set) {
-#pragma unroll
-            for (int j = 0; j < NQ; j++) {
-                const int qi = tid + 256 * j;
-                if (qi < 4 * R) {
-                    *(half8*)&Ah[buf][qi >> 2][(qi & 3) * 8] = rah[j];
-                    *(half8*)&Al[buf][qi >> 2][(qi & 3) * 8] = ral[j];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                *(half8*)&Bh[buf][bc + 64 * c][bq] = rbh[set][c];
-                *(half8*)&Bl[buf][bc + 64 * c][bq] = rbl[set][c];
-            }
-        };
+        const GroupTile tile = A.tiles[it];
+        M2LTileLoads<R, Kp, NQ> ld(A, tile, tid);
+        _Float16 rs[NQ], cs[2];
+        i32x4 rah[NQ], ral[NQ];
+        i32x4 rbh[BD][2], rbl[BD][2];   // [set][c]: the multipole columns of BD K steps in flight
         f32x4 acc[NB0][4];
 #pragma unroll
         for (int a = 0; a < NB0; a++)
 #pragma unroll
             for (int c = 0; c < 4; c++) acc[a][c] = f32x4{0, 0, 0, 0};
-        // the multipole columns (gathered from HBM) are loaded BD K steps ahead, the operator
-        // rows (shared by the tiles of one class, mostly L2 hits) one step ahead; the K loop is
-        // unrolled so the register sets are indexed statically
-        aload(0);
+        int m = tile.mask, buf = 0;   // m: the children left (at least one)
+        int o_cur = __builtin_ctz(m);
+        ld.set_columns(o_cur);
+        ld.set_rows(o_cur);
+        ld.scales(o_cur, rs, cs);
+        ld.aload(0, rah, ral);
 #pragma unroll
-        for (int d = 0; d < BD; d++)
-            if (d < NKS) bload(d, d * BK);
-        lstore(0, 0);
+        for (int d = 0; d < BD; d++) ld.bload(d * BK, rbh[d], rbl[d]);
+        ld.template store<S>(rs, cs, rah, ral, rbh[0], rbl[0], Ah[0], Al[0], Bh[0], Bl[0]);
+        ld.aload(BK, rah, ral);
+        ld.bload(BD * BK, rbh[0], rbl[0]);
         __syncthreads();
+        for (bool more = true; more;) {
+            m &= m - 1;
+            more = m != 0;
+            // the next child; after the last one its operator's first steps are loaded and the first
+            // stored again, unused, and no column: the K loop stays free of branches
+            const int o = more ? __builtin_ctz(m) : o_cur;
+            o_cur = o;
+            _Float16 nrs[NQ], ncs[2];
+            for (int kt0 = 0; kt0 < NKS; kt0 += BD)
 #pragma unroll
-        for (int kt = 0; kt < NKS; kt++) {
-            const int cur = kt & 1;
-            if (kt + 1 < NKS) aload((kt + 1) * BK);
-            if (kt + BD < NKS) bload(kt % BD, (kt + BD) * BK);   // this set held step kt, stored already
-            const int kk = 8 * g;
-            half8 bh[4], bl[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                bh[c] = *(const half8*)&Bh[cur][wc * 64 + 16 * c + li][kk];
-                bl[c] = *(const half8*)&Bl[cur][wc * 64 + 16 * c + li][kk];
-            }
-            // all of this K step's operator fragments are read up front: the MFMAs of a row block
-            // wait only for its own reads, which land while the earlier blocks' MFMAs run
-            half8 ah[NB0], al[NB0];
-#pragma unroll
-            for (int a = 0; a < NB0; a++) {
-                // the second row half's last block is past NB when NB is odd: it reads the block
-                // NB - 1 instead (in bounds) and its MFMAs are skipped
-                const int row = min(rb0 + a, NB - 1) * 16 + li;
-                ah[a] = *(const half8*)&Ah[cur][row][kk];
-                al[a] = *(const half8*)&Al[cur][row][kk];
-            }
-#pragma unroll
-            for (int a = 0; a < NB0; a++) {
-                if (rb0 + a >= NB) continue;   // uniform over the wave
+            for (int d = 0; d < BD; d++) {
+                // register sets (and for even NKS the LDS buffers) by constant indexes
+                const int kt = kt0 + d, cb = BD % 2 ? buf : d & 1, ob = cb ^ 1, set = (d + 1) % BD;
+                const int ka = kt + 2 < NKS ? kt + 2 : kt + 2 - NKS;               // steps loaded now
+                const int kb = kt + 1 + BD < NKS ? kt + 1 + BD : kt + 1 + BD - NKS;
+                const int kk = 8 * lds_chunk(g, li);
+                half8 bh[4], bl[4];
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[a], bh[c], acc[a][c], 0, 0, 0);
-                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[a], bl[c], acc[a][c], 0, 0, 0);
-                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[a], bh[c], acc[a][c], 0, 0, 0);
+                    bh[c] = *(const half8*)&Bh[cb][wc * 64 + 16 * c + li][kk];
+                    bl[c] = *(const half8*)&Bl[cb][wc * 64 + 16 * c + li][kk];
                 }
+                // row block by row block, each block's operator fragments read during the previous block's
+                // MFMAs.  Between the blocks, spread over the step: the next step (loaded during the
+                // previous one) goes to the other LDS buffer, last read before the previous barrier, and
+                // its registers take the step after it; from the last steps on these are the next child's.
+                // The scheduling barriers keep the pieces apart: left alone the compiler gathers the loads
+                // and runs out of registers
+                half8 fh[2], fl[2];
+                auto frag = [&](int a) {
+                    // the second row half's last block is past NB when NB is odd: it reads the block
+                    // NB - 1 instead (in bounds) and its MFMAs are skipped
+                    const int row = min(rb0 + a, NB - 1) * 16 + li;
+                    fh[a & 1] = *(const half8*)&Ah[cb][row][kk];
+                    fl[a & 1] = *(const half8*)&Al[cb][row][kk];
+                };
+                frag(0);
+                static_assert(NQ + 2 <= NB0, "the pieces of the staging fit between the row blocks");
+#pragma unroll
+                for (int a = 0; a < NB0; a++) {
+                    if (a + 1 < NB0) frag(a + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (rb0 + a < NB) {   // uniform over the wave
+#pragma unroll
+                        for (int c = 0; c < 4; c++) {
+                            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[a & 1], bh[c], acc[a][c], 0, 0, 0);
+                            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bl[c], acc[a][c], 0, 0, 0);
+                            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bh[c], acc[a][c], 0, 0, 0);
+                        }
+                    }
+                    if (a == 0) {
+                        if (kt + 1 == NKS) {
+#pragma unroll
+                            for (int j = 0; j < NQ; j++) rs[j] = nrs[j];
+                            cs[0] = ncs[0];
+                            cs[1] = ncs[1];
+                        }
+                        if (kt + 1 + BD == NKS) {
+                            ld.set_columns(o, more);
+                            ld.scales(o, nrs, ncs);
+                        }
+                        if (kt + 2 == NKS) ld.set_rows(o);
+                        ld.template bstore<S>(cs, rbh[set], rbl[set], Bh[ob], Bl[ob]);
+                    }
+                    if (a >= 1 && a <= NQ) {
+                        ld.template astore1<S>(a - 1, rs[a - 1], rah[a - 1], ral[a - 1], Ah[ob], Al[ob]);
+                        ld.aload1(a - 1, ka * BK, rah[a - 1], ral[a - 1]);
+                    }
+                    if (a == NQ + 1) ld.bload(kb * BK, rbh[set], rbl[set]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                __syncthreads();
+                if (BD % 2) buf = ob;
             }
-            // the other LDS buffer was last read before the previous barrier
-            if (kt + 1 < NKS) lstore(cur ^ 1, (kt + 1) % BD);
-            __syncthreads();
         }
-        const float* rv = ops_rinv + (size_t)op * R;
+        const float* rv = A.cls_rinv + (size_t)tile.cls * R;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             const int cl = wc * 64 + 16 * c + li;
-            if (cl >= tile.ncol) continue;
-            const int col = tile.col0 + cl, pair = col / 3, comp = col - 3 * pair;
-            const float sinv = 1.0f / cscale[pair_src[pair] * 3 + comp];
-            float* out = slab + (size_t)col * R;
+            if (cl >= 3 * tile.ng) continue;
+            float sinv;
+            float* out = ld.column(cl, sinv);
 #pragma unroll
             for (int a = 0; a < NB0; a++) {
                 if (rb0 + a >= NB) break;
@@ -755,13 +846,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
 }
 
 // per multipole column c (node * 3 + component): the power of 2 s_c that brings
-// max_i |M[c][i] dm[i]| into [0.5, 1) (1 for a zero column), and the column's equilibrated values
+// max_i |M[c][i] dm[i]| into [0.5, 1) (column_scale), and the column's equilibrated values
 // x_i = M[c][i] dm[i] s_c split into FP16 hi = fp16(x) and lo = fp16(x - hi) (zero beyond L): the
 // B operand of the F16X3 M2L, split once per evaluation instead of once per tile.  Layout
 // [column][K step][hi 32 | lo 32]: the hi and lo halves of one K step share a 128-byte line.
 // A wave per column, lane j owning the 8 coefficients [8j, 8j + 8) (Kp <= 8 * 64): two 16-byte
 // loads, a maximum over the wave, two 16-byte stores; the waves of a capped grid stride over the
-// columns and keep their lanes' dm in registers.
+// columns and keep their lanes' dm in registers.  Column ncols is written as zeros.
 __global__ __launch_bounds__(256) void k_split_columns(const float* __restrict__ M, int ncols, int L, int Lp, int Kp,
                                                        const float* __restrict__ dm, float* __restrict__ scale,
                                                        _Float16* __restrict__ hl,
@@ -773,7 +864,12 @@ __global__ __launch_bounds__(256) void k_split_columns(const float* __restrict__
     float d[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) d[e] = act && i0 + e < L ? dm[i0 + e] : 0.0f;
-    for (int c = blockIdx.x * 4 + (threadIdx.x >> 6); c < ncols; c += gridDim.x * 4) {
+    for (int c = blockIdx.x * 4 + (threadIdx.x >> 6); c <= ncols; c += gridDim.x * 4) {
+        if (c == ncols) {   // the column of zeros
+            _Float16* z = hl + (size_t)c * 2 * Kp + off;
+            if (act) *(half8*)z = *(half8*)(z + 32) = half8{0, 0, 0, 0, 0, 0, 0, 0};
+            break;
+        }
         if (skip_first_child) {   // leaves with points: split by the P2M already
             const int node = c / 3;
             if (skip_first_child[node] < 0 && skip_npts[node] > 0) continue;
@@ -789,7 +885,7 @@ __global__ __launch_bounds__(256) void k_split_columns(const float* __restrict__
             for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(x[e]));
         }
         for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        const float sc = mx > 0.0f ? exp2f((float)(-(ilogbf(mx) + 1))) : 1.0f;
+        const float sc = column_scale(mx);
         if (lane == 0) scale[c] = sc;
         if (act) {
             half8 h, l;
@@ -811,7 +907,7 @@ void split_columns(const float* M, int ncols, int L, int Lp, int Kp, const float
     if (ncols <= 0) return;
     if (Kp > 8 * 64 || Kp % 32 || Lp % 8 || Kp > Lp) throw Error(4, "FP16 split: column length out of range");
     if (!skip_first_child != !skip_npts) throw Error(1, "FP16 split: node flags come in pairs");
-    const int grid = std::min((ncols + 3) / 4, 8 * num_cus());
+    const int grid = std::min((ncols + 4) / 4, 8 * num_cus());
     k_split_columns<<<grid, 256, 0, st>>>(M, ncols, L, Lp, Kp, dm, scale, hl, skip_first_child, skip_npts);
     FMM_HIP(hipGetLastError());
 }
@@ -823,46 +919,77 @@ bool m2l_f16x3_persistent(int L) {
 }
 int m2l_f16_kpad(int L) { return 32 * ((L + 31) / 32); }
 
-// 128-column tiles: the double-buffered 2 x 2 kernel where the single-buffered one's
-// accumulators leave one workgroup per CU anyway (R >= 224, p >= 13) and its two LDS buffers fit
-// (R <= 368, p <= 18); the single-buffered kernel (two or more workgroups per CU below) otherwise
-template <int NB, int NKS>
-static void launch_f16x3_128(int ntiles, const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv,
-                             const GemmTile* d_tiles, const int* pair_src, const _Float16* src_hl,
-                             const float* cscale, float* slab, int op_base, int* queues, hipStream_t st) {
-    if constexpr (NB >= 14 && NB <= 23) {
-        // one workgroup per CU (the two LDS buffers), 8 per XCD round
-        const int grid = std::min(8 * ((ntiles + 7) / 8), 8 * ((num_cus() + 7) / 8));
-        FMM_HIP(hipMemsetAsync(queues, 0, 8 * sizeof(int), st));
-        k_gemm_m2l_f16x3_q<NB, NKS, 2><<<grid, 256, 0, st>>>(ops_hi, ops_lo, ops_rinv, d_tiles, pair_src, src_hl,
-                                                             cscale, slab, op_base, ntiles, queues);
-    }
-    else
-        k_gemm_m2l_f16x3<NB, NKS, 2><<<ntiles, 256, 0, st>>>(ops_hi, ops_lo, ops_rinv, d_tiles, pair_src, src_hl,
-                                                             cscale, slab, op_base);
+__global__ void k_sibling_scales(const int* __restrict__ parent, const int* __restrict__ first_child, int n,
+                                 const float* __restrict__ cscale, float* __restrict__ ratio,
+                                 float* __restrict__ pinv) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == n) ratio[i] = pinv[i] = 0.0f;   // the column of zeros
+    if (i >= n) return;
+    const int v = i / 3, p = parent[v];
+    float mn = cscale[i];
+    if (p >= 0)
+        for (int o = 0; o < 8; o++) mn = fminf(mn, cscale[3 * (first_child[p] + o) + (i - 3 * v)]);
+    ratio[i] = mn / cscale[i];
+    pinv[i] = 1.0f / mn;
+}
+void sibling_scales(const int* parent, const int* first_child, int nnodes, const float* cscale, float* ratio,
+                    float* pinv, hipStream_t st) {
+    if (!nnodes) return;
+    k_sibling_scales<<<blocks(3ll * nnodes + 1), 256, 0, st>>>(parent, first_child, 3 * nnodes, cscale, ratio, pinv);
+    FMM_HIP(hipGetLastError());
 }
 
-void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, int op_base,
-                    const GemmTile* d_tiles, int ntiles, int tile_cols, const int* pair_src, const _Float16* src_hl,
-                    const float* cscale, float* slab, int L, int* queues, hipStream_t st) {
-    if (ntiles == 0) return;
-    const int nb = m2l_f16_rows(L) / 16, nks = m2l_f16_kpad(L) / 32;
-    if (tile_cols != 64 && tile_cols != 128) throw Error(4, "FP16 M2L: tiles of 64 or 128 columns");
-#define FMM_F16(NBV, NKV)                                                                                            \
-    if (nb == NBV && nks == NKV) {                                                                                   \
-        if (tile_cols == 128)                                                                                        \
-            launch_f16x3_128<NBV, NKV>(ntiles, ops_hi, ops_lo, ops_rinv, d_tiles, pair_src, src_hl, cscale, slab,    \
-                                       op_base, queues, st);                                                         \
-        else                                                                                                         \
-            k_gemm_m2l_f16x3<NBV, NKV, 1><<<ntiles, 256, 0, st>>>(ops_hi, ops_lo, ops_rinv, d_tiles, pair_src,       \
-                                                                  src_hl, cscale, slab, op_base);                    \
-        FMM_HIP(hipGetLastError());                                                                                  \
-        return;                                                                                                      \
+__global__ void k_group_row_scales(const int* __restrict__ cls_ops, const int* __restrict__ cls_mask, int ncls, int R,
+                                   const float* __restrict__ ops_rinv, float* __restrict__ cls_rinv) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (long long)ncls * R) return;
+    const int c = (int)(i / R), row = (int)(i - (long long)c * R);
+    float r = 0.0f;
+    for (int m = cls_mask[c]; m; m &= m - 1)
+        r = fmaxf(r, ops_rinv[(size_t)cls_ops[8 * (size_t)c + __builtin_ctz(m)] * R + row]);
+    cls_rinv[i] = r;
+}
+void group_row_scales(FarGroups& G, const float* ops_rinv, int L, hipStream_t st) {
+    if (!G.num_classes) return;
+    const int R = m2l_f16_rows(L);
+    const size_t n = (size_t)G.num_classes * R;
+    k_group_row_scales<<<blocks((long long)n), 256, 0, st>>>(G.cls_ops.as<int>(), G.cls_mask.as<int>(), G.num_classes, R,
+                                                             ops_rinv, G.cls_rinv.get<float>(n));
+    FMM_HIP(hipGetLastError());
+}
+
+// The double-buffered 2 x 2 kernel where the single-buffered one's accumulators leave one workgroup per
+// CU anyway (R >= 224, p >= 14) and its two LDS buffers fit (R <= 368, p <= 18); the single-buffered
+// kernel (two or more workgroups per CU below) otherwise
+template <int NB, int NKS>
+static void launch_f16x3(const M2LGroupArgs& A, int* queues, hipStream_t st) {
+    if constexpr (NB >= 14 && NB <= 23) {
+        // one workgroup per CU (the two LDS buffers), 8 per XCD round
+        const int grid = std::min(8 * ((A.ntiles + 7) / 8), 8 * ((num_cus() + 7) / 8));
+        FMM_HIP(hipMemsetAsync(queues, 0, 8 * sizeof(int), st));
+        k_gemm_m2l_f16x3_q<NB, NKS, NKS % 2 ? 1 : 2><<<grid, 256, 0, st>>>(A, queues);
+    } else {
+        k_gemm_m2l_f16x3<NB, NKS><<<A.ntiles, 256, 0, st>>>(A);
     }
-    FMM_F16(1, 1) FMM_F16(2, 1) FMM_F16(3, 2) FMM_F16(4, 2) FMM_F16(4, 3) FMM_F16(5, 3) FMM_F16(6, 3) FMM_F16(7, 4)
-    FMM_F16(8, 4) FMM_F16(9, 5) FMM_F16(10, 5) FMM_F16(11, 6) FMM_F16(12, 6) FMM_F16(13, 7) FMM_F16(14, 7)
-    FMM_F16(15, 8) FMM_F16(16, 8) FMM_F16(17, 9) FMM_F16(18, 9) FMM_F16(19, 10) FMM_F16(20, 10) FMM_F16(21, 11)
-    FMM_F16(22, 11) FMM_F16(23, 12) FMM_F16(24, 12) FMM_F16(25, 13) FMM_F16(26, 13) FMM_F16(27, 14) FMM_F16(28, 14)
+}
+
+void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, const FarGroups& G,
+                    const _Float16* src_hl, const float* ratio, const float* pinv, int zero_col, float* slab, int L,
+                    int* queues, hipStream_t st) {
+    if (!G.num_tiles) return;
+    const M2LGroupArgs A{ops_hi, ops_lo, ops_rinv, G.tiles.as<GroupTile>(), G.cls_ops.as<int>(), G.cls_rinv.as<float>(),
+                         G.fc.as<int>(), G.mask.as<int>(), src_hl, ratio, pinv, slab, G.num_tiles, zero_col};
+    const int nb = m2l_f16_rows(L) / 16, nks = m2l_f16_kpad(L) / 32;
+    // the row and K counts of the orders 1 .. 20
+#define FMM_F16(NBV, NKV)                                      \
+    if (nb == NBV && nks == NKV) {                             \
+        launch_f16x3<NBV, NKV>(A, queues, st);                 \
+        FMM_HIP(hipGetLastError());                            \
+        return;                                                \
+    }
+    FMM_F16(1, 1) FMM_F16(2, 1) FMM_F16(3, 2) FMM_F16(4, 2) FMM_F16(6, 3) FMM_F16(7, 4) FMM_F16(8, 4) FMM_F16(9, 5)
+    FMM_F16(11, 6) FMM_F16(13, 7) FMM_F16(15, 8) FMM_F16(16, 8) FMM_F16(19, 10) FMM_F16(21, 11) FMM_F16(23, 12)
+    FMM_F16(25, 13) FMM_F16(28, 14)
 #undef FMM_F16
     throw Error(4, "FP16 M2L: no kernel instance for this order");
 }
@@ -1015,20 +1142,14 @@ static int key_bits(int nnodes) {
     return b;
 }
 
-void build_pair_index(const int* key, int npairs, int nnodes, PairIndex& ix, hipStream_t st) {
+void index_sorted_pairs(const int* key, int npairs, int nnodes, PairIndex& ix, hipStream_t st) {
     ix.npairs = npairs;
     ix.nnodes = nnodes;
     int* b = ix.begin.get<int>(std::max(nnodes, 1));
     int* e = ix.end.get<int>(std::max(nnodes, 1));
     if (nnodes) k_zero_ranges<<<blocks(nnodes), 256, 0, st>>>(b, e, nnodes);
     if (!npairs) return;
-    int* io = ix.iota.get<int>(npairs);
-    k_iota<<<blocks(npairs), 256, 0, st>>>(io, npairs);
-    uint32_t* ks = ix.keys_sorted.get<uint32_t>(npairs);
-    int* ord = ix.order.get<int>(npairs);
-    // stable radix sort: pairs of one node stay in ascending pair order
-    sort_pairs_u32((const uint32_t*)key, ks, io, ord, npairs, key_bits(nnodes), ix.tmp, st);
-    k_key_ranges<<<blocks(npairs), 256, 0, st>>>(ks, npairs, b, e);
+    k_key_ranges<<<blocks(npairs), 256, 0, st>>>((const uint32_t*)key, npairs, b, e);
     // segments of at most PAIR_SEGMENT pairs per node, numbered node by node
     uint32_t* cnt = ix.seg_count.get<uint32_t>(nnodes + 1);
     uint32_t* off = ix.seg_off.get<uint32_t>(nnodes + 1);
@@ -1037,6 +1158,18 @@ void build_pair_index(const int* key, int npairs, int nnodes, PairIndex& ix, hip
     ix.max_segments = npairs / PAIR_SEGMENT + std::min(npairs, nnodes);
     k_segment_nodes<<<blocks(nnodes), 256, 0, st>>>(off, nnodes, ix.seg_node.get<int>(ix.max_segments));
     FMM_HIP(hipGetLastError());
+}
+
+void build_pair_index(const int* key, int npairs, int nnodes, PairIndex& ix, hipStream_t st) {
+    uint32_t* ks = nullptr;
+    if (npairs) {
+        int* io = ix.iota.get<int>(npairs);
+        k_iota<<<blocks(npairs), 256, 0, st>>>(io, npairs);
+        ks = ix.keys_sorted.get<uint32_t>(npairs);
+        // stable radix sort: pairs of one node stay in ascending pair order
+        sort_pairs_u32((const uint32_t*)key, ks, io, ix.order.get<int>(npairs), npairs, key_bits(nnodes), ix.tmp, st);
+    }
+    index_sorted_pairs((const int*)ks, npairs, nnodes, ix, st);
 }
 
 // Two passes, so that nodes with hundreds of pairs do not serialise the launch: (1) one wave

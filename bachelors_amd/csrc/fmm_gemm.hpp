@@ -43,6 +43,8 @@ struct PairIndex {
     DevBuf keys, keys_sorted, iota, order, begin, end, tmp, seg_count, seg_off, seg_node, partial;
 };
 void build_pair_index(const int* key, int npairs, int nnodes, PairIndex& ix, hipStream_t st);
+// the same with ix.order given and key sorted: node v receives order[k] for the k with key[k] = v
+void index_sorted_pairs(const int* key, int npairs, int nnodes, PairIndex& ix, hipStream_t st);
 
 // out[v][c][0 .. R) = sum over the pairs of v, in ascending pair order, of slab[pair][c][0 .. R),
 // out[v][c][R .. Lp) = 0, for every node v < ix.nnodes (written, not added: nothing needs to clear
@@ -61,21 +63,33 @@ void m2l_gemm(Precision prec, const void* ops, const void* ops_lo, const GemmTil
 // F16X3 M2L (FP16 split products on MFMA, equilibrated by powers of 2): operator rows
 // m2l_f16_rows(L), K padded to Kp = m2l_f16_kpad(L); the multipoles enter split by split_columns
 // (src_hl [node * 3 + comp][Kp / 32][hi 32 | lo 32], equilibrated by dm[>= Kp], the per-coefficient
-// scales the tables were built with, and by cscale[node * 3 + comp]); the slab rows are
-// m2l_f16_rows(L) long.  Tile operator k is table entry k - op_base; tiles hold at most tile_cols
-// (64 or 128) columns.  queues: 8 device ints, the per-XCD tile counters of the persistent kernel.
+// scales the tables were built with, and by cscale[node * 3 + comp]).
+// The column scale: the power of 2 that brings the column's largest value mx into [0.5, 1); 2^126, which
+// never is the smallest scale among siblings, for a column of zeros
+__device__ __forceinline__ float column_scale(float mx) {
+    return mx > 0.0f ? exp2f((float)min(-(ilogbf(mx) + 1), 126)) : 0x1p126f;
+}
 int m2l_f16_rows(int L);
 // whether the F16X3 M2L of order (L = (p + 1)^2) runs as the persistent one-workgroup-per-CU kernel
 // (128-column tiles) that leaves room for a near-field workgroup per CU
 bool m2l_f16x3_persistent(int L);
 int m2l_f16_kpad(int L);
 // skip_first_child / skip_npts (per node, both or neither): columns of leaves with points are
-// left as they are (the P2M writes them, see launch_p2m)
+// left as they are (the P2M writes them, see launch_p2m); column ncols is set to zeros
 void split_columns(const float* M, int ncols, int L, int Lp, int Kp, const float* dm, float* scale, _Float16* hl,
                    hipStream_t st, const int* skip_first_child = nullptr, const int* skip_npts = nullptr);
-void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, int op_base,
-                    const GemmTile* d_tiles, int ntiles, int tile_cols, const int* pair_src, const _Float16* src_hl,
-                    const float* cscale, float* slab, int L, int* queues, hipStream_t st);
+// per column: ratio = (smallest column scale of the node's siblings) / (its own), a power of 2 <= 1, and
+// pinv = 1 / that smallest scale (the same for all siblings), by which a group's sum is scaled back;
+// both have an entry 3 nnodes for the column of zeros
+void sibling_scales(const int* parent, const int* first_child, int nnodes, const float* cscale, float* ratio,
+                    float* pinv, hipStream_t st);
+// The M2L of all groups of far pairs (fmm_groups.hpp): slab[3 * group + comp][m2l_f16_rows(L)] = the sum
+// over the group's children.  queues: 8 device ints, the per-XCD tile counters of the persistent kernel.
+struct FarGroups;
+void group_row_scales(FarGroups& G, const float* ops_rinv, int L, hipStream_t st);
+void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, const FarGroups& G,
+                    const _Float16* src_hl, const float* ratio, const float* pinv, int zero_col, float* slab, int L,
+                    int* queues, hipStream_t st);
 
 // tiles of at most width columns (default 64) over the classes' columns 3 * class_begin
 void plan_tiles(const std::vector<int>& class_begin, const std::vector<int>& class_op, std::vector<GemmTile>& tiles,

@@ -411,6 +411,7 @@ void build_lists(Lists& out, ListScratch& L, const TreeDev& S, const TreeDev& T,
             out.num_far = nfar;
             // classes
             out.num_classes = 0;
+            out.wide = false;
             out.h_class_begin.clear();
             if (nfar > 0 && classes) {
                 uint32_t* flag = L.flag.get<uint32_t>(nfar);
@@ -425,6 +426,7 @@ void build_lists(Lists& out, ListScratch& L, const TreeDev& S, const TreeDev& T,
                 if (hc[1] & ERR_LATTICE)
                     throw Error(4, "interaction offset off the box lattice (the shared frame needs lattice-aligned boxes)");
                 if (hc[1] & ERR_RANGE) {
+                    out.wide = true;
                     // offsets or level differences beyond the compact code (deep, strongly adaptive
                     // trees): classes by the wide code, sorted in two stable passes (by target, then
                     // by code), so the order is still (class, target)

@@ -21,6 +21,7 @@ struct Lists {
     DevBuf far_t, far_s, far_code;          // int, int, uint32 class code
     DevBuf class_begin;                     // int[num_classes]
     std::vector<int> h_class_begin;         // num_classes + 1
+    bool wide = false;                      // classes keyed by the wide code
     DevBuf close_t, close_s;                // int
     DevBuf close_begin, close_end;          // per target node
 };
