@@ -168,7 +168,7 @@ struct fmm_ctx {
     // multipole column scales; down_l2l = L2L operators ahead of the M2L ones in the down tables
     DevBuf dm, m2l_hi, m2l_lo, m2l_rinv, m2l_work, cscale, Mhl;   // Mhl: split multipoles (hi | lo)
     DevBuf cratio, cpinv;                        // column scales against the siblings' smallest, and 1 / that
-    DevBuf queues;   // work counters: [0, 8) the M2L GEMM's per-XCD tiles, [8] the near-field leaves
+    DevBuf queues;   // work counters: [0, 8) the M2L GEMM's per-XCD tiles, [8] the near-field leaves; [14, 16) probe
     int down_l2l = 0;
     const OpSpec* down_specs = nullptr;          // device specs of the down tables
     DevBuf m2l_slab;                             // M2L result per (pair or group, component)
@@ -188,6 +188,7 @@ struct fmm_ctx {
                j_start = nullptr, j_tables = nullptr,   // j_tables: everything the side stream builds for M2L
                j_src = nullptr, j_tgt = nullptr,        // source tree on the main / target side on the side stream
                j_caller = nullptr;                      // the caller's default-stream work before a _dev read
+    bool side_checked = false;   // the side stream was seen to run beside the main one (or none does)
     long long near_inter = -1;
     bool lists_ready = false;
     bool leaves_split = false;   // F16X3: the last P2M also wrote its leaves' split M2L columns
@@ -767,7 +768,7 @@ void translate_gemm(fmm_ctx* c, hipEvent_t gemm_after = nullptr, bool split_done
     const int R = m2l_slab_rows(c->prec, c->L, c->Lp);
     if (f16) {
         group_row_scales(c->groups, c->m2l_rinv.as<float>(), c->L, st);
-        FMM_HIP(hipMemsetAsync(c->queues.as<int>() + 8, 0, sizeof(int), st));   // the near field's leaves
+        FMM_HIP(hipMemsetAsync(c->queues.as<int>(), 0, 9 * sizeof(int), st));   // tiles, the near field's leaves
     }
     c->rec(E_GEMM0);
     if (P.npairs && f16) {
@@ -856,7 +857,8 @@ __global__ void k_fill_nan(double* p, size_t n) {
 void p2p_from_queue(fmm_ctx* c, hipStream_t ps, int grid, bool beside) {
     launch_p2p_queue(c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S, c->lists.close_begin.as<int>(),
                      c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->nP0.ptr, c->nP1.ptr, c->nP2.ptr,
-                     c->txyz.as<double>(), c->Bnear.as<double>(), c->queues.as<int>() + 8, grid, beside, ps);
+                     c->txyz.as<double>(), c->Bnear.as<double>(), c->queues.as<int>() + 8, c->queues.as<int>(),
+                     c->groups.num_tiles, grid, beside, ps);
 }
 
 // near field on stream ps (needs the lists and the packed sources)
@@ -961,6 +963,51 @@ void direct_sum(fmm_ctx* c, bool pot, double current, size_t m, const double* xy
                   nsplit, c->stream);
 }
 
+// Waits for *flag (set by k_probe_set on another stream) and says whether it came; gives up after
+// PROBE_TICKS of the constant 100 MHz clock, so the wait ends in any case.
+constexpr long long PROBE_TICKS = 20000;   // 200 us: a launch on an idle queue takes some 10
+__global__ void k_probe_wait(const int* flag, int* seen) {
+    const long long t0 = wall_clock64();
+    int v;
+    do v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (!v && wall_clock64() - t0 < PROBE_TICKS);
+    *seen = v;
+}
+__global__ void k_probe_set(int* flag) { __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// The fused evaluation lives on its two streams running at the same time, but the runtime maps all streams
+// of a process to a few hardware queues, and streams that share one run one after the other: of three
+// contexts alive at once one took 43.9 instead of 28.5 ms per evaluation of the 4M shells.  Before a
+// context's first fused evaluation (and after a change of its main stream) a kernel on the main stream
+// waits, for a bounded time, for one on the side stream; if it waits in vain another side stream is
+// tried, a few times, the failed ones held until then so that their queues are not handed out again.
+void check_side_stream(fmm_ctx* c) {
+    if (c->side_checked) return;
+    int* d = c->queues.as<int>() + 14;   // flag, seen
+    std::vector<hipStream_t> failed;
+    for (int attempt = 0; attempt < 4; attempt++) {
+        if (attempt) {
+            failed.push_back(c->side);
+            c->side = nullptr;
+            FMM_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+        }
+        k_probe_set<<<1, 1, 0, c->side>>>(d + 1);   // the streams' first launches set up their queues
+        FMM_HIP(hipStreamSynchronize(c->side));
+        FMM_HIP(hipMemsetAsync(d, 0, 2 * sizeof(int), c->stream));
+        FMM_HIP(hipStreamSynchronize(c->stream));
+        k_probe_wait<<<1, 1, 0, c->stream>>>(d, d + 1);
+        k_probe_set<<<1, 1, 0, c->side>>>(d);
+        FMM_HIP(hipGetLastError());
+        int seen = 0;
+        FMM_HIP(hipMemcpyAsync(&seen, d + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        FMM_HIP(hipStreamSynchronize(c->stream));
+        FMM_HIP(hipStreamSynchronize(c->side));
+        if (seen) break;
+    }
+    for (hipStream_t s : failed) FMM_HIP(hipStreamDestroy(s));
+    c->side_checked = true;
+}
+
 // The whole evaluation with the side stream: the lists are built (on a host thread, since
 // their compaction reads counts back) while P2M and M2M run, and the near field runs beside the
 // M2L GEMM (persistent F16X3 GEMM) or after it, beside the memory-bound slab reduction, L2L and
@@ -975,6 +1022,7 @@ void run_fused(fmm_ctx* c, double current, double* Bdev) {
         stage_evaluate(c, current, Bdev);
         return;
     }
+    check_side_stream(c);
     hipStream_t A = c->stream, Bs = c->side;
     // Side thread (stream Bs): target tree, targets in slot order, then -- once the source tree
     // is built -- the far lists (E_FAR), the close lists and the pair index (j_lists).  This
@@ -1242,6 +1290,7 @@ const char* fmm_last_error(const fmm_ctx* c) { return c ? c->err.c_str() : "null
 int fmm_set_stream(fmm_ctx* c, void* s) {
     return guard(c, [&] {
         FMM_HIP(hipStreamSynchronize(c->stream));
+        c->side_checked = false;
         if (s) {
             if (c->own_stream) FMM_HIP(hipStreamDestroy(c->stream));
             c->own_stream = false;

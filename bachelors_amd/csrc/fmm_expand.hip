@@ -596,9 +596,13 @@ __global__ __launch_bounds__(256) void k_p2p_transposed(
 // The same near field as a persistent grid taking leaves from a queue (an atomic counter that starts at
 // 0), two forms of which may share a queue: BESIDE with a register budget of 56 per lane (no unrolling),
 // one workgroup of which fits on a CU beside the F16X3 M2L GEMM's, so the near field runs on the VALU
-// slots the GEMM leaves idle, and the plain one for the leaves left when the GEMM is done.
+// slots the GEMM leaves idle, and the plain one for the leaves left when the GEMM is done.  A BESIDE
+// workgroup that starts when the GEMM's tiles are all taken (their streams share a hardware queue and
+// run one after the other) leaves the leaves to the other form: one workgroup per CU alone takes 25 ms
+// for the 7 ms of near field of the 4M shells.
 template <class R, bool POT, bool BESIDE>
 __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, int nleaves, int* __restrict__ queue,
+                                               const int* __restrict__ gemm_queues, int gemm_tiles,
                                                const int* __restrict__ tbegin, const int* __restrict__ tend,
                                                const int* __restrict__ close_begin, const int* __restrict__ close_end,
                                                const int* __restrict__ close_s, const double* __restrict__ origin,
@@ -611,6 +615,19 @@ __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, i
     __shared__ R s2[4][64];
     __shared__ double red[4][3][64];
     __shared__ int next;
+    if (BESIDE) {
+        if (threadIdx.x == 0) {
+            int left = 0;   // tiles of the XCDs' eighths not yet taken
+            for (int x = 0; x < 8; x++)
+                left += max(0, (gemm_tiles >> 3) + (x < (gemm_tiles & 7) ? 1 : 0) -
+                                   __hip_atomic_load(gemm_queues + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            next = left;
+        }
+        __syncthreads();
+        const bool gone = next == 0;
+        __syncthreads();
+        if (gone) return;
+    }
     for (;;) {
         if (threadIdx.x == 0) next = atomicAdd(queue, 1);
         __syncthreads();
@@ -623,22 +640,24 @@ __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, i
 }
 template <class R, bool POT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(10))) void k_p2p_queue(
-    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ tbegin,
+    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ gemm_queues,
+    int gemm_tiles, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
     const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
     const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
     const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
-    p2p_queue_body<R, POT, true>(leaves, nleaves, queue, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+    p2p_queue_body<R, POT, true>(leaves, nleaves, queue, gemm_queues, gemm_tiles, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
                                  send, P0, P1, P2, txyz, Bnear);
 }
 template <class R, bool POT>
 __global__ __launch_bounds__(256) void k_p2p_queue_rest(
-    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ tbegin,
+    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ gemm_queues,
+    int gemm_tiles, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
     const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
     const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
     const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
-    p2p_queue_body<R, POT, false>(leaves, nleaves, queue, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+    p2p_queue_body<R, POT, false>(leaves, nleaves, queue, gemm_queues, gemm_tiles, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
                                   send, P0, P1, P2, txyz, Bnear);
 }
 
@@ -1052,11 +1071,12 @@ void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, cons
 }
 void launch_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                       const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                      const double* txyz, double* Bnear, int* queue, int grid, bool beside, hipStream_t st) {
+                      const double* txyz, double* Bnear, int* queue, const int* gemm_queues, int gemm_tiles, int grid,
+                      bool beside, hipStream_t st) {
     if (!nleaves) return;
     if (grid < 1) throw Error(1, "near field: empty persistent grid");
     (beside ? k_p2p_queue<float, false> : k_p2p_queue_rest<float, false>)<<<grid, 256, 0, st>>>(
-        leaves, nleaves, queue, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
+        leaves, nleaves, queue, gemm_queues, gemm_tiles, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
         S.center.as<double>(), S.begin.as<int>(), S.end.as<int>(), (const float4*)P0, (const float4*)P1,
         (const float*)P2, txyz, Bnear);
     FMM_HIP(hipGetLastError());

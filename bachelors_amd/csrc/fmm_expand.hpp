@@ -30,10 +30,11 @@ void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, cons
                 const double* txyz, double* Bnear, hipStream_t st);
 // launch_p2p in FP32 as a persistent grid of `grid` workgroups taking leaves from the counter *queue (0
 // at the start; several grids may share it); beside: with a small register budget that lets a workgroup
-// share its CU with one of the M2L GEMM's
+// share its CU with one of the M2L GEMM's, whose tile counters and tiles are given
 void launch_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                       const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                      const double* txyz, double* Bnear, int* queue, int grid, bool beside, hipStream_t st);
+                      const double* txyz, double* Bnear, int* queue, const int* gemm_queues, int gemm_tiles, int grid,
+                      bool beside, hipStream_t st);
 // the transposed near field at the sources (slot order, written whole for the leaves given): the
 // targets are packed by launch_pack_sources with their strengths, relative to the same origin (the
 // source root's centre); close_begin / close_end / close_t: the close targets of every source node

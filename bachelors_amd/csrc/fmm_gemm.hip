@@ -966,7 +966,6 @@ static void launch_f16x3(const M2LGroupArgs& A, int* queues, hipStream_t st) {
     if constexpr (NB >= 14 && NB <= 23) {
         // one workgroup per CU (the two LDS buffers), 8 per XCD round
         const int grid = std::min(8 * ((A.ntiles + 7) / 8), 8 * ((num_cus() + 7) / 8));
-        FMM_HIP(hipMemsetAsync(queues, 0, 8 * sizeof(int), st));
         k_gemm_m2l_f16x3_q<NB, NKS, NKS % 2 ? 1 : 2><<<grid, 256, 0, st>>>(A, queues);
     } else {
         k_gemm_m2l_f16x3<NB, NKS><<<A.ntiles, 256, 0, st>>>(A);

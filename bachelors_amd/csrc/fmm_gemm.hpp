@@ -84,7 +84,8 @@ void split_columns(const float* M, int ncols, int L, int Lp, int Kp, const float
 void sibling_scales(const int* parent, const int* first_child, int nnodes, const float* cscale, float* ratio,
                     float* pinv, hipStream_t st);
 // The M2L of all groups of far pairs (fmm_groups.hpp): slab[3 * group + comp][m2l_f16_rows(L)] = the sum
-// over the group's children.  queues: 8 device ints, the per-XCD tile counters of the persistent kernel.
+// over the group's children.  queues: 8 device ints, the per-XCD tile counters of the persistent kernel
+// (0 at the launch).
 struct FarGroups;
 void group_row_scales(FarGroups& G, const float* ops_rinv, int L, hipStream_t st);
 void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, const FarGroups& G,
