@@ -313,3 +313,31 @@ def test_fused_run_matches_staged_run(fm, precision, tol):
         F.run_B_dev(1.0, out.data_ptr())
         F.synchronize()
         assert rel_l2(out.cpu().numpy(), B_staged) < tol
+
+
+@pytest.mark.parametrize("nt", [1, 255, 257, 32767, 32768, 70001])
+def test_target_extent_on_device_equals_host(fm, nt):
+    """The target tree of the reference frame (root = the targets' bounding box) is the same from a host
+    array (extent by the host loop below 32,768 points) and from a device pointer (extent by a kernel),
+    bit for bit, with NaN coordinates and coordinates of one sign among the targets."""
+    import ctypes
+
+    import torch
+    rng = np.random.default_rng(nt)
+    tgt = rng.uniform(0.5, 2, (nt, 3)) * [1, -1, 1]
+    if nt > 300:
+        tgt[rng.integers(1, nt, 5), rng.integers(0, 3, 5)] = np.nan
+    trees = []
+    d = torch.from_numpy(tgt).cuda()
+    for dev in (False, True):
+        F = fm.FMM(order=2, source_leaf_capacity=8, target_leaf_capacity=50)
+        F.set_sources(np.array([[1.0, 0.0, 0.0]]), np.array([1.0]))
+        if dev:
+            F.set_targets_dev(nt, ctypes.c_void_p(d.data_ptr()))
+        else:
+            F.set_targets(tgt)
+        F.build_trees()
+        trees.append(F.tree(1))
+        F.close()
+    for k in trees[0]:
+        assert np.array_equal(trees[0][k], trees[1][k]), k
