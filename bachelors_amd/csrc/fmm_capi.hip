@@ -177,6 +177,7 @@ struct fmm_ctx {
     // evaluation
     DevBuf Bfar, Bnear, Bout;
     DevBuf Afar, Anear, Aout;                    // vector potential (calcA)
+    TreecodeScratch tc_scratch;
     DevBuf direct_part, pts, tc_B, tc_A;         // direct-sum partials; host query points and results
     double current = 1.0;
     // adjoint state
@@ -952,8 +953,8 @@ void stage_treecode(fmm_ctx* c, double current, size_t m, const double* xyz, dou
     require(c->stage >= ST_UP, FMM_ERR_STATE, "Multipoles are not ready!");
     require(m < (size_t)INT32_MAX / 3, FMM_ERR_LIMIT, "too many points");
     require(m == 0 || xyz, FMM_ERR_ARG, "null point array");
-    launch_treecode_points(c->f64(), c->S, c->sigS, c->M.ptr, c->p, c->Lp, xyz, (int)m,
-                           current * REF_MU0 / (4.0 * REF_PI), current / (4.0 * REF_PI), B, A, c->stream);
+    launch_treecode_points(c->f64(), c->S, c->sigS, c->M.ptr, c->p, c->Lp, c->cfg.source_root_center, xyz, (int)m,
+                           current * REF_MU0 / (4.0 * REF_PI), current / (4.0 * REF_PI), B, A, c->tc_scratch, c->stream);
 }
 
 // FP64 direct sum of B (pot: A) at m device targets into out, partial sums in part (nsplit *
