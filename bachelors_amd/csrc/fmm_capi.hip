@@ -161,7 +161,6 @@ struct fmm_ctx {
     // their launch data; operator specs go first in a copy of their own, so the table kernels
     // run while the host plans the passes
     Staging up_specs, up_stage, down_stage, m2l_specs, m2l_stage, adj_stage;
-    DevBuf pp_tiles;                             // per-pair path: tiles of one chunk
     Lists lists;
     ListScratch lscr;
     PairIndex m2l_ix;                            // far pairs (F16X3: their groups) by target node
@@ -584,35 +583,9 @@ void stage_upward(fmm_ctx* c, int alg = FMM_M2M_MATRICES) {
     c->stage = ST_UP;
 }
 
-// Reference frame: every M2L and L2L translation vector is unique (bounding-box target
-// root, float-rounded centres), so operators are built per pair, in chunks, and applied
-// with the same GEMM kernels (one 3-column tile per pair).  A correctness path: the
-// shared frame is the fast one.
-void run_per_pair(fmm_ctx* c, int kind, const int* d_src, const int* d_dst, int npairs, const TreeDev& Tsrc,
-                  const TreeDev& Tdst, const ScaleTable& sg_src, const ScaleTable& sg_dst, const void* src_exp,
-                  void* dst_exp, bool atomic) {
-    hipStream_t st = c->stream;
-    OpTables& O = c->down_ops;
-    const size_t per = (size_t)c->Lp * c->Lp * sizeof(double);
-    int chunk = (int)std::max<size_t>(1, ((size_t)256 << 20) / per);
-    std::vector<GemmTile> tiles;
-    for (int b = 0; b < npairs; b += chunk) {
-        int n = std::min(chunk, npairs - b);
-        OpSpec* sp = O.specs.get<OpSpec>(n);
-        make_pair_specs(d_src + b, d_dst + b, n, Tsrc.center.as<double>(), Tdst.center.as<double>(),
-                        Tsrc.level.as<int>(), Tdst.level.as<int>(), sg_src, sg_dst, kind, c->cfg.m2l_full, sp, st);
-        O.nops = n;
-        build_tables(c, O, sp, st);
-        tiles.resize(n);
-        for (int i = 0; i < n; i++) tiles[i] = GemmTile{i, 3 * (b + i), 3};
-        GemmTile* dt = c->pp_tiles.get<GemmTile>(n);
-        FMM_HIP(hipMemcpyAsync(dt, tiles.data(), n * sizeof(GemmTile), hipMemcpyHostToDevice, st));
-        class_gemm(c->pass_prec(), ops_ptr(c, O), O.lo.ptr, dt, n, d_src, d_dst, src_exp, dst_exp, c->Lp,
-                   atomic ? EPI_ATOMIC : EPI_ADD, st, false, 1, kind == OPK_L2L ? TRI_UPPER : TRI_NONE);
-        FMM_HIP(hipStreamSynchronize(st));   // the chunk buffers are reused
-    }
-}
-
+// Reference frame: every M2L and L2L translation vector is unique (bounding-box target root,
+// float-rounded centres), so no operator is shared and the translations are applied pair by pair
+// (translate_pairs).  The shared frame is the fast one.
 void downward_per_pair(fmm_ctx* c) {
     hipStream_t st = c->stream;
     const TreeDev& S = c->S;
@@ -621,8 +594,8 @@ void downward_per_pair(fmm_ctx* c) {
     void* Lx = c->Lx.reserve(n * c->esize());
     FMM_HIP(hipMemsetAsync(Lx, 0, n * c->esize(), st));
     c->rec(E_TABLES);
-    run_per_pair(c, OPK_M2L, c->lists.far_s.as<int>(), c->lists.far_t.as<int>(), c->lists.num_far, S, T, c->sigS,
-                 c->sigT, c->M.ptr, Lx, true);
+    translate_pairs(OPK_M2L, c->f64(), c->lists.far_s.as<int>(), c->lists.far_t.as<int>(), c->lists.num_far, S, T,
+                    c->sigS, c->sigT, c->p, c->cfg.m2l_full, c->Lp, c->M.ptr, Lx, st);
     c->rec(E_M2L);
     // L2L with each child's exact translation (calculation_point_octree.cpp:277-299)
     Staging& sg = c->down_stage;
@@ -644,7 +617,7 @@ void downward_per_pair(fmm_ctx* c) {
         resolve_pass(P, dev);
         P.ntiles = 0;   // per-pair operators: this pass has no shared tiles (no adjoint)
         if (P.npairs)
-            run_per_pair(c, OPK_L2L, P.src, P.dst, P.npairs, T, T, c->sigT, c->sigT, Lx, Lx, false);
+            translate_pairs(OPK_L2L, c->f64(), P.src, P.dst, P.npairs, T, T, c->sigT, c->sigT, c->p, 0, c->Lp, Lx, Lx, st);
     }
     c->down_ops.nops = 0;
     c->m2l_pass = Pass();

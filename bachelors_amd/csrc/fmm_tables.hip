@@ -521,24 +521,6 @@ void make_m2l_specs(const int* class_begin, int nc, const int* far_t, const int*
 
 namespace fmm {
 
-// one operator per (src, dst) node pair: t = c_src - c_dst (M2L: source - target,
-// L2L: parent - child, M2M: child - parent)
-__global__ void k_pair_specs(const int* __restrict__ src, const int* __restrict__ dst, int n,
-                             const double* __restrict__ csrc, const double* __restrict__ cdst,
-                             const int* __restrict__ lsrc, const int* __restrict__ ldst, ScaleTable sig_src,
-                             ScaleTable sig_dst, int kind, int m2l_full, OpSpec* __restrict__ out) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int s = src[i], d = dst[i];
-    OpSpec o;
-    for (int a = 0; a < 3; a++) o.t[a] = csrc[3 * s + a] - cdst[3 * d + a];
-    o.sig_in = sig_src.s[lsrc[s]];
-    o.sig_out = sig_dst.s[ldst[d]];
-    o.kind = kind;
-    o.m2l_full = m2l_full;
-    out[i] = o;
-}
-
 // M2M operator specs per (child level k, orientation o), as the reference builds them
 // (multipole_solver.cpp:472-534): from the first non-empty child of orientation o at level k (the
 // lowest node id, BFS order) and its parent, so the translation is the float-rounded offset of
@@ -594,11 +576,168 @@ void make_m2m_specs(const TreeDev& S, const ScaleTable& sig, const double* d_nom
     FMM_HIP(hipGetLastError());
 }
 
-void make_pair_specs(const int* src, const int* dst, int n, const double* csrc, const double* cdst, const int* lsrc,
-                     const int* ldst, const ScaleTable& sig_src, const ScaleTable& sig_dst, int kind, int m2l_full,
-                     OpSpec* out, hipStream_t st) {
-    if (n) k_pair_specs<<<(n + 255) / 256, 256, 0, st>>>(src, dst, n, csrc, cdst, lsrc, ldst, sig_src, sig_dst, kind,
-                                                         m2l_full, out);
+// Translations whose vector no other pair shares (the reference frame: bounding-box target root,
+// float-rounded centres): the complex formula applied to each pair without forming its operator.  Per
+// pair wave 0 puts the harmonics X of the translation into LDS while waves 1-3 put the source's complex
+// coefficients C(a, b), b >= 0, scaled to the target and times (-1)^a there; then thread (output
+// (l, m >= 0), part) adds X C over the input degrees a = part, part + parts, ...  With real expansions
+// C(a, -b) = conj C(a, b), so the orders b and -b share a read of C and
+//   s1 X1 C + s2 X2 conj C = ((X1 + X2).re C.re + (X2 - X1).im C.im, (X1 + X2).im C.re + (X1 - X2).re C.im)
+// with the signs in X1, X2 takes half the products; the outputs at -m are the conjugates.  That is
+//   M2L  out(l, m) += sum_{a, |b| <= a} (-1)^(b > 0 ? min(m, b) : 0) X(l + a, m - b) (-1)^a C(a, b)
+//   L2L  out(l, m) += (-1)^l sum_{a >= l, b} (-1)^(b <= 0 ? m : b <= m ? m - b : 0) X(a - l, m - b) (-1)^a C(a, b)
+// (multipole_translator.cpp:148-176, 201-232).  The arithmetic is FP64 for every precision.  An M2L
+// workgroup takes 4 consecutive pairs and keeps the sums of one destination in registers (the lists are
+// sorted by it); an L2L child has one pair, and a level of few children is a matter of latency.
+//
+// Bound by the latency of a pair's tables and sums.  An L x L operator per pair, written and read back by
+// a GEMM that used it for 3 columns, in chunks of 256 MB with a host wait each, cost 2.8 of the 6.2 ms of a
+// BEM solve (p = 10, 22 thousand far pairs); this costs 0.25 + 0.04 of 3.2 ms, and 0.04 + 0.03 of the
+// 3.85 ms (4.2 before) of the drop-in coil.
+template <int KIND, int PAIRS, class T>
+__global__ __launch_bounds__(256) void k_translate_pairs(const int* __restrict__ src, const int* __restrict__ dst,
+                                                         int npairs, const double* __restrict__ csrc,
+                                                         const double* __restrict__ cdst,
+                                                         const int* __restrict__ lsrc, const int* __restrict__ ldst,
+                                                         ScaleTable sg_src, ScaleTable sg_dst, int p, int pH, int Lp,
+                                                         const T* __restrict__ in, T* __restrict__ out) {
+    extern __shared__ cplx sh[];
+    const int NT = (p + 1) * (p + 2) / 2, nX = (pH + 1) * (pH + 2) / 2, parts = max(1, 256 / NT);
+    cplx* X = sh;              // packed (n, k >= 0), n <= pH
+    cplx* C = X + nX;          // [3][NT], packed (a, b >= 0)
+    double(*red)[6] = (double(*)[6])(C + 3 * NT);   // [256]
+    const int tid = threadIdx.x, t = tid % NT, part = tid / NT;
+    const bool act = part < parts;   // NT <= 231
+    int l = 0;
+    while ((l + 1) * (l + 2) / 2 <= t) l++;
+    const int m = t - l * (l + 1) / 2;
+    const double c = 0.70710678118654752440, r2_ = 1.41421356237309504880;
+    double acc[6] = {0, 0, 0, 0, 0, 0};   // Re, Im of the three components
+    const int i0 = blockIdx.x * PAIRS, i1 = min(npairs, i0 + PAIRS);
+    for (int i = i0; i < i1; i++) {
+        const int s = src[i], d = dst[i];
+        const double si = sg_src.s[lsrc[s]], so = sg_dst.s[ldst[d]];
+        const double ux = (csrc[3 * s] - cdst[3 * d]) / so, uy = (csrc[3 * s + 1] - cdst[3 * d + 1]) / so,
+                     uz = (csrc[3 * s + 2] - cdst[3 * d + 2]) / so;
+        const double r2 = ux * ux + uy * uy + uz * uz;
+        __syncthreads();   // the previous pair's tables are no longer read
+        if (tid < 64) {
+            if (tid <= pH) {   // column k = tid of the harmonics, pH <= 40
+                const int k = tid;
+                const double inv = 1.0 / r2;
+                cplx h = {KIND == OPK_M2L ? 1.0 / sqrt(r2) : 1.0, 0};
+                for (int q = 1; q <= k; q++)
+                    h = cscale(cmul(h, {ux, uy}), KIND == OPK_M2L ? (2.0 * q - 1) * inv : recip(2 * q));
+                cplx pm2 = {0, 0}, pm1 = h;
+                X[tri(k, k)] = cscale(h, sgn_pow(k));
+                for (int n = k + 1; n <= pH; n++) {
+                    cplx v;
+                    if (KIND == OPK_M2L)
+                        v = cscale(cadd(cscale(pm1, (2.0 * n - 1) * uz), cscale(pm2, -(double)((n - 1) * (n - 1) - k * k))),
+                                   inv);
+                    else
+                        v = cscale(cadd(cscale(pm1, (2.0 * n - 1) * uz), cscale(pm2, -r2)), recip(n * n - k * k));
+                    X[tri(n, k)] = cscale(v, sgn_pow(n));
+                    pm2 = pm1;
+                    pm1 = v;
+                }
+            }
+        } else {
+            // (sig_s / sig_t)^a for the M2L, (sig_child / sig_parent)^(a + 1) for the L2L
+            const double ratio = KIND == OPK_M2L ? si / so : so / si;
+            const T* Ms = in + (size_t)s * 3 * Lp;
+            for (int e = tid - 64; e < 3 * NT; e += 192) {
+                const int comp = e / NT, q = e - comp * NT;
+                int a = (int)((sqrtf(8.0f * q + 1.0f) - 1.0f) * 0.5f);
+                while ((a + 1) * (a + 2) / 2 <= q) a++;
+                while (a * (a + 1) / 2 > q) a--;
+                const int b = q - a * (a + 1) / 2, o = comp * Lp + a * a + a;
+                double f = sgn_pow(a), w = ratio;
+                for (int ex = KIND == OPK_M2L ? a : a + 1; ex; ex >>= 1, w *= w)
+                    if (ex & 1) f *= w;
+                C[e] = b == 0 ? cplx{f * (double)Ms[o], 0.0}
+                              : cplx{f * (c * (double)Ms[o + b]), f * (c * (double)Ms[o - b])};
+            }
+        }
+        __syncthreads();
+        if (act)
+            for (int a = KIND == OPK_M2L ? part : l + part; a <= p; a += parts) {
+                const int n = KIND == OPK_M2L ? l + a : a - l;
+                if (n > pH) break;
+                const cplx* Xn = X + n * (n + 1) / 2;
+                const cplx* Ca = C + a * (a + 1) / 2;
+                if (KIND == OPK_M2L || m <= n) {   // b = 0, where C is real
+                    cplx x = Xn[m];
+                    if (KIND == OPK_L2L && (m & 1)) x = {-x.re, -x.im};
+#pragma unroll
+                    for (int comp = 0; comp < 3; comp++) {
+                        const double v = Ca[comp * NT].re;
+                        acc[2 * comp] = __builtin_fma(x.re, v, acc[2 * comp]);
+                        acc[2 * comp + 1] = __builtin_fma(x.im, v, acc[2 * comp + 1]);
+                    }
+                }
+#pragma unroll 2
+                for (int b = 1; b <= a; b++) {
+                    const int k1 = m - b < 0 ? b - m : m - b, k2 = m + b;
+                    // an M2L has |m -+ b| <= l + a = n; an L2L has no such term beyond n
+                    const bool in1 = KIND == OPK_M2L || k1 <= n, in2 = KIND == OPK_M2L || k2 <= n;
+                    cplx x1 = Xn[in1 ? k1 : 0], x2 = Xn[in2 ? k2 : 0];
+                    const int odd1 = KIND == OPK_M2L ? min(m, b) : b <= m ? m - b : 0;
+                    const double s1 = !in1 ? 0.0 : (odd1 & 1) ? -1.0 : 1.0;
+                    const double s2 = !in2 ? 0.0 : KIND == OPK_L2L && (m & 1) ? -1.0 : 1.0;
+                    x1 = {s1 * x1.re, (m < b ? -s1 : s1) * x1.im};
+                    x2 = {s2 * x2.re, s2 * x2.im};
+                    const double pr = x1.re + x2.re, pi = x1.im + x2.im, qi = x2.im - x1.im, qr = x1.re - x2.re;
+#pragma unroll
+                    for (int comp = 0; comp < 3; comp++) {
+                        const cplx v = Ca[comp * NT + b];
+                        acc[2 * comp] = __builtin_fma(pr, v.re, __builtin_fma(qi, v.im, acc[2 * comp]));
+                        acc[2 * comp + 1] = __builtin_fma(pi, v.re, __builtin_fma(qr, v.im, acc[2 * comp + 1]));
+                    }
+                }
+            }
+        if (i + 1 < i1 && dst[i + 1] == d) continue;   // uniform over the workgroup
+        for (int e = 0; e < 6; e++) {
+            red[tid][e] = acc[e];
+            acc[e] = 0.0;
+        }
+        __syncthreads();
+        if (tid < NT) {
+            T* o = out + (size_t)d * 3 * Lp + l * l + l;
+            const double sl = KIND == OPK_L2L ? sgn_pow(l) : 1.0;
+            for (int comp = 0; comp < 3; comp++) {
+                double re = 0, im = 0;
+                for (int q = 0; q < parts; q++) {
+                    re += red[tid + q * NT][2 * comp];
+                    im += red[tid + q * NT][2 * comp + 1];
+                }
+                if (m == 0) unsafeAtomicAdd(o + comp * Lp, (T)(sl * re));
+                else {
+                    unsafeAtomicAdd(o + comp * Lp + m, (T)(sl * (r2_ * re)));
+                    unsafeAtomicAdd(o + comp * Lp - m, (T)(sl * (r2_ * im)));
+                }
+            }
+        }
+    }
+}
+
+void translate_pairs(int kind, bool f64, const int* src, const int* dst, int npairs, const TreeDev& Tsrc,
+                     const TreeDev& Tdst, const ScaleTable& sg_src, const ScaleTable& sg_dst, int p, int m2l_full,
+                     int Lp, const void* in, void* out, hipStream_t st) {
+    if (npairs <= 0) return;
+    if (p > MAX_ORDER) throw Error(4, "expansion order above 20");
+    const int pH = kind == OPK_M2L && m2l_full ? 2 * p : p, NT = (p + 1) * (p + 2) / 2;
+    const size_t lds = ((size_t)(pH + 1) * (pH + 2) / 2 + 3 * NT) * sizeof(cplx) + 256 * 6 * sizeof(double);
+    auto go = [&](auto kern, int per_wg, auto* in_, auto* out_) {
+        kern<<<(npairs + per_wg - 1) / per_wg, 256, lds, st>>>(
+            src, dst, npairs, Tsrc.center.as<double>(), Tdst.center.as<double>(), Tsrc.level.as<int>(),
+            Tdst.level.as<int>(), sg_src, sg_dst, p, pH, Lp, in_, out_);
+    };
+    if (kind == OPK_M2L && f64) go(k_translate_pairs<OPK_M2L, 4, double>, 4, (const double*)in, (double*)out);
+    else if (kind == OPK_M2L) go(k_translate_pairs<OPK_M2L, 4, float>, 4, (const float*)in, (float*)out);
+    else if (f64) go(k_translate_pairs<OPK_L2L, 1, double>, 1, (const double*)in, (double*)out);
+    else go(k_translate_pairs<OPK_L2L, 1, float>, 1, (const float*)in, (float*)out);
+    FMM_HIP(hipGetLastError());
 }
 
 }  // namespace fmm

@@ -48,8 +48,11 @@ void m2m_per_node(bool f64, const int* parents, int nparents, const TreeDev& S, 
 // node of each (the reference's choice, multipole_solver.cpp:472-534); d_nominal [(k - 1) * 8 + o][3]
 // holds the offsets used where a level has no node of an orientation
 void make_m2m_specs(const TreeDev& S, const ScaleTable& sig, const double* d_nominal, OpSpec* out, hipStream_t st);
-void make_pair_specs(const int* src, const int* dst, int n, const double* csrc, const double* cdst, const int* lsrc,
-                     const int* ldst, const ScaleTable& sig_src, const ScaleTable& sig_dst, int kind, int m2l_full,
-                     OpSpec* out, hipStream_t st);
+// One translation per pair without its operator (the reference frame, where no two pairs share one):
+// out[dst] += A(c_src - c_dst) in[src] for the three components, rows of Lp real coefficients of type
+// double (f64) or float, the arithmetic in FP64.
+void translate_pairs(int kind, bool f64, const int* src, const int* dst, int npairs, const TreeDev& Tsrc,
+                     const TreeDev& Tdst, const ScaleTable& sg_src, const ScaleTable& sg_dst, int p, int m2l_full,
+                     int Lp, const void* in, void* out, hipStream_t st);
 
 }  // namespace fmm

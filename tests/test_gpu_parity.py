@@ -298,6 +298,27 @@ def test_reference_frame_fmm_matches_oracle(fm, orc, precision, tol):
     assert rel_l2(B[ok], Bo[ok]) < tol
 
 
+@pytest.mark.parametrize("p", [1, 2, 11, 20])
+def test_reference_frame_orders_match_oracle(fm, orc, p):
+    """The per-pair translations at the smallest and largest orders (3 and 231 outputs (l, m >= 0) over
+    256 threads) and at a padded row length; M2L workgroups take 4 pairs, destinations end anywhere.  FP64
+    to 1e-10 (the oracle's 10-digit 1/sqrt 2), the 32-bit expansions to 3e-6."""
+    src, w, tgt = _inputs(14, 2000, 601)
+    R = orc.FMMRun(src, w, tgt, p=p, cap_s=32, cap_t=32, flags=orc.CORRECTED)
+    Bo = R.B_input_order(len(tgt))
+    ok = np.isfinite(Bo[:, 0])
+    for precision, tol in (("fp64", 1e-10), ("fp32", 3e-6), ("f16x3", 3e-6)):
+        print("order", p, precision, flush=True)
+        F = fm.FMM(order=p, source_leaf_capacity=32, target_leaf_capacity=32, precision=precision, frame=0)
+        F.set_sources(src, w)
+        F.set_targets(tgt)
+        B = F.run(1.0)
+        assert F.stats()["far_pairs"] > 100
+        assert np.array_equal(np.isfinite(B[:, 0]), ok)
+        assert rel_l2(B[ok], Bo[ok]) < tol
+        F.close()
+
+
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 1e-6), ("f16x3", 1e-6)])
 def test_fused_run_matches_staged_run(fm, precision, tol):
     """fmm_run_B_dev (lists and near field on a side stream) equals the stage-by-stage calls; the
