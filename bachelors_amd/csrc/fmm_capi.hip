@@ -957,8 +957,9 @@ __global__ void k_probe_set(int* flag) { __hip_atomic_store(flag, 1, __ATOMIC_RE
 // context's first fused evaluation (and after a change of its main stream) a kernel on the main stream
 // waits, for a bounded time, for one on the side stream; if it waits in vain another side stream is
 // tried, a few times, the failed ones held until then so that their queues are not handed out again.
+// The check costs 0.3 ms once, so it waits for the first evaluation of 16,384 points or more (some 1 ms).
 void check_side_stream(fmm_ctx* c) {
-    if (c->side_checked) return;
+    if (c->side_checked || (size_t)c->ns + (size_t)c->nt < 16384) return;
     int* d = c->queues.as<int>() + 14;   // flag, seen
     std::vector<hipStream_t> failed;
     for (int attempt = 0; attempt < 4; attempt++) {
@@ -1184,22 +1185,29 @@ void set_targets_common(fmm_ctx* c, size_t m, const double* xyz, hipMemcpyKind k
     if (m) FMM_HIP(hipMemcpyAsync(c->tgt_xyz.get<double>(3 * mm), xyz, 3 * m * sizeof(double), kind, c->stream));
     else c->tgt_xyz.get<double>(3);
     // target extent, once per target set (math::max / math::min, math.cpp:60-84): on the device, except
-    // for few points of a host array (below about 32,768 the launch and the wait cost more than the loop)
-    const bool on_device = m && (kind == hipMemcpyDeviceToDevice || m >= 32768);
+    // for few points, where the launch and the wait cost more than the loop over a host array (below about
+    // 32,768) or than a copy of the points to the host and the loop (below about 16,384: for 121 points in
+    // a new context 0.54 instead of 0.86 ms, most of it the stream's first launch)
+    const bool from_dev = kind == hipMemcpyDeviceToDevice;
+    const bool on_device = m >= (from_dev ? 16384u : 32768u);
     const int nb = on_device ? (int)std::min<size_t>(num_cus(), (m + 255) / 256) : 0;
-    PinnedVec<double>& h = c->h_extent;   // per workgroup: maxima xyz, minima xyz
+    PinnedVec<double>& h = c->h_extent;   // per workgroup: maxima xyz, minima xyz; or the points
     if (on_device) {
         double* part = c->extent.get<double>(6 * (size_t)nb);
         k_extent<<<nb, 256, 0, c->stream>>>(c->tgt_xyz.as<double>(), (int)m, part);
         h.resize(6 * (size_t)nb);
         FMM_HIP(hipMemcpyAsync(h.data(), part, 6 * (size_t)nb * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    } else if (from_dev && m) {
+        h.resize(3 * m);
+        FMM_HIP(hipMemcpyAsync(h.data(), xyz, 3 * m * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     }
+    const double* pts = from_dev ? h.data() : xyz;
     FMM_HIP(hipStreamSynchronize(c->stream));
     for (int a = 0; a < 3; a++) {
         double mx = -1e+16, mn = 1e+16;
         for (size_t i = 0; i < (on_device ? (size_t)nb : m); i++) {
-            const double vmax = on_device ? h[6 * i + a] : xyz[3 * i + a];
-            const double vmin = on_device ? h[6 * i + 3 + a] : xyz[3 * i + a];
+            const double vmax = on_device ? h[6 * i + a] : pts[3 * i + a];
+            const double vmin = on_device ? h[6 * i + 3 + a] : pts[3 * i + a];
             if (vmax > mx) mx = vmax;
             if (vmin < mn) mn = vmin;
         }
