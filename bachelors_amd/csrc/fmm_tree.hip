@@ -410,18 +410,10 @@ __device__ __forceinline__ int octant_of(bool sx, bool sy, bool sz) {
     return (sz ? 4 : 0) + (sx ? (sy ? 2 : 1) : (sy ? 3 : 0));
 }
 
-__global__ void k_paths(const double* __restrict__ P, int n, double3 rc, double3 rh, LevelHalves H, int depth,
-                        uint64_t* __restrict__ key, int* __restrict__ irregular, uint32_t* __restrict__ inroot) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double x = P[3 * i], y = P[3 * i + 1], z = P[3 * i + 2];
-    bool in = in_range(x, rc.x, rh.x) && in_range(y, rc.y, rh.y) && in_range(z, rc.z, rh.z);
-    inroot[i] = in ? 1u : 0u;
-    if (!in) {
-        key[i] = 0;
-        irregular[i] = 0;
-        return;
-    }
+// the octants of a point of the root down to level `depth` (level 1 in the top digit); returns the level
+// whose child is not unique (the digits from there are 0), PATH_LEVELS + 1 if there is none
+__device__ __forceinline__ int point_path(double x, double y, double z, double3 rc, const LevelHalves& H, int depth,
+                                          uint64_t& path) {
     float cx = (float)rc.x, cy = (float)rc.y, cz = (float)rc.z;
     uint64_t k = 0;
     int irr = PATH_LEVELS + 1;
@@ -444,8 +436,20 @@ __global__ void k_paths(const double* __restrict__ P, int n, double3 rc, double3
         cy = y1 ? uy : ly;
         cz = z1 ? uz : lz;
     }
+    path = k;
+    return irr;
+}
+
+__global__ void k_paths(const double* __restrict__ P, int n, double3 rc, double3 rh, LevelHalves H, int depth,
+                        uint64_t* __restrict__ key, int* __restrict__ irregular, uint32_t* __restrict__ inroot) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double x = P[3 * i], y = P[3 * i + 1], z = P[3 * i + 2];
+    bool in = in_range(x, rc.x, rh.x) && in_range(y, rc.y, rh.y) && in_range(z, rc.z, rh.z);
+    inroot[i] = in ? 1u : 0u;
+    uint64_t k = 0;
+    irregular[i] = in ? point_path(x, y, z, rc, H, depth, k) : 0;
     key[i] = k;
-    irregular[i] = irr;
 }
 
 // the root's points, compacted in input order, keyed by the top `levels` levels of their path
@@ -885,6 +889,282 @@ static bool build_from_sorted(TreeDev& T, TreeScratch& S, const K* sk, int n0, i
     return true;
 }
 
+// ---------------------------------------------------------------- small trees in one launch
+// The same tree for n <= SMALL_TREE points by one workgroup: the paths (to SHORT_LEVELS levels), a bitonic
+// sort by (path, input index) in registers, shuffles and LDS, the levels top-down with the children's
+// ranges by binary search in the sorted paths, the ranges of every node, and a second sort by (leaf, input
+// index) for the slots.  pack: header (SP_*), then the first SMALL_MIRROR entries of first_child and of
+// npts, so one copy brings the host all it needs.  What this build does not hold -- a node below the
+// paths' depth that would subdivide, a point whose child is not unique at or above its leaf, more nodes
+// than node_cap -- sets SP_FLAGS and the general build starts over.
+//
+// Such trees are a matter of latency: the general build is some 45 launches and 4 host waits (300 points:
+// 130 us a tree, half of the launches for the levels); this is one launch and one wait (20 us; 80 us at
+// 4,096 points, most of it the two sorts): an evaluation of 300 sources and 121 targets 0.53 -> 0.345 ms, a
+// BEM solve with 1,999 targets 3.2 -> 2.3 ms.
+constexpr int SMALL_TREE = 4096, SMALL_MIRROR = 2048, SMALL_IDX_BITS = 12;
+enum { SP_FLAGS = 0, SP_ROOT = 1, SP_LEVELS = 2, SP_LEVEL_BEGIN = 3, SP_HEADER = SP_LEVEL_BEGIN + MAX_LEVELS + 2 };
+
+__device__ __forceinline__ uint32_t shfl_xor_u(uint32_t v, int m) { return (uint32_t)__shfl_xor((int)v, m, 64); }
+__device__ __forceinline__ uint64_t shfl_xor_u(uint64_t v, int m) {
+    return (uint64_t)shfl_xor_u((uint32_t)(v >> 32), m) << 32 | shfl_xor_u((uint32_t)v, m);
+}
+
+// ascending bitonic sort of N (a power of 2, 256 .. 4096) values, 4 consecutive ones a thread: strides 1, 2
+// in registers, up to 128 by shuffles, the rest through xch[N].  All threads of the workgroup call it;
+// those from 4 tid >= N on hold nothing.
+template <class K> __device__ __forceinline__ void bitonic_sort(K v[4], int N, K* xch) {
+    const int e0 = 4 * threadIdx.x;
+    const bool act = e0 < N;
+    for (int k = 2; k <= N; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            if (j >= 256) {
+                __syncthreads();
+                if (act)
+                    for (int r = 0; r < 4; r++) xch[e0 + r] = v[r];
+                __syncthreads();
+                if (act)
+                    for (int r = 0; r < 4; r++) {
+                        const K o = xch[(e0 + r) ^ j];
+                        const bool lower = (((e0 + r) & j) == 0) == (((e0 + r) & k) == 0);
+                        v[r] = lower == (o < v[r]) ? o : v[r];
+                    }
+            } else if (j >= 4) {
+                for (int r = 0; r < 4; r++) {
+                    const K o = shfl_xor_u(v[r], j >> 2);
+                    const bool lower = ((e0 & j) == 0) == ((e0 & k) == 0);
+                    v[r] = lower == (o < v[r]) ? o : v[r];
+                }
+            } else if (j == 2) {
+                for (int r = 0; r < 2; r++) {
+                    const bool up = ((e0 + r) & k) == 0;
+                    const K a = v[r], b = v[r + 2];
+                    const bool swap = up == (b < a);
+                    v[r] = swap ? b : a;
+                    v[r + 2] = swap ? a : b;
+                }
+            } else {
+                for (int r = 0; r < 4; r += 2) {
+                    const bool up = ((e0 + r) & k) == 0;
+                    const K a = v[r], b = v[r + 1];
+                    const bool swap = up == (b < a);
+                    v[r] = swap ? b : a;
+                    v[r + 1] = swap ? a : b;
+                }
+            }
+        }
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(1024) void k_small_tree(const double* __restrict__ P, int n, double3 rc, double3 rh,
+                                                     LevelHalves H, int depth, int max_depth, int thr, int node_cap,
+                                                     double* __restrict__ center, int* first_child,
+                                                     int* parent, int* __restrict__ level, int* __restrict__ npts,
+                                                     int* begin, int* end, int* __restrict__ slots,
+                                                     int* __restrict__ pack) {
+    __shared__ uint64_t ks[SMALL_TREE];    // (path, input index) in sorted order; exchange buffer of the sorts
+    __shared__ uint32_t mark[SMALL_TREE];  // (leaf's begin, level) at its first point
+    __shared__ uint8_t irr[SMALL_TREE];
+    __shared__ int wsum[16], hdr[SP_HEADER], n_root, flags;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
+    int N = 256;
+    while (N < n) N <<= 1;   // blockDim.x = max(64, N / 4)
+    if (tid == 0) n_root = flags = 0;
+    __syncthreads();
+    uint64_t v[4];
+    int cnt = 0;
+    for (int r = 0; r < 4; r++) {
+        const int i = 4 * tid + r;
+        v[r] = ~(uint64_t)0;
+        if (i < n) {
+            const double x = P[3 * i], y = P[3 * i + 1], z = P[3 * i + 2];
+            if (in_range(x, rc.x, rh.x) && in_range(y, rc.y, rh.y) && in_range(z, rc.z, rh.z)) {
+                uint64_t path;
+                irr[i] = (uint8_t)point_path(x, y, z, rc, H, depth, path);
+                v[r] = path << SMALL_IDX_BITS | (uint64_t)i;
+                cnt++;
+            }
+        }
+    }
+    if (cnt) atomicAdd(&n_root, cnt);
+    bitonic_sort(v, N, ks);
+    for (int r = 0; r < 4; r++) {
+        if (4 * tid + r < N) ks[4 * tid + r] = v[r];
+        mark[4 * tid + r] = 0;
+    }
+    if (tid == 0) {
+        center[0] = rc.x;
+        center[1] = rc.y;
+        center[2] = rc.z;
+        parent[0] = -1;
+        level[0] = 0;
+        begin[0] = 0;
+        end[0] = n_root;
+    }
+    __syncthreads();
+    const int n0 = n_root;
+    // the levels: number the subdividing nodes in node order, then make their children
+    int lb = 0, le = 1, k = 0;
+    if (tid == 0) hdr[SP_LEVEL_BEGIN] = 0;
+    for (;; k++) {
+        const bool allow = level_allows(k, depth, max_depth), deeper = level_deeper(k, depth, max_depth);
+        int made = 0;
+        for (int i0 = lb; i0 < le; i0 += blockDim.x) {
+            const int i = i0 + tid;
+            bool sub = false;
+            int b = 0, e = 0;
+            if (i < le) {
+                b = begin[i];
+                e = end[i];
+                sub = e - b >= thr;
+                if (sub && deeper) flags = 1;
+                sub = sub && allow;
+            }
+            const unsigned long long ballot = __ballot(sub);
+            if (lane == 0) wsum[wave] = __popcll(ballot);
+            __syncthreads();
+            int rank = made + __popcll(ballot & ((1ull << lane) - 1));
+            for (int q = 0; q < nw; q++) {
+                if (q < wave) rank += wsum[q];
+                made += wsum[q];
+            }
+            __syncthreads();
+            if (i < le) {
+                const int fc = le + 8 * rank;
+                if (sub && fc + 8 > node_cap) {
+                    flags = 1;
+                    sub = false;
+                }
+                first_child[i] = sub ? fc : -1;
+                npts[i] = sub ? 0 : e - b;
+                if (sub) parent[fc] = i;
+                else if (e > b) mark[b] = (uint32_t)b << 8 | (uint32_t)k;
+            }
+        }
+        __syncthreads();
+        if (tid == 0) hdr[SP_LEVEL_BEGIN + k + 1] = le;
+        if (!made || flags) break;   // uniform: flags is written before the barrier only
+        const int sh = SMALL_IDX_BITS + 3 * (depth - k - 1);
+        const float w2 = (float)H.h[k][0] / 2.0f, h2 = (float)H.h[k][1] / 2.0f, d2 = (float)H.h[k][2] / 2.0f;
+        for (int c0 = le; c0 < le + 8 * made; c0 += blockDim.x) {   // whole families: blockDim is a multiple of 8
+            const int c = c0 + tid, o = (c - le) & 7;
+            const bool in = c < le + 8 * made;
+            int par = 0, pb = 0, pe = 0, b = 0;
+            if (in) {
+                par = parent[c - o];
+                pb = begin[par];
+                pe = end[par];
+                // the first point of the parent's range whose octant is >= o
+                int l = pb, h = pe;
+                while (l < h) {
+                    const int mid = (l + h) >> 1;
+                    if ((int)((ks[mid] >> sh) & 7) < o) l = mid + 1;
+                    else h = mid;
+                }
+                b = l;
+            }
+            const int next = __shfl_down(b, 1, 64);
+            if (in) {
+                const float x = (float)center[3 * par], y = (float)center[3 * par + 1], z = (float)center[3 * par + 2];
+                center[3 * c] = c_child_sign[o][0] < 0 ? __fsub_rn(x, w2) : __fadd_rn(x, w2);
+                center[3 * c + 1] = c_child_sign[o][1] < 0 ? __fsub_rn(y, h2) : __fadd_rn(y, h2);
+                center[3 * c + 2] = c_child_sign[o][2] < 0 ? __fsub_rn(z, d2) : __fadd_rn(z, d2);
+                if (o) parent[c] = par;
+                level[c] = k + 1;
+                begin[c] = b;
+                end[c] = o == 7 ? pe : next;
+            }
+        }
+        lb = le;
+        le += 8 * made;
+        __syncthreads();
+    }
+    // every point's leaf: the last mark at or before it (the leaves' ranges follow each other)
+    uint32_t m[4], run = 0;
+    for (int r = 0; r < 4; r++) m[r] = run = max(run, 4 * tid + r < n0 ? mark[4 * tid + r] : 0u);
+    uint32_t incl = run;
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t u = (uint32_t)__shfl_up((int)incl, d, 64);
+        if (lane >= d) incl = max(incl, u);
+    }
+    if (lane == 63) wsum[wave] = (int)incl;
+    uint32_t before = (uint32_t)__shfl_up((int)incl, 1, 64);
+    if (lane == 0) before = 0;
+    __syncthreads();
+    for (int q = 0; q < wave; q++) before = max(before, (uint32_t)wsum[q]);
+    uint32_t s[4];
+    for (int r = 0; r < 4; r++) {
+        s[r] = ~0u;
+        if (4 * tid + r < n0) {
+            const uint32_t q = (uint32_t)ks[4 * tid + r] & ((1u << SMALL_IDX_BITS) - 1), lf = max(before, m[r]);
+            if (irr[q] <= (lf & 255)) flags = 1;
+            s[r] = (lf >> 8) << SMALL_IDX_BITS | q;
+        }
+    }
+    __syncthreads();   // ks is the exchange buffer now
+    bitonic_sort(s, N, (uint32_t*)ks);
+    for (int r = 0; r < 4; r++)
+        if (4 * tid + r < n0) slots[4 * tid + r] = (int)(s[r] & ((1u << SMALL_IDX_BITS) - 1));
+    if (tid == 0) {
+        pack[SP_FLAGS] = flags;
+        pack[SP_ROOT] = n0;
+        pack[SP_LEVELS] = k + 1;
+    }
+    for (int i = tid; i < MAX_LEVELS + 2; i += blockDim.x)
+        pack[SP_LEVEL_BEGIN + i] = i <= k + 1 ? hdr[SP_LEVEL_BEGIN + i] : le;
+    for (int i = tid; i < min(le, SMALL_MIRROR); i += blockDim.x) {
+        pack[SP_HEADER + i] = first_child[i];
+        pack[SP_HEADER + SMALL_MIRROR + i] = npts[i];
+    }
+}
+
+// false: the tree needs the general build
+static bool build_small_tree(TreeDev& T, TreeScratch& S, const double* d_xyz, int n, const double root_c[3],
+                             const double root_h[3], const LevelHalves& H, int thr, int max_depth, hipStream_t st) {
+    const int depth = std::min(max_depth, SHORT_LEVELS);
+    // a level has at most 8 n / thr nodes
+    const int node_cap = (int)std::min<size_t>(1 + 8 * ((size_t)n / thr + 1) * depth, 65536);
+    int N = 256;
+    while (N < n) N <<= 1;
+    const int np = SP_HEADER + 2 * SMALL_MIRROR;
+    double* center = T.center.get<double>(3 * (size_t)node_cap);
+    int* first_child = T.first_child.get<int>(node_cap);
+    int* parent = T.parent.get<int>(node_cap);
+    int* level = T.level.get<int>(node_cap);
+    int* npts = T.npts.get<int>(node_cap);
+    int* begin = T.begin.get<int>(node_cap);
+    int* end = T.end.get<int>(node_cap);
+    int* slots = T.slots.get<int>(n);
+    int* pack = S.pack.get<int>(np);
+    k_small_tree<<<1, std::max(64, N / 4), 0, st>>>(d_xyz, n, make_double3(root_c[0], root_c[1], root_c[2]),
+                                                    make_double3(root_h[0], root_h[1], root_h[2]), H, depth, max_depth,
+                                                    thr, node_cap, center, first_child, parent, level, npts, begin, end,
+                                                    slots, pack);
+    FMM_HIP(hipGetLastError());
+    // received in the first mirror: a pinned array of its own would cost a new tree 0.15 ms
+    T.h_first_child.resize(np);
+    int* h = T.h_first_child.data();
+    FMM_HIP(hipMemcpyAsync(h, pack, np * sizeof(int), hipMemcpyDeviceToHost, st));
+    FMM_HIP(hipStreamSynchronize(st));
+    if (h[SP_FLAGS]) return false;
+    T.num_levels = h[SP_LEVELS];
+    T.num_nodes = h[SP_LEVEL_BEGIN + T.num_levels];
+    T.num_slots = h[SP_ROOT];
+    T.dropped = n - h[SP_ROOT];
+    for (int i = 0; i < MAX_LEVELS + 2; i++) T.level_begin[i] = h[SP_LEVEL_BEGIN + i];
+    T.sorted_build = true;
+    if (T.num_nodes > SMALL_MIRROR) {
+        copy_host_mirrors(T, st);
+        return true;
+    }
+    T.h_npts.resize(T.num_nodes);
+    T.details_on_host = false;
+    std::copy_n(h + SP_HEADER + SMALL_MIRROR, T.num_nodes, T.h_npts.data());
+    std::copy_n(h + SP_HEADER, T.num_nodes, h);   // down by SP_HEADER places, in order
+    T.h_first_child.resize(T.num_nodes);
+    return true;
+}
+
 void build_tree(TreeDev& T, TreeScratch& S, const double* d_xyz, int n, const double root_c[3],
                 const double root_h[3], int thr, int max_depth, bool cubic_scale, hipStream_t st) {
     if (thr < 2) throw Error(1, "leaf capacity too small: a node would subdivide forever");
@@ -896,6 +1176,7 @@ void build_tree(TreeDev& T, TreeScratch& S, const double* d_xyz, int n, const do
         LevelHalves H;
         for (int l = 0; l <= PATH_LEVELS; l++)
             for (int a = 0; a < 3; a++) H.h[l][a] = (float)T.half[std::min(l, MAX_LEVELS - 1)][a];
+        if (n <= SMALL_TREE && build_small_tree(T, S, d_xyz, n, root_c, root_h, H, thr, max_depth, st)) return;
         uint64_t* key = S.k64.get<uint64_t>(n);
         int* irr = S.irr.get<int>(n);
         uint32_t* inroot = S.flag.get<uint32_t>(n + 1);

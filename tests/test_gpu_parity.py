@@ -121,6 +121,54 @@ def test_trees_bit_exact_depth_capped(fm, orc, max_depth):
     _cmp_tree(F.tree(1), orc.target_tree(tgt, 24, root=SHARED_ROOT, max_depth=max_depth))
 
 
+def _grown_root(tgt):
+    """The shared frame's target root: the source root doubled along its lattice until it holds the targets."""
+    sc = 1.0
+    while True:
+        j = np.maximum(np.ceil((-3.0 - tgt.min(0)) / 6.0), 0.0)
+        lo = -3.0 - 6.0 * j
+        if np.all(j <= sc - 1) and np.all(tgt.max(0) < lo + 6.0 * sc):
+            return lo + 3.0 * sc, np.full(3, 3.0 * sc)
+        sc *= 2
+
+
+@pytest.mark.parametrize("ns,nt,cap", [(1, 1, 20), (2, 255, 2), (256, 257, 2), (300, 121, 20), (1025, 1023, 3),
+                                       (2048, 2049, 5000), (4095, 4096, 20), (4096, 4095, 64), (4096, 4097, 2)])
+def test_small_trees_bit_exact(fm, orc, ns, nt, cap):
+    """Trees of up to 4,096 points take one launch; at the edges of its sorts (powers of 2 from 256), of
+    the mirror it returns (2,048 nodes) and of the range itself the tree is the oracle's."""
+    src, w, tgt = _inputs(40 + ns, ns, nt)
+    tgt[::7] *= 1.6   # some of them outside the source root
+    F = fm.FMM(order=4, source_leaf_capacity=cap, target_leaf_capacity=cap, frame=1)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    F.build_trees()
+    print(F.stats()["source_nodes"], F.stats()["target_nodes"], flush=True)
+    _cmp_tree(F.tree(0), orc.source_tree(src, cap))
+    _cmp_tree(F.tree(1), orc.target_tree(tgt, cap, root=_grown_root(tgt)))
+
+
+def test_small_trees_what_the_one_launch_build_leaves(fm, orc):
+    """Points in gaps and overlaps of the float-rounded boxes, a cluster deeper than 10 levels, a depth
+    cap, targets far from the sources and sources that are all or in part outside the root give the
+    oracle's tree at these sizes too."""
+    rng = np.random.default_rng(29)
+    src, w, tgt = _inputs(6, 2000, 1500)
+    gap, _ = gap_overlap_targets(orc, tgt, 24, rng)
+    deep = np.concatenate([src, 0.3 + rng.uniform(-1e-5, 1e-5, (600, 3))])
+    assert len(gap) <= 4096
+    for frame, s, t, depth in ((0, src, gap, None), (1, deep, tgt, None), (1, src, tgt, 2), (1, src, tgt + 50.0, None),
+                               (1, src + 50.0, tgt, None), (1, 3.2 * src, tgt, None)):
+        kw = {} if depth is None else dict(max_depth=depth)
+        F = fm.FMM(order=4, source_leaf_capacity=20, target_leaf_capacity=24, frame=frame, **kw)
+        F.set_sources(s, np.full(len(s), 1.0 / len(s)))
+        F.set_targets(t)
+        F.build_trees()
+        _cmp_tree(F.tree(0), orc.source_tree(s, 20, **kw))
+        _cmp_tree(F.tree(1), orc.target_tree(t, 24, root=_grown_root(t) if frame == 1 else None, **kw))
+        assert F.stats()["target_tree_sorted"] == (0 if t is gap else 1)
+
+
 @pytest.mark.parametrize("frame", [0, 1])
 def test_interaction_lists_bit_exact(fm, orc, frame):
     src, w, tgt = _inputs(4, 12000, 4000)
