@@ -150,6 +150,8 @@ struct fmm_ctx {
     ScaleTable sigS, sigT;
     DevBuf sxyz, sq, sJ, txyz;                   // slot order
     DevBuf nP0, nP1, nP2;                        // near-field sources packed per leaf (slot order)
+    DevBuf bP0, bP1, bP2;                        // the same for the near field of the BEM potential
+    DevBuf p2p_parts;                            // near-field sums of leaves shared by several workgroups
     PinnedVec<int> h_src_leaves, h_tgt_leaves;   // useful (non-empty) leaves
     DevBuf src_leaves, tgt_leaves;
     // expansions [node][3][Lp]
@@ -854,7 +856,7 @@ void stage_p2p(fmm_ctx* c, hipStream_t ps, bool queue = false) {
     } else if (c->cfg.near_field) {
         launch_p2p(c->f64(), c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S, c->lists.close_begin.as<int>(),
                    c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->nP0.ptr, c->nP1.ptr, c->nP2.ptr,
-                   c->txyz.as<double>(), Bnear, ps);
+                   c->txyz.as<double>(), Bnear, c->p2p_parts, ps);
     } else {
         FMM_HIP(hipMemsetAsync(Bnear, 0, 3 * (size_t)std::max(nts, 1) * sizeof(double), ps));
     }
@@ -906,14 +908,20 @@ void stage_evaluate_A(fmm_ctx* c, double current, double* Adev) {
         launch_m2p_close(c->f64(), c->S, c->sigS, c->M.ptr, c->p, c->Lp, c->tgt_leaves.as<int>(), nl, c->T,
                          c->lists.close_begin.as<int>(), c->lists.close_end.as<int>(), c->lists.close_s.as<int>(),
                          c->txyz.as<double>(), nullptr, An, st);
-    else if (c->cfg.near_field && c->bem)
+    else if (c->cfg.near_field && c->bem) {
+        const size_t nss = (size_t)std::max(c->S.num_slots, 1);
+        void* P0 = c->bP0.get<double4>(nss);
+        void* P1 = c->bP1.get<double4>(nss);
+        void* P2 = c->bP2.get<double>(nss);
+        launch_pack_sources(true, c->S.num_slots, c->S.center.as<double>(), c->sxyz.as<double>(), c->sq.as<double>(), P0, P1,
+                            P2, st, c->sbd.as<double>());
         launch_p2p_bem(c->tgt_leaves.as<int>(), nl, c->T, c->S, c->lists.close_begin.as<int>(),
-                       c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->sxyz.as<double>(),
-                       c->sq.as<double>(), c->sbd.as<double>(), c->txyz.as<double>(), An, st);
-    else if (c->cfg.near_field)
+                       c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), P0, P1, P2, c->txyz.as<double>(), An,
+                       c->p2p_parts, st);
+    } else if (c->cfg.near_field)
         launch_p2p_A(c->f64(), c->tgt_leaves.as<int>(), nl, c->T, c->S, c->lists.close_begin.as<int>(),
                      c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->nP0.ptr, c->nP1.ptr, c->nP2.ptr,
-                     c->txyz.as<double>(), An, st);
+                     c->txyz.as<double>(), An, c->p2p_parts, st);
     const size_t nout = 3 * (size_t)c->nt;
     if (nout) k_fill_nan<<<(unsigned)((nout + 255) / 256), 256, 0, st>>>(Adev, nout);
     launch_assemble(c->T.slots.as<int>(), nts, Af, An, current / (4.0 * REF_PI), Adev, st);

@@ -419,17 +419,19 @@ __device__ __forceinline__ float inv_power(float x) {
     const float ri = x > 0.0f ? __builtin_amdgcn_rsqf(x) : 0.0f;
     return POT ? ri : ri * ri * ri;
 }
-// P0[j] = (hi(y_j - o), q_x), P1[j] = (lo(y_j - o), q_y), P2[j] = q_z for every source slot j
+// P0[j] = (hi(y_j - o), q_x), P1[j] = (lo(y_j - o), q_y), P2[j] = q_z for every source slot j; in FP64,
+// where the low parts are zero, P1[j].x holds sd[j] if there is one (BEM)
 template <class R>
 __global__ void k_pack_sources(int n, const double* __restrict__ origin, const double* __restrict__ sxyz,
-                               const double* __restrict__ sq, typename V4<R>::t* __restrict__ P0,
-                               typename V4<R>::t* __restrict__ P1, R* __restrict__ P2) {
+                               const double* __restrict__ sq, const double* __restrict__ sd,
+                               typename V4<R>::t* __restrict__ P0, typename V4<R>::t* __restrict__ P1,
+                               R* __restrict__ P2) {
     constexpr bool split = sizeof(R) == 4;
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     double dx = sxyz[3 * j] - origin[0], dy = sxyz[3 * j + 1] - origin[1], dz = sxyz[3 * j + 2] - origin[2];
     R hx = (R)dx, hy = (R)dy, hz = (R)dz;
-    R lx = split ? (R)(dx - (double)hx) : (R)0, ly = split ? (R)(dy - (double)hy) : (R)0;
+    R lx = split ? (R)(dx - (double)hx) : sd ? (R)sd[j] : (R)0, ly = split ? (R)(dy - (double)hy) : (R)0;
     R lz = split ? (R)(dz - (double)hz) : (R)0;
     P0[j] = V4<R>::make(hx, hy, hz, (R)sq[3 * j]);
     P1[j] = V4<R>::make(lx, ly, lz, (R)sq[3 * j + 1]);
@@ -441,11 +443,14 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
 // sweep it, G = floor(64 / n) lanes per target for a leaf of 8 <= n <= 64 targets (64 / 2^ceil(log2 n)
 // below 8; lane = target * G + g takes sources g, g + G, ...).  Lane partials are summed over
 // the G lanes, then over the 4 waves in a fixed order, and written once.
-// POT: the vector potential sum_j q_j / |x - y_j| instead of B.
+// KIND: B, the vector potential sum_j q_j / |x - y_j|, or the BEM potential (FP64), whose source has a
+// strength v = q and a number d (in the place of the low part of its x).
+// The chunks may be shared by `parts` (a power of 2) workgroups per leaf, each writing its own sums.
 // UP: the leaf takes the lists of its ancestors as well (parent[] up to the root): the transposed
 // near field, where a source leaf is reached through the close pairs of any node that holds it.
-template <class R, bool POT, int UNROLL, bool UP = false>
-__device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegin, const int* __restrict__ tend,
+enum { NEAR_B, NEAR_A, NEAR_BEM };
+template <class R, int KIND, int UNROLL, bool UP = false>
+__device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const int* __restrict__ tbegin, const int* __restrict__ tend,
                                          const int* __restrict__ close_begin, const int* __restrict__ close_end,
                                          const int* __restrict__ close_s, const double* __restrict__ origin,
                                          const int* __restrict__ sbegin, const int* __restrict__ send,
@@ -456,7 +461,9 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
                                          double (*red)[3][64], const int* __restrict__ parent = nullptr) {
     typedef typename V4<R>::t v4;
     constexpr bool split = sizeof(R) == 4;
+    static_assert(KIND != NEAR_BEM || !split, "the BEM potential is FP64");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nw = 4 * parts, w0 = 4 * part + wave;
     const int tb = tbegin[leaf], te = tend[leaf];
     if (!UP && close_begin[leaf] >= close_end[leaf]) {
         for (int k = tb + tid; k < te; k += 256) Bnear[3 * k] = Bnear[3 * k + 1] = Bnear[3 * k + 2] = 0.0;
@@ -489,7 +496,7 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
             const int s = close_s[ci];
             const int sb = sbegin[s], se = send[s];
             const int nch = (se - sb + 63) >> 6;
-            for (int j0 = sb + 64 * ((wave - run) & 3); j0 < se; j0 += 4 * 64) {
+            for (int j0 = sb + 64 * ((w0 - run) & (nw - 1)); j0 < se; j0 += 64 * nw) {
                 const int nj = min(64, se - j0);
                 __syncwarp();
                 if (lane < nj) {
@@ -512,8 +519,12 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
                     }
                     // fused multiply-adds (explicit: this library is built without contraction)
                     const R r2 = fma_t(dx, dx, fma_t(dy, dy, dz * dz));
-                    const R ip = inv_power<POT>(r2);
-                    if (POT) {
+                    const R ip = inv_power<KIND == NEAR_A>(r2);
+                    if (KIND == NEAR_BEM) {   // (d (y - x) + (y - x) x v) / |y - x|^3
+                        f0 = fma_t(-fma_t(dx, yl.x, fma_t(dy, qz, -dz * qy)), ip, f0);
+                        f1 = fma_t(-fma_t(dy, yl.x, fma_t(dz, qx, -dx * qz)), ip, f1);
+                        f2 = fma_t(-fma_t(dz, yl.x, fma_t(dx, qy, -dy * qx)), ip, f2);
+                    } else if (KIND == NEAR_A) {
                         f0 = fma_t(qx, ip, f0);
                         f1 = fma_t(qy, ip, f1);
                         f2 = fma_t(qz, ip, f2);
@@ -556,19 +567,39 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int* __restrict__ tbegi
     }
 }
 
-template <class R, bool POT>
-__global__ __launch_bounds__(256) void k_p2p(const int* __restrict__ leaves, const int* __restrict__ tbegin,
-                                             const int* __restrict__ tend, const int* __restrict__ close_begin,
-                                             const int* __restrict__ close_end, const int* __restrict__ close_s,
-                                             const double* __restrict__ origin, const int* __restrict__ sbegin,
-                                             const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0,
+// Part 0 of a leaf writes `near`, part q its sums into partial[q - 1][n3] (n3 = 3 x target slots).
+//
+// A workgroup per leaf leaves the chip idle when the leaves are few: their lists are walked one chunk of
+// a wave after the other, and the time is that of the longest list.  32,768 sources and 4,096 targets in
+// 276 leaves (3.3e7 pairs, FP64): 470 -> 112 us; the drop-in coil (38,400 sources in leaves of 1,000, 4,096
+// targets in leaves of 100) 1275 -> 150 us; a BEM solve (6,000, 1,999; one lane per target of a leaf in one
+// wave before) 375 -> 27 + 5 us.
+template <class R, int KIND>
+__global__ __launch_bounds__(256) void k_p2p(const int* __restrict__ leaves, int lg_parts,
+                                             const int* __restrict__ tbegin, const int* __restrict__ tend,
+                                             const int* __restrict__ close_begin, const int* __restrict__ close_end,
+                                             const int* __restrict__ close_s, const double* __restrict__ origin,
+                                             const int* __restrict__ sbegin, const int* __restrict__ send,
+                                             const typename V4<R>::t* __restrict__ P0,
                                              const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
-                                             const double* __restrict__ txyz, double* __restrict__ Bnear) {
+                                             const double* __restrict__ txyz, double* __restrict__ near,
+                                             double* __restrict__ partial, size_t n3) {
     __shared__ typename V4<R>::t s0[4][64];
     __shared__ typename V4<R>::t s1[4][64];
     __shared__ R s2[4][64];
     __shared__ double red[4][3][64];
-    p2p_leaf<R, POT, 4>(leaves[blockIdx.x], tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send, P0, P1, P2, txyz, Bnear, s0, s1, s2, red);
+    const int part = blockIdx.x & ((1 << lg_parts) - 1);
+    p2p_leaf<R, KIND, 4>(leaves[blockIdx.x >> lg_parts], part, 1 << lg_parts, tbegin, tend, close_begin, close_end, close_s,
+                         origin, sbegin, send, P0, P1, P2, txyz, part ? partial + (part - 1) * n3 : near, s0, s1, s2,
+                         red);
+}
+
+__global__ void k_add_parts(const double* __restrict__ partial, int nparts, size_t n3, double* __restrict__ near) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n3) return;
+    double v = near[i];
+    for (int q = 0; q < nparts; q++) v += partial[q * n3 + i];
+    near[i] = v;
 }
 
 // The transposed near field (adjoint): per useful source leaf, sum_i g_i x (y_j - x_i) / |y_j - x_i|^3
@@ -589,7 +620,7 @@ __global__ __launch_bounds__(256) void k_p2p_transposed(
     __shared__ typename V4<R>::t s1[4][64];
     __shared__ R s2[4][64];
     __shared__ double red[4][3][64];
-    p2p_leaf<R, false, 4, true>(leaves[blockIdx.x], sbegin, send, close_begin, close_end, close_t, origin, tbegin, tend,
+    p2p_leaf<R, NEAR_B, 4, true>(leaves[blockIdx.x], 0, 1, sbegin, send, close_begin, close_end, close_t, origin, tbegin, tend,
                                 P0, P1, P2, sxyz, out, s0, s1, s2, red, parent);
 }
 
@@ -634,7 +665,7 @@ __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, i
         const int i = next;
         __syncthreads();   // every thread has read next before thread 0 takes the following leaf
         if (i >= nleaves) break;
-        p2p_leaf<R, POT, BESIDE ? 1 : 4>(leaves[i], tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send,
+        p2p_leaf<R, POT ? NEAR_A : NEAR_B, BESIDE ? 1 : 4>(leaves[i], 0, 1, tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send,
                                          P0, P1, P2, txyz, Bnear, s0, s1, s2, red);
     }
 }
@@ -778,37 +809,6 @@ __global__ __launch_bounds__(64) void k_p2m_bem(const int* __restrict__ leaves, 
     }
 }
 
-// near field of the BEM potential, FP64: one thread per target of a useful target leaf, over the
-// sources of every node of the leaf's close list
-__global__ __launch_bounds__(64) void k_p2p_bem(const int* __restrict__ leaves, const int* __restrict__ tbegin,
-                                                const int* __restrict__ tend, const int* __restrict__ close_begin,
-                                                const int* __restrict__ close_end, const int* __restrict__ close_s,
-                                                const int* __restrict__ sbegin, const int* __restrict__ send,
-                                                const double* __restrict__ sxyz, const double* __restrict__ sv,
-                                                const double* __restrict__ sd, const double* __restrict__ txyz,
-                                                double* __restrict__ out) {
-    const int leaf = leaves[blockIdx.x];
-    for (int k = tbegin[leaf] + threadIdx.x; k < tend[leaf]; k += blockDim.x) {
-        const double x = txyz[3 * k], y = txyz[3 * k + 1], z = txyz[3 * k + 2];
-        double a0 = 0, a1 = 0, a2 = 0;
-        for (int ci = close_begin[leaf]; ci < close_end[leaf]; ci++) {
-            const int s = close_s[ci];
-            for (int j = sbegin[s]; j < send[s]; j++) {
-                const double q0 = sxyz[3 * j] - x, q1 = sxyz[3 * j + 1] - y, q2 = sxyz[3 * j + 2] - z;
-                const double r2 = q0 * q0 + q1 * q1 + q2 * q2;
-                const double r3 = inv_power<false>(r2), d = sd[j];
-                const double v0 = sv[3 * j], v1 = sv[3 * j + 1], v2 = sv[3 * j + 2];
-                a0 += (q0 * d + (q1 * v2 - q2 * v1)) * r3;
-                a1 += (q1 * d + (q2 * v0 - q0 * v2)) * r3;
-                a2 += (q2 * d + (q0 * v1 - q1 * v0)) * r3;
-            }
-        }
-        out[3 * k] = a0;
-        out[3 * k + 1] = a1;
-        out[3 * k + 2] = a2;
-    }
-}
-
 void launch_bem_charges(const int* slots, int n, const double* xyz, const double* w, const double* Bv,
                         const double* nrm, double* sxyz, double* sv, double* sd, hipStream_t st) {
     if (n) k_bem_charges<<<blocks(n), 256, 0, st>>>(slots, n, xyz, w, Bv, nrm, sxyz, sv, sd);
@@ -827,15 +827,6 @@ void launch_p2m_bem(bool f64, const int* leaves, int nleaves, const TreeDev& S, 
                                                    S.level.as<int>(), sig, sxyz, sv, sd, p, Lp, (float*)M);
     FMM_HIP(hipGetLastError());
 }
-void launch_p2p_bem(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
-                    const int* close_end, const int* close_s, const double* sxyz, const double* sv, const double* sd,
-                    const double* txyz, double* out, hipStream_t st) {
-    if (!nleaves) return;
-    k_p2p_bem<<<nleaves, 64, 0, st>>>(leaves, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
-                                      S.begin.as<int>(), S.end.as<int>(), sxyz, sv, sd, txyz, out);
-    FMM_HIP(hipGetLastError());
-}
-
 // ---------------------------------------------------------------- assembly
 __global__ void k_assemble(const int* __restrict__ slots, int n, const double* __restrict__ Bfar,
                            const double* __restrict__ Bnear, double scale, double* __restrict__ B) {
@@ -1039,35 +1030,51 @@ void launch_l2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, co
     l2p_launch<true>(f64, leaves, nleaves, T, sig, txyz, Lexp, p, Lp, Afar, st);
 }
 void launch_pack_sources(bool f64, int n, const double* origin, const double* sxyz, const double* sq, void* P0,
-                         void* P1, void* P2, hipStream_t st) {
+                         void* P1, void* P2, hipStream_t st, const double* sd) {
     if (!n) return;
     if (f64)
-        k_pack_sources<double><<<blocks(n), 256, 0, st>>>(n, origin, sxyz, sq, (double4*)P0, (double4*)P1, (double*)P2);
+        k_pack_sources<double><<<blocks(n), 256, 0, st>>>(n, origin, sxyz, sq, sd, (double4*)P0, (double4*)P1, (double*)P2);
     else
-        k_pack_sources<float><<<blocks(n), 256, 0, st>>>(n, origin, sxyz, sq, (float4*)P0, (float4*)P1, (float*)P2);
+        k_pack_sources<float><<<blocks(n), 256, 0, st>>>(n, origin, sxyz, sq, nullptr, (float4*)P0, (float4*)P1, (float*)P2);
     FMM_HIP(hipGetLastError());
 }
-template <bool POT>
+// workgroups per leaf, a power of 2: enough for some 8 to 16 workgroups a CU in all (6 to 8 are resident at
+// a time; the rest evens out the lists), at most 16, and one where there are few sources to share
+static int p2p_lg_parts(int nleaves, int nsources) {
+    int lg = 0;
+    while (lg < 4 && ((long long)nleaves << lg) <= 8LL * num_cus() && (nsources >> (lg + 9)) > 0) lg++;
+    return lg;
+}
+template <int KIND>
 static void p2p_launch(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S,
                        const int* close_begin, const int* close_end, const int* close_s, const void* P0,
-                       const void* P1, const void* P2, const double* txyz, double* out, hipStream_t st) {
+                       const void* P1, const void* P2, const double* txyz, double* out, DevBuf& scratch, hipStream_t st) {
     if (!nleaves) return;
+    const int lg = p2p_lg_parts(nleaves, S.num_slots), more = (1 << lg) - 1;
+    const size_t n3 = 3 * (size_t)T.num_slots;
+    double* partial = more ? scratch.get<double>(more * n3) : nullptr;
     if (f64)
-        k_p2p<double, POT><<<nleaves, 256, 0, st>>>(leaves, T.begin.as<int>(), T.end.as<int>(),
-                                                    close_begin, close_end, close_s, S.center.as<double>(),
-                                                    S.begin.as<int>(), S.end.as<int>(), (const double4*)P0,
-                                                    (const double4*)P1, (const double*)P2, txyz, out);
-    else
-        k_p2p<float, POT><<<nleaves, 256, 0, st>>>(leaves, T.begin.as<int>(), T.end.as<int>(),
-                                                   close_begin, close_end, close_s, S.center.as<double>(),
-                                                   S.begin.as<int>(), S.end.as<int>(), (const float4*)P0,
-                                                   (const float4*)P1, (const float*)P2, txyz, out);
+        k_p2p<double, KIND><<<nleaves << lg, 256, 0, st>>>(leaves, lg, T.begin.as<int>(), T.end.as<int>(),
+                                                           close_begin, close_end, close_s, S.center.as<double>(),
+                                                           S.begin.as<int>(), S.end.as<int>(), (const double4*)P0,
+                                                           (const double4*)P1, (const double*)P2, txyz, out, partial, n3);
+    else if constexpr (KIND != NEAR_BEM)
+        k_p2p<float, KIND><<<nleaves << lg, 256, 0, st>>>(leaves, lg, T.begin.as<int>(), T.end.as<int>(),
+                                                          close_begin, close_end, close_s, S.center.as<double>(),
+                                                          S.begin.as<int>(), S.end.as<int>(), (const float4*)P0,
+                                                          (const float4*)P1, (const float*)P2, txyz, out, partial, n3);
+    if (more) k_add_parts<<<blocks((long long)n3), 256, 0, st>>>(partial, more, n3, out);
     FMM_HIP(hipGetLastError());
 }
 void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                 const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                const double* txyz, double* Bnear, hipStream_t st) {
-    p2p_launch<false>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Bnear, st);
+                const double* txyz, double* Bnear, DevBuf& scratch, hipStream_t st) {
+    p2p_launch<NEAR_B>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Bnear, scratch, st);
+}
+void launch_p2p_bem(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                    const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
+                    const double* txyz, double* out, DevBuf& scratch, hipStream_t st) {
+    p2p_launch<NEAR_BEM>(true, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, out, scratch, st);
 }
 void launch_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                       const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
@@ -1099,8 +1106,8 @@ void launch_p2p_transposed(bool f64, const int* leaves, int nleaves, const TreeD
 }
 void launch_p2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                   const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                  const double* txyz, double* Anear, hipStream_t st) {
-    p2p_launch<true>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Anear, st);
+                  const double* txyz, double* Anear, DevBuf& scratch, hipStream_t st) {
+    p2p_launch<NEAR_A>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Anear, scratch, st);
 }
 void launch_assemble(const int* slots, int n, const double* Bfar, const double* Bnear, double scale, double* B,
                      hipStream_t st) {

@@ -22,12 +22,13 @@ void launch_zero_unwritten(const TreeDev& S, int Lp, size_t esize, void* M, hipS
 void launch_l2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const ScaleTable& sig, const double* txyz,
                 const void* Lexp, int p, int Lp, double* Bfar, hipStream_t st);
 // near-field sources in slot order relative to origin[3] (a device pointer); P0, P1: 4 x R per
-// slot, P2: R per slot, R = double if f64 else float
+// slot, P2: R per slot, R = double if f64 else float; sd (f64 only): the BEM sources' d
 void launch_pack_sources(bool f64, int n, const double* origin, const double* sxyz, const double* sq, void* P0,
-                         void* P1, void* P2, hipStream_t st);
+                         void* P1, void* P2, hipStream_t st, const double* sd = nullptr);
+// few leaves are shared by several workgroups each, whose sums go through scratch
 void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                 const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                const double* txyz, double* Bnear, hipStream_t st);
+                const double* txyz, double* Bnear, DevBuf& scratch, hipStream_t st);
 // launch_p2p in FP32 as a persistent grid of `grid` workgroups taking leaves from the counter *queue (0
 // at the start; several grids may share it); beside: with a small register budget that lets a workgroup
 // share its CU with one of the M2L GEMM's, whose tile counters and tiles are given
@@ -48,16 +49,17 @@ void launch_l2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, co
                   const void* Lexp, int p, int Lp, double* Afar, hipStream_t st);
 void launch_p2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                   const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                  const double* txyz, double* Anear, hipStream_t st);
+                  const double* txyz, double* Anear, DevBuf& scratch, hipStream_t st);
 // Problem::BEM: slot-order strengths v = w (B x n) (3) and d = w (B . n) of BEMQuadrature sources;
-// their multipoles (P2M of the gradient of R); the near field of their potential (FP64, unscaled)
+// their multipoles (P2M of the gradient of R); the near field of their potential (FP64, unscaled) from
+// sources packed in FP64 with q = v and their d
 void launch_bem_charges(const int* slots, int n, const double* xyz, const double* w, const double* Bv,
                         const double* nrm, double* sxyz, double* sv, double* sd, hipStream_t st);
 void launch_p2m_bem(bool f64, const int* leaves, int nleaves, const TreeDev& S, const ScaleTable& sig,
                     const double* sxyz, const double* sv, const double* sd, int p, int Lp, void* M, hipStream_t st);
 void launch_p2p_bem(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
-                    const int* close_end, const int* close_s, const double* sxyz, const double* sv, const double* sd,
-                    const double* txyz, double* out, hipStream_t st);
+                    const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
+                    const double* txyz, double* out, DevBuf& scratch, hipStream_t st);
 // FP64 direct sum of B (pot: A) at nt targets over the ns slot-order sources, scaled; the sources
 // are cut into nsplit ranges whose partial sums (partial: nsplit * nt * 3 doubles) are added in
 // range order.  direct_splits: the number of ranges that fills the GPU.

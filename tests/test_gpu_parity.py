@@ -313,6 +313,23 @@ def test_B_matches_oracle(fm, orc, small_case, precision, tol):
     assert rel_l2(Bf, R.Bfar) < tol * 10
 
 
+@pytest.mark.parametrize("ns,nt,cap", [(511, 3, 8), (1023, 130, 100), (2500, 65, 64), (9000, 65, 100), (9000, 1, 500)])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
+def test_near_field_of_few_leaves(fm, orc, ns, nt, cap, precision, tol):
+    """Few target leaves: their close lists are shared by 1 to 16 workgroups, some without a chunk."""
+    rng = np.random.default_rng(ns + nt)
+    src = shell_sources(rng, ns)
+    w = rng.uniform(0.5, 1.5, ns) / ns
+    tgt = shell_sources(rng, nt)
+    R = _oracle_run(orc, src, w, tgt, 3, cap, cap)
+    F = fm.FMM(order=3, source_leaf_capacity=cap, target_leaf_capacity=cap, precision=precision, frame=1)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    F.run(1.0)
+    assert np.abs(R.Bnear).max() > 0
+    assert rel_l2(F.B_parts()[1], R.Bnear) < tol
+
+
 def test_direct_sum_gpu_vs_oracle(fm, orc):
     import ctypes
     src, w, tgt = _inputs(12, 3000, 500)
