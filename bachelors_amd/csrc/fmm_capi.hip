@@ -300,19 +300,20 @@ void resolve_pass(Pass& P, const char* dev) {
     P.tiles = (const GemmTile*)(dev + P.o_tiles);
 }
 
-// O.nops operators from device specs, written in the precision the GEMMs apply
-// O.nops operators (from device specs) in the precision of the passes that apply them
-void build_tables(fmm_ctx* c, OpTables& O, const OpSpec* d_specs, hipStream_t st, int nops = -1) {
-    if (nops < 0) nops = O.nops;
-    size_t n = (size_t)nops * c->Lp * c->Lp;
-    if (!n) return;
+// operators from device specs in the precision of the passes that apply them: n M2M or L2L ones, then
+// nm2l M2L ones
+void build_tables(fmm_ctx* c, OpTables& O, const OpSpec* d_specs, hipStream_t st, int n, int nm2l = 0) {
+    const size_t one = (size_t)c->Lp * c->Lp, all = (size_t)(n + nm2l) * one;
+    if (!all) return;
+    void* work = nm2l ? c->m2l_work.reserve(m2l_work_bytes(nm2l, c->p)) : nullptr;
+    auto make = [&](int mode, auto* out, __bf16* lo) {
+        make_operators(d_specs, n, c->p, c->Lp, mode, out, lo, st);
+        make_m2l(d_specs + n, nm2l, c->p, c->Lp, mode, out + n * one, lo ? lo + n * one : nullptr, work, st);
+    };
     const Precision pr = c->pass_prec();
-    if (pr == Precision::F64)
-        make_operators(d_specs, nops, c->p, c->Lp, 0, O.f64.get<double>(n), nullptr, st);
-    else if (pr == Precision::F32)
-        make_operators(d_specs, nops, c->p, c->Lp, 1, O.f32.get<float>(n), nullptr, st);
-    else
-        make_operators(d_specs, nops, c->p, c->Lp, 2, O.hi.get<__bf16>(n), O.lo.get<__bf16>(n), st);
+    if (pr == Precision::F64) make(0, O.f64.get<double>(all), nullptr);
+    else if (pr == Precision::F32) make(1, O.f32.get<float>(all), nullptr);
+    else make(2, O.hi.get<__bf16>(all), O.lo.get<__bf16>(all));
 }
 
 const void* ops_ptr(const fmm_ctx* c, const OpTables& O) {
@@ -533,7 +534,7 @@ void stage_upward(fmm_ctx* c, int alg = FMM_M2M_MATRICES) {
         const double* d_nominal = (const double*)(sp.send(c->stream) + o);
         OpSpec* d_specs = O.specs.get<OpSpec>(O.nops);
         make_m2m_specs(S, c->sigS, d_nominal, d_specs, c->stream);
-        build_tables(c, O, d_specs, c->stream);
+        build_tables(c, O, d_specs, c->stream, O.nops);
     }
     if (alg != FMM_M2M_MATRICES) {
         upward_without_matrices(c, alg);
@@ -692,10 +693,10 @@ void translate_tables(fmm_ctx* c, hipStream_t st) {
             f.lo = c->m2l_lo.get<_Float16>((size_t)nc * f.R * f.Kp);
             f.rinv = c->m2l_rinv.get<float>((size_t)nc * f.R);
             f.dm = c->dm.as<float>();
-            make_m2l_f16(d + n_l2l, nc, c->p, f, c->m2l_work.reserve(m2l_f16_work_bytes(nc, c->p)), st);
+            make_m2l_f16(d + n_l2l, nc, c->p, f, c->m2l_work.reserve(m2l_work_bytes(nc, c->p)), st);
         }
-    } else if (O.nops) {
-        build_tables(c, O, d, st);
+    } else {
+        build_tables(c, O, d, st, n_l2l, nc);
     }
     // the M2L tiles (planned while the tables are built; F16X3: those of the groups, made with the lists)
     Pass& P = c->m2l_pass;
@@ -1426,7 +1427,7 @@ int fmm_adjoint_weights_dev(fmm_ctx* c, double current, const double* dLdB, doub
         a.prec = c->pass_prec();
         if (c->prec == Precision::F16X3 && c->down_ops.nops > c->down_l2l)
             // the transposed passes apply the down operators in FP32: the M2L ones too
-            build_tables(c, c->down_ops, c->down_specs, c->stream);
+            build_tables(c, c->down_ops, c->down_specs, c->stream, c->down_l2l, c->down_ops.nops - c->down_l2l);
         a.p = c->p;
         a.Lp = c->Lp;
         a.S = &c->S;

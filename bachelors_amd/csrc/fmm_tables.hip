@@ -213,11 +213,52 @@ __global__ void k_m2l_harmonics(const OpSpec* __restrict__ specs, int nops, int 
     }
 }
 
-// M2L operators as FP16 splits (F16Split), one item per (output degree l, order |m|) x (input
-// degree a, order |b|): the complex kernel entries K(+-m, +-b) = f(+-m, +-b) X(l + a, +-m -+ b)
-// take two harmonics, X(n, m - b) and X(n, m + b), and their conjugates, and give the up to four
-// real entries of rows (l, +-m) and columns (a, +-b) with the same operations, in the same
-// order, as the entry-wise kernel.  Workgroup s of an operator owns the row pairs (l, |m|) of
+// One item of an M2L operator: the row pair (l, m), (l, -m) of packed index lm and the column pair (a, b),
+// (a, -b) of packed index ab.  The complex kernel entries K(+-m, +-b) = f(+-m, +-b) X(l + a, +-m -+ b)
+// take two harmonics, X(n, m - b) and X(n, m + b), and their conjugates, and give the up to four real
+// entries with the same operations, in the same order, as the entry-wise kernel: put(0 for +m or 1 for
+// -m, column, value without the factor of degree a).
+template <class Put>
+__device__ __forceinline__ void m2l_item(const cplx* X, int pH, short2 lm, short2 ab, Put put) {
+    const double c = 0.70710678118654752440;
+    const int l = lm.x, m = lm.y, a = ab.x, b = ab.y, n = l + a;
+    // K(s1 m, s2 b), s = +-1: f(m', b') = (-1)^|(|m'-b'| - |m'| - |b'|) / 2| (-1)^a
+    cplx kpp = {0, 0}, kpm = {0, 0}, kmp = {0, 0}, kmm = {0, 0};
+    if (n <= pH) {
+        const cplx A = harm(X, n, m - b), Bq = harm(X, n, m + b);
+        const double sa = sgn_pow(a);
+        kpp = cscale(A, sgn_pow(abs((abs(m - b) - m - b) / 2)) * sa);
+        kpm = cscale(Bq, sgn_pow(abs((abs(m + b) - m - b) / 2)) * sa);
+        kmp = cscale(cplx{Bq.re, -Bq.im}, sgn_pow(abs((abs(-m - b) - m - b) / 2)) * sa);
+        kmm = cscale(cplx{A.re, -A.im}, sgn_pow(abs((abs(b - m) - m - b) / 2)) * sa);
+    }
+    const int jp = a * a + a + b, jm = a * a + a - b;   // columns (a, +-b)
+    if (b == 0) {   // column (a, 0): out_c(m') = K(m', 0)
+        if (m == 0) put(0, jp, kpp.re);
+        else {
+            put(0, jp, c * (kpp.re + kmp.re));
+            put(1, jp, c * (kpp.im - kmp.im));
+        }
+        return;
+    }
+    // column (a, +b): out_c(m') = c K(m', b) + c K(m', -b)
+    // column (a, -b): out_c(m') = (-c Im K(m', b) + c Im K(m', -b), c Re K(m', b) - c Re K(m', -b))
+    const cplx opP = {c * kpp.re + c * kpm.re, c * kpp.im + c * kpm.im};       // m' = m, col +b
+    const cplx opM = {-(c * kpp.im) + c * kpm.im, c * kpp.re + -(c * kpm.re)};  // m' = m, col -b
+    if (m == 0) {
+        put(0, jp, opP.re);
+        put(0, jm, opM.re);
+        return;
+    }
+    const cplx omP = {c * kmp.re + c * kmm.re, c * kmp.im + c * kmm.im};       // m' = -m, col +b
+    const cplx omM = {-(c * kmp.im) + c * kmm.im, c * kmp.re + -(c * kmm.re)};  // m' = -m, col -b
+    put(0, jp, c * (opP.re + omP.re));
+    put(1, jp, c * (opP.im - omP.im));
+    put(0, jm, c * (opM.re + omM.re));
+    put(1, jm, c * (opM.im - omM.im));
+}
+
+// M2L operators as FP16 splits (F16Split).  Workgroup s of an operator owns the row pairs (l, |m|) of
 // packed index [s pps, (s+1) pps), staged in LDS as FP32 rows (scaled by fac[a] and 1 / dm_j),
 // two per pair (+m, then -m; m = 0 leaves the second unused); each wave then takes whole rows:
 // the row maximum by a shuffle reduction, the power-of-2 row scale and the hi + lo split into
@@ -247,55 +288,18 @@ __global__ __launch_bounds__(256) void k_make_m2l_f16(const OpSpec* __restrict__
     for (int n = threadIdx.x; n <= p; n += blockDim.x) cf[n] = facall[(size_t)opi * (p + 1) + n];
     for (int j = threadIdx.x; j < L; j += blockDim.x) idm[j] = (double)(1.0f / f16.dm[j]);   // exact: dm is 2^k
     __syncthreads();
-    const double c = 0.70710678118654752440;
     const int rp0 = slice * pps, nrp = min(NP, rp0 + pps) - rp0;
     // items e = rp NP + q, (rp, q) advanced by the stride instead of divided out
     int rp = threadIdx.x / NP, q = threadIdx.x - (threadIdx.x / NP) * NP;
     const int drp = blockDim.x / NP, dq = blockDim.x - drp * NP;
     for (int e = threadIdx.x; e < nrp * NP; e += blockDim.x, rp += drp, q += dq) {
         if (q >= NP) { q -= NP; rp++; }
-        const short2 lm = tri_lm[rp0 + rp], ab = tri_lm[q];
-        const int l = lm.x, m = lm.y, a = ab.x, b = ab.y, n = l + a;
-        // K(s1 m, s2 b), s = +-1: f(m', b') = (-1)^|(|m'-b'| - |m'| - |b'|) / 2| (-1)^a
-        cplx kpp = {0, 0}, kpm = {0, 0}, kmp = {0, 0}, kmm = {0, 0};
-        if (n <= pH) {
-            const cplx A = harm(X, n, m - b), Bq = harm(X, n, m + b);
-            const double sa = sgn_pow(a);
-            kpp = cscale(A, sgn_pow(abs((abs(m - b) - m - b) / 2)) * sa);
-            kpm = cscale(Bq, sgn_pow(abs((abs(m + b) - m - b) / 2)) * sa);
-            kmp = cscale(cplx{Bq.re, -Bq.im}, sgn_pow(abs((abs(-m - b) - m - b) / 2)) * sa);
-            kmm = cscale(cplx{A.re, -A.im}, sgn_pow(abs((abs(b - m) - m - b) / 2)) * sa);
-        }
-        const double fa = cf[a];
-        const int rp_ = 2 * rp, rm_ = 2 * rp + 1;   // staged rows (l, +-m)
-        const int jp = a * a + a + b, jm = a * a + a - b;   // columns (a, +-b)
-        auto put = [&](int r, int j, double val) {
+        const short2 ab = tri_lm[q];
+        const double fa = cf[ab.x];
+        m2l_item(X, pH, tri_lm[rp0 + rp], ab, [&](int minus, int j, double val) {
             val *= fa;
-            stg[r * L + j] = (float)(val * idm[j]);
-        };
-        if (b == 0) {   // column (a, 0): out_c(m') = K(m', 0)
-            if (m == 0) put(rp_, jp, kpp.re);
-            else {
-                put(rp_, jp, c * (kpp.re + kmp.re));
-                put(rm_, jp, c * (kpp.im - kmp.im));
-            }
-        } else {
-            // column (a, +b): out_c(m') = c K(m', b) + c K(m', -b)
-            // column (a, -b): out_c(m') = (-c Im K(m', b) + c Im K(m', -b), c Re K(m', b) - c Re K(m', -b))
-            const cplx opP = {c * kpp.re + c * kpm.re, c * kpp.im + c * kpm.im};       // m' = m, col +b
-            const cplx opM = {-(c * kpp.im) + c * kpm.im, c * kpp.re + -(c * kpm.re)};  // m' = m, col -b
-            if (m == 0) {
-                put(rp_, jp, opP.re);
-                put(rp_, jm, opM.re);
-            } else {
-                const cplx omP = {c * kmp.re + c * kmm.re, c * kmp.im + c * kmm.im};       // m' = -m, col +b
-                const cplx omM = {-(c * kmp.im) + c * kmm.im, c * kmp.re + -(c * kmm.re)};  // m' = -m, col -b
-                put(rp_, jp, c * (opP.re + omP.re));
-                put(rm_, jp, c * (opP.im - omP.im));
-                put(rp_, jm, c * (opM.re + omM.re));
-                put(rm_, jm, c * (opM.im - omM.im));
-            }
-        }
+            stg[(2 * rp + minus) * L + j] = (float)(val * idm[j]);
+        });
     }
     __syncthreads();
     // rows: maximum, scale, split.  Lane g takes the columns 4g .. 4g + 3 of each group of 256.
@@ -342,11 +346,78 @@ __global__ __launch_bounds__(256) void k_make_m2l_f16(const OpSpec* __restrict__
     }
 }
 
-// row pairs per workgroup of k_make_m2l_f16: as many as the staging budget holds (two rows of
+// M2L operators in the layout of k_make_ops (MODE as there), by the items and the slices of
+// k_make_m2l_f16: rows staged in LDS as they are written, then whole rows of Lp elements, the padding of
+// the columns with them and rows L .. Lp-1 by the last slice.
+//
+// Bound by the FP64 arithmetic of the entries (a column of harmonics per thread of every workgroup and
+// four times the sign and basis work per entry cost k_make_ops more), in FP64 also by the writes.  Tables of
+// 3,256 classes in FP64 at p = 10 (0.43 GB) 280 -> 122 us (3.5 TB/s), of 1M points at p = 12 360 -> 146 us, the
+// FP32 ones of the adjoint of 262,147 x 131,101 clustered points (p = 14) 2.26 -> 0.89 ms.
+template <int MODE>
+__global__ __launch_bounds__(256) void k_make_m2l(const OpSpec* __restrict__ specs, int p, int pI_full, int nX, int Lp,
+                                                  const cplx* __restrict__ Xall, const double* __restrict__ facall,
+                                                  void* __restrict__ out, __bf16* __restrict__ out_lo, int pps,
+                                                  int nsplit) {
+    typedef typename std::conditional<MODE == 0, double, float>::type T;
+    extern __shared__ cplx X[];   // packed (n, k>=0), n <= pH
+    const int opi = blockIdx.x / nsplit, slice = blockIdx.x - opi * nsplit;
+    const int pH = specs[opi].m2l_full ? pI_full : p;
+    const int L = (p + 1) * (p + 1), NP = (p + 1) * (p + 2) / 2;
+    short2* tri_lm = (short2*)(X + nX);                 // (n, k) of packed index t (degree <= p)
+    double* cf = (double*)(tri_lm + ((NP + 1) & ~1));   // fac[a]
+    T* stg = (T*)(cf + (p + 1));                        // the slice's rows, [row][L]
+    {
+        const cplx* Xg = Xall + (size_t)opi * nX;
+        const int nXh = (pH + 1) * (pH + 2) / 2;
+        for (int t = threadIdx.x; t < nXh; t += blockDim.x) X[t] = Xg[t];
+    }
+    for (int t = threadIdx.x; t < NP; t += blockDim.x) {
+        int n = 0;
+        while ((n + 1) * (n + 2) / 2 <= t) n++;
+        tri_lm[t] = make_short2((short)n, (short)(t - n * (n + 1) / 2));
+    }
+    for (int n = threadIdx.x; n <= p; n += blockDim.x) cf[n] = facall[(size_t)opi * (p + 1) + n];
+    __syncthreads();
+    const int rp0 = slice * pps, nrp = min(NP, rp0 + pps) - rp0;
+    int rp = threadIdx.x / NP, q = threadIdx.x - (threadIdx.x / NP) * NP;
+    const int drp = blockDim.x / NP, dq = blockDim.x - drp * NP;
+    for (int e = threadIdx.x; e < nrp * NP; e += blockDim.x, rp += drp, q += dq) {
+        if (q >= NP) { q -= NP; rp++; }
+        const short2 ab = tri_lm[q];
+        const double fa = cf[ab.x];
+        m2l_item(X, pH, tri_lm[rp0 + rp], ab,
+                 [&](int minus, int j, double val) { stg[(2 * rp + minus) * L + j] = (T)(val * fa); });
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nst = 2 * nrp, r_end = nst + (slice == nsplit - 1 ? Lp - L : 0);
+    for (int r = wave; r < r_end; r += 4) {
+        const bool pad = r >= nst;
+        int i = L + (r - nst);
+        if (!pad) {
+            const short2 lm = tri_lm[rp0 + (r >> 1)];
+            if ((r & 1) && lm.y == 0) continue;   // m = 0: one row per pair (uniform over the wave)
+            i = lm.x * lm.x + lm.x + ((r & 1) ? -lm.y : lm.y);
+        }
+        const size_t o = ((size_t)opi * Lp + i) * Lp;
+        for (int j = lane; j < Lp; j += 64) {
+            const T v = !pad && j < L ? stg[r * L + j] : (T)0;
+            if (MODE == 2) {
+                const __bf16 h = (__bf16)(float)v;
+                ((__bf16*)out)[o + j] = h;
+                out_lo[o + j] = (__bf16)((float)v - (float)h);
+            } else
+                ((T*)out)[o + j] = v;
+        }
+    }
+}
+
+// row pairs per workgroup of k_make_m2l_f16 and k_make_m2l: as many as the staging budget holds (two rows of
 // L floats each), so that several workgroups share a CU
 constexpr size_t M2L_F16_STAGE = 16 * 1024;   // p = 12: 12 pairs, 23 KB in all, 7 workgroups per CU
 
-size_t m2l_f16_work_bytes(int nops, int p) {
+size_t m2l_work_bytes(int nops, int p) {
     const int pI = 2 * p, nX = (pI + 1) * (pI + 2) / 2;
     return (size_t)nops * nX * sizeof(cplx) + (size_t)nops * (p + 1) * sizeof(double);
 }
@@ -368,6 +439,28 @@ void make_m2l_f16(const OpSpec* d_specs, int nops, int p, const F16Split& f16, v
                        (size_t)(p + 1 + L) * sizeof(double) + per_pair * pps;
     if (lds > 64 * 1024) throw Error(4, "FP16 split tables: order too large for the LDS staging");
     k_make_m2l_f16<<<nops * nsplit, 256, lds, st>>>(d_specs, p, pI, nX, Xall, facall, f16, pps, nsplit);
+    FMM_HIP(hipGetLastError());
+}
+
+void make_m2l(const OpSpec* d_specs, int nops, int p, int Lp, int out_mode, void* d_out, __bf16* d_out_lo, void* work,
+              hipStream_t st) {
+    if (nops == 0) return;
+    const int L = (p + 1) * (p + 1), NP = (p + 1) * (p + 2) / 2, pI = 2 * p, nX = (pI + 1) * (pI + 2) / 2;
+    cplx* Xall = (cplx*)work;
+    double* facall = (double*)(Xall + (size_t)nops * nX);
+    k_m2l_harmonics<<<blocks((long long)nops * (pI + 1)), 256, 0, st>>>(d_specs, nops, p, pI, nX, Xall, facall);
+    FMM_HIP(hipGetLastError());
+    const size_t per_pair = 2 * (size_t)L * (out_mode == 0 ? sizeof(double) : sizeof(float));
+    const int pps = (int)std::max<size_t>(1, std::min<size_t>(NP, M2L_F16_STAGE / per_pair));
+    const int nsplit = (NP + pps - 1) / pps;
+    const size_t lds = (size_t)nX * sizeof(cplx) + (size_t)((NP + 1) & ~1) * sizeof(short2) +
+                       (size_t)(p + 1) * sizeof(double) + per_pair * pps;
+    auto go = [&](auto kern) {
+        kern<<<nops * nsplit, 256, lds, st>>>(d_specs, p, pI, nX, Lp, Xall, facall, d_out, d_out_lo, pps, nsplit);
+    };
+    if (out_mode == 0) go(k_make_m2l<0>);
+    else if (out_mode == 1) go(k_make_m2l<1>);
+    else go(k_make_m2l<2>);
     FMM_HIP(hipGetLastError());
 }
 

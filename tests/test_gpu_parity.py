@@ -300,6 +300,29 @@ def test_expansions_fp64(fm, orc, small_case):
     assert checked > 20
 
 
+@pytest.mark.parametrize("p", [1, 2, 9, 20])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-9), ("fp32", 1e-5), ("bf16x3", 1e-4)])
+def test_local_expansions_of_the_short_m2l(fm, orc, p, precision, tol):
+    """M2L tables with l + lambda <= p (m2l_full = 0), whole rows and padding, at the smallest and largest
+    orders: a node's largest coefficient to 1e-9 in FP64 (as test_expansions_fp64), 100 units of the last
+    place in FP32 and as much above it with bf16 splits (2^-16 a factor) as in the tests of B."""
+    src, w, tgt = _inputs(31, 3000, 800)
+    R = orc.FMMRun(src, w, tgt, p=p, cap_s=32, cap_t=32, flags=orc.SECTORAL_FIX | orc.FACT_FIX, target_root=SHARED_ROOT)
+    F = fm.FMM(order=p, source_leaf_capacity=32, target_leaf_capacity=32, precision=precision, frame=1, m2l_full=0)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    F.run(1.0)
+    T = orc.target_tree(tgt, 32, root=SHARED_ROOT)
+    checked = 0
+    for b in range(0, len(T.level), max(1, len(T.level) // 40)):
+        if T.first_child[b] < 0 and T.npts[b] == 0:
+            continue
+        Lo = R.local(b)
+        assert np.abs(F.expansion(1, b) - Lo).max() <= tol * np.abs(Lo).max()
+        checked += 1
+    assert checked > 10
+
+
 # measured: fp32 2.2e-7, bf16x3 9.6e-7, f16x3 2.1e-7
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("fp32", 1e-6), ("bf16x3", 1e-5), ("f16x3", 1e-6)])
 def test_B_matches_oracle(fm, orc, small_case, precision, tol):
