@@ -438,46 +438,55 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
     P2[j] = (R)sq[3 * j + 2];
 }
 
-// One workgroup (4 waves) per target leaf.  The 64-source chunks of the leaf's close list are
-// dealt round-robin to the waves; each wave stages a chunk in its own LDS slice and its lanes
-// sweep it, G = floor(64 / n) lanes per target for a leaf of 8 <= n <= 64 targets (64 / 2^ceil(log2 n)
-// below 8; lane = target * G + g takes sources g, g + G, ...).  Lane partials are summed over
-// the G lanes, then over the 4 waves in a fixed order, and written once.
+// One workgroup (4 waves) per target leaf.  The sources of the close list are taken 256 at a time
+// whatever nodes they come from: 64 list entries at a time give a table of slot ranges in LDS, each
+// thread finds its source in it, and the batch after the current one is on its way while the current
+// one is summed from LDS.  The leaf's targets go in even blocks of at most 128, n of them spread over
+// the workgroup with G = floor(256 / n) lanes each: lane g n + t takes the sources g, g + G, ... for target
+// t, so the lanes of a wave read one or a few sources at a time (broadcasts).  Partial sums of at most 64
+// terms in R are added up in FP64, over the G lanes in a fixed order.
 // KIND: B, the vector potential sum_j q_j / |x - y_j|, or the BEM potential (FP64), whose source has a
 // strength v = q and a number d (in the place of the low part of its x).
-// The chunks may be shared by `parts` (a power of 2) workgroups per leaf, each writing its own sums.
+// The batches may be shared by `parts` workgroups per leaf, each writing its own sums.
 // UP: the leaf takes the lists of its ancestors as well (parent[] up to the root): the transposed
 // near field, where a source leaf is reached through the close pairs of any node that holds it.
+//
+// Bound by VALU issue (26 instructions a pair in FP32).  With a wave per 64-source chunk of a node and
+// floor(64 / n) lanes a target, a leaf of 33 .. 63 targets left 2 to 48 % of the lanes idle and a node's
+// last chunk was short: B and A of 250,000 shell points 0.53 + 0.41 -> 0.36 + 0.31 ms, the transposed
+// near field of 262,147 x 131,101 clustered points (3.6e8 pairs) 2.14 -> 1.27 ms.
 enum { NEAR_B, NEAR_A, NEAR_BEM };
+template <class R> struct P2PShared {
+    typename V4<R>::t s0[256], s1[256];
+    R s2[256];
+    int nbegin[64], nfirst[65];   // the table: first slot and first source of each entry, and their number
+};
 template <class R, int KIND, int UNROLL, bool UP = false>
-__device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const int* __restrict__ tbegin, const int* __restrict__ tend,
-                                         const int* __restrict__ close_begin, const int* __restrict__ close_end,
-                                         const int* __restrict__ close_s, const double* __restrict__ origin,
-                                         const int* __restrict__ sbegin, const int* __restrict__ send,
-                                         const typename V4<R>::t* __restrict__ P0,
+__device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const int* __restrict__ tbegin,
+                                         const int* __restrict__ tend, const int* __restrict__ close_begin,
+                                         const int* __restrict__ close_end, const int* __restrict__ close_s,
+                                         const double* __restrict__ origin, const int* __restrict__ sbegin,
+                                         const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0,
                                          const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
-                                         const double* __restrict__ txyz, double* __restrict__ Bnear,
-                                         typename V4<R>::t (*s0)[64], typename V4<R>::t (*s1)[64], R (*s2)[64],
-                                         double (*red)[3][64], const int* __restrict__ parent = nullptr) {
+                                         const double* __restrict__ txyz, double* __restrict__ Bnear, P2PShared<R>& sh,
+                                         const int* __restrict__ parent = nullptr) {
     typedef typename V4<R>::t v4;
     constexpr bool split = sizeof(R) == 4;
     static_assert(KIND != NEAR_BEM || !split, "the BEM potential is FP64");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nw = 4 * parts, w0 = 4 * part + wave;
+    static_assert(sizeof(sh.s0) + sizeof(sh.s1) >= 256 * 3 * sizeof(double), "the sums reuse the source buffers");
+    double(*red)[3] = (double(*)[3])sh.s0;
+    const int tid = threadIdx.x;
     const int tb = tbegin[leaf], te = tend[leaf];
     if (!UP && close_begin[leaf] >= close_end[leaf]) {
         for (int k = tb + tid; k < te; k += 256) Bnear[3 * k] = Bnear[3 * k + 1] = Bnear[3 * k + 2] = 0.0;
         return;
     }
-    for (int k0 = tb; k0 < te; k0 += 64) {
-        const int n = min(64, te - k0);
-        // G lanes per target: 64 / n (n >= 8, at most 8 lanes, summed through LDS), else the power
-        // of 2 64 / 2^ceil(log2 n) (summed by shuffles)
-        const bool pow2 = n < 8;
-        const int lgG = 6 - (n <= 1 ? 0 : 32 - __clz(n - 1));
-        const int G = pow2 ? 1 << lgG : 64 / n;
-        const int ti = pow2 ? lane >> lgG : lane / G, g = lane - ti * G;
-        const bool valid = ti < n;
+    const int nblk = (te - tb + 127) / 128;
+    for (int blk = 0; blk < nblk; blk++) {
+        const int k0 = tb + (int)((long long)(te - tb) * blk / nblk);
+        const int n = tb + (int)((long long)(te - tb) * (blk + 1) / nblk) - k0;
+        const int G = 256 / n, g = tid / n, ti = tid - g * n;
+        const bool valid = g < G;
         double ux = 0, uy = 0, uz = 0;
         if (valid) {
             ux = txyz[3 * (k0 + ti)] - origin[0];
@@ -488,82 +497,105 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
         const R ulx = split ? (R)(ux - (double)uhx) : (R)0, uly = split ? (R)(uy - (double)uhy) : (R)0;
         const R ulz = split ? (R)(uz - (double)uhz) : (R)0;
         double a0 = 0, a1 = 0, a2 = 0;
-        // the close list's 64-source chunks, in list order, dealt round-robin to the waves (an
-        // internal close node can hold most of a leaf's sources)
-        int run = 0;   // chunks of the close nodes before ci
+        int run = 0;   // batches of the list entries before c0
         for (int node = leaf; node >= 0; node = UP ? parent[node] : -1)
-        for (int ci = close_begin[node], ce = close_end[node]; ci < ce; ci++) {
-            const int s = close_s[ci];
-            const int sb = sbegin[s], se = send[s];
-            const int nch = (se - sb + 63) >> 6;
-            for (int j0 = sb + 64 * ((w0 - run) & (nw - 1)); j0 < se; j0 += 64 * nw) {
-                const int nj = min(64, se - j0);
-                __syncwarp();
-                if (lane < nj) {
-                    s0[wave][lane] = P0[j0 + lane];
-                    s1[wave][lane] = P1[j0 + lane];
-                    s2[wave][lane] = P2[j0 + lane];
+        for (int c0 = close_begin[node], ce = close_end[node]; c0 < ce; c0 += 64) {
+            __syncthreads();   // the last table is no longer read
+            if (tid < 64) {
+                int b = 0, cnt = 0;
+                if (c0 + tid < ce) {
+                    const int s = close_s[c0 + tid];
+                    b = sbegin[s];
+                    cnt = send[s] - b;
                 }
-                __syncwarp();
-                R f0 = 0, f1 = 0, f2 = 0;
+                int incl = cnt;
+                for (int d = 1; d < 64; d <<= 1) {
+                    const int u = __shfl_up(incl, d, 64);
+                    if (tid >= d) incl += u;
+                }
+                sh.nbegin[tid] = b;
+                sh.nfirst[tid + 1] = incl;
+                if (tid == 0) sh.nfirst[0] = 0;
+            }
+            __syncthreads();
+            const int total = sh.nfirst[64], nbatch = (total + 255) >> 8;
+            // slot of source x of the table: the last entry with nfirst <= x that is not empty
+            auto slot = [&](int x) {
+                x = min(x, total - 1);
+                int e = 0;
+#pragma unroll
+                for (int d = 32; d > 0; d >>= 1)
+                    if (sh.nfirst[e + d] <= x) e += d;
+                return sh.nbegin[e] + (x - sh.nfirst[e]);
+            };
+            int b = (part - run) & (parts - 1);   // parts is a power of 2
+            run += nbatch;
+            if (b >= nbatch) continue;
+            int j = slot(256 * b + tid);
+            v4 p0 = P0[j], p1 = P1[j];
+            R p2 = P2[j];
+            for (; b < nbatch; b += parts) {
+                __syncthreads();   // the last batch is no longer read
+                sh.s0[tid] = p0;
+                sh.s1[tid] = p1;
+                sh.s2[tid] = p2;
+                const int nj = min(256, total - 256 * b);
+                j = slot(256 * (b + parts) + tid);   // beyond the end: the last source again
+                p0 = P0[j];
+                p1 = P1[j];
+                p2 = P2[j];
+                __syncthreads();
+                for (int q = valid ? g : nj; q < nj;) {
+                    const int qe = min(nj, q + 64 * G);
+                    R f0 = 0, f1 = 0, f2 = 0;
 #pragma unroll UNROLL
-                for (int jj = g; jj < nj; jj += G) {
-                    const v4 yh = s0[wave][jj];
-                    const v4 yl = s1[wave][jj];
-                    const R qx = yh.w, qy = yl.w, qz = s2[wave][jj];
-                    R dx = uhx - yh.x, dy = uhy - yh.y, dz = uhz - yh.z;
-                    if (split) {
-                        dx += ulx - yl.x;
-                        dy += uly - yl.y;
-                        dz += ulz - yl.z;
+                    for (; q < qe; q += G) {
+                        const v4 yh = sh.s0[q];
+                        const v4 yl = sh.s1[q];
+                        const R qx = yh.w, qy = yl.w, qz = sh.s2[q];
+                        R dx = uhx - yh.x, dy = uhy - yh.y, dz = uhz - yh.z;
+                        if (split) {
+                            dx += ulx - yl.x;
+                            dy += uly - yl.y;
+                            dz += ulz - yl.z;
+                        }
+                        // fused multiply-adds (explicit: this library is built without contraction)
+                        const R r2 = fma_t(dx, dx, fma_t(dy, dy, dz * dz));
+                        const R ip = inv_power<KIND == NEAR_A>(r2);
+                        if (KIND == NEAR_BEM) {   // (d (y - x) + (y - x) x v) / |y - x|^3
+                            f0 = fma_t(-fma_t(dx, yl.x, fma_t(dy, qz, -dz * qy)), ip, f0);
+                            f1 = fma_t(-fma_t(dy, yl.x, fma_t(dz, qx, -dx * qz)), ip, f1);
+                            f2 = fma_t(-fma_t(dz, yl.x, fma_t(dx, qy, -dy * qx)), ip, f2);
+                        } else if (KIND == NEAR_A) {
+                            f0 = fma_t(qx, ip, f0);
+                            f1 = fma_t(qy, ip, f1);
+                            f2 = fma_t(qz, ip, f2);
+                        } else {
+                            f0 = fma_t(fma_t(qy, dz, -qz * dy), ip, f0);
+                            f1 = fma_t(fma_t(qz, dx, -qx * dz), ip, f1);
+                            f2 = fma_t(fma_t(qx, dy, -qy * dx), ip, f2);
+                        }
                     }
-                    // fused multiply-adds (explicit: this library is built without contraction)
-                    const R r2 = fma_t(dx, dx, fma_t(dy, dy, dz * dz));
-                    const R ip = inv_power<KIND == NEAR_A>(r2);
-                    if (KIND == NEAR_BEM) {   // (d (y - x) + (y - x) x v) / |y - x|^3
-                        f0 = fma_t(-fma_t(dx, yl.x, fma_t(dy, qz, -dz * qy)), ip, f0);
-                        f1 = fma_t(-fma_t(dy, yl.x, fma_t(dz, qx, -dx * qz)), ip, f1);
-                        f2 = fma_t(-fma_t(dz, yl.x, fma_t(dx, qy, -dy * qx)), ip, f2);
-                    } else if (KIND == NEAR_A) {
-                        f0 = fma_t(qx, ip, f0);
-                        f1 = fma_t(qy, ip, f1);
-                        f2 = fma_t(qz, ip, f2);
-                    } else {
-                        f0 = fma_t(fma_t(qy, dz, -qz * dy), ip, f0);
-                        f1 = fma_t(fma_t(qz, dx, -qx * dz), ip, f1);
-                        f2 = fma_t(fma_t(qx, dy, -qy * dx), ip, f2);
-                    }
+                    a0 += f0;
+                    a1 += f1;
+                    a2 += f2;
                 }
-                a0 += f0;
-                a1 += f1;
-                a2 += f2;
-            }
-            run += nch;
-        }
-        if (pow2)
-            for (int off = 1; off < G; off <<= 1) {
-                a0 += __shfl_xor(a0, off);
-                a1 += __shfl_xor(a1, off);
-                a2 += __shfl_xor(a2, off);
-            }
-        red[wave][0][lane] = a0;
-        red[wave][1][lane] = a1;
-        red[wave][2][lane] = a2;
-        __syncthreads();
-        if (wave == 0 && valid && g == 0) {
-            const int k = k0 + ti;
-            for (int c = 0; c < 3; c++) {
-                double t[4];
-                for (int w = 0; w < 4; w++) {
-                    double sw = red[w][c][lane];
-                    if (!pow2)
-                        for (int gg = 1; gg < G; gg++) sw += red[w][c][lane + gg];
-                    t[w] = sw;
-                }
-                Bnear[3 * k + c] = ((t[0] + t[1]) + t[2]) + t[3];
             }
         }
-        __syncthreads();
+        __syncthreads();   // the last batch is no longer read
+        red[tid][0] = a0;
+        red[tid][1] = a1;
+        red[tid][2] = a2;
+        for (int h = G; h > 1;) {
+            const int half = (h + 1) >> 1;
+            __syncthreads();
+            if (g + half < h)
+                for (int c = 0; c < 3; c++) red[tid][c] += red[tid + half * n][c];
+            h = half;
+        }
+        if (tid < n)
+            for (int c = 0; c < 3; c++) Bnear[3 * (k0 + tid) + c] = red[tid][c];
+        __syncthreads();   // the next leaf or block writes the buffers again
     }
 }
 
@@ -584,14 +616,10 @@ __global__ __launch_bounds__(256) void k_p2p(const int* __restrict__ leaves, int
                                              const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
                                              const double* __restrict__ txyz, double* __restrict__ near,
                                              double* __restrict__ partial, size_t n3) {
-    __shared__ typename V4<R>::t s0[4][64];
-    __shared__ typename V4<R>::t s1[4][64];
-    __shared__ R s2[4][64];
-    __shared__ double red[4][3][64];
+    __shared__ P2PShared<R> sh;
     const int part = blockIdx.x & ((1 << lg_parts) - 1);
     p2p_leaf<R, KIND, 4>(leaves[blockIdx.x >> lg_parts], part, 1 << lg_parts, tbegin, tend, close_begin, close_end, close_s,
-                         origin, sbegin, send, P0, P1, P2, txyz, part ? partial + (part - 1) * n3 : near, s0, s1, s2,
-                         red);
+                         origin, sbegin, send, P0, P1, P2, txyz, part ? partial + (part - 1) * n3 : near, sh);
 }
 
 __global__ void k_add_parts(const double* __restrict__ partial, int nparts, size_t n3, double* __restrict__ near) {
@@ -607,7 +635,7 @@ __global__ void k_add_parts(const double* __restrict__ partial, int nparts, size
 // leaf or to one of its ancestors.  The roles of the forward near field are swapped, so the pairs run
 // in the same body: no atomics, and a sum whose order is fixed.  Bound by VALU issue like the forward
 // one; one wave per target leaf adding to the sources by FP64 atomics, its differences in plain FP32,
-// took 14.2 ms where this takes about 2 (262,147 x 131,101 clustered points, 3.6e8 pairs) and had put
+// took 14.2 ms where this takes 1.3 (262,147 x 131,101 clustered points, 3.6e8 pairs) and had put
 // 1.5e-6 into the FP32 gradient, now 1.4e-7.
 template <class R>
 __global__ __launch_bounds__(256) void k_p2p_transposed(
@@ -616,12 +644,9 @@ __global__ __launch_bounds__(256) void k_p2p_transposed(
     const int* __restrict__ close_t, const double* __restrict__ origin, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
     const R* __restrict__ P2, const double* __restrict__ sxyz, double* __restrict__ out) {
-    __shared__ typename V4<R>::t s0[4][64];
-    __shared__ typename V4<R>::t s1[4][64];
-    __shared__ R s2[4][64];
-    __shared__ double red[4][3][64];
+    __shared__ P2PShared<R> sh;
     p2p_leaf<R, NEAR_B, 4, true>(leaves[blockIdx.x], 0, 1, sbegin, send, close_begin, close_end, close_t, origin, tbegin, tend,
-                                P0, P1, P2, sxyz, out, s0, s1, s2, red, parent);
+                                P0, P1, P2, sxyz, out, sh, parent);
 }
 
 // The same near field as a persistent grid taking leaves from a queue (an atomic counter that starts at
@@ -641,10 +666,7 @@ __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, i
                                                const typename V4<R>::t* __restrict__ P0,
                                                const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
                                                const double* __restrict__ txyz, double* __restrict__ Bnear) {
-    __shared__ typename V4<R>::t s0[4][64];
-    __shared__ typename V4<R>::t s1[4][64];
-    __shared__ R s2[4][64];
-    __shared__ double red[4][3][64];
+    __shared__ P2PShared<R> sh;
     __shared__ int next;
     if (BESIDE) {
         if (threadIdx.x == 0) {
@@ -666,7 +688,7 @@ __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, i
         __syncthreads();   // every thread has read next before thread 0 takes the following leaf
         if (i >= nleaves) break;
         p2p_leaf<R, POT ? NEAR_A : NEAR_B, BESIDE ? 1 : 4>(leaves[i], 0, 1, tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send,
-                                         P0, P1, P2, txyz, Bnear, s0, s1, s2, red);
+                                         P0, P1, P2, txyz, Bnear, sh);
     }
 }
 template <class R, bool POT>
