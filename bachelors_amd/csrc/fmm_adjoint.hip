@@ -262,7 +262,7 @@ void run_adjoint(AdjointState& S, const AdjointArgs& a, const double* dLdB, doub
         k_gather_close<<<blocks(L.num_close), 256, 0, st>>>(S.close_ix.order.as<int>(), L.close_t.as<int>(),
                                                             L.num_close, ct);
         launch_p2p_transposed(f64, a.src_leaves, a.n_src_leaves, Ts, Tt, S.close_ix.begin.as<int>(),
-                              S.close_ix.end.as<int>(), ct, P0, P1, P2, a.sxyz, gn, st);
+                              S.close_ix.end.as<int>(), ct, P0, P1, P2, a.sxyz, gn, S.near, st);
     }
     // dL/dw = J . dL/dq (input order; sources outside the root keep 0)
     FMM_HIP(hipMemsetAsync(dLdw, 0, (size_t)std::max(a.ns, 1) * sizeof(double), st));

@@ -1,4 +1,5 @@
 #pragma once
+#include "fmm_expand.hpp"
 #include "fmm_gemm.hpp"
 #include "fmm_lists.hpp"
 
@@ -44,6 +45,7 @@ struct AdjointState {
     PairIndex m2l_ix;   // far pairs by source node
     DevBuf gn;          // near field at the sources
     PairIndex close_ix; // close pairs by source node
+    NearScratch near;   // of the transposed near field
     DevBuf close_t, P0, P1, P2;   // their targets in that order; the targets packed with g
 };
 

@@ -151,7 +151,7 @@ struct fmm_ctx {
     DevBuf sxyz, sq, sJ, txyz;                   // slot order
     DevBuf nP0, nP1, nP2;                        // near-field sources packed per leaf (slot order)
     DevBuf bP0, bP1, bP2;                        // the same for the near field of the BEM potential
-    DevBuf p2p_parts;                            // near-field sums of leaves shared by several workgroups
+    NearScratch p2p_parts;                       // work items and partial sums of the near field
     PinnedVec<int> h_src_leaves, h_tgt_leaves;   // useful (non-empty) leaves
     DevBuf src_leaves, tgt_leaves;
     // expansions [node][3][Lp]
@@ -171,7 +171,7 @@ struct fmm_ctx {
     // multipole column scales; down_l2l = L2L operators ahead of the M2L ones in the down tables
     DevBuf dm, m2l_hi, m2l_lo, m2l_rinv, m2l_work, cscale, Mhl;   // Mhl: split multipoles (hi | lo)
     DevBuf cratio, cpinv;                        // column scales against the siblings' smallest, and 1 / that
-    DevBuf queues;   // work counters: [0, 8) the M2L GEMM's per-XCD tiles, [8] the near-field leaves; [14, 16) probe
+    DevBuf queues;   // work counters: [0, 8) the M2L GEMM's per-XCD tiles, [14, 16) probe
     int down_l2l = 0;
     const OpSpec* down_specs = nullptr;          // device specs of the down tables
     DevBuf m2l_slab;                             // M2L result per (pair or group, component)
@@ -747,7 +747,7 @@ void translate_gemm(fmm_ctx* c, hipEvent_t gemm_after = nullptr, bool split_done
     const int R = m2l_slab_rows(c->prec, c->L, c->Lp);
     if (f16) {
         group_row_scales(c->groups, c->m2l_rinv.as<float>(), c->L, st);
-        FMM_HIP(hipMemsetAsync(c->queues.as<int>(), 0, 9 * sizeof(int), st));   // tiles, the near field's leaves
+        FMM_HIP(hipMemsetAsync(c->queues.as<int>(), 0, 8 * sizeof(int), st));
     }
     c->rec(E_GEMM0);
     if (P.npairs && f16) {
@@ -832,11 +832,11 @@ __global__ void k_fill_nan(double* p, size_t n) {
     if (i < n) p[i] = __longlong_as_double(0x7ff8000000000000ll);
 }
 
-// near field of the target leaves left in the queue, by a persistent grid on stream ps
+// near field of the items left in the queue, by a persistent grid on stream ps
 void p2p_from_queue(fmm_ctx* c, hipStream_t ps, int grid, bool beside) {
     launch_p2p_queue(c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S, c->lists.close_begin.as<int>(),
                      c->lists.close_end.as<int>(), c->lists.close_s.as<int>(), c->nP0.ptr, c->nP1.ptr, c->nP2.ptr,
-                     c->txyz.as<double>(), c->Bnear.as<double>(), c->queues.as<int>() + 8, c->queues.as<int>(),
+                     c->txyz.as<double>(), c->Bnear.as<double>(), c->p2p_parts, c->queues.as<int>(),
                      c->groups.num_tiles, grid, beside, ps);
 }
 
@@ -1047,6 +1047,10 @@ void run_fused(fmm_ctx* c, double current, double* Bdev) {
             if (src_state == 1) {
                 FMM_HIP(hipStreamWaitEvent(Bs, c->j_src, 0));   // the source tree on stream A
                 stage_lists(c, Bs, c->ev[E_FAR], [&] { post(far_state, 1); });   // E_FAR also joins
+                if (p2p_beside)
+                    prepare_p2p_queue(c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->S,
+                                      c->lists.close_begin.as<int>(), c->lists.close_end.as<int>(),
+                                      c->lists.close_s.as<int>(), c->p2p_parts, Bs);
                 FMM_HIP(hipEventRecord(c->j_lists, Bs));
                 post(lists_state, 1);
                 if (p2p_beside) {
@@ -1116,10 +1120,12 @@ void run_fused(fmm_ctx* c, double current, double* Bdev) {
         FMM_HIP(hipEventRecord(c->j_p2p, Bs));
     }
     stage_l2p(c);
-    // the leaves that the near field beside the GEMM has not taken: the chip is free now, and one
+    // the items that the near field beside the GEMM has not taken: the chip is free now, and one
     // workgroup per CU would take until long after
     if (p2p_beside) p2p_from_queue(c, A, 8 * num_cus(), false);
     FMM_HIP(hipStreamWaitEvent(A, c->j_p2p, 0));
+    if (p2p_beside)
+        finish_p2p_queue(c->tgt_leaves.as<int>(), (int)c->h_tgt_leaves.size(), c->T, c->Bnear.as<double>(), c->p2p_parts, A);
     stage_assemble(c, current, Bdev);
 }
 

@@ -447,7 +447,8 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
 // terms in R are added up in FP64, over the G lanes in a fixed order.
 // KIND: B, the vector potential sum_j q_j / |x - y_j|, or the BEM potential (FP64), whose source has a
 // strength v = q and a number d (in the place of the low part of its x).
-// The batches may be shared by `parts` workgroups per leaf, each writing its own sums.
+// The batches may be shared by `parts` workgroups per leaf, each writing its own sums; out: the leaf's
+// first row.
 // UP: the leaf takes the lists of its ancestors as well (parent[] up to the root): the transposed
 // near field, where a source leaf is reached through the close pairs of any node that holds it.
 //
@@ -461,14 +462,14 @@ template <class R> struct P2PShared {
     R s2[256];
     int nbegin[64], nfirst[65];   // the table: first slot and first source of each entry, and their number
 };
-template <class R, int KIND, int UNROLL, bool UP = false>
+template <class R, int KIND, bool UP>
 __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const int* __restrict__ tbegin,
                                          const int* __restrict__ tend, const int* __restrict__ close_begin,
                                          const int* __restrict__ close_end, const int* __restrict__ close_s,
                                          const double* __restrict__ origin, const int* __restrict__ sbegin,
                                          const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0,
                                          const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
-                                         const double* __restrict__ txyz, double* __restrict__ Bnear, P2PShared<R>& sh,
+                                         const double* __restrict__ txyz, double* __restrict__ out, P2PShared<R>& sh,
                                          const int* __restrict__ parent = nullptr) {
     typedef typename V4<R>::t v4;
     constexpr bool split = sizeof(R) == 4;
@@ -478,7 +479,7 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
     const int tid = threadIdx.x;
     const int tb = tbegin[leaf], te = tend[leaf];
     if (!UP && close_begin[leaf] >= close_end[leaf]) {
-        for (int k = tb + tid; k < te; k += 256) Bnear[3 * k] = Bnear[3 * k + 1] = Bnear[3 * k + 2] = 0.0;
+        for (int k = tid; k < te - tb; k += 256) out[3 * k] = out[3 * k + 1] = out[3 * k + 2] = 0.0;
         return;
     }
     const int nblk = (te - tb + 127) / 128;
@@ -548,7 +549,7 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
                 for (int q = valid ? g : nj; q < nj;) {
                     const int qe = min(nj, q + 64 * G);
                     R f0 = 0, f1 = 0, f2 = 0;
-#pragma unroll UNROLL
+#pragma unroll 1
                     for (; q < qe; q += G) {
                         const v4 yh = sh.s0[q];
                         const v4 yl = sh.s1[q];
@@ -594,40 +595,160 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
             h = half;
         }
         if (tid < n)
-            for (int c = 0; c < 3; c++) Bnear[3 * (k0 + tid) + c] = red[tid][c];
+            for (int c = 0; c < 3; c++) out[3 * (k0 - tb + tid) + c] = red[tid][c];
         __syncthreads();   // the next leaf or block writes the buffers again
     }
 }
 
-// Part 0 of a leaf writes `near`, part q its sums into partial[q - 1][n3] (n3 = 3 x target slots).
+// What the near field's workgroups work on: part 0 of every leaf, and the further parts of the leaves with
+// long lists, extra[] = (leaf, part).  desc[leaf] = (parts, first row of `partial` of the further parts).
+// counters: extra items made, rows made, items taken (by the grids that share them).  The first
+// extra_wgs workgroups of a grid of its own share the extra items in equal strides (they are of one size),
+// the others take a leaf each: a counter for all of 32,768 leaves, most of them short, took 0.4 ms more.
+// Without desc every leaf is one item.
 //
-// A workgroup per leaf leaves the chip idle when the leaves are few: their lists are walked one chunk of
-// a wave after the other, and the time is that of the longest list.  32,768 sources and 4,096 targets in
-// 276 leaves (3.3e7 pairs, FP64): 470 -> 112 us; the drop-in coil (38,400 sources in leaves of 1,000, 4,096
-// targets in leaves of 100) 1275 -> 150 us; a BEM solve (6,000, 1,999; one lane per target of a leaf in one
-// wave before) 375 -> 27 + 5 us.
+// A few leaves near the sources can hold most of the pairs: with one workgroup per leaf the time is that
+// of the longest list, or of the last ones to start (1M uniform targets around a coil of 1M sources: 1.0
+// ms in FP32, 2.7 ms in FP64; 32,768 x 4,096 points in 276 leaves, FP64: 470 us).  A part is therefore
+// at most `batches` batches of 256 sources (near_batches), and the register budget is that of 7 (FP64: 5) waves a
+// SIMD (no unrolling), since the short lists are a matter of latency: 1M points 1007 (items alone: 1230) ->
+// 660 us in FP32, 2.7 -> 2.0 ms in FP64, beside the slab reduction; 262,147 x 131,101 clustered points 1520
+// -> 330 us, transposed 1270 -> 420 us; B and A of 250,000 points 365 + 307 -> 267 + 237 us; 276 leaves 90
+// -> 75 us.
+struct NearWork {
+    const int* leaves;
+    int nleaves;
+    int2* desc;
+    int2* extra;
+    int* counters;
+    double* partial;
+    int extra_cap, extra_wgs;
+};
+
+// the parts of every leaf; 16 leaves a workgroup, 16 lanes a leaf.  Where the extra items or the rows run
+// out, a workgroup's leaves keep one part each.
+constexpr int NEAR_MAX_PARTS = 32;
+template <bool UP>
+__global__ __launch_bounds__(256) void k_near_items(NearWork w, int batches, int rows_cap, const int* __restrict__ tbegin,
+                                                    const int* __restrict__ tend, const int* __restrict__ parent,
+                                                    const int* __restrict__ close_begin,
+                                                    const int* __restrict__ close_end, const int* __restrict__ close_s,
+                                                    const int* __restrict__ sbegin, const int* __restrict__ send) {
+    __shared__ int first_item[16], first_row[16], parts_of[16], fits;
+    const int tid = threadIdx.x, u = tid >> 4, lane = tid & 15, li = 16 * blockIdx.x + u;
+    int n = 0;
+    long long load = 0;
+    if (li < w.nleaves) {
+        const int leaf = w.leaves[li];
+        n = tend[leaf] - tbegin[leaf];
+        for (int node = leaf; node >= 0; node = UP ? parent[node] : -1)
+            for (int ci = close_begin[node] + lane, ce = close_end[node]; ci < ce; ci += 16) {
+                const int s = close_s[ci];
+                load += send[s] - sbegin[s];
+            }
+    }
+    for (int d = 1; d < 16; d <<= 1) load += __shfl_xor(load, d);
+    int parts = 1;
+    while (parts < NEAR_MAX_PARTS && (long long)parts * batches * 256 < load) parts *= 2;
+    while (parts > 1 && (long long)(parts - 1) * n > 1 << 24) parts >>= 1;   // the sums below stay in 32 bits
+    if (lane == 0) {
+        parts_of[u] = parts;
+        first_row[u] = (parts - 1) * n;
+    }
+    __syncthreads();
+    if (tid < 16) {
+        const int p = parts_of[tid] - 1, r = first_row[tid];
+        int ip = p, ir = r;
+        for (int d = 1; d < 16; d <<= 1) {
+            const int vp = __shfl_up(ip, d, 16), vr = __shfl_up(ir, d, 16);
+            if (tid >= d) {
+                ip += vp;
+                ir += vr;
+            }
+        }
+        int bp = 0, br = 0;
+        if (tid == 15 && ip) {
+            bp = atomicAdd(&w.counters[0], ip);
+            br = atomicAdd(&w.counters[1], ir);
+        }
+        bp = __shfl(bp, 15, 16);
+        br = __shfl(br, 15, 16);
+        const int np = __shfl(ip, 15, 16), nr = __shfl(ir, 15, 16);
+        const bool ok = bp >= 0 && br >= 0 && bp <= w.extra_cap - np && br <= rows_cap - nr;
+        first_item[tid] = bp + ip - p;
+        first_row[tid] = br + ir - r;
+        if (tid == 0) fits = ok;
+        if (!ok)   // the items that this workgroup took are nobody's
+            for (int q = bp + tid; bp >= 0 && q < min(w.extra_cap, bp + np); q += 16) w.extra[q] = make_int2(-1, 0);
+    }
+    __syncthreads();
+    if (li >= w.nleaves) return;
+    if (!fits) parts = 1;
+    if (lane == 0) w.desc[li] = make_int2(parts, first_row[u]);
+    for (int q = 1 + lane; q < parts; q += 16) w.extra[first_item[u] + q - 1] = make_int2(li, q);
+}
+
+// near[leaf] += the sums of its further parts, in their order; a wave per leaf
+__global__ __launch_bounds__(256) void k_add_parts(NearWork w, const int* __restrict__ tbegin,
+                                                   const int* __restrict__ tend, double* __restrict__ near) {
+    const int li = 4 * blockIdx.x + (threadIdx.x >> 6);
+    if (li >= w.nleaves) return;
+    const int2 d = w.desc[li];
+    if (d.x == 1) return;
+    const int leaf = w.leaves[li], tb = tbegin[leaf], n = tend[leaf] - tb;
+    for (int e = threadIdx.x & 63; e < 3 * n; e += 64) {
+        double v = near[3 * (size_t)tb + e];
+#pragma unroll 8
+        for (int q = 0; q < d.x - 1; q++) v += w.partial[3 * ((size_t)d.y + (size_t)q * n) + e];
+        near[3 * (size_t)tb + e] = v;
+    }
+}
+
+// QUEUE: items from the counter (leaves, then extra items); else those of this workgroup
+template <class R, int KIND, bool UP, bool QUEUE>
+__device__ __forceinline__ void p2p_items(const NearWork& w, const int* __restrict__ tbegin,
+                                          const int* __restrict__ tend, const int* __restrict__ close_begin,
+                                          const int* __restrict__ close_end, const int* __restrict__ close_s,
+                                          const double* __restrict__ origin, const int* __restrict__ sbegin,
+                                          const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0,
+                                          const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
+                                          const double* __restrict__ txyz, double* __restrict__ near,
+                                          const int* __restrict__ parent = nullptr) {
+    __shared__ P2PShared<R> sh;
+    __shared__ int next;
+    const int nextra = w.desc ? min(w.counters[0], w.extra_cap) : 0;
+    // i < nleaves: part 0 of leaf i, else extra item i - nleaves
+    const bool own = !QUEUE && (int)blockIdx.x >= w.extra_wgs;   // one leaf
+    for (int i = own ? blockIdx.x - w.extra_wgs : w.nleaves + blockIdx.x;; i += w.extra_wgs) {
+        if (QUEUE) {
+            if (threadIdx.x == 0) next = atomicAdd(&w.counters[2], 1);
+            __syncthreads();
+            i = next;
+            __syncthreads();   // every thread has read next before thread 0 takes the following item
+        }
+        if (i >= w.nleaves + nextra) break;
+        const int2 it = i < w.nleaves ? make_int2(i, 0) : w.extra[i - w.nleaves];
+        if (it.x >= 0) {
+            const int leaf = w.leaves[it.x], tb = tbegin[leaf];
+            const int2 d = w.desc ? w.desc[it.x] : make_int2(1, 0);
+            double* out = it.y ? w.partial + 3 * ((size_t)d.y + (size_t)(it.y - 1) * (tend[leaf] - tb)) : near + 3 * (size_t)tb;
+            p2p_leaf<R, KIND, UP>(leaf, it.y, d.x, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+                                          send, P0, P1, P2, txyz, out, sh, parent);
+        }
+        if (own) break;
+    }
+}
+
 template <class R, int KIND>
-__global__ __launch_bounds__(256) void k_p2p(const int* __restrict__ leaves, int lg_parts,
-                                             const int* __restrict__ tbegin, const int* __restrict__ tend,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 7 : 5))) void k_p2p(NearWork w, const int* __restrict__ tbegin, const int* __restrict__ tend,
                                              const int* __restrict__ close_begin, const int* __restrict__ close_end,
                                              const int* __restrict__ close_s, const double* __restrict__ origin,
                                              const int* __restrict__ sbegin, const int* __restrict__ send,
                                              const typename V4<R>::t* __restrict__ P0,
                                              const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
-                                             const double* __restrict__ txyz, double* __restrict__ near,
-                                             double* __restrict__ partial, size_t n3) {
-    __shared__ P2PShared<R> sh;
-    const int part = blockIdx.x & ((1 << lg_parts) - 1);
-    p2p_leaf<R, KIND, 4>(leaves[blockIdx.x >> lg_parts], part, 1 << lg_parts, tbegin, tend, close_begin, close_end, close_s,
-                         origin, sbegin, send, P0, P1, P2, txyz, part ? partial + (part - 1) * n3 : near, sh);
-}
-
-__global__ void k_add_parts(const double* __restrict__ partial, int nparts, size_t n3, double* __restrict__ near) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n3) return;
-    double v = near[i];
-    for (int q = 0; q < nparts; q++) v += partial[q * n3 + i];
-    near[i] = v;
+                                             const double* __restrict__ txyz, double* __restrict__ near) {
+    p2p_items<R, KIND, false, false>(w, tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send, P0, P1, P2,
+                                        txyz, near);
 }
 
 // The transposed near field (adjoint): per useful source leaf, sum_i g_i x (y_j - x_i) / |y_j - x_i|^3
@@ -638,27 +759,24 @@ __global__ void k_add_parts(const double* __restrict__ partial, int nparts, size
 // took 14.2 ms where this takes 1.3 (262,147 x 131,101 clustered points, 3.6e8 pairs) and had put
 // 1.5e-6 into the FP32 gradient, now 1.4e-7.
 template <class R>
-__global__ __launch_bounds__(256) void k_p2p_transposed(
-    const int* __restrict__ leaves, const int* __restrict__ sbegin, const int* __restrict__ send,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 7 : 5))) void k_p2p_transposed(
+    NearWork w, const int* __restrict__ sbegin, const int* __restrict__ send,
     const int* __restrict__ parent, const int* __restrict__ close_begin, const int* __restrict__ close_end,
     const int* __restrict__ close_t, const double* __restrict__ origin, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
     const R* __restrict__ P2, const double* __restrict__ sxyz, double* __restrict__ out) {
-    __shared__ P2PShared<R> sh;
-    p2p_leaf<R, NEAR_B, 4, true>(leaves[blockIdx.x], 0, 1, sbegin, send, close_begin, close_end, close_t, origin, tbegin, tend,
-                                P0, P1, P2, sxyz, out, sh, parent);
+    p2p_items<R, NEAR_B, true, false>(w, sbegin, send, close_begin, close_end, close_t, origin, tbegin, tend, P0, P1,
+                                         P2, sxyz, out, parent);
 }
 
-// The same near field as a persistent grid taking leaves from a queue (an atomic counter that starts at
-// 0), two forms of which may share a queue: BESIDE with a register budget of 56 per lane (no unrolling),
-// one workgroup of which fits on a CU beside the F16X3 M2L GEMM's, so the near field runs on the VALU
-// slots the GEMM leaves idle, and the plain one for the leaves left when the GEMM is done.  A BESIDE
-// workgroup that starts when the GEMM's tiles are all taken (their streams share a hardware queue and
-// run one after the other) leaves the leaves to the other form: one workgroup per CU alone takes 25 ms
-// for the 7 ms of near field of the 4M shells.
+// The near field by two persistent grids that take their items from the one counter: BESIDE with a small
+// register budget, one workgroup of which fits on a CU beside the F16X3 M2L GEMM's, so the
+// near field runs on the VALU slots the GEMM leaves idle, and the plain one for the items left when the
+// GEMM is done.  A BESIDE workgroup that starts when the GEMM's tiles are all taken (their streams share a
+// hardware queue and run one after the other) leaves the items to the other form: one workgroup per CU
+// alone takes 25 ms for the 7 ms of near field of the 4M shells.
 template <class R, bool POT, bool BESIDE>
-__device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, int nleaves, int* __restrict__ queue,
-                                               const int* __restrict__ gemm_queues, int gemm_tiles,
+__device__ __forceinline__ void p2p_queue_body(const NearWork& w, const int* __restrict__ gemm_queues, int gemm_tiles,
                                                const int* __restrict__ tbegin, const int* __restrict__ tend,
                                                const int* __restrict__ close_begin, const int* __restrict__ close_end,
                                                const int* __restrict__ close_s, const double* __restrict__ origin,
@@ -666,51 +784,39 @@ __device__ __forceinline__ void p2p_queue_body(const int* __restrict__ leaves, i
                                                const typename V4<R>::t* __restrict__ P0,
                                                const typename V4<R>::t* __restrict__ P1, const R* __restrict__ P2,
                                                const double* __restrict__ txyz, double* __restrict__ Bnear) {
-    __shared__ P2PShared<R> sh;
-    __shared__ int next;
     if (BESIDE) {
+        __shared__ int tiles;
         if (threadIdx.x == 0) {
             int left = 0;   // tiles of the XCDs' eighths not yet taken
             for (int x = 0; x < 8; x++)
                 left += max(0, (gemm_tiles >> 3) + (x < (gemm_tiles & 7) ? 1 : 0) -
                                    __hip_atomic_load(gemm_queues + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            next = left;
+            tiles = left;
         }
         __syncthreads();
-        const bool gone = next == 0;
-        __syncthreads();
-        if (gone) return;
+        if (tiles == 0) return;
     }
-    for (;;) {
-        if (threadIdx.x == 0) next = atomicAdd(queue, 1);
-        __syncthreads();
-        const int i = next;
-        __syncthreads();   // every thread has read next before thread 0 takes the following leaf
-        if (i >= nleaves) break;
-        p2p_leaf<R, POT ? NEAR_A : NEAR_B, BESIDE ? 1 : 4>(leaves[i], 0, 1, tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send,
-                                         P0, P1, P2, txyz, Bnear, sh);
-    }
+    p2p_items<R, POT ? NEAR_A : NEAR_B, false, true>(w, tbegin, tend, close_begin, close_end, close_s,
+                                                                     origin, sbegin, send, P0, P1, P2, txyz, Bnear);
 }
 template <class R, bool POT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(10))) void k_p2p_queue(
-    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ gemm_queues,
-    int gemm_tiles, const int* __restrict__ tbegin,
+    NearWork w, const int* __restrict__ gemm_queues, int gemm_tiles, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
     const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
     const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
     const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
-    p2p_queue_body<R, POT, true>(leaves, nleaves, queue, gemm_queues, gemm_tiles, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+    p2p_queue_body<R, POT, true>(w, gemm_queues, gemm_tiles, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
                                  send, P0, P1, P2, txyz, Bnear);
 }
 template <class R, bool POT>
-__global__ __launch_bounds__(256) void k_p2p_queue_rest(
-    const int* __restrict__ leaves, int nleaves, int* __restrict__ queue, const int* __restrict__ gemm_queues,
-    int gemm_tiles, const int* __restrict__ tbegin,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_p2p_queue_rest(
+    NearWork w, const int* __restrict__ gemm_queues, int gemm_tiles, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
     const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
     const int* __restrict__ send, const typename V4<R>::t* __restrict__ P0, const typename V4<R>::t* __restrict__ P1,
     const R* __restrict__ P2, const double* __restrict__ txyz, double* __restrict__ Bnear) {
-    p2p_queue_body<R, POT, false>(leaves, nleaves, queue, gemm_queues, gemm_tiles, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
+    p2p_queue_body<R, POT, false>(w, gemm_queues, gemm_tiles, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
                                   send, P0, P1, P2, txyz, Bnear);
 }
 
@@ -1060,76 +1166,129 @@ void launch_pack_sources(bool f64, int n, const double* origin, const double* sx
         k_pack_sources<float><<<blocks(n), 256, 0, st>>>(n, origin, sxyz, sq, nullptr, (float4*)P0, (float4*)P1, (float*)P2);
     FMM_HIP(hipGetLastError());
 }
-// workgroups per leaf, a power of 2: enough for some 8 to 16 workgroups a CU in all (6 to 8 are resident at
-// a time; the rest evens out the lists), at most 16, and one where there are few sources to share
-static int p2p_lg_parts(int nleaves, int nsources) {
-    int lg = 0;
-    while (lg < 4 && ((long long)nleaves << lg) <= 8LL * num_cus() && (nsources >> (lg + 9)) > 0) lg++;
-    return lg;
+// batches per part: 16 (4,096 sources) where there are leaves enough for 8 workgroups a CU, fewer where
+// the parts have to fill the chip
+static int near_batches(int nleaves) { return std::max(2, std::min(16, 2 * nleaves / num_cus())); }
+constexpr int NEAR_SPLIT_SOURCES = 1024;   // below, the items cost more launches than they save
+
+static NearWork near_work(const int* leaves, int nleaves, size_t rows, NearScratch& scratch) {
+    NearWork w;
+    w.leaves = leaves;
+    w.nleaves = nleaves;
+    w.extra_cap = 4 * nleaves + 65536;
+    w.extra_wgs = 0;
+    w.desc = scratch.desc.get<int2>(nleaves);
+    w.extra = scratch.extra.get<int2>(w.extra_cap);
+    w.counters = scratch.counters.get<int>(4);
+    w.partial = scratch.partial.get<double>(3 * rows);
+    return w;
 }
+// rows of partial sums: of 2 more parts per target, and what small problems take
+static size_t near_rows(int nslots) { return 2 * (size_t)nslots + 262144; }
+
+template <bool UP>
+static void make_items(const NearWork& w, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                       const int* close_end, const int* close_s, hipStream_t st) {
+    FMM_HIP(hipMemsetAsync(w.counters, 0, 3 * sizeof(int), st));
+    k_near_items<UP><<<(w.nleaves + 15) / 16, 256, 0, st>>>(
+        w, near_batches(w.nleaves), (int)std::min<size_t>(near_rows(T.num_slots), INT32_MAX), T.begin.as<int>(),
+        T.end.as<int>(), T.parent.as<int>(), close_begin, close_end, close_s, S.begin.as<int>(), S.end.as<int>());
+    FMM_HIP(hipGetLastError());
+}
+static void add_parts(const NearWork& w, const TreeDev& T, double* near, hipStream_t st) {
+    k_add_parts<<<(w.nleaves + 3) / 4, 256, 0, st>>>(w, T.begin.as<int>(), T.end.as<int>(), near);
+    FMM_HIP(hipGetLastError());
+}
+// the items of a near field into scratch, and its grid
+template <bool UP>
+static NearWork start_near(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                           const int* close_end, const int* close_s, NearScratch& scratch, int& grid, hipStream_t st) {
+    NearWork w{leaves, nleaves, nullptr, nullptr, nullptr, nullptr, 0, 0};
+    grid = nleaves;
+    if (S.num_slots > NEAR_SPLIT_SOURCES) {
+        w = near_work(leaves, nleaves, near_rows(T.num_slots), scratch);
+        make_items<UP>(w, T, S, close_begin, close_end, close_s, st);
+        w.extra_wgs = (int)std::min<long long>(8LL * num_cus(), (long long)NEAR_MAX_PARTS * nleaves);
+        grid += w.extra_wgs;
+    }
+    return w;
+}
+
 template <int KIND>
 static void p2p_launch(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S,
                        const int* close_begin, const int* close_end, const int* close_s, const void* P0,
-                       const void* P1, const void* P2, const double* txyz, double* out, DevBuf& scratch, hipStream_t st) {
+                       const void* P1, const void* P2, const double* txyz, double* out, NearScratch& scratch,
+                       hipStream_t st) {
     if (!nleaves) return;
-    const int lg = p2p_lg_parts(nleaves, S.num_slots), more = (1 << lg) - 1;
-    const size_t n3 = 3 * (size_t)T.num_slots;
-    double* partial = more ? scratch.get<double>(more * n3) : nullptr;
+    int grid;
+    const NearWork w = start_near<false>(leaves, nleaves, T, S, close_begin, close_end, close_s, scratch, grid, st);
     if (f64)
-        k_p2p<double, KIND><<<nleaves << lg, 256, 0, st>>>(leaves, lg, T.begin.as<int>(), T.end.as<int>(),
-                                                           close_begin, close_end, close_s, S.center.as<double>(),
-                                                           S.begin.as<int>(), S.end.as<int>(), (const double4*)P0,
-                                                           (const double4*)P1, (const double*)P2, txyz, out, partial, n3);
+        k_p2p<double, KIND><<<grid, 256, 0, st>>>(w, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
+                                                  S.center.as<double>(), S.begin.as<int>(), S.end.as<int>(),
+                                                  (const double4*)P0, (const double4*)P1, (const double*)P2, txyz, out);
     else if constexpr (KIND != NEAR_BEM)
-        k_p2p<float, KIND><<<nleaves << lg, 256, 0, st>>>(leaves, lg, T.begin.as<int>(), T.end.as<int>(),
-                                                          close_begin, close_end, close_s, S.center.as<double>(),
-                                                          S.begin.as<int>(), S.end.as<int>(), (const float4*)P0,
-                                                          (const float4*)P1, (const float*)P2, txyz, out, partial, n3);
-    if (more) k_add_parts<<<blocks((long long)n3), 256, 0, st>>>(partial, more, n3, out);
+        k_p2p<float, KIND><<<grid, 256, 0, st>>>(w, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
+                                                 S.center.as<double>(), S.begin.as<int>(), S.end.as<int>(),
+                                                 (const float4*)P0, (const float4*)P1, (const float*)P2, txyz, out);
     FMM_HIP(hipGetLastError());
+    if (w.desc) add_parts(w, T, out, st);
 }
 void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                 const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                const double* txyz, double* Bnear, DevBuf& scratch, hipStream_t st) {
+                const double* txyz, double* Bnear, NearScratch& scratch, hipStream_t st) {
     p2p_launch<NEAR_B>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Bnear, scratch, st);
 }
 void launch_p2p_bem(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                     const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                    const double* txyz, double* out, DevBuf& scratch, hipStream_t st) {
+                    const double* txyz, double* out, NearScratch& scratch, hipStream_t st) {
     p2p_launch<NEAR_BEM>(true, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, out, scratch, st);
+}
+void launch_p2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                  const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
+                  const double* txyz, double* Anear, NearScratch& scratch, hipStream_t st) {
+    p2p_launch<NEAR_A>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Anear, scratch, st);
+}
+void prepare_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                       const int* close_end, const int* close_s, NearScratch& scratch, hipStream_t st) {
+    if (!nleaves) return;
+    make_items<false>(near_work(leaves, nleaves, near_rows(T.num_slots), scratch), T, S, close_begin, close_end, close_s, st);
 }
 void launch_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                       const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                      const double* txyz, double* Bnear, int* queue, const int* gemm_queues, int gemm_tiles, int grid,
-                      bool beside, hipStream_t st) {
+                      const double* txyz, double* Bnear, NearScratch& scratch, const int* gemm_queues, int gemm_tiles,
+                      int grid, bool beside, hipStream_t st) {
     if (!nleaves) return;
     if (grid < 1) throw Error(1, "near field: empty persistent grid");
+    const NearWork w = near_work(leaves, nleaves, near_rows(T.num_slots), scratch);
     (beside ? k_p2p_queue<float, false> : k_p2p_queue_rest<float, false>)<<<grid, 256, 0, st>>>(
-        leaves, nleaves, queue, gemm_queues, gemm_tiles, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
+        w, gemm_queues, gemm_tiles, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
         S.center.as<double>(), S.begin.as<int>(), S.end.as<int>(), (const float4*)P0, (const float4*)P1,
         (const float*)P2, txyz, Bnear);
     FMM_HIP(hipGetLastError());
 }
+void finish_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, double* Bnear, NearScratch& scratch,
+                      hipStream_t st) {
+    if (nleaves) add_parts(near_work(leaves, nleaves, near_rows(T.num_slots), scratch), T, Bnear, st);
+}
 void launch_p2p_transposed(bool f64, const int* leaves, int nleaves, const TreeDev& S, const TreeDev& T,
                            const int* close_begin, const int* close_end, const int* close_t, const void* P0,
-                           const void* P1, const void* P2, const double* sxyz, double* out, hipStream_t st) {
+                           const void* P1, const void* P2, const double* sxyz, double* out, NearScratch& scratch,
+                           hipStream_t st) {
     if (!nleaves) return;
+    int grid;
+    const NearWork w = start_near<true>(leaves, nleaves, S, T, close_begin, close_end, close_t, scratch, grid, st);
     if (f64)
-        k_p2p_transposed<double><<<nleaves, 256, 0, st>>>(
-            leaves, S.begin.as<int>(), S.end.as<int>(), S.parent.as<int>(), close_begin, close_end, close_t,
+        k_p2p_transposed<double><<<grid, 256, 0, st>>>(
+            w, S.begin.as<int>(), S.end.as<int>(), S.parent.as<int>(), close_begin, close_end, close_t,
             S.center.as<double>(), T.begin.as<int>(), T.end.as<int>(), (const double4*)P0, (const double4*)P1,
             (const double*)P2, sxyz, out);
     else
-        k_p2p_transposed<float><<<nleaves, 256, 0, st>>>(
-            leaves, S.begin.as<int>(), S.end.as<int>(), S.parent.as<int>(), close_begin, close_end, close_t,
+        k_p2p_transposed<float><<<grid, 256, 0, st>>>(
+            w, S.begin.as<int>(), S.end.as<int>(), S.parent.as<int>(), close_begin, close_end, close_t,
             S.center.as<double>(), T.begin.as<int>(), T.end.as<int>(), (const float4*)P0, (const float4*)P1,
             (const float*)P2, sxyz, out);
     FMM_HIP(hipGetLastError());
-}
-void launch_p2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
-                  const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                  const double* txyz, double* Anear, DevBuf& scratch, hipStream_t st) {
-    p2p_launch<NEAR_A>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Anear, scratch, st);
+    if (w.desc) add_parts(w, S, out, st);
 }
 void launch_assemble(const int* slots, int n, const double* Bfar, const double* Bnear, double scale, double* B,
                      hipStream_t st) {

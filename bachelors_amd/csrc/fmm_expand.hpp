@@ -25,23 +25,33 @@ void launch_l2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, cons
 // slot, P2: R per slot, R = double if f64 else float; sd (f64 only): the BEM sources' d
 void launch_pack_sources(bool f64, int n, const double* origin, const double* sxyz, const double* sq, void* P0,
                          void* P1, void* P2, hipStream_t st, const double* sd = nullptr);
-// few leaves are shared by several workgroups each, whose sums go through scratch
+// the work items of a near field (leaves with long close lists are shared by several workgroups) and the
+// sums of their further parts; 48 bytes a target and 6 MB
+struct NearScratch {
+    DevBuf desc, extra, counters, partial;
+};
 void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                 const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                const double* txyz, double* Bnear, DevBuf& scratch, hipStream_t st);
-// launch_p2p in FP32 as a persistent grid of `grid` workgroups taking leaves from the counter *queue (0
-// at the start; several grids may share it); beside: with a small register budget that lets a workgroup
-// share its CU with one of the M2L GEMM's, whose tile counters and tiles are given
+                const double* txyz, double* Bnear, NearScratch& scratch, hipStream_t st);
+// launch_p2p in FP32 in pieces: prepare makes the items (needs the lists only); then one or more
+// persistent grids of `grid` workgroups, on streams of their own, take them from one counter; finish, after
+// all of them, adds the parts up.  beside: with a small register budget that lets a workgroup share its CU
+// with one of the M2L GEMM's, whose tile counters and tiles are given
+void prepare_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                       const int* close_end, const int* close_s, NearScratch& scratch, hipStream_t st);
 void launch_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                       const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                      const double* txyz, double* Bnear, int* queue, const int* gemm_queues, int gemm_tiles, int grid,
-                      bool beside, hipStream_t st);
+                      const double* txyz, double* Bnear, NearScratch& scratch, const int* gemm_queues, int gemm_tiles,
+                      int grid, bool beside, hipStream_t st);
+void finish_p2p_queue(const int* leaves, int nleaves, const TreeDev& T, double* Bnear, NearScratch& scratch,
+                      hipStream_t st);
 // the transposed near field at the sources (slot order, written whole for the leaves given): the
 // targets are packed by launch_pack_sources with their strengths, relative to the same origin (the
 // source root's centre); close_begin / close_end / close_t: the close targets of every source node
 void launch_p2p_transposed(bool f64, const int* leaves, int nleaves, const TreeDev& S, const TreeDev& T,
                            const int* close_begin, const int* close_end, const int* close_t, const void* P0,
-                           const void* P1, const void* P2, const double* sxyz, double* out, hipStream_t st);
+                           const void* P1, const void* P2, const double* sxyz, double* out, NearScratch& scratch,
+                           hipStream_t st);
 void launch_assemble(const int* slots, int n, const double* Bfar, const double* Bnear, double scale, double* B,
                      hipStream_t st);
 // L2P / P2P of the vector potential A (the calcA counterparts of launch_l2p / launch_p2p)
@@ -49,7 +59,7 @@ void launch_l2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, co
                   const void* Lexp, int p, int Lp, double* Afar, hipStream_t st);
 void launch_p2p_A(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                   const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                  const double* txyz, double* Anear, DevBuf& scratch, hipStream_t st);
+                  const double* txyz, double* Anear, NearScratch& scratch, hipStream_t st);
 // Problem::BEM: slot-order strengths v = w (B x n) (3) and d = w (B . n) of BEMQuadrature sources;
 // their multipoles (P2M of the gradient of R); the near field of their potential (FP64, unscaled) from
 // sources packed in FP64 with q = v and their d
@@ -59,7 +69,7 @@ void launch_p2m_bem(bool f64, const int* leaves, int nleaves, const TreeDev& S, 
                     const double* sxyz, const double* sv, const double* sd, int p, int Lp, void* M, hipStream_t st);
 void launch_p2p_bem(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                     const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                    const double* txyz, double* out, DevBuf& scratch, hipStream_t st);
+                    const double* txyz, double* out, NearScratch& scratch, hipStream_t st);
 // FP64 direct sum of B (pot: A) at nt targets over the ns slot-order sources, scaled; the sources
 // are cut into nsplit ranges whose partial sums (partial: nsplit * nt * 3 doubles) are added in
 // range order.  direct_splits: the number of ranges that fills the GPU.
