@@ -11,6 +11,13 @@
 
 namespace fmm {
 
+// Far pairs per class from which groups are made.  A class of few pairs falls into group classes of fewer
+// still, whose tiles are mostly empty and read more operators, and the grouping waits twice for counts.
+// Grouped / single, whole evaluations: 375 pairs a class (p = 8) 3.5 / 3.9 ms, 1,860 (p = 12) 7.5 / 8.4, but 73
+// (p = 12) 6.2 / 5.3, 75 (p = 13) 1.80 / 1.45, 20 (p = 10) 1.92 / 1.54; the training clusters (182, p = 14) gain in
+// the slab what their GEMM loses.
+constexpr int GROUP_MIN_PAIRS = 128;
+
 static int bits_of(int n) {   // smallest b with 2^b >= n (at least 1)
     int b = 1;
     while (b < 31 && (1 << b) < n) b++;
@@ -184,6 +191,24 @@ __global__ void k_group_tiles(const int* __restrict__ mask, const uint32_t* __re
     tiles[toff[c] + (i - b) / GROUP_TILE] = t;
 }
 
+// every pair a group of its own (child 0 of its source), in class order as the pairs are
+__global__ void k_single_groups(const int* __restrict__ far_s, const uint32_t* __restrict__ class_flag,
+                                const uint32_t* __restrict__ class_pos, int n, int* __restrict__ fc,
+                                int* __restrict__ mask, int* __restrict__ cls_begin, int* __restrict__ cls_mask,
+                                int* __restrict__ cls_ops) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int c = (int)(class_pos[i] + class_flag[i]) - 1;
+    fc[i] = far_s[i];
+    mask[i] = 1;
+    if (class_flag[i]) {
+        cls_begin[c] = i;
+        cls_mask[c] = 1;
+        cls_ops[8 * (size_t)c] = c;
+    }
+    if (i == n - 1) cls_begin[c + 1] = n;
+}
+
 static HalfSizes half_sizes(const TreeDev& T) {
     HalfSizes h;
     for (int k = 0; k < MAX_LEVELS; k++)
@@ -197,6 +222,23 @@ void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_
     G.num = G.num_classes = G.num_tiles = 0;
     if (!n) {
         build_pair_index(nullptr, 0, T.num_nodes, ix, st);
+        return;
+    }
+    if (n < (long long)GROUP_MIN_PAIRS * L.num_classes) {
+        uint32_t *tcount = G.tcount.get<uint32_t>(n + 1), *toff = G.toff.get<uint32_t>(n + 1);
+        int *fc = G.fc.get<int>(n), *mask = G.mask.get<int>(n), *cb = G.cls_begin.get<int>(n + 1);
+        const int nc = L.num_classes;
+        k_single_groups<<<blocks(n), 256, 0, st>>>(L.far_s.as<int>(), class_flag, class_pos, n, fc, mask, cb,
+                                                   G.cls_mask.get<int>(nc), G.cls_ops.get<int>(8 * (size_t)nc));
+        k_group_tile_counts<<<blocks(n + 1), 256, 0, st>>>(cb, class_pos, class_flag, n, tcount);
+        exclusive_scan_u32(tcount, toff, n + 1, G.tmp, st);
+        k_group_tiles<<<blocks(n), 256, 0, st>>>(mask, class_pos, class_flag, cb, toff, n, G.tiles.get<GroupTile>(n),
+                                                 G.counts.get<unsigned>(4));
+        build_pair_index(L.far_t.as<int>(), n, T.num_nodes, ix, st);
+        FMM_HIP(hipGetLastError());
+        G.num = n;
+        G.num_classes = nc;
+        for (int c = 0; c < nc; c++) G.num_tiles += ceil_div(L.h_class_begin[c + 1] - L.h_class_begin[c], GROUP_TILE);
         return;
     }
     const int sb = bits_of(S.num_nodes + 1), tb = bits_of(T.num_nodes);

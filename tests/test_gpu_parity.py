@@ -353,6 +353,27 @@ def test_near_field_of_few_leaves(fm, orc, ns, nt, cap, precision, tol):
     assert rel_l2(F.B_parts()[1], R.Bnear) < tol
 
 
+@pytest.mark.parametrize("p", [1, 8, 12, 13, 14, 16, 18, 20])
+def test_f16x3_with_and_without_groups(fm, p):
+    """The F16X3 M2L over groups of far pairs (uniform points: many pairs per class) and over single pairs
+    (few per class) against FP64 on the same trees: 1e-6, as against the oracle."""
+    rng = np.random.default_rng(p)
+    for n, grouped in ((30000, True), (1500, False)):
+        src, tgt = rng.uniform(-2.9, 2.9, (n, 3)), rng.uniform(-2.9, 2.9, (n, 3))
+        w = rng.uniform(0.5, 1.5, n) / n
+        B = {}
+        for precision in ("fp64", "f16x3"):
+            F = fm.FMM(order=p, source_leaf_capacity=32, target_leaf_capacity=32, precision=precision, frame=1)
+            F.set_sources(src, w)
+            F.set_targets(tgt)
+            F.run(1.0)
+            B[precision] = F.B_parts()[0]
+            st = F.stats()
+            F.close()
+        assert (st["far_pairs"] >= 128 * st["m2l_classes"]) == grouped
+        assert rel_l2(B["f16x3"], B["fp64"]) < 1e-6
+
+
 def test_direct_sum_gpu_vs_oracle(fm, orc):
     import ctypes
     src, w, tgt = _inputs(12, 3000, 500)
