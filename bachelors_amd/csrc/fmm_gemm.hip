@@ -917,6 +917,13 @@ bool m2l_f16x3_persistent(int L) {
     const int nb = m2l_f16_rows(L) / 16;
     return nb >= 14 && nb <= 23;   // the 128-column tiles of launch_f16x3_128 below
 }
+// A class of few pairs falls into group classes of fewer still, whose tiles are mostly empty and read more
+// operators, and the grouping waits twice for counts; the persistent kernel loses least by it.  Grouped
+// against single pairs, GEMM alone or whole evaluations: persistent, 182 to 450 pairs a class (p = 14, 16) 0.87
+// to 1.0 of the time, 75 (p = 13, then the other kernel) 1.45 / 1.80 ms for single pairs; the other kernel, 2,094
+// pairs (p = 8) 1.11 / 1.66 ms for groups, 1,149 (p = 12) 6.14 / 6.3, but 184 (p = 12) 4.0 / 2.7 ms, 214 (p = 13)
+// 1.68 / 0.64 and 516 (p = 10) 0.89 / 0.51 for single pairs.
+int m2l_group_min_pairs(int L) { return m2l_f16x3_persistent(L) ? 128 : 1024; }
 int m2l_f16_kpad(int L) { return 32 * ((L + 31) / 32); }
 
 __global__ void k_sibling_scales(const int* __restrict__ parent, const int* __restrict__ first_child, int n,

@@ -73,6 +73,7 @@ int m2l_f16_rows(int L);
 // whether the F16X3 M2L of order (L = (p + 1)^2) runs as the persistent one-workgroup-per-CU kernel
 // (128-column tiles) that leaves room for a near-field workgroup per CU
 bool m2l_f16x3_persistent(int L);
+int m2l_group_min_pairs(int L);   // far pairs per class from which the F16X3 M2L runs over groups
 int m2l_f16_kpad(int L);
 // skip_first_child / skip_npts (per node, both or neither): columns of leaves with points are
 // left as they are (the P2M writes them, see launch_p2m); column ncols is set to zeros

@@ -11,13 +11,6 @@
 
 namespace fmm {
 
-// Far pairs per class from which groups are made.  A class of few pairs falls into group classes of fewer
-// still, whose tiles are mostly empty and read more operators, and the grouping waits twice for counts.
-// Grouped / single, whole evaluations: 375 pairs a class (p = 8) 3.5 / 3.9 ms, 1,860 (p = 12) 7.5 / 8.4, but 73
-// (p = 12) 6.2 / 5.3, 75 (p = 13) 1.80 / 1.45, 20 (p = 10) 1.92 / 1.54; the training clusters (182, p = 14) gain in
-// the slab what their GEMM loses.
-constexpr int GROUP_MIN_PAIRS = 128;
-
 static int bits_of(int n) {   // smallest b with 2^b >= n (at least 1)
     int b = 1;
     while (b < 31 && (1 << b) < n) b++;
@@ -217,14 +210,14 @@ static HalfSizes half_sizes(const TreeDev& T) {
 }
 
 void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_t* class_flag,
-                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, hipStream_t st) {
+                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, hipStream_t st) {
     const int n = L.num_far;
     G.num = G.num_classes = G.num_tiles = 0;
     if (!n) {
         build_pair_index(nullptr, 0, T.num_nodes, ix, st);
         return;
     }
-    if (n < (long long)GROUP_MIN_PAIRS * L.num_classes) {
+    if (n < (long long)min_pairs * L.num_classes) {
         uint32_t *tcount = G.tcount.get<uint32_t>(n + 1), *toff = G.toff.get<uint32_t>(n + 1);
         int *fc = G.fc.get<int>(n), *mask = G.mask.get<int>(n), *cb = G.cls_begin.get<int>(n + 1);
         const int nc = L.num_classes;

@@ -28,8 +28,9 @@ struct FarGroups {
 
 // Groups of the far pairs L (sorted by class; class_flag / class_pos: the class starts and their
 // exclusive scan, so pair i has class class_pos[i] + class_flag[i] - 1), and the index of the groups by
-// target node for reduce_pairs.  The host waits for the counts.
+// target node for reduce_pairs.  The host waits for the counts.  With fewer than min_pairs far pairs per
+// class every pair is a group of its own (no counts, no waits).
 void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_t* class_flag,
-                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, hipStream_t st);
+                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, hipStream_t st);
 
 }  // namespace fmm

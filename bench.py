@@ -144,8 +144,9 @@ def m2l_roofline(st, L, prec, traffic):
 def other_stage_rooflines(st, L, n_src, n_tgt, prec):
     """Achieved rates of the other stages from the stage-by-stage (no overlap) event times, with the
     algorithmic units of each: P2M and L2P bytes (positions, strengths, FP32 coefficients, FP64 B),
-    P2P pair interactions at 20 flop, the M2L slab reduction's bytes (one FP32 slab per far pair
-    read, the local expansions read and written)."""
+    P2P pair interactions at 20 flop, the M2L slab reduction's bytes (one slab block per far pair
+    read, the local expansions read and written; F16X3 stores one block per group of far pairs, whose
+    number the statistics do not hold: no bytes there)."""
     Lp = (L + 63) // 64 * 64
     b_coef = 4 if prec != "fp64" else 8
     rows = {}
@@ -162,11 +163,13 @@ def other_stage_rooflines(st, L, n_src, n_tgt, prec):
     red_ms = st["t_m2l"] - st["t_m2l_gemm"]
     R = Lp if prec == "bf16x3" else min(Lp, (L + 15) // 16 * 16)
     red_bytes = st["far_pairs"] * 3 * R * b_coef + 2 * st["target_nodes"] * 3 * Lp * b_coef
+    if prec == "f16x3":
+        red_bytes = None
     rows["m2l_reduction"] = {"ms": red_ms, "bytes": red_bytes, "bound": "hbm",
-                             "achieved_GBs": red_bytes / (red_ms * 1e-3) / 1e9 if red_ms > 0 else 0.0}
+                             "achieved_GBs": red_bytes / (red_ms * 1e-3) / 1e9 if red_bytes and red_ms > 0 else None}
     for r in rows.values():
         if r["bound"] == "hbm":
-            r["frac"] = r["achieved_GBs"] / HBM_GBS
+            r["frac"] = r["achieved_GBs"] / HBM_GBS if r["achieved_GBs"] is not None else None
         else:
             r["frac"] = r["achieved_TFs_at_20_flop"] / r["peak_TFs"]
     return rows
