@@ -501,7 +501,8 @@ struct M2LGroupArgs {
 // load is unconditional (rows beyond R are clamped and not stored, columns whose group lacks the child
 // read the column of zeros behind the nodes'): after a load that may have been skipped the compiler
 // cannot count the loads in flight and waits for all of them, the ones issued steps ahead included.
-template <int R, int Kp, int NQ>
+// SINGLE: every group is one pair, child 0 with the class's one operator: no scales to even out.
+template <int R, int Kp, int NQ, bool SINGLE = false>
 struct M2LTileLoads {
     const M2LGroupArgs& A;
     GroupTile tile;
@@ -518,7 +519,7 @@ struct M2LTileLoads {
             const bool valid = cl < 3 * tile.ng;
             const int g = tile.g0 + (valid ? cl / 3 : 0);
             col[c] = 3 * A.grp_fc[g] + cl % 3;
-            gm[c] = valid ? A.grp_mask[g] : 0;
+            gm[c] = !valid ? 0 : SINGLE ? 1 : A.grp_mask[g];
         }
     }
     __device__ __forceinline__ int row(int j) const {
@@ -527,7 +528,9 @@ struct M2LTileLoads {
     }
     // a wave stages 16 rows at a time: all of them exist or none
     __device__ __forceinline__ bool has_rows(int j) const { return 64 * (j + 1) <= R || 16 * wave + 64 * j < R; }
-    __device__ __forceinline__ size_t op(int o) const { return (size_t)A.cls_ops[8 * (size_t)tile.cls + o]; }
+    __device__ __forceinline__ size_t op(int o) const {
+        return SINGLE ? (size_t)tile.cls : (size_t)A.cls_ops[8 * (size_t)tile.cls + o];
+    }
     __device__ __forceinline__ void set_columns(int o, bool any = true) {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
@@ -540,6 +543,7 @@ struct M2LTileLoads {
         al = A.ops_lo + op(o) * R * Kp;
     }
     __device__ __forceinline__ void scales(int o, _Float16 (&rs)[NQ], _Float16 (&cs)[2]) const {
+        if (SINGLE) return;
 #pragma unroll
         for (int c = 0; c < 2; c++) cs[c] = (_Float16)A.ratio[(gm[c] >> o) & 1 ? col[c] + 3 * o : A.zero_col];
         const float *ro = A.ops_rinv + op(o) * R, *rc = A.cls_rinv + (size_t)tile.cls * R;
@@ -566,7 +570,7 @@ struct M2LTileLoads {
     template <int S>
     __device__ __forceinline__ void astore1(int j, _Float16 rs, const i32x4& h, const i32x4& l, _Float16 (*Ah)[S],
                                             _Float16 (*Al)[S]) const {
-        const i32x4 hs = scaled(h, rs), ls = scaled(l, rs);
+        const i32x4 hs = SINGLE ? h : scaled(h, rs), ls = SINGLE ? l : scaled(l, rs);
         if (has_rows(j)) {
             *(i32x4*)&Ah[(tid >> 2) + 64 * j][sq] = hs;
             *(i32x4*)&Al[(tid >> 2) + 64 * j][sq] = ls;
@@ -577,8 +581,8 @@ struct M2LTileLoads {
                                            _Float16 (*Bh)[S], _Float16 (*Bl)[S]) const {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            *(i32x4*)&Bh[(tid >> 2) + 64 * c][sq] = scaled(h[c], cs[c]);
-            *(i32x4*)&Bl[(tid >> 2) + 64 * c][sq] = scaled(l[c], cs[c]);
+            *(i32x4*)&Bh[(tid >> 2) + 64 * c][sq] = SINGLE ? h[c] : scaled(h[c], cs[c]);
+            *(i32x4*)&Bl[(tid >> 2) + 64 * c][sq] = SINGLE ? l[c] : scaled(l[c], cs[c]);
         }
     }
     template <int S>
@@ -593,15 +597,17 @@ struct M2LTileLoads {
     // column cl of the tile: the slab block's column and the scale to undo
     __device__ __forceinline__ float* column(int cl, float& sinv) const {
         const int g = tile.g0 + cl / 3, comp = cl % 3;
-        sinv = A.pinv[3 * A.grp_fc[g] + comp];
+        const int col = 3 * A.grp_fc[g] + comp;
+        sinv = SINGLE ? A.pinv[col] * A.ratio[col] : A.pinv[col];   // of the column itself or of its family
         return A.slab + (3 * (size_t)g + comp) * R;
     }
 };
 
 // Small orders (and the largest, whose two LDS buffers do not fit): wave w owns the tile's columns
 // [32w, 32w + 32) and all NB row blocks; one LDS buffer refilled from registers whose loads overlap the
-// MFMAs, two workgroups per CU.
-template <int NB, int NKS>
+// MFMAs, two workgroups per CU.  Single pairs are one operator a tile, so the work before and after its few
+// K steps counts: without the class tables and the scales 54,762 x 253,324 clustered points (p = 12) MEAS
+template <int NB, int NKS, bool SINGLE>
 __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
     constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK;
     constexpr int NQ = (4 * R + 255) / 256;                          // A: 8-half vectors per thread and part
@@ -614,7 +620,7 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
     const int t = xcd * q + min(xcd, rem) + (blockIdx.x >> 3);
     const GroupTile tile = A.tiles[t];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
-    M2LTileLoads<R, Kp, NQ> ld(A, tile, tid);
+    M2LTileLoads<R, Kp, NQ, SINGLE> ld(A, tile, tid);
     _Float16 rs[NQ], cs[2];
     i32x4 rah[NQ], ral[NQ], rbh[2], rbl[2];
     f32x4 acc[NB][2];
@@ -622,7 +628,7 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
     for (int a = 0; a < NB; a++)
 #pragma unroll
         for (int c = 0; c < 2; c++) acc[a][c] = f32x4{0, 0, 0, 0};
-    int m = tile.mask;
+    int m = SINGLE ? 1 : tile.mask;
     auto open = [&](int o) {
         ld.set_columns(o);
         ld.set_rows(o);
@@ -636,8 +642,8 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
         for (int kt = 0; kt < NKS; kt++) {
             ld.template store<S>(rs, cs, rah, ral, rbh, rbl, Ah, Al, Bh, Bl);
             __syncthreads();
-            if (kt + 1 < NKS || m) {
-                if (kt + 1 == NKS) open(__builtin_ctz(m));
+            if (kt + 1 < NKS || (!SINGLE && m)) {
+                if (!SINGLE && kt + 1 == NKS) open(__builtin_ctz(m));
                 const int k0 = kt + 1 < NKS ? (kt + 1) * BK : 0;
                 ld.aload(k0, rah, ral);
                 ld.bload(k0, rbh, rbl);
@@ -664,7 +670,7 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
         }
     }
     // epilogue: undo the scales; the slab is written once and read once (nontemporal)
-    const float* rv = A.cls_rinv + (size_t)tile.cls * R;
+    const float* rv = (SINGLE ? A.ops_rinv : A.cls_rinv) + (size_t)tile.cls * R;
 #pragma unroll
     for (int c = 0; c < 2; c++) {
         const int cl = wave * 32 + 16 * c + li;
@@ -969,13 +975,13 @@ void group_row_scales(FarGroups& G, const float* ops_rinv, int L, hipStream_t st
 // CU anyway (R >= 224, p >= 14) and its two LDS buffers fit (R <= 368, p <= 18); the single-buffered
 // kernel (two or more workgroups per CU below) otherwise
 template <int NB, int NKS>
-static void launch_f16x3(const M2LGroupArgs& A, int* queues, hipStream_t st) {
+static void launch_f16x3(const M2LGroupArgs& A, bool single, int* queues, hipStream_t st) {
     if constexpr (NB >= 14 && NB <= 23) {
         // one workgroup per CU (the two LDS buffers), 8 per XCD round
         const int grid = std::min(8 * ((A.ntiles + 7) / 8), 8 * ((num_cus() + 7) / 8));
         k_gemm_m2l_f16x3_q<NB, NKS, NKS % 2 ? 1 : 2><<<grid, 256, 0, st>>>(A, queues);
     } else {
-        k_gemm_m2l_f16x3<NB, NKS><<<A.ntiles, 256, 0, st>>>(A);
+        (single ? k_gemm_m2l_f16x3<NB, NKS, true> : k_gemm_m2l_f16x3<NB, NKS, false>)<<<A.ntiles, 256, 0, st>>>(A);
     }
 }
 
@@ -989,7 +995,7 @@ void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float*
     // the row and K counts of the orders 1 .. 20
 #define FMM_F16(NBV, NKV)                                      \
     if (nb == NBV && nks == NKV) {                             \
-        launch_f16x3<NBV, NKV>(A, queues, st);                 \
+        launch_f16x3<NBV, NKV>(A, G.single, queues, st);       \
         FMM_HIP(hipGetLastError());                            \
         return;                                                \
     }

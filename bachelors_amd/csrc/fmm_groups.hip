@@ -213,6 +213,7 @@ void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_
                       const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, hipStream_t st) {
     const int n = L.num_far;
     G.num = G.num_classes = G.num_tiles = 0;
+    G.single = false;
     if (!n) {
         build_pair_index(nullptr, 0, T.num_nodes, ix, st);
         return;
@@ -231,6 +232,7 @@ void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_
         FMM_HIP(hipGetLastError());
         G.num = n;
         G.num_classes = nc;
+        G.single = true;
         for (int c = 0; c < nc; c++) G.num_tiles += ceil_div(L.h_class_begin[c + 1] - L.h_class_begin[c], GROUP_TILE);
         return;
     }

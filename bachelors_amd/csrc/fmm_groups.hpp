@@ -17,6 +17,7 @@ constexpr int GROUP_TILE = 42;   // groups per tile: 126 of the 128 columns
 
 struct FarGroups {
     int num = 0, num_classes = 0, num_tiles = 0;
+    bool single = false;             // every pair a group of its own, group class = far class
     DevBuf fc, mask;                 // per group: first child of the sources' parent, child mask
     DevBuf cls_ops, cls_mask;        // per group class: far class (operator) of child o at [8 c + o]; children in use
     DevBuf cls_rinv;                 // [class][R]: largest row scale 1 / rs over the class's operators
