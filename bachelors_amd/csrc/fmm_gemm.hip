@@ -670,19 +670,32 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
         }
     }
     // epilogue: undo the scales; the slab is written once and read once (nontemporal)
+    // All scales are read before the first store: a load after a store could alias it, so it stayed there and
+    // its wait was one for the store as well, and the pieces of a 128-byte line reached memory one by one
+    // (209,062 x 506,545 clustered points, p = 12: 6.9 instead of 5.3 GB written, 3.9 instead of 2.9 ms)
     const float* rv = (SINGLE ? A.ops_rinv : A.cls_rinv) + (size_t)tile.cls * R;
+    float sinv[2];
+    float* out[2];
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-        const int cl = wave * 32 + 16 * c + li;
-        if (cl >= 3 * tile.ng) continue;
-        float sinv;
-        float* out = ld.column(cl, sinv);
+    for (int c = 0; c < 2; c++) out[c] = ld.column(min(wave * 32 + 16 * c + li, 3 * tile.ng - 1), sinv[c]);
+    constexpr int EB = NB < 14 ? NB : 7;   // row blocks at a time
 #pragma unroll
-        for (int a = 0; a < NB; a++) {
-            const float4 r = *(const float4*)(rv + a * 16 + 4 * g);
-            const f32x4 v = f32x4{acc[a][c][0] * r.x * sinv, acc[a][c][1] * r.y * sinv, acc[a][c][2] * r.z * sinv,
-                                  acc[a][c][3] * r.w * sinv};
-            __builtin_nontemporal_store(v, (f32x4*)(out + a * 16 + 4 * g));
+    for (int a0 = 0; a0 < NB; a0 += EB) {
+        float4 r[EB];
+#pragma unroll
+        for (int a = 0; a < EB; a++)
+            if (a0 + a < NB) r[a] = *(const float4*)(rv + (a0 + a) * 16 + 4 * g);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            if (wave * 32 + 16 * c + li >= 3 * tile.ng) continue;
+#pragma unroll
+            for (int a = 0; a < EB; a++) {
+                if (a0 + a >= NB) continue;
+                const f32x4 x = acc[a0 + a][c];
+                const f32x4 v = f32x4{x[0] * r[a].x * sinv[c], x[1] * r[a].y * sinv[c], x[2] * r[a].z * sinv[c],
+                                      x[3] * r[a].w * sinv[c]};
+                __builtin_nontemporal_store(v, (f32x4*)(out[c] + (a0 + a) * 16 + 4 * g));
+            }
         }
     }
 }
@@ -832,20 +845,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
                 if (BD % 2) buf = ob;
             }
         }
+        // the scales before the first store, as in k_gemm_m2l_f16x3
         const float* rv = A.cls_rinv + (size_t)tile.cls * R;
+        float4 r[NB0];
+        float sinv[4];
+        float* out[4];
+#pragma unroll
+        for (int a = 0; a < NB0; a++) r[a] = *(const float4*)(rv + min(rb0 + a, NB - 1) * 16 + 4 * g);
+#pragma unroll
+        for (int c = 0; c < 4; c++) out[c] = ld.column(min(wc * 64 + 16 * c + li, 3 * tile.ng - 1), sinv[c]);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const int cl = wc * 64 + 16 * c + li;
-            if (cl >= 3 * tile.ng) continue;
-            float sinv;
-            float* out = ld.column(cl, sinv);
+            if (wc * 64 + 16 * c + li >= 3 * tile.ng) continue;
 #pragma unroll
             for (int a = 0; a < NB0; a++) {
                 if (rb0 + a >= NB) break;
-                const float4 r = *(const float4*)(rv + (rb0 + a) * 16 + 4 * g);
-                const f32x4 v = f32x4{acc[a][c][0] * r.x * sinv, acc[a][c][1] * r.y * sinv, acc[a][c][2] * r.z * sinv,
-                                      acc[a][c][3] * r.w * sinv};
-                __builtin_nontemporal_store(v, (f32x4*)(out + (rb0 + a) * 16 + 4 * g));
+                const f32x4 v = f32x4{acc[a][c][0] * r[a].x * sinv[c], acc[a][c][1] * r[a].y * sinv[c],
+                                      acc[a][c][2] * r[a].z * sinv[c], acc[a][c][3] * r[a].w * sinv[c]};
+                __builtin_nontemporal_store(v, (f32x4*)(out[c] + (rb0 + a) * 16 + 4 * g));
             }
         }
     }
