@@ -170,7 +170,6 @@ struct fmm_ctx {
     // F16X3: per-coefficient scales dm, the M2L tables split in FP16 (their FP32 staging), the
     // multipole column scales; down_l2l = L2L operators ahead of the M2L ones in the down tables
     DevBuf dm, m2l_hi, m2l_lo, m2l_rinv, m2l_work, cscale, Mhl;   // Mhl: split multipoles (hi | lo)
-    DevBuf cratio, cpinv;                        // column scales against the siblings' smallest, and 1 / that
     DevBuf queues;   // work counters: [0, 8) the M2L GEMM's per-XCD tiles, [14, 16) probe
     int down_l2l = 0;
     const OpSpec* down_specs = nullptr;          // device specs of the down tables
@@ -729,8 +728,6 @@ void split_for_gemm(fmm_ctx* c) {
     split_columns(c->M.as<float>(), ncols, c->L, c->Lp, kp, c->dm.as<float>(), c->cscale.get<float>(ncols),
                   c->Mhl.get<_Float16>((size_t)2 * (ncols + 1) * kp), c->stream,
                   leaves ? c->S.first_child.as<int>() : nullptr, leaves ? c->S.npts.as<int>() : nullptr);
-    sibling_scales(c->S.parent.as<int>(), c->S.first_child.as<int>(), c->S.num_nodes, c->cscale.as<float>(),
-                   c->cratio.get<float>(ncols + 1), c->cpinv.get<float>(ncols + 1), c->stream);
 }
 
 // Part 2 (stream A, after the tables and the multipoles): the M2L of all classes in one launch
@@ -745,16 +742,13 @@ void translate_gemm(fmm_ctx* c, hipEvent_t gemm_after = nullptr, bool split_done
     if (f16 && P.npairs && !split_done) split_for_gemm(c);
     if (gemm_after) FMM_HIP(hipStreamWaitEvent(st, gemm_after, 0));
     const int R = m2l_slab_rows(c->prec, c->L, c->Lp);
-    if (f16) {
-        group_row_scales(c->groups, c->m2l_rinv.as<float>(), c->L, st);
-        FMM_HIP(hipMemsetAsync(c->queues.as<int>(), 0, 8 * sizeof(int), st));
-    }
+    if (f16) FMM_HIP(hipMemsetAsync(c->queues.as<int>(), 0, 8 * sizeof(int), st));
     c->rec(E_GEMM0);
     if (P.npairs && f16) {
         void* slab = c->m2l_slab.reserve((size_t)3 * c->groups.num * R * c->esize());
         m2l_gemm_f16x3(c->m2l_hi.as<_Float16>(), c->m2l_lo.as<_Float16>(), c->m2l_rinv.as<float>(), c->groups,
-                       c->Mhl.as<_Float16>(), c->cratio.as<float>(), c->cpinv.as<float>(), 3 * c->S.num_nodes, (float*)slab,
-                       c->L, c->queues.get<int>(16), st);
+                       c->Mhl.as<_Float16>(), c->cscale.as<float>(), 3 * c->S.num_nodes, (float*)slab, c->L,
+                       c->queues.get<int>(16), st);
     } else if (P.npairs) {
         void* slab = c->m2l_slab.reserve((size_t)3 * P.npairs * R * c->esize());
         m2l_gemm(c->prec, ops_ptr(c, O), O.lo.ptr, P.tiles, P.ntiles, c->lists.far_s.as<int>(), c->M.ptr, slab, c->L,

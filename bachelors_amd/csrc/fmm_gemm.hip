@@ -452,24 +452,21 @@ __global__ __launch_bounds__(256) void k_gemm_m2l(const T* __restrict__ ops, con
 //                                   coefficient; the tables hold A_eq split, rinv = 1 / rs)
 //   B_eq = diag(dm) M diag(s)      (multipoles: dm per coefficient, s per column, split once per
 //                                   evaluation by k_split_columns into FP16 hi and lo parts)
-// so T M = diag(rinv) (A_eq B_eq) diag(1/s), applied in the epilogue.  Rows R = 16 NB >= L,
-// K padded to Kp = 32 NKS >= L (zero operator columns and multipole rows beyond L).
+// so T M = diag(rinv) (A_eq B_eq) diag(1/s).  Rows R = 16 NB >= L, K padded to Kp = 32 NKS >= L
+// (zero operator columns and multipole rows beyond L).
 //
 // A column is a component of one group of far pairs: up to 8 children of one source node that are far
 // from one target (fmm_groups.hpp).  A tile runs over the K steps of every child in the union of its
-// groups' masks, one operator per child; columns whose group lacks that child take zeros.  The children
-// have operators and columns of their own scales, so on the way into LDS the operator rows are brought
-// to the largest 1 / rs of the class (rows times rinv / cls_rinv) and the columns to the smallest
-// scale of the siblings (ratio), powers of 2 at most 1: a value keeps FP16's 22 split bits relative to
-// the largest term of the group's sum.  The epilogue applies cls_rinv and 1 / that scale (pinv) and
-// stores one slab block per group.
+// groups' masks, one operator per child; columns whose group lacks that child take zeros.  Every child
+// has scales of its own, so its product is accumulated by itself, scaled back, and added to the group's
+// sum in FP32: the roundings are those of one pair, whatever its siblings.  In one accumulator through
+// all children, brought to common scales in FP16, the sum took up to 8 times the roundings at its full
+// size, and a child far below a sibling lost its bits even where that sibling is no far pair (a leaf of
+// 2^20 times the weight: the far field beside it off by 1e-4 of itself).
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 // eight halves on their way from memory to LDS.  As a half vector the compiler takes each register apart
 // and together again wherever a load is conditional (300 instructions per K step, more than all others)
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ i32x4 scaled(i32x4 v, _Float16 s) {
-    return __builtin_bit_cast(i32x4, __builtin_bit_cast(half8, v) * s);
-}
 
 // LDS rows of 32 halves without padding, their four 16-byte chunks permuted by the row: chunk q of row r
 // lies at q ^ f(r / 4 mod 4), f = 0, 2, 3, 1.  16-byte LDS reads are served in lane groups
@@ -486,127 +483,107 @@ struct M2LGroupArgs {
     const float* ops_rinv;
     const GroupTile* tiles;
     const int* cls_ops;
-    const float* cls_rinv;
     const int* grp_fc;
     const int* grp_mask;
     const _Float16* src_hl;
-    const float* ratio;
-    const float* pinv;
+    const float* cscale;
     float* slab;
     int ntiles, zero_col;   // the column of zeros
 };
 
-// What the threads of a workgroup load of the current child of a tile: the operator's rows
-// (tid >> 2) + 64 j and the columns (tid >> 2) + 64 c, 8 consecutive k each, and their scales.  Every
-// load is unconditional (rows beyond R are clamped and not stored, columns whose group lacks the child
-// read the column of zeros behind the nodes'): after a load that may have been skipped the compiler
-// cannot count the loads in flight and waits for all of them, the ones issued steps ahead included.
-// SINGLE: every group is one pair, child 0 with the class's one operator: no scales to even out.
-template <int R, int Kp, int NQ, bool SINGLE = false>
-struct M2LTileLoads {
+// The columns (tid >> 2) + 64 c of a tile that a thread loads, and the operators of its children.
+// Columns whose group lacks a child read the column of zeros behind the nodes'.
+// SINGLE: every group is one pair, child 0 with the class's one operator.
+template <int R, int Kp, bool SINGLE>
+struct M2LTile {
     const M2LGroupArgs& A;
     GroupTile tile;
+    int col[2], gm[2];   // multipole column of child 0 and child mask of the columns' groups
+    __device__ __forceinline__ M2LTile(const M2LGroupArgs& A_, const GroupTile& t, int tid) : A(A_), tile(t) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) find((tid >> 2) + 64 * c, col[c], gm[c]);
+    }
+    __device__ __forceinline__ void find(int cl, int& col0, int& mask) const {
+        const bool valid = cl < 3 * tile.ng;
+        const int g = tile.g0 + (valid ? cl / 3 : 0);
+        col0 = 3 * A.grp_fc[g] + cl % 3;
+        mask = !valid ? 0 : SINGLE ? 1 : A.grp_mask[g];
+    }
+    __device__ __forceinline__ size_t op(int o) const {
+        return SINGLE ? (size_t)tile.cls : (size_t)A.cls_ops[8 * (size_t)tile.cls + o];
+    }
+    // the parts of column c of child o, K step by K step hi | lo
+    __device__ __forceinline__ const _Float16* column(int c, int o, bool any = true) const {
+        return A.src_hl + (size_t)(any && ((gm[c] >> o) & 1) ? col[c] + 3 * o : A.zero_col) * 2 * Kp;
+    }
+    // what undoes the scale of a column of child o (0 where the group lacks the child: that product is 0)
+    __device__ __forceinline__ float column_inv(int col0, int mask, int o) const {
+        return (mask >> o) & 1 ? 1.0f / A.cscale[col0 + 3 * o] : 0.0f;
+    }
+    __device__ __forceinline__ float* slab(int cl) const {   // the block's column of the tile's column cl
+        return A.slab + (3 * (size_t)tile.g0 + cl) * R;
+    }
+};
+
+// What the threads of a workgroup load of the current child of a tile into registers: the operator's rows
+// (tid >> 2) + 64 j and the columns, 8 consecutive k each.  Every load is unconditional (rows beyond R
+// are clamped and not stored): after a load that may have been skipped the compiler cannot count the loads
+// in flight and waits for all of them.
+template <int R, int Kp, int NQ, bool SINGLE>
+struct M2LTileLoads : M2LTile<R, Kp, SINGLE> {
     int tid, wave, bq, sq;           // wave: uniform; bq, sq: first k of this thread's chunk, its place in LDS
-    int col[2], gm[2];               // multipole column of child 0 and child mask of the columns' groups
     const _Float16 *ah, *al;         // operator parts (uniform)
     const _Float16* b[2];
     __device__ __forceinline__ M2LTileLoads(const M2LGroupArgs& A_, const GroupTile& t, int tid_)
-        : A(A_), tile(t), tid(tid_), wave(__builtin_amdgcn_readfirstlane(tid_ >> 6)), bq((tid_ & 3) * 8),
-          sq(8 * lds_chunk(tid_ & 3, tid_ >> 2)) {
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int cl = (tid >> 2) + 64 * c;
-            const bool valid = cl < 3 * tile.ng;
-            const int g = tile.g0 + (valid ? cl / 3 : 0);
-            col[c] = 3 * A.grp_fc[g] + cl % 3;
-            gm[c] = !valid ? 0 : SINGLE ? 1 : A.grp_mask[g];
-        }
-    }
+        : M2LTile<R, Kp, SINGLE>(A_, t, tid_), tid(tid_), wave(__builtin_amdgcn_readfirstlane(tid_ >> 6)),
+          bq((tid_ & 3) * 8), sq(8 * lds_chunk(tid_ & 3, tid_ >> 2)) {}
     __device__ __forceinline__ int row(int j) const {
         const int r = (tid >> 2) + 64 * j;
         return 64 * (j + 1) <= R ? r : min(r, R - 1);
     }
     // a wave stages 16 rows at a time: all of them exist or none
     __device__ __forceinline__ bool has_rows(int j) const { return 64 * (j + 1) <= R || 16 * wave + 64 * j < R; }
-    __device__ __forceinline__ size_t op(int o) const {
-        return SINGLE ? (size_t)tile.cls : (size_t)A.cls_ops[8 * (size_t)tile.cls + o];
+    __device__ __forceinline__ void open(int o) {
+        for (int c = 0; c < 2; c++) b[c] = this->column(c, o) + bq;
+        ah = this->A.ops_hi + this->op(o) * R * Kp;
+        al = this->A.ops_lo + this->op(o) * R * Kp;
     }
-    __device__ __forceinline__ void set_columns(int o, bool any = true) {
+    __device__ __forceinline__ void load(int k0, i32x4 (&ah_)[NQ], i32x4 (&al_)[NQ], i32x4 (&bh)[2],
+                                         i32x4 (&bl)[2]) const {
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const bool in = any && ((gm[c] >> o) & 1);
-            b[c] = A.src_hl + (size_t)(in ? col[c] + 3 * o : A.zero_col) * 2 * Kp + bq;
+        for (int j = 0; j < NQ; j++) {
+            const unsigned o = (unsigned)(row(j) * Kp + k0 + bq);
+            ah_[j] = *(const i32x4*)(ah + o);
+            al_[j] = *(const i32x4*)(al + o);
         }
-    }
-    __device__ __forceinline__ void set_rows(int o) {
-        ah = A.ops_hi + op(o) * R * Kp;
-        al = A.ops_lo + op(o) * R * Kp;
-    }
-    __device__ __forceinline__ void scales(int o, _Float16 (&rs)[NQ], _Float16 (&cs)[2]) const {
-        if (SINGLE) return;
-#pragma unroll
-        for (int c = 0; c < 2; c++) cs[c] = (_Float16)A.ratio[(gm[c] >> o) & 1 ? col[c] + 3 * o : A.zero_col];
-        const float *ro = A.ops_rinv + op(o) * R, *rc = A.cls_rinv + (size_t)tile.cls * R;
-#pragma unroll
-        for (int j = 0; j < NQ; j++)   // both are powers of 2: the quotient by their exponents
-            rs[j] = (_Float16)__int_as_float(__float_as_int(ro[row(j)]) - __float_as_int(rc[row(j)]) + 0x3f800000);
-    }
-    __device__ __forceinline__ void aload1(int j, int k0, i32x4& h, i32x4& l) const {
-        const unsigned o = (unsigned)(row(j) * Kp + k0 + bq);
-        h = *(const i32x4*)(ah + o);
-        l = *(const i32x4*)(al + o);
-    }
-    __device__ __forceinline__ void aload(int k0, i32x4 (&h)[NQ], i32x4 (&l)[NQ]) const {
-#pragma unroll
-        for (int j = 0; j < NQ; j++) aload1(j, k0, h[j], l[j]);
-    }
-    __device__ __forceinline__ void bload(int k0, i32x4 (&h)[2], i32x4 (&l)[2]) const {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            h[c] = *(const i32x4*)(b[c] + 2 * k0);
-            l[c] = *(const i32x4*)(b[c] + 2 * k0 + 32);
+            bh[c] = *(const i32x4*)(b[c] + 2 * k0);
+            bl[c] = *(const i32x4*)(b[c] + 2 * k0 + 32);
         }
     }
     template <int S>
-    __device__ __forceinline__ void astore1(int j, _Float16 rs, const i32x4& h, const i32x4& l, _Float16 (*Ah)[S],
-                                            _Float16 (*Al)[S]) const {
-        const i32x4 hs = SINGLE ? h : scaled(h, rs), ls = SINGLE ? l : scaled(l, rs);
-        if (has_rows(j)) {
-            *(i32x4*)&Ah[(tid >> 2) + 64 * j][sq] = hs;
-            *(i32x4*)&Al[(tid >> 2) + 64 * j][sq] = ls;
-        }
-    }
-    template <int S>
-    __device__ __forceinline__ void bstore(const _Float16 (&cs)[2], const i32x4 (&h)[2], const i32x4 (&l)[2],
-                                           _Float16 (*Bh)[S], _Float16 (*Bl)[S]) const {
+    __device__ __forceinline__ void store(const i32x4 (&ah_)[NQ], const i32x4 (&al_)[NQ], const i32x4 (&bh)[2],
+                                          const i32x4 (&bl)[2], _Float16 (*Ah)[S], _Float16 (*Al)[S],
+                                          _Float16 (*Bh)[S], _Float16 (*Bl)[S]) const {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            *(i32x4*)&Bh[(tid >> 2) + 64 * c][sq] = SINGLE ? h[c] : scaled(h[c], cs[c]);
-            *(i32x4*)&Bl[(tid >> 2) + 64 * c][sq] = SINGLE ? l[c] : scaled(l[c], cs[c]);
+            *(i32x4*)&Bh[(tid >> 2) + 64 * c][sq] = bh[c];
+            *(i32x4*)&Bl[(tid >> 2) + 64 * c][sq] = bl[c];
         }
-    }
-    template <int S>
-    __device__ __forceinline__ void store(const _Float16 (&rs)[NQ], const _Float16 (&cs)[2], const i32x4 (&ah_)[NQ],
-                                          const i32x4 (&al_)[NQ], const i32x4 (&bh)[2], const i32x4 (&bl)[2],
-                                          _Float16 (*Ah)[S], _Float16 (*Al)[S], _Float16 (*Bh)[S],
-                                          _Float16 (*Bl)[S]) const {
-        bstore<S>(cs, bh, bl, Bh, Bl);
 #pragma unroll
-        for (int j = 0; j < NQ; j++) astore1<S>(j, rs[j], ah_[j], al_[j], Ah, Al);
-    }
-    // column cl of the tile: the slab block's column and the scale to undo
-    __device__ __forceinline__ float* column(int cl, float& sinv) const {
-        const int g = tile.g0 + cl / 3, comp = cl % 3;
-        const int col = 3 * A.grp_fc[g] + comp;
-        sinv = SINGLE ? A.pinv[col] * A.ratio[col] : A.pinv[col];   // of the column itself or of its family
-        return A.slab + (3 * (size_t)g + comp) * R;
+        for (int j = 0; j < NQ; j++) {
+            if (!has_rows(j)) continue;
+            *(i32x4*)&Ah[(tid >> 2) + 64 * j][sq] = ah_[j];
+            *(i32x4*)&Al[(tid >> 2) + 64 * j][sq] = al_[j];
+        }
     }
 };
 
-// Small orders (and the largest, whose two LDS buffers do not fit): wave w owns the tile's columns
+// Single pairs up to p = 13 and above 18, and groups up to p = 7: wave w owns the tile's columns
 // [32w, 32w + 32) and all NB row blocks; one LDS buffer refilled from registers whose loads overlap the
 // MFMAs, two workgroups per CU.  Single pairs are one operator a tile, so the work before and after its few
-// K steps counts: without the class tables and the scales 13,693 x 710,485 points (p = 10) 0.65 -> 0.50 ms.
+// K steps counts: without the class tables 13,693 x 710,485 points (p = 10) 0.65 -> 0.50 ms.
 template <int NB, int NKS, bool SINGLE>
 __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
     constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK;
@@ -621,32 +598,35 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
     const GroupTile tile = A.tiles[t];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
     M2LTileLoads<R, Kp, NQ, SINGLE> ld(A, tile, tid);
-    _Float16 rs[NQ], cs[2];
+    int wcol[2], wgm[2];   // of the columns whose products this lane holds
+#pragma unroll
+    for (int c = 0; c < 2; c++) ld.find(wave * 32 + 16 * c + li, wcol[c], wgm[c]);
     i32x4 rah[NQ], ral[NQ], rbh[2], rbl[2];
-    f32x4 acc[NB][2];
+    f32x4 acc[NB][2], sum[SINGLE ? 1 : NB][2];
 #pragma unroll
     for (int a = 0; a < NB; a++)
 #pragma unroll
         for (int c = 0; c < 2; c++) acc[a][c] = f32x4{0, 0, 0, 0};
-    int m = SINGLE ? 1 : tile.mask;
-    auto open = [&](int o) {
-        ld.set_columns(o);
-        ld.set_rows(o);
-        ld.scales(o, rs, cs);
-    };
-    open(__builtin_ctz(m));
-    ld.aload(0, rah, ral);
-    ld.bload(0, rbh, rbl);
+#pragma unroll
+    for (int a = 0; a < (SINGLE ? 1 : NB); a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) sum[a][c] = f32x4{0, 0, 0, 0};
+    constexpr int EB = NB < 14 ? NB : 7;   // row blocks whose scales are read at a time
+    int m = SINGLE ? 1 : tile.mask, o = __builtin_ctz(m);
+    ld.open(o);
+    ld.load(0, rah, ral, rbh, rbl);
     while (m) {
         m &= m - 1;
+        const int cur = o;
         for (int kt = 0; kt < NKS; kt++) {
-            ld.template store<S>(rs, cs, rah, ral, rbh, rbl, Ah, Al, Bh, Bl);
+            ld.template store<S>(rah, ral, rbh, rbl, Ah, Al, Bh, Bl);
             __syncthreads();
             if (kt + 1 < NKS || (!SINGLE && m)) {
-                if (!SINGLE && kt + 1 == NKS) open(__builtin_ctz(m));
-                const int k0 = kt + 1 < NKS ? (kt + 1) * BK : 0;
-                ld.aload(k0, rah, ral);
-                ld.bload(k0, rbh, rbl);
+                if (!SINGLE && kt + 1 == NKS) {
+                    o = __builtin_ctz(m);
+                    ld.open(o);
+                }
+                ld.load(kt + 1 < NKS ? (kt + 1) * BK : 0, rah, ral, rbh, rbl);
             }
             const int kk = 8 * lds_chunk(g, li);
             half8 bh[2], bl[2];
@@ -668,65 +648,236 @@ __global__ __launch_bounds__(256) void k_gemm_m2l_f16x3(M2LGroupArgs A) {
             }
             __syncthreads();
         }
+        if (SINGLE) break;
+        // the child's product, scaled back, into the group's sum
+        const float* rv = A.ops_rinv + ld.op(cur) * R;
+        float sinv[2];
+#pragma unroll
+        for (int c = 0; c < 2; c++) sinv[c] = ld.column_inv(wcol[c], wgm[c], cur);
+#pragma unroll
+        for (int a = 0; a < (SINGLE ? 0 : NB); a++) {
+            const float4 r = *(const float4*)(rv + a * 16 + 4 * g);
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const f32x4 x = acc[a][c];
+                const float rr[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[a][c][e] = __builtin_fmaf(x[e] * rr[e], sinv[c], sum[a][c][e]);
+                acc[a][c] = f32x4{0, 0, 0, 0};
+            }
+        }
     }
-    // epilogue: undo the scales; the slab is written once and read once (nontemporal)
-    // All scales are read before the first store: a load after a store could alias it, so it stayed there and
+    // epilogue: the slab is written once and read once (nontemporal).  A single pair's scales are undone here, all
+    // of them read before the first store: a load after a store could alias it, so it stayed there and
     // its wait was one for the store as well, and the pieces of a 128-byte line reached memory one by one
     // (209,062 x 506,545 clustered points, p = 12: 6.9 instead of 5.3 GB written, 3.9 instead of 2.9 ms)
-    const float* rv = (SINGLE ? A.ops_rinv : A.cls_rinv) + (size_t)tile.cls * R;
+    const float* rv = A.ops_rinv + (size_t)tile.cls * R;
     float sinv[2];
-    float* out[2];
 #pragma unroll
-    for (int c = 0; c < 2; c++) out[c] = ld.column(min(wave * 32 + 16 * c + li, 3 * tile.ng - 1), sinv[c]);
-    constexpr int EB = NB < 14 ? NB : 7;   // row blocks at a time
+    for (int c = 0; c < 2; c++) sinv[c] = SINGLE ? ld.column_inv(wcol[c], wgm[c], 0) : 0.0f;
 #pragma unroll
     for (int a0 = 0; a0 < NB; a0 += EB) {
         float4 r[EB];
+        if (SINGLE)
 #pragma unroll
-        for (int a = 0; a < EB; a++)
-            if (a0 + a < NB) r[a] = *(const float4*)(rv + (a0 + a) * 16 + 4 * g);
+            for (int a = 0; a < EB; a++)
+                if (a0 + a < NB) r[a] = *(const float4*)(rv + (a0 + a) * 16 + 4 * g);
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            if (wave * 32 + 16 * c + li >= 3 * tile.ng) continue;
+            const int cl = wave * 32 + 16 * c + li;
+            if (cl >= 3 * tile.ng) continue;
+            float* out = ld.slab(cl);
 #pragma unroll
             for (int a = 0; a < EB; a++) {
                 if (a0 + a >= NB) continue;
-                const f32x4 x = acc[a0 + a][c];
-                const f32x4 v = f32x4{x[0] * r[a].x * sinv[c], x[1] * r[a].y * sinv[c], x[2] * r[a].z * sinv[c],
-                                      x[3] * r[a].w * sinv[c]};
-                __builtin_nontemporal_store(v, (f32x4*)(out[c] + (a0 + a) * 16 + 4 * g));
+                f32x4 v = sum[SINGLE ? 0 : a0 + a][c];
+                if (SINGLE) {
+                    const f32x4 x = acc[a0 + a][c];
+                    v = f32x4{x[0] * r[a].x * sinv[c], x[1] * r[a].y * sinv[c], x[2] * r[a].z * sinv[c],
+                              x[3] * r[a].w * sinv[c]};
+                }
+                __builtin_nontemporal_store(v, (f32x4*)(out + (a0 + a) * 16 + 4 * g));
             }
         }
     }
 }
 
+// 64 lanes' 16 bytes from memory into 1 KB of LDS, without registers: lane i's to lds + 16 i (lds: uniform).
+// Counted by vmcnt like any load: dma_barrier waits for it and then for the workgroup.
+__device__ __forceinline__ void dma16(const _Float16* p, _Float16* lds) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p,
+                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+// Waits for all but the last LEFT loads of this wave and for its LDS accesses, then for the workgroup.  A
+// __syncthreads would wait for all loads.
+template <int LEFT> __device__ __forceinline__ void dma_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// A workgroup's part of the persistent kernel below: the tile's columns and operators, and the loads into LDS.
+// A buffer of rows is [hi | lo][R][32 halves], one of columns [hi | lo][128][32].
+template <int NB, int NKS, bool SINGLE>
+struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
+    static constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK, W = 128;
+    static constexpr int NQ = (4 * R + 255) / 256;   // 16-byte chunks per thread and part of the rows
+    static constexpr int NB0 = (NB + 1) / 2, NS = (R + 255) / 256;
+    const _Float16 *ah, *al;   // operator parts (uniform)
+    const _Float16* b[2];
+    int tid, wave, lane, rb0, wc, kk;
+    unsigned aq, bq;   // lane's place in LDS row (tid >> 2) is slot tid & 3: the chunk that belongs there
+    f32x4 acc[NB0][4], sum[SINGLE ? 1 : NB0][4];
+    __device__ __forceinline__ M2LTileDma(const M2LGroupArgs& A_, const GroupTile& t, int tid_)
+        : M2LTile<R, Kp, SINGLE>(A_, t, tid_), tid(tid_), wave(__builtin_amdgcn_readfirstlane(tid_ >> 6)),
+          lane(tid_ & 63), rb0((wave & 1) * NB0), wc(wave >> 1), kk(8 * lds_chunk(lane >> 4, lane & 15)),
+          aq((unsigned)((tid_ >> 2) * Kp + 8 * lds_chunk(tid_ & 3, tid_ >> 2))),
+          bq((unsigned)(8 * lds_chunk(tid_ & 3, tid_ >> 2))) {
+#pragma unroll
+        for (int a = 0; a < NB0; a++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                acc[a][c] = f32x4{0, 0, 0, 0};
+                if (!SINGLE) sum[SINGLE ? 0 : a][c] = f32x4{0, 0, 0, 0};
+            }
+    }
+    __device__ __forceinline__ f32x4 result(int a, int c) const { return SINGLE ? acc[a][c] : sum[SINGLE ? 0 : a][c]; }
+    __device__ __forceinline__ void rows(int o) {
+        ah = this->A.ops_hi + this->op(o) * R * Kp;
+        al = this->A.ops_lo + this->op(o) * R * Kp;
+    }
+    __device__ __forceinline__ void columns(int o, bool any) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) b[c] = this->column(c, o, any) + bq;
+    }
+    __device__ __forceinline__ void aload(int kt, _Float16* buf) const {
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            // a wave takes 16 rows at a time: all of them exist or none
+            if (64 * (j + 1) > R && 16 * wave + 64 * j >= R) continue;
+            dma16(ah + (size_t)64 * j * Kp + kt * BK + aq, buf + (16 * wave + 64 * j) * S);
+            dma16(al + (size_t)64 * j * Kp + kt * BK + aq, buf + (R + 16 * wave + 64 * j) * S);
+        }
+    }
+    __device__ __forceinline__ void bload(int kt, _Float16* buf) const {   // BLOADS loads of every wave
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            dma16(b[c] + 2 * kt * BK, buf + (16 * wave + 64 * c) * S);
+            dma16(b[c] + 2 * kt * BK + 32, buf + (W + 16 * wave + 64 * c) * S);
+        }
+    }
+    static constexpr int BLOADS = 4;
+    // K step kt of child o; on: the next child (any: there is one).  ac, bc: the operands of this step; an, bn: the
+    // rows of the next step and the columns of the one after it, their buffers last read before the previous
+    // barrier; sc: the scales of the current child's rows and columns [R + W].  The buffers are different ones,
+    // which the compiler has to know (it waits for loads into LDS before every read that could be of them).
+    // LAST: the child's last step, after which its product is scaled back and added to the sum.
+    template <bool LAST>
+    __device__ __forceinline__ void step(int kt, int o, int on, bool any, const _Float16* __restrict__ ac,
+                                         const _Float16* __restrict__ bc, _Float16* __restrict__ an,
+                                         _Float16* __restrict__ bn, float* __restrict__ sc) {
+        if (LAST) rows(on);
+        aload(LAST ? 0 : kt + 1, an);
+        __builtin_amdgcn_sched_barrier(0);   // dma_barrier counts on the columns' loads being the last
+        if (kt + 2 == NKS) columns(on, any);
+        bload(kt + 2 < NKS ? kt + 2 : kt + 2 - NKS, bn);
+        __builtin_amdgcn_sched_barrier(0);
+        float sv[NS], cv = 0;   // the child's scales on their way to LDS
+        if (!LAST && kt == 0) {
+            const float* rv = this->A.ops_rinv + this->op(o) * R;
+#pragma unroll
+            for (int i = 0; i < NS; i++) sv[i] = rv[min(tid + 256 * i, R - 1)];
+            const int c = tid & 3;
+            if (c < 2) cv = this->column_inv(c ? this->col[1] : this->col[0], c ? this->gm[1] : this->gm[0], o);
+        }
+        const int li = lane & 15, g = lane >> 4;
+        half8 bh[4], bl[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            bh[c] = *(const half8*)(bc + (wc * 64 + 16 * c + li) * S + kk);
+            bl[c] = *(const half8*)(bc + (W + wc * 64 + 16 * c + li) * S + kk);
+        }
+        // row block by row block, each block's operator fragments read during the previous block's
+        // MFMAs (the scheduling barriers keep the reads from gathering at the start)
+        half8 fh[2], fl[2];
+#pragma unroll
+        for (int a = -1; a < NB0; a++) {
+            if (a + 1 < NB0) {
+                // the second row half's last block is past NB when NB is odd: it is the block NB - 1 again, in
+                // bounds and not stored (a branch around it costs copies of the accumulators, and the other
+                // half's waves would be waited for anyway)
+                const int row = min(rb0 + a + 1, NB - 1) * 16 + li;
+                fh[(a + 1) & 1] = *(const half8*)(ac + row * S + kk);
+                fl[(a + 1) & 1] = *(const half8*)(ac + (R + row) * S + kk);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (a < 0) continue;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[a & 1], bh[c], acc[a][c], 0, 0, 0);
+                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bl[c], acc[a][c], 0, 0, 0);
+                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bh[c], acc[a][c], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!LAST && kt == 0) {   // last read at the end of the previous child, a barrier ago
+#pragma unroll
+            for (int i = 0; i < NS; i++)
+                if (tid + 256 * i < R) sc[tid + 256 * i] = sv[i];
+            if ((tid & 3) < 2) sc[R + (tid >> 2) + 64 * (tid & 3)] = cv;
+        }
+        if (LAST) {
+            float ci[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) ci[c] = sc[R + wc * 64 + 16 * c + li];
+#pragma unroll
+            for (int a = 0; a < NB0; a++) {
+                const f32x4 r = *(const f32x4*)(sc + min(rb0 + a, NB - 1) * 16 + 4 * g);
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    f32x4 x = acc[a][c];
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        x[e] = SINGLE ? x[e] * r[e] * ci[c] : __builtin_fmaf(x[e] * r[e], ci[c], sum[SINGLE ? 0 : a][c][e]);
+                    if (!SINGLE) sum[SINGLE ? 0 : a][c] = x;
+                    acc[a][c] = SINGLE ? x : f32x4{0, 0, 0, 0};
+                }
+            }
+        }
+    }
+};
+
 // The waves on a 2 x 2 grid: wave (wr, wc) owns the row blocks [wr NB0, wr NB0 + NB0) below NB
 // (NB0 = ceil(NB / 2)) and the tile columns [64 wc, 64 wc + 64), so it reads half the operator rows and
 // half the columns from LDS per K step (a wave tile of 16 NB0 x 64 instead of 16 NB x 32: about a
-// third less LDS traffic per MFMA).  Two LDS buffers, one barrier per K step; the multipole columns
-// (gathered from HBM) are loaded BD K steps ahead, the operator rows (shared by the tiles of one
-// class, mostly L2 hits) one step ahead, across the boundary from one child to the next.
-template <int NB, int NKS, int BD>
+// third less LDS traffic per MFMA).  The operands go to LDS without passing registers (dma16), which hold
+// two sets of accumulators instead, a child's and the group's: two buffers for the operator rows (shared by
+// the tiles of one class, mostly L2 hits), loaded one K step ahead, three for the multipole columns (gathered
+// from HBM), loaded two steps ahead, one barrier per K step, all across the boundary from one child to the
+// next.  Measured against one set of accumulators fed through registers: 4M shells, p = 16, 26.1 and 26.2 ms an
+// evaluation; GEMM of 1M points, p = 8, 12 and 13, 0.65 -> 0.58, 1.93 -> 1.86 and 6.9 -> 4.2 ms (then the
+// kernel above).  Far field of 999,983 x 750,019 clustered points, p = 14, against FP64: 3.8e-7 -> 3.4e-7, as
+// pair by pair; a second set in the kernel above leaves one workgroup per CU (p = 12: 3.3 ms).
+template <int NB, int NKS, bool SINGLE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_gemm_m2l_f16x3_q(M2LGroupArgs A,
                                                                                                 int* __restrict__ xq) {
-    static_assert(NKS % BD == 0 && (BD == 2 || BD == 1), "the column register sets are indexed statically");
-    constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK;
-    constexpr int NQ = (4 * R + 255) / 256;                          // A: 8-half vectors per thread and part
-    constexpr int W = 128, NB0 = (NB + 1) / 2;
-    __shared__ __attribute__((aligned(16))) _Float16 Ah[2][R][S];
-    __shared__ __attribute__((aligned(16))) _Float16 Al[2][R][S];
-    __shared__ __attribute__((aligned(16))) _Float16 Bh[2][W][S];
-    __shared__ __attribute__((aligned(16))) _Float16 Bl[2][W][S];
+    typedef M2LTileDma<NB, NKS, SINGLE> Tile;
+    static_assert(NKS >= 3, "two steps ahead reach at most the next child; its scales have a step of their own");
+    constexpr int R = Tile::R, W = Tile::W, S = Tile::S, RBUF = 2 * R * S, CBUF = 2 * W * S;
+    // one variable: with several the compiler labels the accesses by variable, and then a read waits for
+    // every load into LDS under way to its variable, that of the other buffers too
+    __shared__ struct {
+        __attribute__((aligned(16))) _Float16 rows[2 * RBUF], columns[3 * CBUF];
+        __attribute__((aligned(16))) float scales[R + W];   // the current child's
+        int next_tile;
+    } sh;
     // persistent: the grid (a multiple of 8, workgroup b on XCD b mod 8) walks the tiles, each
     // XCD a contiguous eighth of them (one class's operators shared in one L2) taken from that
     // XCD's counter xq[xcd] (zero at launch), so a workgroup that starts late (its CU busy)
     // takes fewer tiles, and then from the other XCDs' eighths; a workgroup starts its next tile
     // while its last stores drain.  The
     // register budget leaves room for one near-field workgroup (k_p2p_queue) per CU.
-    const int xcd = blockIdx.x & 7, q = A.ntiles >> 3, rem = A.ntiles & 7;
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, li = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave & 1, wc = wave >> 1, rb0 = wr * NB0;
-    __shared__ int next_tile;
+    const int xcd = blockIdx.x & 7, q = A.ntiles >> 3, rem = A.ntiles & 7, tid = threadIdx.x;
     int from = xcd;   // (thread 0) the eighth this workgroup draws from: its XCD's, then the others'
     for (;;) {
         if (tid == 0) {
@@ -741,128 +892,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
                     from = x;
                 }
             }
-            next_tile = t;
+            sh.next_tile = t;
         }
-        __syncthreads();
+        __syncthreads();   // also: no load into LDS of the previous tile is under way in any wave
         // read before the K loop's barriers, rewritten only after them; the same in every lane, so what
         // follows from it stays in scalar registers
-        const int it = __builtin_amdgcn_readfirstlane(next_tile);
+        const int it = __builtin_amdgcn_readfirstlane(sh.next_tile);
         if (it < 0) break;
-        const GroupTile tile = A.tiles[it];
-        M2LTileLoads<R, Kp, NQ> ld(A, tile, tid);
-        _Float16 rs[NQ], cs[2];
-        i32x4 rah[NQ], ral[NQ];
-        i32x4 rbh[BD][2], rbl[BD][2];   // [set][c]: the multipole columns of BD K steps in flight
-        f32x4 acc[NB0][4];
-#pragma unroll
-        for (int a = 0; a < NB0; a++)
-#pragma unroll
-            for (int c = 0; c < 4; c++) acc[a][c] = f32x4{0, 0, 0, 0};
-        int m = tile.mask, buf = 0;   // m: the children left (at least one)
-        int o_cur = __builtin_ctz(m);
-        ld.set_columns(o_cur);
-        ld.set_rows(o_cur);
-        ld.scales(o_cur, rs, cs);
-        ld.aload(0, rah, ral);
-#pragma unroll
-        for (int d = 0; d < BD; d++) ld.bload(d * BK, rbh[d], rbl[d]);
-        ld.template store<S>(rs, cs, rah, ral, rbh[0], rbl[0], Ah[0], Al[0], Bh[0], Bl[0]);
-        ld.aload(BK, rah, ral);
-        ld.bload(BD * BK, rbh[0], rbl[0]);
-        __syncthreads();
+        Tile ld(A, A.tiles[it], tid);
+        int m = SINGLE ? 1 : ld.tile.mask, o = __builtin_ctz(m);   // m: the children left after the current one o
+        m &= m - 1;
+        ld.rows(o);
+        ld.columns(o, true);
+        ld.aload(0, sh.rows);
+        ld.bload(0, sh.columns);
+        __builtin_amdgcn_sched_barrier(0);
+        ld.bload(1, sh.columns + CBUF);
+        dma_barrier<Tile::BLOADS>();
+        int ab = 0, bb = 0;   // the buffers of the current step
+        auto next = [&] {
+            dma_barrier<Tile::BLOADS>();   // all but the columns two steps ahead
+            ab ^= 1;
+            bb = bb == 2 ? 0 : bb + 1;
+        };
         for (bool more = true; more;) {
+            more = !SINGLE && m != 0;
+            // the next child; after the last one the loads ahead are of its first rows and the column of zeros, unused
+            const int on = more ? __builtin_ctz(m) : o;
             m &= m - 1;
-            more = m != 0;
-            // the next child; after the last one its operator's first steps are loaded and the first
-            // stored again, unused, and no column: the K loop stays free of branches
-            const int o = more ? __builtin_ctz(m) : o_cur;
-            o_cur = o;
-            _Float16 nrs[NQ], ncs[2];
-            for (int kt0 = 0; kt0 < NKS; kt0 += BD)
-#pragma unroll
-            for (int d = 0; d < BD; d++) {
-                // register sets (and for even NKS the LDS buffers) by constant indexes
-                const int kt = kt0 + d, cb = BD % 2 ? buf : d & 1, ob = cb ^ 1, set = (d + 1) % BD;
-                const int ka = kt + 2 < NKS ? kt + 2 : kt + 2 - NKS;               // steps loaded now
-                const int kb = kt + 1 + BD < NKS ? kt + 1 + BD : kt + 1 + BD - NKS;
-                const int kk = 8 * lds_chunk(g, li);
-                half8 bh[4], bl[4];
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    bh[c] = *(const half8*)&Bh[cb][wc * 64 + 16 * c + li][kk];
-                    bl[c] = *(const half8*)&Bl[cb][wc * 64 + 16 * c + li][kk];
-                }
-                // row block by row block, each block's operator fragments read during the previous block's
-                // MFMAs.  Between the blocks, spread over the step: the next step (loaded during the
-                // previous one) goes to the other LDS buffer, last read before the previous barrier, and
-                // its registers take the step after it; from the last steps on these are the next child's.
-                // The scheduling barriers keep the pieces apart: left alone the compiler gathers the loads
-                // and runs out of registers
-                half8 fh[2], fl[2];
-                auto frag = [&](int a) {
-                    // the second row half's last block is past NB when NB is odd: it reads the block
-                    // NB - 1 instead (in bounds) and its MFMAs are skipped
-                    const int row = min(rb0 + a, NB - 1) * 16 + li;
-                    fh[a & 1] = *(const half8*)&Ah[cb][row][kk];
-                    fl[a & 1] = *(const half8*)&Al[cb][row][kk];
-                };
-                frag(0);
-                static_assert(NQ + 2 <= NB0, "the pieces of the staging fit between the row blocks");
-#pragma unroll
-                for (int a = 0; a < NB0; a++) {
-                    if (a + 1 < NB0) frag(a + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (rb0 + a < NB) {   // uniform over the wave
-#pragma unroll
-                        for (int c = 0; c < 4; c++) {
-                            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[a & 1], bh[c], acc[a][c], 0, 0, 0);
-                            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bl[c], acc[a][c], 0, 0, 0);
-                            acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bh[c], acc[a][c], 0, 0, 0);
-                        }
-                    }
-                    if (a == 0) {
-                        if (kt + 1 == NKS) {
-#pragma unroll
-                            for (int j = 0; j < NQ; j++) rs[j] = nrs[j];
-                            cs[0] = ncs[0];
-                            cs[1] = ncs[1];
-                        }
-                        if (kt + 1 + BD == NKS) {
-                            ld.set_columns(o, more);
-                            ld.scales(o, nrs, ncs);
-                        }
-                        if (kt + 2 == NKS) ld.set_rows(o);
-                        ld.template bstore<S>(cs, rbh[set], rbl[set], Bh[ob], Bl[ob]);
-                    }
-                    if (a >= 1 && a <= NQ) {
-                        ld.template astore1<S>(a - 1, rs[a - 1], rah[a - 1], ral[a - 1], Ah[ob], Al[ob]);
-                        ld.aload1(a - 1, ka * BK, rah[a - 1], ral[a - 1]);
-                    }
-                    if (a == NQ + 1) ld.bload(kb * BK, rbh[set], rbl[set]);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                __syncthreads();
-                if (BD % 2) buf = ob;
+            for (int kt = 0; kt + 1 < NKS; kt++) {
+                ld.template step<false>(kt, o, on, more, sh.rows + ab * RBUF, sh.columns + bb * CBUF, sh.rows + (ab ^ 1) * RBUF,
+                                        sh.columns + (bb == 0 ? 2 : bb - 1) * CBUF, sh.scales);
+                next();
             }
+            ld.template step<true>(NKS - 1, o, on, more, sh.rows + ab * RBUF, sh.columns + bb * CBUF,
+                                   sh.rows + (ab ^ 1) * RBUF, sh.columns + (bb == 0 ? 2 : bb - 1) * CBUF, sh.scales);
+            next();
+            o = on;
         }
-        // the scales before the first store, as in k_gemm_m2l_f16x3
-        const float* rv = A.cls_rinv + (size_t)tile.cls * R;
-        float4 r[NB0];
-        float sinv[4];
-        float* out[4];
-#pragma unroll
-        for (int a = 0; a < NB0; a++) r[a] = *(const float4*)(rv + min(rb0 + a, NB - 1) * 16 + 4 * g);
-#pragma unroll
-        for (int c = 0; c < 4; c++) out[c] = ld.column(min(wc * 64 + 16 * c + li, 3 * tile.ng - 1), sinv[c]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the loads ahead that nothing reads
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            if (wc * 64 + 16 * c + li >= 3 * tile.ng) continue;
+            const int cl = ld.wc * 64 + 16 * c + (ld.lane & 15);
+            if (cl >= 3 * ld.tile.ng) continue;
+            float* out = ld.slab(cl) + 4 * (ld.lane >> 4);
 #pragma unroll
-            for (int a = 0; a < NB0; a++) {
-                if (rb0 + a >= NB) break;
-                const f32x4 v = f32x4{acc[a][c][0] * r[a].x * sinv[c], acc[a][c][1] * r[a].y * sinv[c],
-                                      acc[a][c][2] * r[a].z * sinv[c], acc[a][c][3] * r[a].w * sinv[c]};
-                __builtin_nontemporal_store(v, (f32x4*)(out[c] + (rb0 + a) * 16 + 4 * g));
+            for (int a = 0; a < Tile::NB0; a++) {
+                if (ld.rb0 + a >= NB) break;
+                __builtin_nontemporal_store(ld.result(a, c), (f32x4*)(out + (ld.rb0 + a) * 16));
             }
         }
     }
@@ -935,79 +1012,58 @@ void split_columns(const float* M, int ncols, int L, int Lp, int Kp, const float
     FMM_HIP(hipGetLastError());
 }
 
+constexpr int M2L_GROUP_DMA_NB = 6, M2L_GROUP_MAX_NB = 19;   // groups: k_gemm_m2l_f16x3_q from p = 8, up to p = 16
 int m2l_f16_rows(int L) { return 16 * ((L + 15) / 16); }
 bool m2l_f16x3_persistent(int L) {
     const int nb = m2l_f16_rows(L) / 16;
-    return nb >= 14 && nb <= 23;   // the 128-column tiles of launch_f16x3_128 below
+    return nb >= 14 && nb <= 23;   // see launch_f16x3
 }
 // A class of few pairs falls into group classes of fewer still, whose tiles are mostly empty and read more
-// operators, and the grouping waits twice for counts; the persistent kernel loses least by it.  Grouped
-// against single pairs, GEMM alone or whole evaluations: persistent, 182 to 450 pairs a class (p = 14, 16) 0.87
-// to 1.0 of the time, 75 (p = 13, then the other kernel) 1.45 / 1.80 ms for single pairs; the other kernel, 2,094
-// pairs (p = 8) 1.11 / 1.66 ms for groups, 1,149 (p = 12) 6.14 / 6.3, but 184 (p = 12) 4.0 / 2.7 ms, 214 (p = 13)
-// 1.68 / 0.64 and 516 (p = 10) 0.89 / 0.51 for single pairs.
-int m2l_group_min_pairs(int L) { return m2l_f16x3_persistent(L) ? 128 : 1024; }
+// operators, and the grouping waits twice for counts.  Whole evaluations, groups / single pairs in ms, of coils
+// and clusters of 30,000 to 1,000,000 points: p = 8, 261 pairs a class 2.09 / 2.01, 316 7.5 / 8.8, 441 3.36 / 3.50;
+// p = 12, 112 5.3 / 5.0, 261 2.74 / 2.63, 316 12.1 / 14.4; p = 14, 112 6.7 / 6.3, 261 3.31 / 3.23, 316 16.5 / 18.3;
+// p = 16, 112 9.1 / 8.5, 261 4.06 / 4.01, 316 22.7 / 24.3, 450 4.97 / 5.14.  In the kernel of the orders up to 7
+// (p = 5) 261 1.88 / 1.70, 441 3.1 / 2.9, 427 (8 million pairs) 10.1 / 10.0.  Above p = 16 two sets of
+// accumulators do not fit.
+int m2l_group_min_pairs(int L) {
+    const int nb = m2l_f16_rows(L) / 16;
+    return nb > M2L_GROUP_MAX_NB ? INT32_MAX : nb >= M2L_GROUP_DMA_NB ? 300 : 1024;
+}
 int m2l_f16_kpad(int L) { return 32 * ((L + 31) / 32); }
 
-__global__ void k_sibling_scales(const int* __restrict__ parent, const int* __restrict__ first_child, int n,
-                                 const float* __restrict__ cscale, float* __restrict__ ratio,
-                                 float* __restrict__ pinv) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == n) ratio[i] = pinv[i] = 0.0f;   // the column of zeros
-    if (i >= n) return;
-    const int v = i / 3, p = parent[v];
-    float mn = cscale[i];
-    if (p >= 0)
-        for (int o = 0; o < 8; o++) mn = fminf(mn, cscale[3 * (first_child[p] + o) + (i - 3 * v)]);
-    ratio[i] = mn / cscale[i];
-    pinv[i] = 1.0f / mn;
-}
-void sibling_scales(const int* parent, const int* first_child, int nnodes, const float* cscale, float* ratio,
-                    float* pinv, hipStream_t st) {
-    if (!nnodes) return;
-    k_sibling_scales<<<blocks(3ll * nnodes + 1), 256, 0, st>>>(parent, first_child, 3 * nnodes, cscale, ratio, pinv);
-    FMM_HIP(hipGetLastError());
-}
-
-__global__ void k_group_row_scales(const int* __restrict__ cls_ops, const int* __restrict__ cls_mask, int ncls, int R,
-                                   const float* __restrict__ ops_rinv, float* __restrict__ cls_rinv) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)ncls * R) return;
-    const int c = (int)(i / R), row = (int)(i - (long long)c * R);
-    float r = 0.0f;
-    for (int m = cls_mask[c]; m; m &= m - 1)
-        r = fmaxf(r, ops_rinv[(size_t)cls_ops[8 * (size_t)c + __builtin_ctz(m)] * R + row]);
-    cls_rinv[i] = r;
-}
-void group_row_scales(FarGroups& G, const float* ops_rinv, int L, hipStream_t st) {
-    if (!G.num_classes) return;
-    const int R = m2l_f16_rows(L);
-    const size_t n = (size_t)G.num_classes * R;
-    k_group_row_scales<<<blocks((long long)n), 256, 0, st>>>(G.cls_ops.as<int>(), G.cls_mask.as<int>(), G.num_classes, R,
-                                                             ops_rinv, G.cls_rinv.get<float>(n));
-    FMM_HIP(hipGetLastError());
-}
-
-// The double-buffered 2 x 2 kernel where the single-buffered one's accumulators leave one workgroup per
-// CU anyway (R >= 224, p >= 14) and its two LDS buffers fit (R <= 368, p <= 18); the single-buffered
-// kernel (two or more workgroups per CU below) otherwise
+// The 2 x 2 kernel for groups (from three K steps on), and for single pairs where the other one's
+// accumulators leave one workgroup per CU anyway (R >= 224, p >= 14) and the LDS buffers fit (R <= 368, p <= 18)
 template <int NB, int NKS>
 static void launch_f16x3(const M2LGroupArgs& A, bool single, int* queues, hipStream_t st) {
-    if constexpr (NB >= 14 && NB <= 23) {
-        // one workgroup per CU (the two LDS buffers), 8 per XCD round
-        const int grid = std::min(8 * ((A.ntiles + 7) / 8), 8 * ((num_cus() + 7) / 8));
-        k_gemm_m2l_f16x3_q<NB, NKS, NKS % 2 ? 1 : 2><<<grid, 256, 0, st>>>(A, queues);
-    } else {
-        (single ? k_gemm_m2l_f16x3<NB, NKS, true> : k_gemm_m2l_f16x3<NB, NKS, false>)<<<A.ntiles, 256, 0, st>>>(A);
-    }
+    constexpr bool persistent = NB >= 14 && NB <= 23, dma_groups = NB >= M2L_GROUP_DMA_NB && NB <= M2L_GROUP_MAX_NB;
+    // from p = 14 one workgroup per CU, 8 per XCD round, with a near-field workgroup beside it; below, two fit
+    // on a CU at p = 8 (74 KB of LDS, 224 registers; 0.58 ms, one 0.77: 1M points) and do no harm above
+    const int grid = std::min(8 * ((A.ntiles + 7) / 8), (NB >= 14 ? 8 : 16) * ((num_cus() + 7) / 8));
+    if constexpr (persistent)
+        if (single) {
+            k_gemm_m2l_f16x3_q<NB, NKS, true><<<grid, 256, 0, st>>>(A, queues);
+            return;
+        }
+    if constexpr (dma_groups)
+        if (!single) {
+            k_gemm_m2l_f16x3_q<NB, NKS, false><<<grid, 256, 0, st>>>(A, queues);
+            return;
+        }
+    if constexpr (!persistent)
+        if (single) {
+            k_gemm_m2l_f16x3<NB, NKS, true><<<A.ntiles, 256, 0, st>>>(A);
+            return;
+        }
+    if constexpr (NB < M2L_GROUP_DMA_NB) k_gemm_m2l_f16x3<NB, NKS, false><<<A.ntiles, 256, 0, st>>>(A);
+    else throw Error(1, "FP16 M2L: no kernel over groups for this order");
 }
 
 void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, const FarGroups& G,
-                    const _Float16* src_hl, const float* ratio, const float* pinv, int zero_col, float* slab, int L,
-                    int* queues, hipStream_t st) {
+                    const _Float16* src_hl, const float* cscale, int zero_col, float* slab, int L, int* queues,
+                    hipStream_t st) {
     if (!G.num_tiles) return;
-    const M2LGroupArgs A{ops_hi, ops_lo, ops_rinv, G.tiles.as<GroupTile>(), G.cls_ops.as<int>(), G.cls_rinv.as<float>(),
-                         G.fc.as<int>(), G.mask.as<int>(), src_hl, ratio, pinv, slab, G.num_tiles, zero_col};
+    const M2LGroupArgs A{ops_hi, ops_lo, ops_rinv, G.tiles.as<GroupTile>(), G.cls_ops.as<int>(), G.fc.as<int>(),
+                         G.mask.as<int>(), src_hl, cscale, slab, G.num_tiles, zero_col};
     const int nb = m2l_f16_rows(L) / 16, nks = m2l_f16_kpad(L) / 32;
     // the row and K counts of the orders 1 .. 20
 #define FMM_F16(NBV, NKV)                                      \

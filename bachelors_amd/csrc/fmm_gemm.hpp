@@ -64,14 +64,14 @@ void m2l_gemm(Precision prec, const void* ops, const void* ops_lo, const GemmTil
 // m2l_f16_rows(L), K padded to Kp = m2l_f16_kpad(L); the multipoles enter split by split_columns
 // (src_hl [node * 3 + comp][Kp / 32][hi 32 | lo 32], equilibrated by dm[>= Kp], the per-coefficient
 // scales the tables were built with, and by cscale[node * 3 + comp]).
-// The column scale: the power of 2 that brings the column's largest value mx into [0.5, 1); 2^126, which
-// never is the smallest scale among siblings, for a column of zeros
+// The column scale: the power of 2 that brings the column's largest value mx into [0.5, 1); 1 for a column
+// of zeros
 __device__ __forceinline__ float column_scale(float mx) {
-    return mx > 0.0f ? exp2f((float)min(-(ilogbf(mx) + 1), 126)) : 0x1p126f;
+    return mx > 0.0f ? exp2f((float)min(-(ilogbf(mx) + 1), 126)) : 1.0f;
 }
 int m2l_f16_rows(int L);
-// whether the F16X3 M2L of order (L = (p + 1)^2) runs as the persistent one-workgroup-per-CU kernel
-// (128-column tiles) that leaves room for a near-field workgroup per CU
+// whether the F16X3 M2L of order (L = (p + 1)^2) runs as a persistent grid of one workgroup per CU that leaves
+// room for a near-field workgroup beside each
 bool m2l_f16x3_persistent(int L);
 int m2l_group_min_pairs(int L);   // far pairs per class from which the F16X3 M2L runs over groups
 int m2l_f16_kpad(int L);
@@ -79,19 +79,13 @@ int m2l_f16_kpad(int L);
 // left as they are (the P2M writes them, see launch_p2m); column ncols is set to zeros
 void split_columns(const float* M, int ncols, int L, int Lp, int Kp, const float* dm, float* scale, _Float16* hl,
                    hipStream_t st, const int* skip_first_child = nullptr, const int* skip_npts = nullptr);
-// per column: ratio = (smallest column scale of the node's siblings) / (its own), a power of 2 <= 1, and
-// pinv = 1 / that smallest scale (the same for all siblings), by which a group's sum is scaled back;
-// both have an entry 3 nnodes for the column of zeros
-void sibling_scales(const int* parent, const int* first_child, int nnodes, const float* cscale, float* ratio,
-                    float* pinv, hipStream_t st);
 // The M2L of all groups of far pairs (fmm_groups.hpp): slab[3 * group + comp][m2l_f16_rows(L)] = the sum
 // over the group's children.  queues: 8 device ints, the per-XCD tile counters of the persistent kernel
 // (0 at the launch).
 struct FarGroups;
-void group_row_scales(FarGroups& G, const float* ops_rinv, int L, hipStream_t st);
 void m2l_gemm_f16x3(const _Float16* ops_hi, const _Float16* ops_lo, const float* ops_rinv, const FarGroups& G,
-                    const _Float16* src_hl, const float* ratio, const float* pinv, int zero_col, float* slab, int L,
-                    int* queues, hipStream_t st);
+                    const _Float16* src_hl, const float* cscale, int zero_col, float* slab, int L, int* queues,
+                    hipStream_t st);
 
 // tiles of at most width columns (default 64) over the classes' columns 3 * class_begin
 void plan_tiles(const std::vector<int>& class_begin, const std::vector<int>& class_op, std::vector<GemmTile>& tiles,

@@ -20,7 +20,6 @@ struct FarGroups {
     bool single = false;             // every pair a group of its own, group class = far class
     DevBuf fc, mask;                 // per group: first child of the sources' parent, child mask
     DevBuf cls_ops, cls_mask;        // per group class: far class (operator) of child o at [8 c + o]; children in use
-    DevBuf cls_rinv;                 // [class][R]: largest row scale 1 / rs over the class's operators
     DevBuf tiles;                    // GroupTile
     // scratch: pairs and groups in (target, parent) order, keys, scans
     DevBuf key, key2, val, perm, perm2, flag, pos, g_t, g_fc, g_mask, g_start, skey, skey2, code, flag2, pos2, cls_begin,

@@ -471,3 +471,55 @@ def test_target_extent_on_device_equals_host(fm, nt):
         F.close()
     for k in trees[0]:
         assert np.array_equal(trees[0][k], trees[1][k]), k
+
+
+def _far_part(fm, precision, p, src, w, tgt, **kw):
+    F = fm.FMM(order=p, source_leaf_capacity=32, target_leaf_capacity=32, precision=precision, frame=1, **kw)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    F.run(1.0)
+    far, st = F.B_parts()[0], F.stats()
+    F.close()
+    return far, st
+
+
+@pytest.mark.parametrize("p", [8, 12, 14, 16])
+def test_f16x3_groups_beside_a_strong_leaf(fm, p):
+    """One source leaf of 2^20 times the weight: where it is no far pair, its siblings' groups keep the
+    accuracy of their own columns.  Targets whose far field of the strong leaf alone is exactly zero, against
+    FP64 on the same trees: 1e-6, as against the oracle."""
+    rng = np.random.default_rng(50 + p)
+    n = 30000
+    src, tgt = rng.uniform(-2.9, 2.9, (n, 3)), rng.uniform(-2.9, 2.9, (n, 3))
+    strong = np.all((src > 0) & (src < 0.375), axis=1)   # a box of the tree's fourth level, around 8 points
+    assert strong.sum() > 3
+    w = rng.uniform(0.5, 1.5, n) / n
+    w[strong] *= 2.0 ** 20
+    only, _ = _far_part(fm, "fp64", p, src, np.where(strong, w, 0.0), tgt)
+    sel = np.all(only == 0, axis=1)
+    assert sel.sum() > 20
+    exact, st = _far_part(fm, "fp64", p, src, w, tgt)
+    far, _ = _far_part(fm, "f16x3", p, src, w, tgt)
+    assert st["far_pairs"] >= 1024 * st["m2l_classes"]   # groups at every order
+    assert rel_l2(far[sel], exact[sel]) < 1e-6
+
+
+@pytest.mark.parametrize("p", [1, 2, 4, 9, 12, 14, 16])
+def test_f16x3_groups_of_the_short_m2l(fm, p):
+    """M2L with l + lambda <= p over groups: the operators of some children have rows of zeros (an offset in a
+    lattice plane) where their siblings' have none.  Local expansions against FP64 on the same trees: 1e-6, as B
+    against the oracle."""
+    rng = np.random.default_rng(70 + p)
+    n = 30000
+    src, tgt = rng.uniform(-2.9, 2.9, (n, 3)), rng.uniform(-2.9, 2.9, (n, 3))
+    local = {}
+    for precision in ("fp64", "f16x3"):
+        F = fm.FMM(order=p, source_leaf_capacity=32, target_leaf_capacity=32, precision=precision, frame=1, m2l_full=0)
+        F.set_sources(src, np.full(n, 1.0 / n))
+        F.set_targets(tgt)
+        F.run(1.0)
+        st = F.stats()
+        local[precision] = np.array([F.expansion(1, b) for b in range(0, st["target_nodes"], st["target_nodes"] // 300)])
+        F.close()
+    assert st["far_pairs"] >= 1024 * st["m2l_classes"]
+    assert rel_l2(local["f16x3"], local["fp64"]) < 1e-6
