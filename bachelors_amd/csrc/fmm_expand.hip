@@ -443,8 +443,11 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
 // thread finds its source in it, and the batch after the current one is on its way while the current
 // one is summed from LDS.  The leaf's targets go in even blocks of at most 128, n of them spread over
 // the workgroup with G = floor(256 / n) lanes each: lane g n + t takes the sources g, g + G, ... for target
-// t, so the lanes of a wave read one or a few sources at a time (broadcasts).  Partial sums of at most 64
-// terms in R are added up in FP64, over the G lanes in a fixed order.
+// t, so the lanes of a wave read one or a few sources at a time (broadcasts).  Partial sums of at most RUN
+// terms in R are added up in FP64, over the G lanes in a fixed order.  A run does not end at a node's border, so
+// in FP32 it is kept to 8 terms: at 64 the median error of a target among small leaves (100,000 x 400,000 clustered
+// points, 32 a leaf) was 1.27e-7, with runs within nodes 1.22e-7, now 1.20e-7 (999,983 x 750,019, 48 a leaf: 1.36e-7,
+// 1.39e-7, 1.22e-7), for 2 to 5 % of the near field's time (4M shells 5.68 -> 5.98 ms alone).
 // KIND: B, the vector potential sum_j q_j / |x - y_j|, or the BEM potential (FP64), whose source has a
 // strength v = q and a number d (in the place of the low part of its x).
 // The batches may be shared by `parts` workgroups per leaf, each writing its own sums; out: the leaf's
@@ -473,6 +476,7 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
                                          const int* __restrict__ parent = nullptr) {
     typedef typename V4<R>::t v4;
     constexpr bool split = sizeof(R) == 4;
+    constexpr int RUN = split ? 8 : 64;   // terms of a partial sum in R
     static_assert(KIND != NEAR_BEM || !split, "the BEM potential is FP64");
     static_assert(sizeof(sh.s0) + sizeof(sh.s1) >= 256 * 3 * sizeof(double), "the sums reuse the source buffers");
     double(*red)[3] = (double(*)[3])sh.s0;
@@ -547,7 +551,7 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
                 p2 = P2[j];
                 __syncthreads();
                 for (int q = valid ? g : nj; q < nj;) {
-                    const int qe = min(nj, q + 64 * G);
+                    const int qe = min(nj, q + RUN * G);
                     R f0 = 0, f1 = 0, f2 = 0;
 #pragma unroll 1
                     for (; q < qe; q += G) {

@@ -523,3 +523,25 @@ def test_f16x3_groups_of_the_short_m2l(fm, p):
         F.close()
     assert st["far_pairs"] >= 1024 * st["m2l_classes"]
     assert rel_l2(local["f16x3"], local["fp64"]) < 1e-6
+
+
+def test_near_field_sums_few_terms_in_fp32(fm):
+    """One leaf of 64 targets and sources of which one in 64 is 2^25 times the others: a weak term after a strong one
+    is below half a unit of the sum's last place.  Runs of 8 FP32 terms lose 4 2^-25 of a strong term each on
+    average, 1.2e-7, runs of 64 about 32 2^-25, 9.5e-7; the pairs' own roundings (some 5 units of 2^-24 each, of both
+    signs) average out to less than 2e-7 over the 64 strong sources.  5e-7 against FP64."""
+    rng = np.random.default_rng(90)
+    n = 4096
+    src = rng.uniform(0.4, 0.6, (n, 3))
+    w = np.where(np.arange(n) % 64 == 0, 1.0, 2.0 ** -25)[rng.permutation(n)]
+    J = np.tile([1.0, 0.0, 0.0], (n, 1))
+    tgt = rng.uniform(-0.6, -0.4, (64, 3))
+    near = {}
+    for precision in ("fp64", "fp32"):
+        F = fm.FMM(order=4, source_leaf_capacity=5000, target_leaf_capacity=64, precision=precision, frame=1)
+        F.set_sources(src, w, J)
+        F.set_targets(tgt)
+        F.run(1.0)
+        near[precision] = F.B_parts()[1]
+        F.close()
+    assert rel_l2(near["fp32"], near["fp64"]) < 5e-7
