@@ -613,32 +613,37 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
 //
 // A few leaves near the sources can hold most of the pairs: with one workgroup per leaf the time is that
 // of the longest list, or of the last ones to start (1M uniform targets around a coil of 1M sources: 1.0
-// ms in FP32, 2.7 ms in FP64; 32,768 x 4,096 points in 276 leaves, FP64: 470 us).  A part is therefore
-// at most `batches` batches of 256 sources (near_batches), and the register budget is that of 7 (FP64: 5) waves a
+// ms in FP32, 2.7 ms in FP64; 32,768 x 4,096 points in 276 leaves, FP64: 470 us).  A list is therefore cut
+// into 2, 4, .. 32 parts of at most `batches` batches of 256 sources (near_batches; longer ones where 32 parts
+// are not enough), and the register budget is that of 7 (FP64: 5) waves a
 // SIMD (no unrolling), since the short lists are a matter of latency: 1M points 1007 (items alone: 1230) ->
 // 660 us in FP32, 2.7 -> 2.0 ms in FP64, beside the slab reduction; 262,147 x 131,101 clustered points 1520
 // -> 330 us, transposed 1270 -> 420 us; B and A of 250,000 points 365 + 307 -> 267 + 237 us; 276 leaves 90
 // -> 75 us.
+//
+// The order of a target's sum follows from the parts of its leaf, so these follow from the lists alone: where
+// the parts of all leaves together would take more items or rows than there are, all leaves are held to 16 parts,
+// or 8, and so on (sums: what they take at 2, 4, .. 32).  Where the parts lie, by atomics, enters no sum.
+constexpr int NEAR_MAX_PARTS = 32, NEAR_CUTS = 5;
 struct NearWork {
     const int* leaves;
     int nleaves;
     int2* desc;
     int2* extra;
     int* counters;
+    unsigned long long* sums;   // [2 q]: extra items, [2 q + 1]: rows, of all leaves with parts cut to 2 << q
     double* partial;
     int extra_cap, extra_wgs;
 };
 
-// the parts of every leaf; 16 leaves a workgroup, 16 lanes a leaf.  Where the extra items or the rows run
-// out, a workgroup's leaves keep one part each.
-constexpr int NEAR_MAX_PARTS = 32;
+// the parts every leaf asks for, and the sums; 16 leaves a workgroup, 16 lanes a leaf
 template <bool UP>
-__global__ __launch_bounds__(256) void k_near_items(NearWork w, int batches, int rows_cap, const int* __restrict__ tbegin,
+__global__ __launch_bounds__(256) void k_near_loads(NearWork w, int batches, const int* __restrict__ tbegin,
                                                     const int* __restrict__ tend, const int* __restrict__ parent,
                                                     const int* __restrict__ close_begin,
                                                     const int* __restrict__ close_end, const int* __restrict__ close_s,
                                                     const int* __restrict__ sbegin, const int* __restrict__ send) {
-    __shared__ int first_item[16], first_row[16], parts_of[16], fits;
+    __shared__ int parts_of[16], targets_of[16];
     const int tid = threadIdx.x, u = tid >> 4, lane = tid & 15, li = 16 * blockIdx.x + u;
     int n = 0;
     long long load = 0;
@@ -654,42 +659,52 @@ __global__ __launch_bounds__(256) void k_near_items(NearWork w, int batches, int
     for (int d = 1; d < 16; d <<= 1) load += __shfl_xor(load, d);
     int parts = 1;
     while (parts < NEAR_MAX_PARTS && (long long)parts * batches * 256 < load) parts *= 2;
-    while (parts > 1 && (long long)(parts - 1) * n > 1 << 24) parts >>= 1;   // the sums below stay in 32 bits
+    while (parts > 1 && (long long)(parts - 1) * n > 1 << 24) parts >>= 1;   // a wave's rows stay in 32 bits
     if (lane == 0) {
         parts_of[u] = parts;
-        first_row[u] = (parts - 1) * n;
+        targets_of[u] = n;
+        if (li < w.nleaves) w.desc[li] = make_int2(parts, 0);
     }
     __syncthreads();
-    if (tid < 16) {
-        const int p = parts_of[tid] - 1, r = first_row[tid];
-        int ip = p, ir = r;
-        for (int d = 1; d < 16; d <<= 1) {
-            const int vp = __shfl_up(ip, d, 16), vr = __shfl_up(ir, d, 16);
-            if (tid >= d) {
-                ip += vp;
-                ir += vr;
-            }
-        }
-        int bp = 0, br = 0;
-        if (tid == 15 && ip) {
-            bp = atomicAdd(&w.counters[0], ip);
-            br = atomicAdd(&w.counters[1], ir);
-        }
-        bp = __shfl(bp, 15, 16);
-        br = __shfl(br, 15, 16);
-        const int np = __shfl(ip, 15, 16), nr = __shfl(ir, 15, 16);
-        const bool ok = bp >= 0 && br >= 0 && bp <= w.extra_cap - np && br <= rows_cap - nr;
-        first_item[tid] = bp + ip - p;
-        first_row[tid] = br + ir - r;
-        if (tid == 0) fits = ok;
-        if (!ok)   // the items that this workgroup took are nobody's
-            for (int q = bp + tid; bp >= 0 && q < min(w.extra_cap, bp + np); q += 16) w.extra[q] = make_int2(-1, 0);
+    if (tid < 2 * NEAR_CUTS) {
+        unsigned long long s = 0;
+        for (int e = 0; e < 16; e++)
+            s += (unsigned long long)(min(parts_of[e], 2 << (tid >> 1)) - 1) * (tid & 1 ? targets_of[e] : 1);
+        if (s) atomicAdd(w.sums + tid, s);
     }
-    __syncthreads();
+}
+
+// the parts every leaf gets, and their places; a thread per leaf
+__global__ __launch_bounds__(256) void k_near_items(NearWork w, int rows_cap, const int* __restrict__ tbegin,
+                                                    const int* __restrict__ tend) {
+    const int li = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    int cut = 1;
+    for (int q = 0; q < NEAR_CUTS; q++)   // the sums grow with q
+        if (w.sums[2 * q] <= (unsigned)w.extra_cap && w.sums[2 * q + 1] <= (unsigned)rows_cap) cut = 2 << q;
+    int items = 0, rows = 0;
+    if (li < w.nleaves) {
+        const int leaf = w.leaves[li];
+        items = min(w.desc[li].x, cut) - 1;
+        rows = items * (tend[leaf] - tbegin[leaf]);
+    }
+    int ii = items, ir = rows;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int vi = __shfl_up(ii, d, 64), vr = __shfl_up(ir, d, 64);
+        if (lane >= d) {
+            ii += vi;
+            ir += vr;
+        }
+    }
+    int bi = 0, br = 0;
+    if (lane == 63 && ii) {
+        bi = atomicAdd(&w.counters[0], ii);
+        br = atomicAdd(&w.counters[1], ir);
+    }
+    bi = __shfl(bi, 63, 64) + ii - items;
+    br = __shfl(br, 63, 64) + ir - rows;
     if (li >= w.nleaves) return;
-    if (!fits) parts = 1;
-    if (lane == 0) w.desc[li] = make_int2(parts, first_row[u]);
-    for (int q = 1 + lane; q < parts; q += 16) w.extra[first_item[u] + q - 1] = make_int2(li, q);
+    w.desc[li] = make_int2(items + 1, br);
+    for (int q = 0; q < items; q++) w.extra[bi + q] = make_int2(li, q + 1);
 }
 
 // near[leaf] += the sums of its further parts, in their order; a wave per leaf
@@ -720,7 +735,7 @@ __device__ __forceinline__ void p2p_items(const NearWork& w, const int* __restri
                                           const int* __restrict__ parent = nullptr) {
     __shared__ P2PShared<R> sh;
     __shared__ int next;
-    const int nextra = w.desc ? min(w.counters[0], w.extra_cap) : 0;
+    const int nextra = w.desc ? w.counters[0] : 0;
     // i < nleaves: part 0 of leaf i, else extra item i - nleaves
     const bool own = !QUEUE && (int)blockIdx.x >= w.extra_wgs;   // one leaf
     for (int i = own ? blockIdx.x - w.extra_wgs : w.nleaves + blockIdx.x;; i += w.extra_wgs) {
@@ -732,13 +747,11 @@ __device__ __forceinline__ void p2p_items(const NearWork& w, const int* __restri
         }
         if (i >= w.nleaves + nextra) break;
         const int2 it = i < w.nleaves ? make_int2(i, 0) : w.extra[i - w.nleaves];
-        if (it.x >= 0) {
-            const int leaf = w.leaves[it.x], tb = tbegin[leaf];
-            const int2 d = w.desc ? w.desc[it.x] : make_int2(1, 0);
-            double* out = it.y ? w.partial + 3 * ((size_t)d.y + (size_t)(it.y - 1) * (tend[leaf] - tb)) : near + 3 * (size_t)tb;
-            p2p_leaf<R, KIND, UP>(leaf, it.y, d.x, tbegin, tend, close_begin, close_end, close_s, origin, sbegin,
-                                          send, P0, P1, P2, txyz, out, sh, parent);
-        }
+        const int leaf = w.leaves[it.x], tb = tbegin[leaf];
+        const int2 d = w.desc ? w.desc[it.x] : make_int2(1, 0);
+        double* out = it.y ? w.partial + 3 * ((size_t)d.y + (size_t)(it.y - 1) * (tend[leaf] - tb)) : near + 3 * (size_t)tb;
+        p2p_leaf<R, KIND, UP>(leaf, it.y, d.x, tbegin, tend, close_begin, close_end, close_s, origin, sbegin, send, P0,
+                              P1, P2, txyz, out, sh, parent);
         if (own) break;
     }
 }
@@ -1183,7 +1196,8 @@ static NearWork near_work(const int* leaves, int nleaves, size_t rows, NearScrat
     w.extra_wgs = 0;
     w.desc = scratch.desc.get<int2>(nleaves);
     w.extra = scratch.extra.get<int2>(w.extra_cap);
-    w.counters = scratch.counters.get<int>(4);
+    w.sums = scratch.counters.get<unsigned long long>(2 * NEAR_CUTS + 2);
+    w.counters = (int*)(w.sums + 2 * NEAR_CUTS);
     w.partial = scratch.partial.get<double>(3 * rows);
     return w;
 }
@@ -1193,10 +1207,12 @@ static size_t near_rows(int nslots) { return 2 * (size_t)nslots + 262144; }
 template <bool UP>
 static void make_items(const NearWork& w, const TreeDev& T, const TreeDev& S, const int* close_begin,
                        const int* close_end, const int* close_s, hipStream_t st) {
-    FMM_HIP(hipMemsetAsync(w.counters, 0, 3 * sizeof(int), st));
-    k_near_items<UP><<<(w.nleaves + 15) / 16, 256, 0, st>>>(
-        w, near_batches(w.nleaves), (int)std::min<size_t>(near_rows(T.num_slots), INT32_MAX), T.begin.as<int>(),
-        T.end.as<int>(), T.parent.as<int>(), close_begin, close_end, close_s, S.begin.as<int>(), S.end.as<int>());
+    FMM_HIP(hipMemsetAsync(w.sums, 0, (2 * NEAR_CUTS + 2) * sizeof(unsigned long long), st));
+    k_near_loads<UP><<<(w.nleaves + 15) / 16, 256, 0, st>>>(w, near_batches(w.nleaves), T.begin.as<int>(), T.end.as<int>(),
+                                                            T.parent.as<int>(), close_begin, close_end, close_s,
+                                                            S.begin.as<int>(), S.end.as<int>());
+    k_near_items<<<blocks(w.nleaves), 256, 0, st>>>(w, (int)std::min<size_t>(near_rows(T.num_slots), INT32_MAX),
+                                                    T.begin.as<int>(), T.end.as<int>());
     FMM_HIP(hipGetLastError());
 }
 static void add_parts(const NearWork& w, const TreeDev& T, double* near, hipStream_t st) {
@@ -1207,7 +1223,7 @@ static void add_parts(const NearWork& w, const TreeDev& T, double* near, hipStre
 template <bool UP>
 static NearWork start_near(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                            const int* close_end, const int* close_s, NearScratch& scratch, int& grid, hipStream_t st) {
-    NearWork w{leaves, nleaves, nullptr, nullptr, nullptr, nullptr, 0, 0};
+    NearWork w{leaves, nleaves, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
     grid = nleaves;
     if (S.num_slots > NEAR_SPLIT_SOURCES) {
         w = near_work(leaves, nleaves, near_rows(T.num_slots), scratch);

@@ -140,3 +140,33 @@ def test_transposed_m2l_at_every_row_padding(order, precision, tol):
     rhs = float((wt.detach() * wt.grad).sum())
     assert F._fmm.stats()["far_pairs"] > 0
     assert abs(lhs - rhs) <= tol * abs(lhs)
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("fp32", 2e-6)])
+def test_transposed_near_field_out_of_rows(precision, tol):
+    """40,000 sources in some 64 leaves, each with 65,000 close targets in one leaf, ask for more rows of partial
+    sums than there are: equal bits in every run (no far pairs), and the transpose as above."""
+    import ctypes
+
+    import torch
+    import bachelors_amd as fm
+    rng = np.random.default_rng(97)
+    ns, nt = 40000, 65000
+    F = fm.FMM(order=4, source_leaf_capacity=1000, target_leaf_capacity=nt + 2, precision=precision, frame=1)
+    w = rng.uniform(0.5, 1.5, ns)
+    F.set_sources(rng.uniform(-2.9, 2.9, (ns, 3)), w)
+    F.set_targets(rng.uniform(-2.9, 2.9, (nt, 3)))
+    B = F.run(1.0)
+    st = F.stats()
+    assert st["far_pairs"] == 0 and st["source_leaves"] > 32
+    g = torch.from_numpy(B * (1 + rng.uniform(-0.5, 0.5, B.shape))).cuda()
+    runs = []
+    for _ in range(4):
+        gw = torch.empty(ns, dtype=torch.float64, device="cuda")
+        F.adjoint_weights_dev(1.0, ctypes.c_void_p(g.data_ptr()), ctypes.c_void_p(gw.data_ptr()))
+        F.synchronize()
+        runs.append(gw)
+    F.close()
+    assert all(torch.equal(runs[0], r) for r in runs)
+    lhs, rhs = float((B * g.cpu().numpy()).sum()), float((w * runs[0].cpu().numpy()).sum())
+    assert abs(lhs - rhs) <= tol * abs(lhs)

@@ -545,3 +545,37 @@ def test_near_field_sums_few_terms_in_fp32(fm):
         near[precision] = F.B_parts()[1]
         F.close()
     assert rel_l2(near["fp32"], near["fp64"]) < 5e-7
+
+
+@pytest.mark.parametrize("order,precision,tol", [(4, "fp64", 1e-12), (4, "fp32", 1e-6), (14, "f16x3", 1e-6)])
+@pytest.mark.parametrize("cap_t", [50000, 1000])
+def test_near_field_out_of_rows(fm, order, precision, tol, cap_t):
+    """40,000 targets, each with 65,000 close sources in one leaf, ask for 31 rows of partial sums a target, more
+    than there are: the lists are cut into fewer parts, the same in every run (equal bits), for one leaf and for
+    some 64 (in F16X3 taken from a queue).  Against the direct sum in FP64: no far pairs, so rounding alone."""
+    import ctypes
+
+    import torch
+    rng = np.random.default_rng(95)
+    ns, nt = 65000, 40000
+    F = fm.FMM(order=order, source_leaf_capacity=ns + 2, target_leaf_capacity=cap_t, precision=precision, frame=1)
+    src = torch.from_numpy(shell_sources(rng, ns)).cuda()
+    w = torch.from_numpy(rng.uniform(0.5, 1.5, ns)).cuda()
+    tgt = torch.from_numpy(rng.uniform(-2.9, 2.9, (nt, 3))).cuda()
+    B, exact = torch.empty_like(tgt), torch.empty_like(tgt)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    torch.cuda.synchronize()
+    F.set_sources_dev(ns, ptr(src), ptr(w), None)
+    F.set_targets_dev(nt, ptr(tgt))
+    runs = []
+    for _ in range(4):
+        F.run_B_dev(1.0, ptr(B))
+        F.synchronize()
+        runs.append(B.clone())
+    st = F.stats()
+    assert st["far_pairs"] == 0 and (st["target_leaves"] == 1) == (cap_t == 50000)
+    F.direct_B_dev(1.0, nt, ptr(tgt), ptr(exact))
+    F.synchronize()
+    F.close()
+    assert all(torch.equal(runs[0], r) for r in runs)
+    assert rel_l2(runs[0].cpu().numpy(), exact.cpu().numpy()) < tol
