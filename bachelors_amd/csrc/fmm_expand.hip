@@ -636,6 +636,12 @@ struct NearWork {
     int extra_cap, extra_wgs;
 };
 
+// before every near field; a kernel, because a memset recorded into a graph can fail on later replays
+__global__ void k_near_clear(NearWork w) {
+    if (threadIdx.x < 4) w.counters[threadIdx.x] = 0;
+    if (threadIdx.x < 2 * NEAR_CUTS) w.sums[threadIdx.x] = 0;
+}
+
 // the parts every leaf asks for, and the sums; 16 leaves a workgroup, 16 lanes a leaf
 template <bool UP>
 __global__ __launch_bounds__(256) void k_near_loads(NearWork w, int batches, const int* __restrict__ tbegin,
@@ -1207,7 +1213,7 @@ static size_t near_rows(int nslots) { return 2 * (size_t)nslots + 262144; }
 template <bool UP>
 static void make_items(const NearWork& w, const TreeDev& T, const TreeDev& S, const int* close_begin,
                        const int* close_end, const int* close_s, hipStream_t st) {
-    FMM_HIP(hipMemsetAsync(w.sums, 0, (2 * NEAR_CUTS + 2) * sizeof(unsigned long long), st));
+    k_near_clear<<<1, 64, 0, st>>>(w);
     k_near_loads<UP><<<(w.nleaves + 15) / 16, 256, 0, st>>>(w, near_batches(w.nleaves), T.begin.as<int>(), T.end.as<int>(),
                                                             T.parent.as<int>(), close_begin, close_end, close_s,
                                                             S.begin.as<int>(), S.end.as<int>());

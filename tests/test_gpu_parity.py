@@ -579,3 +579,40 @@ def test_near_field_out_of_rows(fm, order, precision, tol, cap_t):
     F.close()
     assert all(torch.equal(runs[0], r) for r in runs)
     assert rel_l2(runs[0].cpu().numpy(), exact.cpu().numpy()) < tol
+
+
+def test_evaluation_replayed_from_a_graph(fm):
+    """fmm_evaluate_B_dev captured into a graph on the caller's stream (nothing allocated, no wait): every
+    replay equals the eager evaluation, with eager evaluations in between."""
+    import ctypes
+
+    import torch
+    rng = np.random.default_rng(96)
+    src, tgt = shell_sources(rng, 20000), rng.uniform(-2, 2, (3001, 3))
+    out = torch.empty((3001, 3), dtype=torch.float64, device="cuda")
+    ref = torch.empty_like(out)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    s = torch.cuda.Stream()
+    F = fm.FMM(order=4, source_leaf_capacity=64, target_leaf_capacity=64, frame=1)
+    F.set_stream(ctypes.c_void_p(s.cuda_stream))
+    F.set_sources(src, np.full(20000, 1.0 / 20000))
+    F.set_targets(tgt)
+    F.build_trees()
+    F.leaf_expansions()
+    F.upward()
+    F.downward()
+    F.evaluate_B_dev(1.0, ptr(ref))
+    F.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        F.evaluate_B_dev(1.0, ptr(out))
+    for _ in range(4):
+        out.zero_()
+        ref.zero_()
+        torch.cuda.synchronize()
+        F.evaluate_B_dev(1.0, ptr(ref))
+        F.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and float(out.abs().max()) > 0
+    F.close()
