@@ -369,11 +369,12 @@ __global__ __launch_bounds__(64) void k_l2p(const int* __restrict__ leaves, cons
 // source node (the close-list loop of FastMultipoleSolver::calcB, fast_multipole_solver.cpp:214-229;
 // a close node may be internal, then all its subtree's sources are summed).
 //
-// Positions are taken relative to one origin o (the source root centre).  For R = float both
+// For R = float positions are taken relative to one origin o (the source root centre), and both
 // sides are unevaluated sums hi + lo of two floats formed in FP64 (~2^-48 of the root size),
 // so the pair difference d = (x_hi - y_hi) + (x_lo - y_lo) stays accurate for very close
 // pairs (x_hi - y_hi is exact when the two are within a factor 2) while the pair arithmetic
-// runs in FP32.  R = double keeps the offsets whole.
+// runs in FP32.  R = double takes the coordinates themselves (o = 0): the difference of two close
+// ones is exact, and an offset from o that is rounded first would not leave it so.
 template <class R> struct V4;
 template <> struct V4<float> {
     typedef float4 t;
@@ -419,8 +420,8 @@ __device__ __forceinline__ float inv_power(float x) {
     const float ri = x > 0.0f ? __builtin_amdgcn_rsqf(x) : 0.0f;
     return POT ? ri : ri * ri * ri;
 }
-// P0[j] = (hi(y_j - o), q_x), P1[j] = (lo(y_j - o), q_y), P2[j] = q_z for every source slot j; in FP64,
-// where the low parts are zero, P1[j].x holds sd[j] if there is one (BEM)
+// P0[j] = (hi(y_j - o), q_x), P1[j] = (lo(y_j - o), q_y), P2[j] = q_z for every source slot j; in FP64 o = 0 and
+// the low parts are zero, P1[j].x holds sd[j] if there is one (BEM)
 template <class R>
 __global__ void k_pack_sources(int n, const double* __restrict__ origin, const double* __restrict__ sxyz,
                                const double* __restrict__ sq, const double* __restrict__ sd,
@@ -429,7 +430,12 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
     constexpr bool split = sizeof(R) == 4;
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
-    double dx = sxyz[3 * j] - origin[0], dy = sxyz[3 * j + 1] - origin[1], dz = sxyz[3 * j + 2] - origin[2];
+    double dx = sxyz[3 * j], dy = sxyz[3 * j + 1], dz = sxyz[3 * j + 2];
+    if (split) {
+        dx -= origin[0];
+        dy -= origin[1];
+        dz -= origin[2];
+    }
     R hx = (R)dx, hy = (R)dy, hz = (R)dz;
     R lx = split ? (R)(dx - (double)hx) : sd ? (R)sd[j] : (R)0, ly = split ? (R)(dy - (double)hy) : (R)0;
     R lz = split ? (R)(dz - (double)hz) : (R)0;
@@ -494,9 +500,9 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
         const bool valid = g < G;
         double ux = 0, uy = 0, uz = 0;
         if (valid) {
-            ux = txyz[3 * (k0 + ti)] - origin[0];
-            uy = txyz[3 * (k0 + ti) + 1] - origin[1];
-            uz = txyz[3 * (k0 + ti) + 2] - origin[2];
+            ux = txyz[3 * (k0 + ti)] - (split ? origin[0] : 0.0);
+            uy = txyz[3 * (k0 + ti) + 1] - (split ? origin[1] : 0.0);
+            uz = txyz[3 * (k0 + ti) + 2] - (split ? origin[2] : 0.0);
         }
         const R uhx = (R)ux, uhy = (R)uy, uhz = (R)uz;
         const R ulx = split ? (R)(ux - (double)uhx) : (R)0, uly = split ? (R)(uy - (double)uhy) : (R)0;

@@ -21,7 +21,7 @@ void launch_p2m(bool f64, const int* leaves, int nleaves, const TreeDev& S, cons
 void launch_zero_unwritten(const TreeDev& S, int Lp, size_t esize, void* M, hipStream_t st);
 void launch_l2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const ScaleTable& sig, const double* txyz,
                 const void* Lexp, int p, int Lp, double* Bfar, hipStream_t st);
-// near-field sources in slot order relative to origin[3] (a device pointer); P0, P1: 4 x R per
+// near-field sources in slot order, in FP32 relative to origin[3] (a device pointer); P0, P1: 4 x R per
 // slot, P2: R per slot, R = double if f64 else float; sd (f64 only): the BEM sources' d
 void launch_pack_sources(bool f64, int n, const double* origin, const double* sxyz, const double* sq, void* P0,
                          void* P1, void* P2, hipStream_t st, const double* sd = nullptr);

@@ -104,3 +104,36 @@ def test_bem_shared_frame_split_precisions(orc):
         print("%s vs fp64 %.3e" % (precision, e), flush=True)
         assert np.array_equal(np.isfinite(V[:, 0]), ok)
         assert e < 2e-6, precision
+
+
+def test_near_field_of_close_points_off_centre():
+    """FP64 near field of a target 1e-9 from its source, in a tree whose root is off the origin: the difference of
+    two coordinates is exact, so B, A and the BEM potential are those of one pair to 1e-12 (a few ulp, whatever
+    the root's centre; coordinates taken relative to it first would be off by 1e-16 / 1e-9)."""
+    import bachelors_amd as fm
+    rng = np.random.default_rng(98)
+    y = np.array([[0.1, 0.2, 0.3]])
+    d = rng.normal(size=(50, 3))
+    x = y + 1e-9 * d / np.linalg.norm(d, axis=1)[:, None]
+    r = x - y   # exact
+    r3 = np.linalg.norm(r, axis=1)[:, None] ** 3
+    q, b, n = np.array([[0.3, -0.5, 0.8]]), np.array([[0.4, 0.1, -0.7]]), np.array([[0.6, 0.0, 0.8]])
+    root = dict(source_root_center=(0.7, -1.3, 0.9), source_root_half=(3, 3, 3))
+    F = fm.FMM(order=2, source_leaf_capacity=16, target_leaf_capacity=64, precision="fp64", frame=1, **root)
+    F.set_sources(y, np.ones(1), q)
+    F.set_targets(x)
+    B, A = F.run(4 * 3.14159265359), F.evaluate_A(4 * 3.14159265359)
+    F.close()
+    assert rel_l2(B, 1.2566370614e-6 * np.cross(q, r) / r3) < 1e-12
+    assert rel_l2(A, q / np.linalg.norm(r, axis=1)[:, None]) < 1e-12
+    F = fm.FMM(order=2, source_leaf_capacity=16, target_leaf_capacity=64, precision="fp64", frame=1, **root)
+    F.set_bem_sources(y, np.ones(1), b, n)
+    F.set_targets(x)
+    F.build_trees()
+    F.leaf_expansions()
+    F.upward()
+    F.downward()
+    V = F.evaluate_bem()
+    F.close()
+    expect = (-r * (b * n).sum() - np.cross(r, np.cross(b, n))) / r3 / (4 * 3.14159265359)
+    assert rel_l2(V, expect) < 1e-12
