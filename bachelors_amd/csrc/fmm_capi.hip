@@ -1764,11 +1764,12 @@ int fmm_make_operator(int kind, int order, const double* t, double sig_in, doubl
         s.sig_out = sig_out;
         s.kind = kind;
         s.m2l_full = m2l_full;
-        DevBuf d, o;
+        DevBuf d, o, work;
         OpSpec* ds = d.get<OpSpec>(1);
         FMM_HIP(hipMemcpy(ds, &s, sizeof(s), hipMemcpyHostToDevice));
         double* dout = o.get<double>((size_t)Lp * Lp);
-        make_operators(ds, 1, order, Lp, 0, dout, nullptr, 0);
+        if (kind == OPK_M2L) make_m2l(ds, 1, order, Lp, 0, dout, nullptr, work.reserve(m2l_work_bytes(1, order)), 0);
+        else make_operators(ds, 1, order, Lp, 0, dout, nullptr, 0);
         std::vector<double> h((size_t)Lp * Lp);
         FMM_HIP(hipMemcpy(h.data(), dout, h.size() * sizeof(double), hipMemcpyDeviceToHost));
         for (int i = 0; i < L; i++)

@@ -33,18 +33,14 @@ __device__ __forceinline__ cplx harm(const cplx* X, int n, int k) {
     return {v.re, -v.im};
 }
 
-// kernel K(l, m; a, b) of the complex translator (see header comment); zero if absent
-__device__ __forceinline__ cplx kernel_entry(int kind, const cplx* X, int pI, int l, int m, int a, int b) {
+// kernel K(l, m; a, b) of the complex M2M or L2L translator (see header comment); zero if absent
+__device__ __forceinline__ cplx kernel_entry(int kind, const cplx* X, int l, int m, int a, int b) {
     int n, k = m - b;
     double f;
     if (kind == OPK_M2M) {
         n = l - a;
         if (n < 0 || k < -n || k > n) return {0, 0};
         f = sgn_pow(abs((abs(m) - abs(k) - abs(m - k)) / 2));
-    } else if (kind == OPK_M2L) {
-        n = l + a;
-        if (n > pI || k < -n || k > n) return {0, 0};
-        f = sgn_pow(abs((abs(m - b) - abs(m) - abs(b)) / 2)) * sgn_pow(a);
     } else {
         n = a - l;
         if (n < 0 || k < -n || k > n) return {0, 0};
@@ -60,47 +56,31 @@ __device__ __forceinline__ void lm_of(int i, int& l, int& m) {
     m = i - l * l - l;
 }
 
-// nsplit workgroups per operator, each owning a contiguous range of output rows (so a launch
+// M2M and L2L operators: nsplit workgroups per operator, each owning a contiguous range of output rows (so a launch
 // of few operators still fills the GPU).  LDS: the harmonic table X(n, k>=0), the degree/order
 // of every coefficient index and the per-degree scale factor of the operator kind.
 // output: 0 = double, 1 = float, 2 = bf16 hi + bf16 lo (of the float value)
 template <int MODE>
-__global__ __launch_bounds__(256) void k_make_ops(const OpSpec* __restrict__ specs, int p, int pI_full, int Lp,
+__global__ __launch_bounds__(256) void k_make_ops(const OpSpec* __restrict__ specs, int p, int Lp,
                                                   void* __restrict__ out, __bf16* __restrict__ out_lo, int nsplit) {
-    extern __shared__ cplx X[];   // packed (n, k>=0), n <= pH
+    extern __shared__ cplx X[];   // packed (n, k>=0), n <= p
     const int opi = blockIdx.x / nsplit, slice = blockIdx.x - opi * nsplit;
     const OpSpec sp = specs[opi];
     const int kind = sp.kind;
-    const int pH = (kind == OPK_M2L) ? (sp.m2l_full ? pI_full : p) : p;
-    const int pI = pH;
     const int L = (p + 1) * (p + 1);
-    short2* lmt = (short2*)(X + (pI_full + 1) * (pI_full + 2) / 2);   // (l, m) of coefficient i
+    short2* lmt = (short2*)(X + (p + 1) * (p + 2) / 2);                // (l, m) of coefficient i
     double* fac = (double*)(lmt + ((L + 1) & ~1));                     // scale factor per degree
     double su = (kind == OPK_M2M) ? sp.sig_in : sp.sig_out;
     double ux = sp.t[0] / su, uy = sp.t[1] / su, uz = sp.t[2] / su;
     double r2 = ux * ux + uy * uy + uz * uz;
     // column k of the harmonic table, one thread per k
-    for (int k = threadIdx.x; k <= pH; k += blockDim.x) {
-        cplx d;
-        if (kind == OPK_M2L) {
-            // Psi_k^k = (2k-1)!! (x+iy)^k / r^(2k+1)
-            double inv = 1.0 / sqrt(r2);
-            d = {inv, 0};
-            for (int i = 1; i <= k; i++) d = cscale(cmul(d, {ux, uy}), (2.0 * i - 1) / r2);
-        } else {
-            // Phi_k^k = (x+iy)^k / (2^k k!)
-            d = {1, 0};
-            for (int i = 1; i <= k; i++) d = cscale(cmul(d, {ux, uy}), recip(2 * i));
-        }
+    for (int k = threadIdx.x; k <= p; k += blockDim.x) {
+        cplx d = {1, 0};   // Phi_k^k = (x+iy)^k / (2^k k!)
+        for (int i = 1; i <= k; i++) d = cscale(cmul(d, {ux, uy}), recip(2 * i));
         cplx pm2 = {0, 0}, pm1 = d;
         X[tri(k, k)] = cscale(d, sgn_pow(k));
-        for (int n = k + 1; n <= pH; n++) {
-            cplx v;
-            if (kind == OPK_M2L)
-                v = cscale(cadd(cscale(pm1, (2.0 * n - 1) * uz), cscale(pm2, -(double)((n - 1) * (n - 1) - k * k))),
-                           1.0 / r2);
-            else
-                v = cscale(cadd(cscale(pm1, (2.0 * n - 1) * uz), cscale(pm2, -r2)), recip(n * n - k * k));
+        for (int n = k + 1; n <= p; n++) {
+            cplx v = cscale(cadd(cscale(pm1, (2.0 * n - 1) * uz), cscale(pm2, -r2)), recip(n * n - k * k));
             X[tri(n, k)] = cscale(v, sgn_pow(n));
             pm2 = pm1;
             pm1 = v;
@@ -112,10 +92,8 @@ __global__ __launch_bounds__(256) void k_make_ops(const OpSpec* __restrict__ spe
         lm_of(i, l, m);
         lmt[i] = make_short2((short)l, (short)m);
     }
-    // scaling of the expansions: M2M (sig_c / sig_p)^l (output degree), L2L (sig_c / sig_p)^(a+1)
-    // and M2L (sig_s / sig_t)^a (input degree a)
-    for (int n = threadIdx.x; n <= p; n += blockDim.x)
-        fac[n] = kind == OPK_M2M ? pow(ratio, n) : kind == OPK_L2L ? pow(1.0 / ratio, n + 1) : pow(ratio, n);
+    // scaling of the expansions: M2M (sig_c / sig_p)^l (output degree), L2L (sig_c / sig_p)^(a+1) (input degree)
+    for (int n = threadIdx.x; n <= p; n += blockDim.x) fac[n] = kind == OPK_M2M ? pow(ratio, n) : pow(1.0 / ratio, n + 1);
     __syncthreads();
     const double c = 0.70710678118654752440;
     const size_t base = (size_t)opi * Lp * Lp;
@@ -142,8 +120,8 @@ __global__ __launch_bounds__(256) void k_make_ops(const OpSpec* __restrict__ spe
             const cplx v0 = br == 0 ? cplx{1, 0} : br > 0 ? cplx{c, 0} : cplx{0, c};
             const cplx v1 = br > 0 ? cplx{c, 0} : cplx{0, -c};
             auto out_c = [&](int m) {
-                cplx s = cmul(kernel_entry(kind, X, pI, l, m, a, b0), v0);
-                if (two) s = cadd(s, cmul(kernel_entry(kind, X, pI, l, m, a, b1), v1));
+                cplx s = cmul(kernel_entry(kind, X, l, m, a, b0), v0);
+                if (two) s = cadd(s, cmul(kernel_entry(kind, X, l, m, a, b1), v1));
                 return s;
             };
             if (mr == 0) val = out_c(0).re;
@@ -532,8 +510,8 @@ __global__ __launch_bounds__(256) void k_m2m_nodes(const int* __restrict__ paren
                 for (int a = 0; a <= l; a++)
                     for (int b = -a; b <= a; b++) {
                         const cplx in = Cc[a * a + a + b];
-                        op = cadd(op, cmul(kernel_entry(OPK_M2M, X, p, l, am, a, b), in));
-                        if (am) om = cadd(om, cmul(kernel_entry(OPK_M2M, X, p, l, -am, a, b), in));
+                        op = cadd(op, cmul(kernel_entry(OPK_M2M, X, l, am, a, b), in));
+                        if (am) om = cadd(om, cmul(kernel_entry(OPK_M2M, X, l, -am, a, b), in));
                     }
                 // complex -> real (harmonics.cpp:304-320)
                 const double v = m == 0 ? op.re : m > 0 ? c * (op.re + om.re) : c * (op.im - om.im);
@@ -569,15 +547,15 @@ void m2m_per_node(bool f64, const int* parents, int nparents, const TreeDev& S, 
 void make_operators(const OpSpec* d_specs, int nops, int p, int Lp, int out_mode, void* d_out, __bf16* d_out_lo,
                     hipStream_t st) {
     if (nops == 0) return;
-    int pI = 2 * p, L = (p + 1) * (p + 1);
-    size_t lds = (size_t)(pI + 1) * (pI + 2) / 2 * sizeof(cplx) + (size_t)((L + 1) & ~1) * sizeof(short2) +
+    int L = (p + 1) * (p + 1);
+    size_t lds = (size_t)(p + 1) * (p + 2) / 2 * sizeof(cplx) + (size_t)((L + 1) & ~1) * sizeof(short2) +
                  (size_t)(p + 1) * sizeof(double);
     // about 2048 workgroups in all, at least 8 rows each
     const int nsplit = std::max(1, std::min((Lp + 7) / 8, 2048 / nops));
     const int grid = nops * nsplit;
-    if (out_mode == 0) k_make_ops<0><<<grid, 256, lds, st>>>(d_specs, p, pI, Lp, d_out, nullptr, nsplit);
-    else if (out_mode == 1) k_make_ops<1><<<grid, 256, lds, st>>>(d_specs, p, pI, Lp, d_out, nullptr, nsplit);
-    else k_make_ops<2><<<grid, 256, lds, st>>>(d_specs, p, pI, Lp, d_out, d_out_lo, nsplit);
+    if (out_mode == 0) k_make_ops<0><<<grid, 256, lds, st>>>(d_specs, p, Lp, d_out, nullptr, nsplit);
+    else if (out_mode == 1) k_make_ops<1><<<grid, 256, lds, st>>>(d_specs, p, Lp, d_out, nullptr, nsplit);
+    else k_make_ops<2><<<grid, 256, lds, st>>>(d_specs, p, Lp, d_out, d_out_lo, nsplit);
     FMM_HIP(hipGetLastError());
 }
 

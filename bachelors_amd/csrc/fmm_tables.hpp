@@ -27,7 +27,7 @@ struct F16Split {
     int R = 0, Kp = 0;
 };
 
-// nops operators of Lp x Lp, row-major [out][in], zero padded, computed in FP64 and written as
+// nops M2M or L2L operators of Lp x Lp, row-major [out][in], zero padded, computed in FP64 and written as
 // out_mode 0: double (d_out), 1: float (d_out), 2: bf16 hi (d_out) + bf16 lo (d_out_lo) of the
 // float value.
 void make_operators(const OpSpec* d_specs, int nops, int p, int Lp, int out_mode, void* d_out, __bf16* d_out_lo,

@@ -616,3 +616,17 @@ def test_evaluation_replayed_from_a_graph(fm):
         torch.cuda.synchronize()
         assert torch.equal(out, ref) and float(out.abs().max()) > 0
     F.close()
+
+
+@pytest.mark.parametrize("p", [1, 2, 7, 20])
+@pytest.mark.parametrize("full", [0, 1])
+def test_m2l_operator_tables(fm, orc, p, full):
+    """The M2L tables that the evaluations use, at orders of one and of many slices of rows, with
+    l + lambda <= p and <= 2 p, off and in the lattice planes (rows of zeros): 1e-10, as above."""
+    flags = orc.CORRECTED if full else orc.SECTORAL_FIX | orc.FACT_FIX
+    deg = np.array([int(np.sqrt(i)) for i in range((p + 1) ** 2)])
+    for t in ([3.5, -1.5, 2.5], [4.0, 0.0, -2.0], [0.0, 0.0, 5.0]):
+        si, so = 0.5, 1.0
+        G = fm.make_operator(1, p, np.array(t), si, so, full)
+        E = orc.operator(1, p, np.array(t), flags) * (so ** (deg[:, None] + 1.0)) * (si ** deg[None, :])
+        assert np.abs(G - E).max() <= 1e-10 * np.abs(E).max()
