@@ -630,3 +630,31 @@ def test_m2l_operator_tables(fm, orc, p, full):
         G = fm.make_operator(1, p, np.array(t), si, so, full)
         E = orc.operator(1, p, np.array(t), flags) * (so ** (deg[:, None] + 1.0)) * (si ** deg[None, :])
         assert np.abs(G - E).max() <= 1e-10 * np.abs(E).max()
+
+
+@pytest.mark.parametrize("p", [8, 13, 14, 16])
+def test_f16x3_groups_with_wide_keys(fm, orc, p):
+    """A tight cluster whose boxes of levels 11 and 12 are far pairs of target leaves of level 4 (its place and
+    the boxes that hold it lie just outside twice the radius of the leaf at (0.1875, 0.1875, 0.1875)): offsets beyond
+    the compact class code, so all pairs and groups are keyed by the wide codes.  The far field of all targets and
+    of that leaf's against FP64 on the same trees: 1e-6, as above."""
+    rng = np.random.default_rng(99)
+    n, m = 30000, 2000
+    box = np.array([-0.37792969, -0.07910156, -0.00292969])
+    src = np.concatenate([rng.uniform(-2.9, 2.9, (n, 3)), box + rng.uniform(-2, 2, (m, 3)) * 3 / 1024])
+    tgt = rng.uniform(-2.9, 2.9, (n, 3))
+    tgt[:20] = 0.1875 + 0.18 * rng.uniform(-1, 1, (20, 3))
+    S, T = orc.source_tree(src, 32), orc.target_tree(tgt, 32, root=SHARED_ROOT)
+    ft, fs = orc.interaction_lists(S, T)[0]
+    unit = 3.0 / 2.0 ** np.maximum(S.level[fs], T.level[ft])
+    wide = (np.abs(S.center[fs] - T.center[ft]).max(axis=1) / unit > 127.5)
+    families = len(np.unique(np.column_stack([ft, S.parent[fs]])[wide], axis=0))
+    assert families > 20 and wide.sum() > 2 * families   # groups of several wide pairs
+    w = np.full(n + m, 1.0 / n)
+    exact, st = _far_part(fm, "fp64", p, src, w, tgt)
+    far, _ = _far_part(fm, "f16x3", p, src, w, tgt)
+    assert st["far_pairs"] == len(ft) and st["far_pairs"] >= 300 * st["m2l_classes"]
+    assert rel_l2(far, exact) < 1e-6
+    hit = np.unique(ft[wide])
+    sel = np.concatenate([np.arange(T.begin[t], T.end[t]) for t in hit if T.first_child[t] < 0])
+    assert len(sel) > 10 and rel_l2(far[sel], exact[sel]) < 1e-6
