@@ -658,3 +658,21 @@ def test_f16x3_groups_with_wide_keys(fm, orc, p):
     hit = np.unique(ft[wide])
     sel = np.concatenate([np.arange(T.begin[t], T.end[t]) for t in hit if T.first_child[t] < 0])
     assert len(sel) > 10 and rel_l2(far[sel], exact[sel]) < 1e-6
+
+
+@pytest.mark.parametrize("ns,nt,cap_t", [(1024, 60, 64), (1025, 60, 64), (16385, 33, 16), (20000, 129, 200)])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 1e-6)])
+def test_near_field_at_the_limits_of_parts(fm, orc, ns, nt, cap_t, precision, tol):
+    """The largest problem without parts and the smallest with them, and lists longer than 32 parts of 512
+    sources (few leaves): near field against the oracle."""
+    rng = np.random.default_rng(ns + nt)
+    src = shell_sources(rng, ns)
+    w = rng.uniform(0.5, 1.5, ns) / ns
+    tgt = shell_sources(rng, nt)
+    R = _oracle_run(orc, src, w, tgt, 3, ns + 2, cap_t)
+    F = fm.FMM(order=3, source_leaf_capacity=ns + 2, target_leaf_capacity=cap_t, precision=precision, frame=1)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    F.run(1.0)
+    assert F.stats()["source_leaves"] == 1 and F.stats()["target_leaves"] < 20
+    assert rel_l2(F.B_parts()[1], R.Bnear) < tol
