@@ -138,6 +138,7 @@ def lib():
         L.fmm_treecode.argtypes = [_vp, ctypes.c_double, ctypes.c_size_t, _vp, _vp, _vp]
         L.fmm_treecode_dev.argtypes = [_vp, ctypes.c_double, ctypes.c_size_t, _vp, _vp, _vp]
         L.fmm_get_stats.argtypes = [_vp, ctypes.POINTER(Stats)]
+        L.fmm_m2l_blocks.argtypes = [_vp, ctypes.POINTER(ctypes.c_longlong)]
         L.fmm_tree_size.argtypes = [_vp, ctypes.c_int, _ip, _ip]
         L.fmm_tree_export.argtypes = [_vp, ctypes.c_int] + [_vp] * 8
         L.fmm_lists_size.argtypes = [_vp] + [ctypes.POINTER(ctypes.c_longlong)] * 3
@@ -311,6 +312,12 @@ class FMM:
         s = Stats()
         self._check(lib().fmm_get_stats(self.h, ctypes.byref(s)))
         return s.as_dict()
+
+    def m2l_blocks(self):
+        """Slab blocks of the M2L: far pairs, in f16x3 groups of them."""
+        n = ctypes.c_longlong()
+        self._check(lib().fmm_m2l_blocks(self.h, ctypes.byref(n)))
+        return n.value
 
     # ---- parity export
     def tree(self, which):

@@ -1695,6 +1695,14 @@ int fmm_lists_size(fmm_ctx* c, long long* nfar, long long* nclose, long long* nc
     });
 }
 
+int fmm_m2l_blocks(fmm_ctx* c, long long* blocks) {
+    return guard(c, [&] {
+        require(blocks != nullptr, FMM_ERR_ARG, "null count");
+        require(c->lists_ready, FMM_ERR_STATE, "lists are not built");
+        *blocks = c->cfg.frame != FMM_FRAME_SHARED ? 0 : c->prec == Precision::F16X3 ? c->groups.num : c->lists.num_far;
+    });
+}
+
 int fmm_lists_export(fmm_ctx* c, int* ft, int* fs, int* ct, int* cs) {
     return guard(c, [&] {
         require(c->lists_ready, FMM_ERR_STATE, "lists are not built");

@@ -120,6 +120,8 @@ def time_fmm(fm, torch, prec, d_src, d_w, d_tgt, p, cap, steps, warmup, subset, 
         F.synchronize()
         runs.append(F.stats())
     staged = {k: (min(r[k] for r in runs) if k.startswith("t_") else runs[-1][k]) for k in runs[-1]} if runs else {}
+    if runs:
+        staged["m2l_blocks"] = F.m2l_blocks()
     F.close()
     return ms, st, staged, err, finite
 
@@ -144,9 +146,8 @@ def m2l_roofline(st, L, prec, traffic):
 def other_stage_rooflines(st, L, n_src, n_tgt, prec):
     """Achieved rates of the other stages from the stage-by-stage (no overlap) event times, with the
     algorithmic units of each: P2M and L2P bytes (positions, strengths, FP32 coefficients, FP64 B),
-    P2P pair interactions at 20 flop, the M2L slab reduction's bytes (one slab block per far pair
-    read, the local expansions read and written; F16X3 stores one block per group of far pairs, whose
-    number the statistics do not hold: no bytes there)."""
+    P2P pair interactions at 20 flop, the M2L slab reduction's bytes (one slab block per far pair, in
+    F16X3 per group of them, read, the local expansions read and written)."""
     Lp = (L + 63) // 64 * 64
     b_coef = 4 if prec != "fp64" else 8
     rows = {}
@@ -162,14 +163,12 @@ def other_stage_rooflines(st, L, n_src, n_tgt, prec):
                    "peak_TFs": PEAK_TFLOPS["fp32"]}
     red_ms = st["t_m2l"] - st["t_m2l_gemm"]
     R = Lp if prec == "bf16x3" else min(Lp, (L + 15) // 16 * 16)
-    red_bytes = st["far_pairs"] * 3 * R * b_coef + 2 * st["target_nodes"] * 3 * Lp * b_coef
-    if prec == "f16x3":
-        red_bytes = None
+    red_bytes = st["m2l_blocks"] * 3 * R * b_coef + 2 * st["target_nodes"] * 3 * Lp * b_coef
     rows["m2l_reduction"] = {"ms": red_ms, "bytes": red_bytes, "bound": "hbm",
-                             "achieved_GBs": red_bytes / (red_ms * 1e-3) / 1e9 if red_bytes and red_ms > 0 else None}
+                             "achieved_GBs": red_bytes / (red_ms * 1e-3) / 1e9 if red_ms > 0 else 0.0}
     for r in rows.values():
         if r["bound"] == "hbm":
-            r["frac"] = r["achieved_GBs"] / HBM_GBS if r["achieved_GBs"] is not None else None
+            r["frac"] = r["achieved_GBs"] / HBM_GBS
         else:
             r["frac"] = r["achieved_TFs_at_20_flop"] / r["peak_TFs"]
     return rows

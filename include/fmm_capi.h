@@ -194,6 +194,9 @@ int fmm_tree_size(fmm_ctx* ctx, int which, int* num_nodes, int* num_slots);
 int fmm_tree_export(fmm_ctx* ctx, int which, int* level, int* parent, int* first_child, int* begin, int* end,
                     int* npts, double* center, int* slots);
 int fmm_lists_size(fmm_ctx* ctx, long long* nfar, long long* nclose, long long* nclasses);
+/* slab blocks that the shared frame's M2L stores and reads back, 3 padded rows of coefficients each: one per far
+ * pair, in FMM_PREC_F16X3 one per group of them (0 in the reference frame) */
+int fmm_m2l_blocks(fmm_ctx* ctx, long long* blocks);
 int fmm_lists_export(fmm_ctx* ctx, int* far_t, int* far_s, int* close_t, int* close_s);
 /* far / near field of the last evaluation, target-leaf order, scaled to tesla */
 int fmm_export_B_parts(fmm_ctx* ctx, double* Bfar, double* Bnear);

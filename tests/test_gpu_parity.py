@@ -676,3 +676,23 @@ def test_near_field_at_the_limits_of_parts(fm, orc, ns, nt, cap_t, precision, to
     F.run(1.0)
     assert F.stats()["source_leaves"] == 1 and F.stats()["target_leaves"] < 20
     assert rel_l2(F.B_parts()[1], R.Bnear) < tol
+
+
+def test_m2l_blocks(fm):
+    """The slab blocks of the M2L: the far pairs, in F16X3 the (target, source parent) families where pairs are
+    grouped and the pairs where they are not; none in the reference frame."""
+    rng = np.random.default_rng(120)
+    for n, grouped in ((30000, True), (1500, False)):
+        src, tgt = rng.uniform(-2.9, 2.9, (n, 3)), rng.uniform(-2.9, 2.9, (n, 3))
+        for precision, frame in (("fp64", 1), ("f16x3", 1), ("fp64", 0)):
+            F = fm.FMM(order=8, source_leaf_capacity=32, target_leaf_capacity=32, precision=precision, frame=frame)
+            F.set_sources(src, np.full(n, 1.0 / n))
+            F.set_targets(tgt)
+            with pytest.raises(fm.FMMError):
+                F.m2l_blocks()
+            F.run(1.0)
+            (ft, fs), _, _ = F.lists()
+            families = len(np.unique(np.column_stack([ft, F.tree(0)["parent"][fs]]), axis=0))
+            expect = 0 if frame == 0 else families if precision == "f16x3" and grouped else len(ft)
+            assert F.m2l_blocks() == expect
+            F.close()
