@@ -777,11 +777,7 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
                                          const _Float16* __restrict__ bc, _Float16* __restrict__ an,
                                          _Float16* __restrict__ bn, float* __restrict__ sc) {
         if (LAST) rows(on);
-        aload(LAST ? 0 : kt + 1, an);
-        __builtin_amdgcn_sched_barrier(0);   // dma_barrier counts on the columns' loads being the last
         if (kt + 2 == NKS) columns(on, any);
-        bload(kt + 2 < NKS ? kt + 2 : kt + 2 - NKS, bn);
-        __builtin_amdgcn_sched_barrier(0);
         float sv[NS], cv = 0;   // the child's scales on their way to LDS
         if (!LAST && kt == 0) {
             const float* rv = this->A.ops_rinv + this->op(o) * R;
@@ -797,8 +793,11 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
             bh[c] = *(const half8*)(bc + (wc * 64 + 16 * c + li) * S + kk);
             bl[c] = *(const half8*)(bc + (W + wc * 64 + 16 * c + li) * S + kk);
         }
-        // row block by row block, each block's operator fragments read during the previous block's
-        // MFMAs (the scheduling barriers keep the reads from gathering at the start)
+        // row block by row block, each block's operator fragments read during the previous block's MFMAs; the loads
+        // for later steps after the first reads, the columns' after the first block's MFMAs; the three products of an
+        // accumulator back to back.  The scheduling barriers keep it so: with the loads first and the order of the
+        // products the compiler's, the GEMM took 13.7 instead of 12.7 ms (4M shells) and 18.1 instead of 16.7
+        // (moving clusters)
         half8 fh[2], fl[2];
 #pragma unroll
         for (int a = -1; a < NB0; a++) {
@@ -811,14 +810,22 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
                 fl[(a + 1) & 1] = *(const half8*)(ac + (R + row) * S + kk);
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (a < 0) continue;
+            if (a < 0) {
+                aload(LAST ? 0 : kt + 1, an);
+                __builtin_amdgcn_sched_barrier(0);   // dma_barrier counts on the columns' loads being the last
+                continue;
+            }
+            if (a == 1) {
+                bload(kt + 2 < NKS ? kt + 2 : kt + 2 - NKS, bn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[a & 1], bh[c], acc[a][c], 0, 0, 0);
                 acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bl[c], acc[a][c], 0, 0, 0);
                 acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bh[c], acc[a][c], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
         }
         if (!LAST && kt == 0) {   // last read at the end of the previous child, a barrier ago
 #pragma unroll
@@ -854,15 +861,16 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
 // two sets of accumulators instead, a child's and the group's: two buffers for the operator rows (shared by
 // the tiles of one class, mostly L2 hits), loaded one K step ahead, three for the multipole columns (gathered
 // from HBM), loaded two steps ahead, one barrier per K step, all across the boundary from one child to the
-// next.  Measured against one set of accumulators fed through registers: 4M shells, p = 16, 26.1 and 26.2 ms an
-// evaluation; GEMM of 1M points, p = 8, 12 and 13, 0.65 -> 0.58, 1.93 -> 1.86 and 6.9 -> 4.2 ms (then the
-// kernel above).  Far field of 999,983 x 750,019 clustered points, p = 14, against FP64: 3.8e-7 -> 3.4e-7, as
+// next.  Measured against one set of accumulators fed through registers: GEMM of the 4M shells, p = 16, 12.9 and
+// 12.7 ms, of the moving clusters, p = 14, 17.7 and 16.7; of 1M points, p = 8, 12 and 13, 1.04 -> 0.91, 1.97 -> 1.75
+// and 6.9 -> 4.2 ms (then the kernel above).  Far field of 999,983 x 750,019 clustered points, p = 14, against FP64: 3.8e-7 -> 3.4e-7, as
 // pair by pair; a second set in the kernel above leaves one workgroup per CU (p = 12: 3.3 ms).
 template <int NB, int NKS, bool SINGLE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_gemm_m2l_f16x3_q(M2LGroupArgs A,
                                                                                                 int* __restrict__ xq) {
     typedef M2LTileDma<NB, NKS, SINGLE> Tile;
     static_assert(NKS >= 3, "two steps ahead reach at most the next child; its scales have a step of their own");
+    static_assert(Tile::NB0 >= 2, "the columns are loaded behind the first of several row blocks");
     constexpr int R = Tile::R, W = Tile::W, S = Tile::S, RBUF = 2 * R * S, CBUF = 2 * W * S;
     // one variable: with several the compiler labels the accesses by variable, and then a read waits for
     // every load into LDS under way to its variable, that of the other buffers too
