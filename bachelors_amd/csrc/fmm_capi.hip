@@ -641,7 +641,7 @@ void stage_lists(fmm_ctx* c, hipStream_t ls, hipEvent_t far_ready, const std::fu
         if (after_far) after_far();
         if (shared && c->prec == Precision::F16X3)
             build_far_groups(c->groups, c->m2l_ix, c->lists, c->lscr.flag.as<uint32_t>(), c->lscr.pos.as<uint32_t>(),
-                             c->S, c->T, m2l_group_min_pairs(c->L), ls);
+                             c->S, c->T, m2l_group_min_pairs(c->L), m2l_group_tile(c->L), ls);
         else if (shared)
             build_pair_index(c->lists.far_t.as<int>(), c->lists.num_far, c->T.num_nodes, c->m2l_ix, ls);
     });

@@ -717,17 +717,17 @@ template <int LEFT> __device__ __forceinline__ void dma_barrier() {
 }
 
 // A workgroup's part of the persistent kernel below: the tile's columns and operators, and the loads into LDS.
-// A buffer of rows is [hi | lo][R][32 halves], one of columns [hi | lo][128][32].
-template <int NB, int NKS, bool SINGLE>
+// A buffer of rows is [hi | lo][R][32 halves], one of columns [hi | lo][W][32].  CB: 16-column blocks per wave.
+template <int NB, int NKS, bool SINGLE, int CB>
 struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
-    static constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK, W = 128;
+    static constexpr int R = 16 * NB, Kp = 32 * NKS, BK = 32, S = BK, W = 32 * CB;
     static constexpr int NQ = (4 * R + 255) / 256;   // 16-byte chunks per thread and part of the rows
     static constexpr int NB0 = (NB + 1) / 2, NS = (R + 255) / 256;
     const _Float16 *ah, *al;   // operator parts (uniform)
     const _Float16* b[2];
     int tid, wave, lane, rb0, wc, kk;
     unsigned aq, bq;   // lane's place in LDS row (tid >> 2) is slot tid & 3: the chunk that belongs there
-    f32x4 acc[NB0][4], sum[SINGLE ? 1 : NB0][4];
+    f32x4 acc[NB0][CB], sum[SINGLE ? 1 : NB0][CB];
     __device__ __forceinline__ M2LTileDma(const M2LGroupArgs& A_, const GroupTile& t, int tid_)
         : M2LTile<R, Kp, SINGLE>(A_, t, tid_), tid(tid_), wave(__builtin_amdgcn_readfirstlane(tid_ >> 6)),
           lane(tid_ & 63), rb0((wave & 1) * NB0), wc(wave >> 1), kk(8 * lds_chunk(lane >> 4, lane & 15)),
@@ -736,7 +736,7 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
 #pragma unroll
         for (int a = 0; a < NB0; a++)
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
+            for (int c = 0; c < CB; c++) {
                 acc[a][c] = f32x4{0, 0, 0, 0};
                 if (!SINGLE) sum[SINGLE ? 0 : a][c] = f32x4{0, 0, 0, 0};
             }
@@ -759,11 +759,15 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
             dma16(al + (size_t)64 * j * Kp + kt * BK + aq, buf + (R + 16 * wave + 64 * j) * S);
         }
     }
-    __device__ __forceinline__ void bload(int kt, _Float16* buf) const {   // BLOADS loads of every wave
+    // BLOADS loads of every wave (dma_barrier counts them): of 96 columns the last two waves load theirs twice
+    __device__ __forceinline__ void bload(int kt, _Float16* buf) const {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            dma16(b[c] + 2 * kt * BK, buf + (16 * wave + 64 * c) * S);
-            dma16(b[c] + 2 * kt * BK + 32, buf + (W + 16 * wave + 64 * c) * S);
+            const bool own = c == 0 || W == 128 || 16 * wave + 64 * c < W;   // uniform over the wave
+            const _Float16* p = (own ? b[c] : b[0]) + 2 * kt * BK;
+            const int row = 16 * wave + (own ? 64 * c : 0);
+            dma16(p, buf + row * S);
+            dma16(p + 32, buf + (W + row) * S);
         }
     }
     static constexpr int BLOADS = 4;
@@ -787,11 +791,11 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
             if (c < 2) cv = this->column_inv(c ? this->col[1] : this->col[0], c ? this->gm[1] : this->gm[0], o);
         }
         const int li = lane & 15, g = lane >> 4;
-        half8 bh[4], bl[4];
+        half8 bh[CB], bl[CB];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            bh[c] = *(const half8*)(bc + (wc * 64 + 16 * c + li) * S + kk);
-            bl[c] = *(const half8*)(bc + (W + wc * 64 + 16 * c + li) * S + kk);
+        for (int c = 0; c < CB; c++) {
+            bh[c] = *(const half8*)(bc + (16 * (wc * CB + c) + li) * S + kk);
+            bl[c] = *(const half8*)(bc + (W + 16 * (wc * CB + c) + li) * S + kk);
         }
         // row block by row block, each block's operator fragments read during the previous block's MFMAs; the loads
         // for later steps after the first reads, the columns' after the first block's MFMAs; the three products of an
@@ -820,7 +824,7 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
+            for (int c = 0; c < CB; c++) {
                 acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[a & 1], bh[c], acc[a][c], 0, 0, 0);
                 acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bl[c], acc[a][c], 0, 0, 0);
                 acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[a & 1], bh[c], acc[a][c], 0, 0, 0);
@@ -831,17 +835,18 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
 #pragma unroll
             for (int i = 0; i < NS; i++)
                 if (tid + 256 * i < R) sc[tid + 256 * i] = sv[i];
-            if ((tid & 3) < 2) sc[R + (tid >> 2) + 64 * (tid & 3)] = cv;
+            const int cl = (tid >> 2) + 64 * (tid & 3);
+            if ((tid & 3) < 2 && (W == 128 || cl < W)) sc[R + cl] = cv;
         }
         if (LAST) {
-            float ci[4];
+            float ci[CB];
 #pragma unroll
-            for (int c = 0; c < 4; c++) ci[c] = sc[R + wc * 64 + 16 * c + li];
+            for (int c = 0; c < CB; c++) ci[c] = sc[R + 16 * (wc * CB + c) + li];
 #pragma unroll
             for (int a = 0; a < NB0; a++) {
                 const f32x4 r = *(const f32x4*)(sc + min(rb0 + a, NB - 1) * 16 + 4 * g);
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
+                for (int c = 0; c < CB; c++) {
                     f32x4 x = acc[a][c];
 #pragma unroll
                     for (int e = 0; e < 4; e++)
@@ -855,7 +860,7 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
 };
 
 // The waves on a 2 x 2 grid: wave (wr, wc) owns the row blocks [wr NB0, wr NB0 + NB0) below NB
-// (NB0 = ceil(NB / 2)) and the tile columns [64 wc, 64 wc + 64), so it reads half the operator rows and
+// (NB0 = ceil(NB / 2)) and half the tile's columns (128, of groups above p = 16 96), so it reads half the operator rows and
 // half the columns from LDS per K step (a wave tile of 16 NB0 x 64 instead of 16 NB x 32: about a
 // third less LDS traffic per MFMA).  The operands go to LDS without passing registers (dma16), which hold
 // two sets of accumulators instead, a child's and the group's: two buffers for the operator rows (shared by
@@ -865,10 +870,10 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
 // 12.7 ms, of the moving clusters, p = 14, 17.7 and 16.7; of 1M points, p = 8, 12 and 13, 1.04 -> 0.91, 1.97 -> 1.75
 // and 6.9 -> 4.2 ms (then the kernel above).  Far field of 999,983 x 750,019 clustered points, p = 14, against FP64: 3.8e-7 -> 3.4e-7, as
 // pair by pair; a second set in the kernel above leaves one workgroup per CU (p = 12: 3.3 ms).
-template <int NB, int NKS, bool SINGLE>
+template <int NB, int NKS, bool SINGLE, int CB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_gemm_m2l_f16x3_q(M2LGroupArgs A,
                                                                                                 int* __restrict__ xq) {
-    typedef M2LTileDma<NB, NKS, SINGLE> Tile;
+    typedef M2LTileDma<NB, NKS, SINGLE, CB> Tile;
     static_assert(NKS >= 3, "two steps ahead reach at most the next child; its scales have a step of their own");
     static_assert(Tile::NB0 >= 2, "the columns are loaded behind the first of several row blocks");
     constexpr int R = Tile::R, W = Tile::W, S = Tile::S, RBUF = 2 * R * S, CBUF = 2 * W * S;
@@ -940,8 +945,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the loads ahead that nothing reads
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int cl = ld.wc * 64 + 16 * c + (ld.lane & 15);
+        for (int c = 0; c < CB; c++) {
+            const int cl = 16 * (ld.wc * CB + c) + (ld.lane & 15);
             if (cl >= 3 * ld.tile.ng) continue;
             float* out = ld.slab(cl) + 4 * (ld.lane >> 4);
 #pragma unroll
@@ -1020,7 +1025,8 @@ void split_columns(const float* M, int ncols, int L, int Lp, int Kp, const float
     FMM_HIP(hipGetLastError());
 }
 
-constexpr int M2L_GROUP_DMA_NB = 6, M2L_GROUP_MAX_NB = 19;   // groups: k_gemm_m2l_f16x3_q from p = 8, up to p = 16
+// groups: k_gemm_m2l_f16x3_q from p = 8 to 18, with 128 columns a tile to p = 16 (two sets of accumulators)
+constexpr int M2L_GROUP_DMA_NB = 6, M2L_GROUP_WIDE_NB = 19, M2L_GROUP_MAX_NB = 23;
 int m2l_f16_rows(int L) { return 16 * ((L + 15) / 16); }
 bool m2l_f16x3_persistent(int L) {
     const int nb = m2l_f16_rows(L) / 16;
@@ -1031,12 +1037,15 @@ bool m2l_f16x3_persistent(int L) {
 // and clusters of 30,000 to 1,000,000 points: p = 8, 261 pairs a class 2.09 / 2.01, 316 7.5 / 8.8, 441 3.36 / 3.50;
 // p = 12, 112 5.3 / 5.0, 261 2.74 / 2.63, 316 12.1 / 14.4; p = 14, 112 6.7 / 6.3, 261 3.31 / 3.23, 316 16.5 / 18.3;
 // p = 16, 112 9.1 / 8.5, 261 4.06 / 4.01, 316 22.7 / 24.3, 450 4.97 / 5.14.  In the kernel of the orders up to 7
-// (p = 5) 261 1.88 / 1.70, 441 3.1 / 2.9, 427 (8 million pairs) 10.1 / 10.0.  Above p = 16 two sets of
-// accumulators do not fit.
+// (p = 5) 261 1.88 / 1.70, 441 3.1 / 2.9, 427 (8 million pairs) 10.1 / 10.0.  Above p = 18 the LDS
+// buffers and two sets of accumulators do not fit.
 int m2l_group_min_pairs(int L) {
     const int nb = m2l_f16_rows(L) / 16;
     return nb > M2L_GROUP_MAX_NB ? INT32_MAX : nb >= M2L_GROUP_DMA_NB ? 300 : 1024;
 }
+// p = 17 and 18: two sets of accumulators of 96 columns fit beside a near-field workgroup, of 128 not at all (1M
+// shell points, p = 18: single pairs 21.6 ms, groups 19.2)
+int m2l_group_tile(int L) { return m2l_f16_rows(L) <= 16 * M2L_GROUP_WIDE_NB ? GROUP_TILE : 32; }
 int m2l_f16_kpad(int L) { return 32 * ((L + 31) / 32); }
 
 // The 2 x 2 kernel for groups (from three K steps on), and for single pairs where the other one's
@@ -1049,12 +1058,12 @@ static void launch_f16x3(const M2LGroupArgs& A, bool single, int* queues, hipStr
     const int grid = std::min(8 * ((A.ntiles + 7) / 8), (NB >= 14 ? 8 : 16) * ((num_cus() + 7) / 8));
     if constexpr (persistent)
         if (single) {
-            k_gemm_m2l_f16x3_q<NB, NKS, true><<<grid, 256, 0, st>>>(A, queues);
+            k_gemm_m2l_f16x3_q<NB, NKS, true, 4><<<grid, 256, 0, st>>>(A, queues);
             return;
         }
     if constexpr (dma_groups)
         if (!single) {
-            k_gemm_m2l_f16x3_q<NB, NKS, false><<<grid, 256, 0, st>>>(A, queues);
+            k_gemm_m2l_f16x3_q<NB, NKS, false, NB <= M2L_GROUP_WIDE_NB ? 4 : 3><<<grid, 256, 0, st>>>(A, queues);
             return;
         }
     if constexpr (!persistent)

@@ -74,6 +74,7 @@ int m2l_f16_rows(int L);
 // room for a near-field workgroup beside each
 bool m2l_f16x3_persistent(int L);
 int m2l_group_min_pairs(int L);   // far pairs per class from which the F16X3 M2L runs over groups
+int m2l_group_tile(int L);        // groups per tile
 int m2l_f16_kpad(int L);
 // skip_first_child / skip_npts (per node, both or neither): columns of leaves with points are
 // left as they are (the P2M writes them, see launch_p2m); column ncols is set to zeros

@@ -161,15 +161,16 @@ __global__ void k_group_place(const int* __restrict__ perm, const uint32_t* __re
 }
 // tiles per class (0 beyond the last class, so the scan's last entry is their number)
 __global__ void k_group_tile_counts(const int* __restrict__ cls_begin, const uint32_t* __restrict__ pos,
-                                    const uint32_t* __restrict__ flag, int ng, uint32_t* __restrict__ count) {
+                                    const uint32_t* __restrict__ flag, int ng, int tile,
+                                    uint32_t* __restrict__ count) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c > ng) return;
     const int nc = (int)(pos[ng - 1] + flag[ng - 1]);
-    count[c] = c < nc ? (uint32_t)(cls_begin[c + 1] - cls_begin[c] + GROUP_TILE - 1) / GROUP_TILE : 0u;
+    count[c] = c < nc ? (uint32_t)(cls_begin[c + 1] - cls_begin[c] + tile - 1) / tile : 0u;
 }
 __global__ void k_group_tiles(const int* __restrict__ mask, const uint32_t* __restrict__ pos,
                               const uint32_t* __restrict__ flag, const int* __restrict__ cls_begin,
-                              const uint32_t* __restrict__ toff, int ng, GroupTile* __restrict__ tiles,
+                              const uint32_t* __restrict__ toff, int ng, int tile, GroupTile* __restrict__ tiles,
                               unsigned* __restrict__ counts) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ng) return;
@@ -178,10 +179,10 @@ __global__ void k_group_tiles(const int* __restrict__ mask, const uint32_t* __re
         counts[1] = pos[ng - 1] + flag[ng - 1];
         counts[2] = toff[ng];
     }
-    if ((i - b) % GROUP_TILE) return;
-    GroupTile t{i, min(GROUP_TILE, e - i), c, 0};
+    if ((i - b) % tile) return;
+    GroupTile t{i, min(tile, e - i), c, 0};
     for (int j = 0; j < t.ng; j++) t.mask |= mask[i + j];
-    tiles[toff[c] + (i - b) / GROUP_TILE] = t;
+    tiles[toff[c] + (i - b) / tile] = t;
 }
 
 // every pair a group of its own (child 0 of its source), in class order as the pairs are
@@ -210,7 +211,7 @@ static HalfSizes half_sizes(const TreeDev& T) {
 }
 
 void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_t* class_flag,
-                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, hipStream_t st) {
+                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, int tile, hipStream_t st) {
     const int n = L.num_far;
     G.num = G.num_classes = G.num_tiles = 0;
     G.single = false;
@@ -224,9 +225,9 @@ void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_
         const int nc = L.num_classes;
         k_single_groups<<<blocks(n), 256, 0, st>>>(L.far_s.as<int>(), class_flag, class_pos, n, fc, mask, cb,
                                                    G.cls_mask.get<int>(nc), G.cls_ops.get<int>(8 * (size_t)nc));
-        k_group_tile_counts<<<blocks(n + 1), 256, 0, st>>>(cb, class_pos, class_flag, n, tcount);
+        k_group_tile_counts<<<blocks(n + 1), 256, 0, st>>>(cb, class_pos, class_flag, n, GROUP_TILE, tcount);
         exclusive_scan_u32(tcount, toff, n + 1, G.tmp, st);
-        k_group_tiles<<<blocks(n), 256, 0, st>>>(mask, class_pos, class_flag, cb, toff, n, G.tiles.get<GroupTile>(n),
+        k_group_tiles<<<blocks(n), 256, 0, st>>>(mask, class_pos, class_flag, cb, toff, n, GROUP_TILE, G.tiles.get<GroupTile>(n),
                                                  G.counts.get<unsigned>(4));
         build_pair_index(L.far_t.as<int>(), n, T.num_nodes, ix, st);
         FMM_HIP(hipGetLastError());
@@ -284,9 +285,9 @@ void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_
     k_group_place<<<blocks(ng), 256, 0, st>>>(perm2, flag2, pos2, ng, g_fc, g_mask, g_start, val, fs, class_flag, class_pos,
                                               fc, mask, order, cb, cm, ops);
     uint32_t *tcount = G.tcount.get<uint32_t>(ng + 1), *toff = G.toff.get<uint32_t>(ng + 1);
-    k_group_tile_counts<<<blocks(ng + 1), 256, 0, st>>>(cb, pos2, flag2, ng, tcount);
+    k_group_tile_counts<<<blocks(ng + 1), 256, 0, st>>>(cb, pos2, flag2, ng, tile, tcount);
     exclusive_scan_u32(tcount, toff, ng + 1, G.tmp, st);
-    k_group_tiles<<<blocks(ng), 256, 0, st>>>(mask, pos2, flag2, cb, toff, ng, G.tiles.get<GroupTile>(ng), counts);
+    k_group_tiles<<<blocks(ng), 256, 0, st>>>(mask, pos2, flag2, cb, toff, ng, tile, G.tiles.get<GroupTile>(ng), counts);
     // the groups of a target are consecutive in (target, parent) order
     index_sorted_pairs(g_t, ng, T.num_nodes, ix, st);
     FMM_HIP(hipGetLastError());

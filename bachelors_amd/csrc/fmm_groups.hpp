@@ -9,11 +9,11 @@ namespace fmm {
 // class (level difference and offset of the parent: equal class = equal operator for each child), then
 // by the mask of the children that are far pairs of t, then by target.
 struct GroupTile {
-    int g0, ng;   // groups [g0, g0 + ng), ng <= GROUP_TILE, of one class
+    int g0, ng;   // groups [g0, g0 + ng) of one class
     int cls;      // group class
     int mask;     // union of the groups' child masks
 };
-constexpr int GROUP_TILE = 42;   // groups per tile: 126 of the 128 columns
+constexpr int GROUP_TILE = 42;   // groups per tile at most (single pairs: always): 126 of 128 columns
 
 struct FarGroups {
     int num = 0, num_classes = 0, num_tiles = 0;
@@ -27,10 +27,10 @@ struct FarGroups {
 };
 
 // Groups of the far pairs L (sorted by class; class_flag / class_pos: the class starts and their
-// exclusive scan, so pair i has class class_pos[i] + class_flag[i] - 1), and the index of the groups by
-// target node for reduce_pairs.  The host waits for the counts.  With fewer than min_pairs far pairs per
+// exclusive scan, so pair i has class class_pos[i] + class_flag[i] - 1), up to `tile` groups a tile, and the index of
+// the groups by target node for reduce_pairs.  The host waits for the counts.  With fewer than min_pairs far pairs per
 // class every pair is a group of its own (no counts, no waits).
 void build_far_groups(FarGroups& G, PairIndex& ix, const Lists& L, const uint32_t* class_flag,
-                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, hipStream_t st);
+                      const uint32_t* class_pos, const TreeDev& S, const TreeDev& T, int min_pairs, int tile, hipStream_t st);
 
 }  // namespace fmm

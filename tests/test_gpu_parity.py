@@ -483,7 +483,7 @@ def _far_part(fm, precision, p, src, w, tgt, **kw):
     return far, st
 
 
-@pytest.mark.parametrize("p", [8, 12, 14, 16])
+@pytest.mark.parametrize("p", [8, 12, 14, 16, 17, 18])
 def test_f16x3_groups_beside_a_strong_leaf(fm, p):
     """One source leaf of 2^20 times the weight: where it is no far pair, its siblings' groups keep the
     accuracy of their own columns.  Targets whose far field of the strong leaf alone is exactly zero, against
@@ -504,7 +504,7 @@ def test_f16x3_groups_beside_a_strong_leaf(fm, p):
     assert rel_l2(far[sel], exact[sel]) < 1e-6
 
 
-@pytest.mark.parametrize("p", [1, 2, 4, 9, 12, 14, 16])
+@pytest.mark.parametrize("p", [1, 2, 4, 9, 12, 14, 16, 17, 18])
 def test_f16x3_groups_of_the_short_m2l(fm, p):
     """M2L with l + lambda <= p over groups: the operators of some children have rows of zeros (an offset in a
     lattice plane) where their siblings' have none.  Local expansions against FP64 on the same trees: 1e-6, as B
@@ -632,7 +632,7 @@ def test_m2l_operator_tables(fm, orc, p, full):
         assert np.abs(G - E).max() <= 1e-10 * np.abs(E).max()
 
 
-@pytest.mark.parametrize("p", [8, 13, 14, 16])
+@pytest.mark.parametrize("p", [8, 13, 14, 16, 18])
 def test_f16x3_groups_with_wide_keys(fm, orc, p):
     """A tight cluster whose boxes of levels 11 and 12 are far pairs of target leaves of level 4 (its place and
     the boxes that hold it lie just outside twice the radius of the leaf at (0.1875, 0.1875, 0.1875)): offsets beyond
