@@ -94,6 +94,8 @@ typedef struct fmm_stats {
     int order, padded_length, bfs_steps;
     /* stage times in ms (HIP events on the context stream) */
     double t_tree, t_p2m, t_m2m, t_lists, t_tables, t_m2l, t_l2l, t_l2p, t_p2p, t_total;
+                                         /* t_p2p of fmm_run_B_dev in FMM_PREC_F16X3 at p = 14..18: the grid
+                                            beside the M2L GEMM, without the items taken after the L2P */
     double t_m2l_gemm;                   /* the M2L translation GEMM alone (part of t_m2l) */
     int source_tree_sorted, target_tree_sorted;   /* 1: built by one sort of point paths;
                                                      0: level by level (gaps/overlaps of child boxes) */
