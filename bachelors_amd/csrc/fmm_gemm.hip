@@ -860,16 +860,17 @@ struct M2LTileDma : M2LTile<16 * NB, 32 * NKS, SINGLE> {
 };
 
 // The waves on a 2 x 2 grid: wave (wr, wc) owns the row blocks [wr NB0, wr NB0 + NB0) below NB
-// (NB0 = ceil(NB / 2)) and half the tile's columns (128, of groups above p = 16 96), so it reads half the operator rows and
-// half the columns from LDS per K step (a wave tile of 16 NB0 x 64 instead of 16 NB x 32: about a
-// third less LDS traffic per MFMA).  The operands go to LDS without passing registers (dma16), which hold
+// (NB0 = ceil(NB / 2)) and half the tile's columns (128, of groups above p = 16 96), so it reads half the
+// operator rows and half the columns from LDS per K step (a wave tile of 16 NB0 x 64 instead of 16 NB x 32:
+// about a third less LDS traffic per MFMA).  The operands go to LDS without passing registers (dma16), which hold
 // two sets of accumulators instead, a child's and the group's: two buffers for the operator rows (shared by
 // the tiles of one class, mostly L2 hits), loaded one K step ahead, three for the multipole columns (gathered
 // from HBM), loaded two steps ahead, one barrier per K step, all across the boundary from one child to the
 // next.  Measured against one set of accumulators fed through registers: GEMM of the 4M shells, p = 16, 12.9 and
 // 12.7 ms, of the moving clusters, p = 14, 17.7 and 16.7; of 1M points, p = 8, 12 and 13, 1.04 -> 0.91, 1.97 -> 1.75
-// and 6.9 -> 4.2 ms (then the kernel above).  Far field of 999,983 x 750,019 clustered points, p = 14, against FP64: 3.8e-7 -> 3.4e-7, as
-// pair by pair; a second set in the kernel above leaves one workgroup per CU (p = 12: 3.3 ms).
+// and 6.9 -> 4.2 ms (then the kernel above).  Far field of 999,983 x 750,019 clustered points, p = 14, against
+// FP64: 3.8e-7 -> 3.4e-7, as pair by pair; a second set in the kernel above leaves one workgroup per CU (p = 12:
+// 3.3 ms).
 template <int NB, int NKS, bool SINGLE, int CB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_gemm_m2l_f16x3_q(M2LGroupArgs A,
                                                                                                 int* __restrict__ xq) {
@@ -934,8 +935,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_num_vgpr(216))) void k_g
             const int on = more ? __builtin_ctz(m) : o;
             m &= m - 1;
             for (int kt = 0; kt + 1 < NKS; kt++) {
-                ld.template step<false>(kt, o, on, more, sh.rows + ab * RBUF, sh.columns + bb * CBUF, sh.rows + (ab ^ 1) * RBUF,
-                                        sh.columns + (bb == 0 ? 2 : bb - 1) * CBUF, sh.scales);
+                ld.template step<false>(kt, o, on, more, sh.rows + ab * RBUF, sh.columns + bb * CBUF,
+                                        sh.rows + (ab ^ 1) * RBUF, sh.columns + (bb == 0 ? 2 : bb - 1) * CBUF, sh.scales);
                 next();
             }
             ld.template step<true>(NKS - 1, o, on, more, sh.rows + ab * RBUF, sh.columns + bb * CBUF,
