@@ -1234,12 +1234,13 @@ static void add_parts(const NearWork& w, const TreeDev& T, double* near, hipStre
 // the items of a near field into scratch, and its grid
 template <bool UP>
 static NearWork start_near(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
-                           const int* close_end, const int* close_s, NearScratch& scratch, int& grid, hipStream_t st) {
+                           const int* close_end, const int* close_s, NearScratch& scratch, int& grid, hipStream_t st,
+                           bool prepared = false) {
     NearWork w{leaves, nleaves, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0};
     grid = nleaves;
     if (S.num_slots > NEAR_SPLIT_SOURCES) {
         w = near_work(leaves, nleaves, near_rows(T.num_slots), scratch);
-        make_items<UP>(w, T, S, close_begin, close_end, close_s, st);
+        if (!prepared) make_items<UP>(w, T, S, close_begin, close_end, close_s, st);
         w.extra_wgs = (int)std::min<long long>(8LL * num_cus(), (long long)NEAR_MAX_PARTS * nleaves);
         grid += w.extra_wgs;
     }
@@ -1250,10 +1251,11 @@ template <int KIND>
 static void p2p_launch(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S,
                        const int* close_begin, const int* close_end, const int* close_s, const void* P0,
                        const void* P1, const void* P2, const double* txyz, double* out, NearScratch& scratch,
-                       hipStream_t st) {
+                       hipStream_t st, bool prepared = false) {
     if (!nleaves) return;
     int grid;
-    const NearWork w = start_near<false>(leaves, nleaves, T, S, close_begin, close_end, close_s, scratch, grid, st);
+    const NearWork w =
+        start_near<false>(leaves, nleaves, T, S, close_begin, close_end, close_s, scratch, grid, st, prepared);
     if (f64)
         k_p2p<double, KIND><<<grid, 256, 0, st>>>(w, T.begin.as<int>(), T.end.as<int>(), close_begin, close_end, close_s,
                                                   S.center.as<double>(), S.begin.as<int>(), S.end.as<int>(),
@@ -1267,8 +1269,14 @@ static void p2p_launch(bool f64, const int* leaves, int nleaves, const TreeDev& 
 }
 void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                 const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                const double* txyz, double* Bnear, NearScratch& scratch, hipStream_t st) {
-    p2p_launch<NEAR_B>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Bnear, scratch, st);
+                const double* txyz, double* Bnear, NearScratch& scratch, hipStream_t st, bool prepared) {
+    p2p_launch<NEAR_B>(f64, leaves, nleaves, T, S, close_begin, close_end, close_s, P0, P1, P2, txyz, Bnear, scratch, st,
+                       prepared);
+}
+void prepare_p2p(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                 const int* close_end, const int* close_s, NearScratch& scratch, hipStream_t st) {
+    int grid;
+    if (nleaves) start_near<false>(leaves, nleaves, T, S, close_begin, close_end, close_s, scratch, grid, st);
 }
 void launch_p2p_bem(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                     const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,

@@ -30,9 +30,12 @@ void launch_pack_sources(bool f64, int n, const double* origin, const double* sx
 struct NearScratch {
     DevBuf desc, extra, counters, partial;
 };
+// prepare_p2p makes the items ahead (needs the lists only); launch_p2p with `prepared` takes them
+void prepare_p2p(const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
+                 const int* close_end, const int* close_s, NearScratch& scratch, hipStream_t st);
 void launch_p2p(bool f64, const int* leaves, int nleaves, const TreeDev& T, const TreeDev& S, const int* close_begin,
                 const int* close_end, const int* close_s, const void* P0, const void* P1, const void* P2,
-                const double* txyz, double* Bnear, NearScratch& scratch, hipStream_t st);
+                const double* txyz, double* Bnear, NearScratch& scratch, hipStream_t st, bool prepared = false);
 // launch_p2p in FP32 in pieces: prepare makes the items (needs the lists only); then one or more
 // persistent grids of `grid` workgroups, on streams of their own, take them from one counter; finish, after
 // all of them, adds the parts up.  beside: with a small register budget that lets a workgroup share its CU
