@@ -453,7 +453,9 @@ __global__ void k_pack_sources(int n, const double* __restrict__ origin, const d
 // terms in R are added up in FP64, over the G lanes in a fixed order.  A run does not end at a node's border, so
 // in FP32 it is kept to 8 terms: at 64 the median error of a target among small leaves (100,000 x 400,000 clustered
 // points, 32 a leaf) was 1.27e-7, with runs within nodes 1.22e-7, now 1.20e-7 (999,983 x 750,019, 48 a leaf: 1.36e-7,
-// 1.39e-7, 1.22e-7), for 2 to 5 % of the near field's time (4M shells 5.68 -> 5.98 ms alone).
+// 1.39e-7, 1.22e-7).  Full runs are unrolled by 2, which pays for the additions in FP64: near field of the 4M shells
+// alone 5.9 ms with runs of 64, 6.2 with runs of 8, 5.9 unrolled; of 250,000 points 0.288, 0.314, 0.298.  By 4
+// and 8: 5.9 and 6.2, 0.299 and 0.304 (more than 64 registers or longer code).
 // KIND: B, the vector potential sum_j q_j / |x - y_j|, or the BEM potential (FP64), whose source has a
 // strength v = q and a number d (in the place of the low part of its x).
 // The batches may be shared by `parts` workgroups per leaf, each writing its own sums; out: the leaf's
@@ -557,10 +559,8 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
                 p2 = P2[j];
                 __syncthreads();
                 for (int q = valid ? g : nj; q < nj;) {
-                    const int qe = min(nj, q + RUN * G);
                     R f0 = 0, f1 = 0, f2 = 0;
-#pragma unroll 1
-                    for (; q < qe; q += G) {
+                    auto pair = [&](int q) {
                         const v4 yh = sh.s0[q];
                         const v4 yl = sh.s1[q];
                         const R qx = yh.w, qy = yl.w, qz = sh.s2[q];
@@ -586,6 +586,15 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
                             f1 = fma_t(fma_t(qz, dx, -qx * dz), ip, f1);
                             f2 = fma_t(fma_t(qx, dy, -qy * dx), ip, f2);
                         }
+                    };
+                    if (split && q + (RUN - 1) * G < nj) {
+#pragma unroll 2
+                        for (int k = 0; k < RUN; k++) pair(q + k * G);
+                        q += RUN * G;
+                    } else {
+                        const int qe = min(nj, q + RUN * G);
+#pragma unroll 1
+                        for (; q < qe; q += G) pair(q);
                     }
                     a0 += f0;
                     a1 += f1;
@@ -622,7 +631,7 @@ __device__ __forceinline__ void p2p_leaf(int leaf, int part, int parts, const in
 // ms in FP32, 2.7 ms in FP64; 32,768 x 4,096 points in 276 leaves, FP64: 470 us).  A list is therefore cut
 // into 2, 4, .. 32 parts of at most `batches` batches of 256 sources (near_batches; longer ones where 32 parts
 // are not enough), and the register budget is that of 7 (FP64: 5) waves a
-// SIMD (no unrolling), since the short lists are a matter of latency: 1M points 1007 (items alone: 1230) ->
+// SIMD (unrolled by 2 at most), since the short lists are a matter of latency: 1M points 1007 (items alone: 1230) ->
 // 660 us in FP32, 2.7 -> 2.0 ms in FP64, beside the slab reduction; 262,147 x 131,101 clustered points 1520
 // -> 330 us, transposed 1270 -> 420 us; B and A of 250,000 points 365 + 307 -> 267 + 237 us; 276 leaves 90
 // -> 75 us.
@@ -798,8 +807,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
                                          P2, sxyz, out, parent);
 }
 
-// The near field by two persistent grids that take their items from the one counter: BESIDE with a small
-// register budget, one workgroup of which fits on a CU beside the F16X3 M2L GEMM's, so the
+// The near field by two persistent grids that take their items from the one counter: BESIDE, one workgroup
+// of which fits on a CU beside the F16X3 M2L GEMM's (at most 432 registers a lane, which leaves 80: 64 here), so the
 // near field runs on the VALU slots the GEMM leaves idle, and the plain one for the items left when the
 // GEMM is done.  A BESIDE workgroup that starts when the GEMM's tiles are all taken (their streams share a
 // hardware queue and run one after the other) leaves the items to the other form: one workgroup per CU
@@ -829,7 +838,7 @@ __device__ __forceinline__ void p2p_queue_body(const NearWork& w, const int* __r
                                                                      origin, sbegin, send, P0, P1, P2, txyz, Bnear);
 }
 template <class R, bool POT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(10))) void k_p2p_queue(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_p2p_queue(
     NearWork w, const int* __restrict__ gemm_queues, int gemm_tiles, const int* __restrict__ tbegin,
     const int* __restrict__ tend, const int* __restrict__ close_begin, const int* __restrict__ close_end,
     const int* __restrict__ close_s, const double* __restrict__ origin, const int* __restrict__ sbegin,
