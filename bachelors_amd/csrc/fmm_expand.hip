@@ -813,6 +813,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
 // GEMM is done.  A BESIDE workgroup that starts when the GEMM's tiles are all taken (their streams share a
 // hardware queue and run one after the other) leaves the items to the other form: one workgroup per CU
 // alone takes 25 ms for the 7 ms of near field of the 4M shells.
+// The plain form's workgroups beyond the number of items left leave at once: of 2,048 that raced for 288 items, some
+// CUs got three and others none (959,985 sources, 273 targets, p = 16: 0.9 to 1.25 ms, now 0.6).
 template <class R, bool POT, bool BESIDE>
 __device__ __forceinline__ void p2p_queue_body(const NearWork& w, const int* __restrict__ gemm_queues, int gemm_tiles,
                                                const int* __restrict__ tbegin, const int* __restrict__ tend,
@@ -833,6 +835,10 @@ __device__ __forceinline__ void p2p_queue_body(const NearWork& w, const int* __r
         }
         __syncthreads();
         if (tiles == 0) return;
+    } else {
+        const int left = w.nleaves + (w.desc ? w.counters[0] : 0) -
+                         __hip_atomic_load(w.counters + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((int)blockIdx.x >= left) return;   // the first workgroup stays until none are left
     }
     p2p_items<R, POT ? NEAR_A : NEAR_B, false, true>(w, tbegin, tend, close_begin, close_end, close_s,
                                                                      origin, sbegin, send, P0, P1, P2, txyz, Bnear);

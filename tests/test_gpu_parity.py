@@ -445,6 +445,27 @@ def test_fused_run_matches_staged_run(fm, precision, tol):
         assert rel_l2(out.cpu().numpy(), B_staged) < tol
 
 
+@pytest.mark.parametrize("ns,nt,cap", [(700, 1, 8), (1023, 130, 100), (9000, 1, 500), (60000, 273, 100), (100003, 40, 8),
+                                       (60000, 30000, 8)])
+def test_fused_near_field_takes_every_item(fm, ns, nt, cap):
+    """The fused near field at p = 14 (two grids on one counter) sums every item: from one item to more than the
+    grids' workgroups, its results are those of the stage-by-stage near field, bit for bit (parts of a leaf and
+    the order of their sums follow from the lists), in every call."""
+    import torch
+    src, w, tgt = _inputs(ns + nt, ns, nt)
+    F = fm.FMM(order=14, source_leaf_capacity=cap, target_leaf_capacity=cap, precision="f16x3", frame=1)
+    F.set_sources(src, w)
+    F.set_targets(tgt)
+    F.run(1.0)
+    near = F.B_parts()[1]
+    assert np.abs(near).max() > 0
+    out = torch.empty((nt, 3), dtype=torch.float64, device="cuda")
+    for _ in range(3):
+        F.run_B_dev(1.0, out.data_ptr())
+        F.synchronize()
+        assert np.array_equal(F.B_parts()[1], near)
+
+
 @pytest.mark.parametrize("nt", [1, 255, 257, 32767, 32768, 70001])
 def test_target_extent_on_device_equals_host(fm, nt):
     """The target tree of the reference frame (root = the targets' bounding box) is the same from a host
